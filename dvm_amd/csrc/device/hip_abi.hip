@@ -18,6 +18,8 @@ extern "C" __global__ void dvm_vm_vec_rx_parts(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_ry_parts(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_sw(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_sw_parts(const VmParam p);
+#define DVM_ROW_DECL(slabs) extern "C" __global__ void dvm_vm_vec_row##slabs(const VmParam p);
+DVM_ROW_DECL(1) DVM_ROW_DECL(2) DVM_ROW_DECL(3) DVM_ROW_DECL(4) DVM_ROW_DECL(5) DVM_ROW_DECL(6) DVM_ROW_DECL(8)
 extern "C" __global__ void dvm_vm_vec_pw_u4(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_u4(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_ry_u4(const VmParam p);
@@ -66,6 +68,11 @@ static const CubeKernel kCubeCombKernels[4][2] = {{dvm_vm_cube_f16_big_comb, dvm
                                                   {dvm_vm_cube_f16_small_comb, dvm_vm_cube_bf16_small_comb},
                                                   {dvm_vm_cube_f16_big8_comb, dvm_vm_cube_bf16_big8_comb}};
 
+// [slabs a lane]: the row build of the vector VM
+typedef void (*VecKernel)(const VmParam);
+static const VecKernel kRowKernels[9] = {nullptr, dvm_vm_vec_row1, dvm_vm_vec_row2, dvm_vm_vec_row3, dvm_vm_vec_row4,
+                                         dvm_vm_vec_row5, dvm_vm_vec_row6, nullptr, dvm_vm_vec_row8};
+
 // The workspace of dvm_hip_launch_vm_static_ws: device memory that belongs to the library's code object, one copy
 // per device. Host code never uses this name as an address: it asks the runtime for the array's address on the
 // current device (hipGetSymbolAddress) and passes that.
@@ -113,6 +120,12 @@ __global__ void dvm_fill_u32_kernel(uint32_t *dst, uint32_t value, size_t n) {
 // registers). The grid is a multiple of what is resident: one workgroup too many per CU costs a whole extra pass.
 uint32_t kernel_waves_per_simd(uint64_t kind) {
   if (kind & VS_WIDE) return 2;
+  switch (DVM_VEC_ROW_SLABS(kind)) {  // (from the builds' register counts, as below)
+    case 0: break;
+    case 1: case 2: return 5;
+    case 3: case 4: return 4;
+    default: return 2;
+  }
   switch (kind & VS_KIND_MASK) {
     case VS_POINTWISE: return 5;
     case VS_REDX: return 4;
@@ -150,6 +163,8 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
                                        reinterpret_cast<const void *>(dvm_vm_vec_rx_sw), reinterpret_cast<const void *>(dvm_vm_vec_rx_sw_parts),
                                        reinterpret_cast<const void *>(dvm_vm_vec_pw_u4), reinterpret_cast<const void *>(dvm_vm_vec_rx_u4),
                                        reinterpret_cast<const void *>(dvm_vm_vec_ry_u4)};
+  for (VecKernel k : kRowKernels)
+    if (k != nullptr) kernels.push_back(reinterpret_cast<const void *>(k));
   for (const auto &tile : kCubeKernels)
     for (const auto &dt : tile)
       for (CubeKernel k : dt) kernels.push_back(reinterpret_cast<const void *>(k));
@@ -241,6 +256,69 @@ static bool sweeps_flag_holds(const VmParam &p) {
   return true;
 }
 
+// The row build reads its words without looking for anything else, accesses rows without guards and holds exactly
+// `slabs` slabs a lane: a blob that carries VS_ROW_* must have that shape.
+static bool row_words_hold(const VmParam &p, uint32_t threads) {
+  const VVecHeader *h = reinterpret_cast<const VVecHeader *>(p.w);
+  const uint32_t slabs = DVM_VEC_ROW_SLABS(h->sched), off = h->row_code & 0xffffu, n = h->row_code >> 16;
+  if (!DVM_VEC_ROW_OK(slabs) || threads > DVM_VEC_ROW_LANES(slabs) || n == 0 || n > DVM_VEC_ROW_WORDS || off + n > DVM_PARAM_WORDS ||
+      off < h->code_off + h->n_code || VI_OP(p.w[off + n - 1]) != VOP_END) return false;
+  const uint64_t team = h->team_is_block ? threads : 64u;
+  if (h->n_rdim != 1 || h->n_kdim > 2 || h->n_mem == 0 || h->n_mem > 64 || h->inner_extent < DVM_VEC_E || h->n_ridx != (h->inner_extent + DVM_VEC_E - 1) / DVM_VEC_E ||
+      h->n_ridx > slabs * team || h->n_ridx <= (slabs - 1) * team || (h->n_kdim == 2 && h->kdims[0].extent == 0)) return false;
+  if (h->team_is_block ? h->n_items > h->n_kidx : static_cast<uint64_t>(h->n_items) * (threads / 64u) >= static_cast<uint64_t>(h->n_kidx) + threads / 64u) return false;
+  const VMemDesc *mems = reinterpret_cast<const VMemDesc *>(p.w + h->mem_off);
+  auto mem_ok = [&](uint32_t a, bool row) {
+    if (a >= h->n_mem) return false;
+    const VMemDesc &m = mems[a];
+    if (m.dtype != VDT_F32 && m.dtype != VDT_F16 && m.dtype != VDT_BF16) return false;
+    if ((m.addr & (m.dtype == VDT_F32 ? 3u : 1u)) != 0) return false;
+    return (m.flags & (VMF_VEC | VMF_GATHER)) == (row ? static_cast<uint32_t>(VMF_VEC) : 0u);
+  };
+  bool in_sweep = false;
+  for (uint32_t i = off; i < off + n; ++i) {
+    const uint64_t w = p.w[i];
+    const uint32_t op = VI_OP(w), kind = VI_KIND(w), a = VI_A(w);
+    const bool ends = (static_cast<uint32_t>(w) & VI_ENDS) != 0;
+    if (op == VOP_END) {
+      if (in_sweep || i != off + n - 1) return false;
+      continue;
+    }
+    if (op == VOP_SWEEP) {
+      if (in_sweep) return false;
+      in_sweep = true;
+      continue;
+    }
+    if (ends && !in_sweep) return false;
+    switch (op) {
+      case VOP_LD: if (kind != VK_MEM || !mem_ok(a, in_sweep)) return false; break;
+      case VOP_ST: if (!mem_ok(a, in_sweep)) return false; break;
+      case VOP_BINF:
+        if (kind == VK_MEM && !mem_ok(a, in_sweep)) return false;
+        if (kind == VK_REG && (!in_sweep || slabs > 2 || a + 1 > h->n_vslot)) return false;
+        if (kind > VK_SREG2) return false;
+        break;
+      case VOP_CMP: case VOP_MSK: case VOP_MOVM:
+        if (in_sweep || kind == VK_REG || (kind == VK_MEM && !mem_ok(a, false))) return false;
+        break;
+      case VOP_LDR: case VOP_STR:
+        if (!in_sweep || slabs > 2 || a + ((VI_SUB(w) & 3u) == VF_F32 ? 2u : 1u) > h->n_vslot) return false;
+        break;
+      case VOP_RED: case VOP_SPLAT: if (!in_sweep) return false; break;
+      case VOP_FIN: case VOP_STS: if (in_sweep) return false; break;
+      case VOP_LDS: case VOP_LDI: case VOP_UN: case VOP_CAST: case VOP_ENDSWEEP: break;
+      default: return false;
+    }
+    if ((static_cast<uint32_t>(w) & VI_LD_PAIR) && op == VOP_LD) {
+      const uint64_t w1 = i + 1 < off + n ? p.w[i + 1] : 0;
+      if (!in_sweep || ends || VI_OP(w1) != VOP_BINF || VI_KIND(w1) != VK_MEM || VI_A(w1) >= h->n_mem || mems[VI_A(w1)].dtype != mems[a].dtype ||
+          mems[a].dtype == VDT_F32) return false;
+    }
+    if (ends) in_sweep = false;
+  }
+  return true;
+}
+
 // Checks one program blob against the launch it is to get and launches the interpreter kernel its entry type names.
 static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads, uint32_t lds_bytes, void *stream, bool check_only = false) {
   if (block_dim == 0 || threads == 0 || threads > 1024 || (threads & 63u) != 0) {
@@ -271,7 +349,9 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     if ((h->sched & VS_KIND_MASK) == VS_REDY && threads > 512) return static_cast<int>(hipErrorInvalidValue);
     // the sweep build trusts the flag: it is only defined for programs that reduce the innermost axis, two slabs a lane
     const bool sweeps = (h->sched & VS_SWEEPS) != 0;
-    if (sweeps && (wide || (h->sched & VS_KIND_MASK) != VS_REDX || !sweeps_flag_holds(p))) return static_cast<int>(hipErrorInvalidValue);
+    const uint32_t row = DVM_VEC_ROW_SLABS(h->sched);
+    if (row != 0 && (wide || h->r_chunk != 0 || (h->sched & VS_KIND_MASK) != VS_REDX || !row_words_hold(p, threads))) return static_cast<int>(hipErrorInvalidValue);
+    if (row == 0 && sweeps && (wide || (h->sched & VS_KIND_MASK) != VS_REDX || !sweeps_flag_holds(p))) return static_cast<int>(hipErrorInvalidValue);
     // a reduce shared between workgroups: its parts are the outermost kept axis and cover the reduced index space
     const bool parts = h->r_chunk != 0;
     if (parts) {
@@ -287,7 +367,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
       const uint64_t u = wide ? DVM_VEC_U_WIDE : 2;
       uint64_t need = static_cast<uint64_t>(DVM_VEC_RED_SCRATCH_DOUBLES(h->sched, threads)) * 8 + static_cast<uint64_t>(h->n_vslot) * u * 16 * threads;
       uint64_t parked = 0;
-      for (uint64_t i = h->code_off; i < code_end; ++i) {
+      for (uint64_t i = h->code_off; row == 0 && i < code_end; ++i) {
         if (VI_OP(p.w[i]) != VOP_LD) continue;
         if (static_cast<uint32_t>(p.w[i]) & (VI_LD_KEEP_WR | VI_LD_KEEP_RD)) {
           if (wide) return static_cast<int>(hipErrorInvalidValue);
@@ -306,7 +386,9 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
         hipLaunchKernelGGL(wide ? dvm_vm_vec_pw_u4 : dvm_vm_vec_pw, dim3(block_dim), dim3(threads), lds_bytes, s, p);
         break;
       case VS_REDX:
-        if (sweeps) {
+        if (row != 0) {
+          hipLaunchKernelGGL(kRowKernels[row], dim3(block_dim), dim3(threads), lds_bytes, s, p);
+        } else if (sweeps) {
           hipLaunchKernelGGL(parts ? dvm_vm_vec_rx_sw_parts : dvm_vm_vec_rx_sw, dim3(block_dim), dim3(threads), lds_bytes, s, p);
         } else {
           hipLaunchKernelGGL(parts ? dvm_vm_vec_rx_parts : (wide ? dvm_vm_vec_rx_u4 : dvm_vm_vec_rx), dim3(block_dim), dim3(threads), lds_bytes, s, p);

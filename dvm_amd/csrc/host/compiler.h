@@ -356,7 +356,7 @@ class Compiler {
   void OrderAndMerge();
   void ChooseSchedule();
   void EmitProgram();
-  void FinishProgram();
+  bool FinishProgram();  // false: the program was laid out for the row build and does not fit it
   void ReplicatePeeled();
 
   // tables of the passes: members, so that a kernel compiled again (dynamic shapes) allocates nothing
@@ -389,6 +389,11 @@ class Compiler {
   void PairLoads();
   void PlanRereads();
   bool FitsSweepBuild();
+  bool RowCandidate() const;
+  bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;
+  bool BuildRowCode();
+  bool row_allowed_ = true;             // (false: the program has turned out to be outside the row build's vocabulary)
+  std::vector<uint64_t> row_code_;
   bool mem_is_view_[DVM_VEC_MAXMEM] = {false};  // memory operand i is a strided view
   int last_mem_ = -1;         // memory operand of the last memory instruction emitted in this round, or -1
   int u_ = 2;                 // slabs per lane per instruction of the program being compiled

@@ -135,6 +135,7 @@ std::string &VKernel::DisAssemble() {
             os << "broadcast_s acc, " << buf;
             break;
           }
+          case VOP_SPLAT: os << "splat acc"; break;
           case VOP_STR: os << "mov v" << VI_A(w) << "." << kFmt[sub & 3] << ", acc"; break;
           case VOP_STS: os << "mov s" << VI_A(w) << ", acc"; break;
           case VOP_ST:
@@ -205,7 +206,9 @@ std::string &VKernel::DisAssemble() {
     const VVecHeader *h = reinterpret_cast<const VVecHeader *>(p.blob.w);
     if (h->entry == VE_VECTOR) {
       static const char *sched[] = {"pointwise", "reduce-x", "reduce-y"};
-      os << "entry vector sched=" << sched[h->sched & VS_KIND_MASK] << ((h->sched & VS_WIDE) ? " wide" : "") << ((h->sched & VS_SWEEPS) ? " sweeps" : "") << " blocks=" << p.grid << " threads=" << p.threads
+      os << "entry vector sched=" << sched[h->sched & VS_KIND_MASK] << ((h->sched & VS_WIDE) ? " wide" : "") << ((h->sched & VS_SWEEPS) ? " sweeps" : "");
+      if (DVM_VEC_ROW_SLABS(h->sched) != 0) os << " row=" << DVM_VEC_ROW_SLABS(h->sched);
+      os << " blocks=" << p.grid << " threads=" << p.threads
          << " lds=" << p.lds_bytes << " items=" << h->n_items << " kept=" << h->n_kidx << " red=" << h->n_ridx
          << " inner=" << h->inner_extent << " team=" << (h->team_is_block ? p.threads : (1u << h->team_log2))
          << " vslots=" << h->n_vslot;
@@ -228,6 +231,10 @@ std::string &VKernel::DisAssemble() {
         os << "]\n";
       }
       print_code(p.blob.w + h->code_off, h->n_code, [&](uint32_t m) { return mems[m].dtype; });
+      if (tuning_.debug && DVM_VEC_ROW_SLABS(h->sched) != 0) {  // the words the row build executes
+        os << "  row build:\n";
+        print_code(p.blob.w + (h->row_code & 0xffffu), h->row_code >> 16, [&](uint32_t m) { return mems[m].dtype; });
+      }
     } else if (h->entry == VE_CUBE) {
       const VCubeHeader *c = reinterpret_cast<const VCubeHeader *>(p.blob.w);
       static const int tile[] = {256, 128, 64, 256};

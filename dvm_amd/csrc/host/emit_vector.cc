@@ -670,7 +670,7 @@ void Compiler::EmitProgram() {
   for (int s = 0; s < n_sec_; ++s) EmitSection(s);
   Emit(VOP_END, 0, 0, 0, 0, 0);
 }
-void Compiler::FinishProgram() {
+bool Compiler::FinishProgram() {
   {
     uint32_t dts[DVM_VEC_MAXMEM];
     for (int i = 0; i < n_mem_; ++i) dts[i] = mems_[i].dtype;
@@ -683,24 +683,35 @@ void Compiler::FinishProgram() {
   if (k_->tuning_.vec_unirun != 0) MarkUniformRuns();
   if (k_->tuning_.vec_pair != 0) PairLoads();
   if (k_->tuning_.vec_sweeps != 0 && FitsSweepBuild()) hdr_.sched |= VS_SWEEPS;
+  row_code_.clear();
+  if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && !BuildRowCode()) return false;
   hdr_.n_mem = n_mem_;
   hdr_.n_code = static_cast<uint32_t>(code_.size());
   hdr_.mem_off = sizeof(VVecHeader) / 8;
   hdr_.code_off = hdr_.mem_off + n_mem_ * (sizeof(VMemDesc) / 8);
   hdr_.n_vslot = max_vslot_;
   if (hdr_.code_off + code_.size() > DVM_PARAM_WORDS) Fail("program larger than 4 KB");
+  if (!row_code_.empty()) {
+    const size_t at = hdr_.code_off + code_.size();
+    if (at + row_code_.size() > DVM_PARAM_WORDS) return false;
+    hdr_.row_code = static_cast<uint32_t>(at | (row_code_.size() << 16));
+  }
   std::memset(&prog_->blob, 0, sizeof(VmParam));
   std::memcpy(prog_->blob.w, &hdr_, sizeof(hdr_));
   std::memcpy(prog_->blob.w + hdr_.mem_off, mems_, sizeof(VMemDesc) * n_mem_);
   std::memcpy(prog_->blob.w + hdr_.code_off, code_.data(), 8 * code_.size());
+  std::memcpy(prog_->blob.w + (hdr_.row_code & 0xffffu), row_code_.data(), 8 * row_code_.size());
   prog_->lds_bytes = DVM_VEC_RED_SCRATCH_DOUBLES(hdr_.sched, prog_->threads) * 8 + static_cast<uint32_t>(max_vslot_) * u_ * 16 * prog_->threads;
+  const uint32_t lds_unparked = prog_->lds_bytes;
   PlanRereads();
+  if (!row_code_.empty()) prog_->lds_bytes = lds_unparked;  // (the row build parks nothing)
   uint64_t gt = (static_cast<uint64_t>(std::min<uint32_t>(hdr_.n_items, g_system.core_num * 4)) << 32) | prog_->threads;
   if (g_system.HasDevice()) {
     gt = g_system.Api().select_block_thread(hdr_.sched, hdr_.n_items, prog_->threads, prog_->lds_bytes);
   }
   prog_->grid = static_cast<uint32_t>(gt >> 32);
   if (prog_->grid == 0) prog_->grid = 1;
+  return true;
 }
 
 void Compiler::CompileArea(int a) {
@@ -747,6 +758,7 @@ void Compiler::CompileArea(int a) {
   }
   UnifyAxes();
   OrderAndMerge();
+  row_allowed_ = true;
   ChooseSchedule();
   // a stored value must span the index space it is stored from, or it would be written several times. (The axis
   // that numbers the parts of a shared reduce is the exception: a value stored inside the sweep over the reduced space
@@ -774,7 +786,17 @@ void Compiler::CompileArea(int a) {
     }
   }
   EmitProgram();
-  FinishProgram();
+  if (!FinishProgram()) {  // laid out for the row build, and outside its vocabulary after all: once more without it
+    row_allowed_ = false;
+    for (int i = 0; i < nn_; ++i) {
+      nodes_[i].mem_idx = nodes_[i].reg = -1;
+      nodes_[i].slot_ready = false;
+    }
+    prog_->patches.clear();
+    ChooseSchedule();
+    EmitProgram();
+    FinishProgram();
+  }
   if (n_peel_ > 0) ReplicatePeeled();
 }
 

@@ -337,6 +337,181 @@ bool Compiler::FitsSweepBuild() {
   return true;
 }
 
+// The row build's instruction words (vm_vector_row.hip), from the finished words of the program: per-output runs lose
+// their brackets (every wave computes them), loads lose what concerns rounds, and a sweep that begins with the very
+// words whose result the accumulator still holds from the sweep before begins behind them. False: a word outside the
+// build's vocabulary.
+bool Compiler::BuildRowCode() {
+  const uint32_t slabs = DVM_VEC_ROW_SLABS(hdr_.sched);
+  if (n_mem_ > 64) return false;
+  row_code_.clear();
+  auto float_type = [&](uint32_t a) { return mems_[a].dtype == VDT_F32 || mems_[a].dtype == VDT_F16 || mems_[a].dtype == VDT_BF16; };
+  auto row_mem = [&](uint32_t a) { return float_type(a) && (mems_[a].flags & (VMF_VEC | VMF_GATHER)) == VMF_VEC; };
+  auto one_mem = [&](uint32_t a) { return float_type(a) && (mems_[a].flags & (VMF_VEC | VMF_GATHER)) == 0; };
+  auto reads_sreg = [](uint64_t w, uint32_t written) {
+    uint32_t used = 0;
+    if (VI_OP(w) == VOP_LDS) used |= 1u << VI_A(w);
+    if (VI_OP(w) == VOP_BINF) {
+      if (VI_KIND(w) == VK_SREG || VI_KIND(w) == VK_SREG2) used |= 1u << VI_A(w);
+      if (VI_KIND(w) == VK_SREG2 || (VI_KIND(w) == VK_MEM && (VI_IMM(w) & VI_PRE_SREG))) used |= 1u << ((VI_IMM(w) >> 8) & 0xffu);
+    }
+    return (used & written) != 0;
+  };
+  // what the accumulator holds behind the last sweep: the words that computed it, if it started from a load
+  std::vector<uint64_t> &held = scratch_code_;
+  held.clear();
+  bool held_ok = false, x_changed = false;
+  uint32_t sregs_written = 0;  // since `held` was computed
+  const size_t n = code_.size();
+  for (size_t i = 0; i < n; ++i) {
+    const uint64_t w = code_[i];
+    const uint32_t op = VI_OP(w), kind = VI_KIND(w), sub = VI_SUB(w);
+    if (op != VOP_SWEEP) {
+      switch (op) {
+        case VOP_UNI_BEGIN: case VOP_UNI_END: case VOP_ENDSWEEP:
+          continue;
+        case VOP_END:
+          break;
+        case VOP_FIN:
+          if (sub & VRF_INT) return false;
+          break;
+        case VOP_LDS: case VOP_LDI:
+          break;
+        case VOP_STS:
+          sregs_written |= 1u << VI_A(w);
+          break;
+        case VOP_UN:
+          if (sub > VU_TRUNC) return false;
+          break;
+        case VOP_CAST:
+          if (sub != VC_RND) return false;
+          break;
+        case VOP_ST:
+          if (!one_mem(VI_A(w))) return false;
+          break;
+        case VOP_LD: case VOP_BINF: case VOP_CMP: case VOP_MSK: case VOP_MOVM:
+          if (kind == VK_REG || (kind == VK_MEM && !one_mem(VI_A(w)))) return false;
+          if (op == VOP_BINF && ((sub & 0x3fu) > VB_MAX || (kind == VK_MEM && (VI_IMM(w) & VI_PRE_SREG)))) return false;
+          if (op == VOP_BINF && kind == VK_SREG2 && (VI_IMM(w) & 0x3fu) > VB_MAX) return false;
+          if (op == VOP_CMP && (sub & VCMP_INT)) return false;
+          break;
+        default:
+          return false;
+      }
+      if (op != VOP_STS && op != VOP_ST && op != VOP_END && op != VOP_MSK) x_changed = true;
+      row_code_.push_back(w);
+      continue;
+    }
+    row_code_.push_back(w & ~(static_cast<uint64_t>(VSW_REVERSE) << 8));
+    // the body, as the row build executes it
+    size_t first = i + 1, last = first;
+    while (last < n && !(static_cast<uint32_t>(code_[last]) & VI_ENDS)) ++last;
+    if (last >= n) return false;
+    auto defines_acc = [](uint32_t o) { return o == VOP_LD || o == VOP_LDR || o == VOP_LDS || o == VOP_LDI; };
+    auto changes_acc = [](uint32_t o) { return o == VOP_LD || o == VOP_LDR || o == VOP_LDS || o == VOP_LDI || o == VOP_BINF || o == VOP_UN || o == VOP_CAST; };
+    auto plain = [&](uint64_t b) -> uint64_t {  // a word without what only the other builds look at
+      uint64_t m = static_cast<uint64_t>(VI_ENDS) | VI_SAME_OFFS | VI_OFFS_ASIDE;
+      if (VI_OP(b) == VOP_LD) return VI_MAKE(VOP_LD, 0, VK_MEM, 0, VI_A(b), 0);
+      if (VI_OP(b) == VOP_BINF && VI_KIND(b) == VK_MEM) return b & ~m;
+      return b & ~static_cast<uint64_t>(VI_ENDS);
+    };
+    for (uint64_t h : held) held_ok = held_ok && !reads_sreg(h, sregs_written);
+    size_t skip = 0;
+    uint64_t code_word = 0;
+    uint64_t rest = 0;  // what is left of a fused word whose first half is the last of `held`
+    if (held_ok && !held.empty()) {
+      while (skip < held.size() && first + skip <= last && plain(code_[first + skip]) == held[skip]) ++skip;
+      if (skip + 1 == held.size() && skip > 0 && first + skip <= last) {
+        const uint64_t b = plain(code_[first + skip]);
+        const uint32_t imm = VI_IMM(b);
+        if (VI_OP(b) == VOP_BINF && VI_KIND(b) == VK_SREG2 && VI_MAKE(VOP_BINF, VI_SUB(b), VK_SREG, VI_RND(b), VI_A(b), 0) == held[skip]) {
+          rest = VI_MAKE(VOP_BINF, imm & 0x3fu, VK_SREG, (imm >> 16) & 3u, (imm >> 8) & 0xffu, 0);
+        } else if (VI_OP(b) == VOP_BINF && VI_KIND(b) == VK_MEM && (imm & VI_PRE_SREG) &&
+                   VI_MAKE(VOP_BINF, imm & 0x3fu, VK_SREG, (imm >> 16) & 3u, (imm >> 8) & 0xffu, 0) == held[skip]) {
+          rest = b & 0xffffffffull;
+        }
+        if (rest != 0) ++skip;
+      }
+      skip = skip == held.size() ? skip : 0;
+      if (skip == 0) rest = 0;
+      if (first + skip > last && rest == 0) skip = 0;
+    }
+    if (rest != 0) {
+      --skip;
+      code_word = rest | (static_cast<uint32_t>(code_[first + skip]) & VI_ENDS);
+    }
+    if (skip == 0 && rest == 0) {
+      if (!defines_acc(VI_OP(code_[first]))) {
+        if (x_changed) {
+          row_code_.push_back(VI_MAKE(VOP_SPLAT, 0, 0, 0, 0, 0));
+          held_ok = false;
+        }
+      } else {
+        held.clear();
+        held_ok = true;
+      }
+    }
+    sregs_written = 0;
+    for (size_t j = first + skip; j <= last; ++j) {
+      const uint64_t b = (rest != 0 && j == first + skip) ? code_word : code_[j];
+      const uint32_t bop = VI_OP(b), bk = VI_KIND(b), bsub = VI_SUB(b);
+      if (static_cast<uint32_t>(b) & VI_UNIFORM) return false;
+      switch (bop) {
+        case VOP_LD:
+          if (bk != VK_MEM || !row_mem(VI_A(b))) return false;
+          break;
+        case VOP_LDR: case VOP_STR:
+          if (slabs > 2) return false;
+          break;
+        case VOP_LDS: case VOP_LDI: case VOP_ENDSWEEP:
+          break;
+        case VOP_BINF:
+          if ((bsub & 0x3fu) > VB_MAX) return false;
+          if (bk == VK_MEM) {
+            if (!row_mem(VI_A(b)) || ((VI_IMM(b) & VI_PRE_SREG) && (VI_IMM(b) & 0x3fu) > VB_MAX)) return false;
+          } else if (bk == VK_SREG2) {
+            if ((VI_IMM(b) & 0x3fu) > VB_MAX) return false;
+          } else if (bk == VK_REG) {
+            if (slabs > 2) return false;
+          } else if (bk != VK_IMM && bk != VK_SREG && bk != VK_ACC) {
+            return false;
+          }
+          break;
+        case VOP_RED:
+          if ((bsub & VRF_INT) || ((bsub & (VRF_SQUARE | VRF_PAIR)) && (bsub & 0xfu) != VR_SUM)) return false;
+          break;
+        case VOP_ST:
+          if (!row_mem(VI_A(b))) return false;
+          break;
+        case VOP_UN:
+          if (bsub != VU_EXP && bsub != VU_ABS) return false;
+          break;
+        case VOP_CAST:
+          if (bsub != VC_RND) return false;
+          break;
+        default:
+          return false;
+      }
+      uint64_t out = plain(b) | (static_cast<uint32_t>(b) & VI_ENDS);
+      if (bop == VOP_LD && j < last && VI_OP(code_[j + 1]) == VOP_BINF && VI_KIND(code_[j + 1]) == VK_MEM && !(VI_IMM(code_[j + 1]) & VI_PRE_SREG)) {
+        const VMemDesc &ma = mems_[VI_A(b)], &mb = mems_[VI_A(code_[j + 1])];
+        if (ma.dtype == mb.dtype && ma.dtype != VDT_F32 && row_mem(VI_A(code_[j + 1]))) out |= VI_LD_PAIR;
+      }
+      row_code_.push_back(out);
+      if (!changes_acc(bop)) continue;
+      if (defines_acc(bop)) {
+        held.clear();
+        held_ok = bop == VOP_LD;
+      }
+      if (bop == VOP_BINF && bk == VK_REG) held_ok = false;  // (V registers change hands)
+      held.push_back(plain(b));
+    }
+    x_changed = false;
+    i = last;
+  }
+  return row_code_.size() <= DVM_VEC_ROW_WORDS;
+}
+
 // A reduce with consumers reads its input twice: once for the statistics, once to apply them. What the
 // second sweep does not have to fetch again from HBM:
 //  * the first rounds of the first sweep stay in the workgroup's spare local memory (VI_LD_KEEP_WR/RD);

@@ -464,6 +464,49 @@ uint32_t Log2(uint32_t v) {
   return l;
 }
 
+// Whether a sub-kernel's operators are worth trying on the row build (vm_vector_row.hip): values that vary along the
+// reduced axis are floats from contiguous rows, combined by the arithmetic that build knows. BuildRowCode has the last
+// word; this only keeps code generation from laying a program out for a build that will refuse it.
+bool Compiler::RowCandidate() const {
+  if (!row_allowed_ || k_->tuning_.vec_sweeps == 0 || k_->tuning_.vec_row == 0 || k_->tuning_.vec_team >= 1) return false;
+  if (nr_ != 1 || nk_ > 2 || n_peel_ > 0 || hdr_.inner_extent < static_cast<uint32_t>(E)) return false;
+  auto is_float = [](DataType t) { return t == kFloat32 || t == kFloat16 || t == kBFloat16; };
+  for (int i = 0; i < nn_; ++i) {
+    const ANode &n = nodes_[i];
+    if (!is_float(n.dtype)) return false;
+    if (n.kind != AK_OP) continue;
+    switch (n.op->kind) {
+      case kObjUnary: case kObjBinary: case kObjBinaryS: case kObjCast: break;
+      default: return false;
+    }
+    if ((n.op->kind == kObjBinary || n.op->kind == kObjBinaryS) && (n.op->op == kPow || n.op->op == kLogicalAnd || n.op->op == kLogicalOr)) return false;
+  }
+  return true;
+}
+
+// Slabs and lanes per row. More slabs a lane mean fewer waves per row: less scalar work between the sweeps, fewer
+// decodes per element, and from one wave per row on no barrier; but the chip wants some 2^17 lanes (two waves per SIMD)
+// in flight before it gives any up. Only the last slab of a row may be ragged. Measured on MI355X (times of a call, us;
+// without the row build / 2 / 4 / 8 slabs): residual RMSNorm bf16 [8192,4096] 63 / 57 / 54 / 51, [8192,8192] 116 / 120 /
+// 93 / 92, softmax fp32 [8192,4096] 87 / 76 / 72 / 68, [4096,16384] 192 / 179 / 139 / 137, [2048,32001] 535 / - / 152 /
+// 164; 37 rows of 4096 take the kernel 10.8 -> 7.7 us.
+bool Compiler::ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const {
+  if (n_r <= 32) return false;  // (up to 256 elements: several rows share a wave on the other builds)
+  uint32_t best = 0, best_team = 0;
+  for (uint32_t u = 1; u <= 8; ++u) {
+    if (!DVM_VEC_ROW_OK(u) || (k_->tuning_.vec_row > 0 && u > static_cast<uint32_t>(k_->tuning_.vec_row))) continue;
+    const uint64_t t = ((n_r + u - 1) / u + 63) / 64 * 64;
+    if (t > DVM_VEC_ROW_LANES(u) || n_r <= t * (u - 1)) continue;
+    if (best != 0 && n_k * t < (1ull << 17)) break;  // (more slabs would leave lanes idle)
+    best = u;
+    best_team = static_cast<uint32_t>(t);
+  }
+  if (best == 0) return false;
+  *slabs = best;
+  *team = best_team;
+  return true;
+}
+
 void Compiler::ChooseSchedule() {
   std::memset(&hdr_, 0, sizeof(hdr_));
   hdr_.entry = VE_VECTOR;
@@ -572,6 +615,9 @@ void Compiler::ChooseSchedule() {
       }
       if (team > cap) team = cap;
     }
+    // The row build, when the operators are in its vocabulary: a lane holds up to eight slabs and the row is one round.
+    uint32_t row_slabs = 0;
+    if (parts == 0 && !wide && RowCandidate() && ChooseRow(n_k, n_r, &row_slabs, &team)) hdr_.sched |= row_slabs << VS_ROW_SHIFT;
     if (team > 64) {
       hdr_.team_is_block = 1;
       threads = team;

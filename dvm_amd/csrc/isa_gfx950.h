@@ -64,7 +64,19 @@ enum {
   // (dvm_vm_vec_rx_sw), which decodes a sweep's body once per sweep instead of once per instruction and round; the
   // generic kernel runs it as well and gives the same bits.
   VS_SWEEPS = 0x20,
+  // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.hip) may run the program from the words at
+  // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space is one axis of n_ridx
+  // groups, more than (slabs - 1) * team and at most slabs * team of them (team: the workgroup when team_is_block, else
+  // one wave), and holds at least eight elements. The words at code_off stay valid for the generic kernel at the same
+  // geometry, with the local memory the rounds they park need.
+  VS_ROW_SHIFT = 8,
+  VS_ROW_MASK = 0xf00,
 };
+#define DVM_VEC_ROW_SLABS(sched) (((sched) & VS_ROW_MASK) >> VS_ROW_SHIFT)
+#define DVM_VEC_ROW_WORDS 64  // instruction words of a row program at most (one per lane of a wave)
+// slabs a lane the row build exists for, and the lanes a workgroup of that build may have
+#define DVM_VEC_ROW_OK(slabs) ((slabs) >= 1u && (slabs) <= 8u && (slabs) != 7u)
+#define DVM_VEC_ROW_LANES(slabs) ((slabs) <= 4u ? 1024u : 512u)
 #define DVM_VEC_SWEEP_BODY 6
 // Local memory at the start of a vector program's segment, in doubles: what the lanes of a workgroup combine their
 // reduce partials through. One double per lane; eight (one per element of a lane's group) on the schedule that keeps
@@ -94,6 +106,7 @@ enum {
                      // first wave executes the run, the others jump to the end
   VOP_UNI_END = 14,  // end of the run: the first wave's S registers and accumulator value are handed to the
                      // other waves through local memory
+  VOP_SPLAT = 15,    // row build only, inside a sweep: every element of acc = the lane's value from between the sweeps
   VOP_SRC_BASE = 16,
   VOP_LD = 16,       // acc = mem[a]             (kind is always VK_MEM)
   VOP_BINF = 17,     // acc = acc (sub = VB_*) src, float class
@@ -250,7 +263,8 @@ typedef struct {
   // that axis is kidx / k_per_chunk, and the lane reduces the indices [c * r_chunk, min(n_ridx, (c + 1) * r_chunk)).
   uint32_t r_chunk;
   uint32_t k_per_chunk;
-  uint32_t pad[2];       // (keeps the axis tables 16-byte aligned: the interpreter reads them as 128-bit words)
+  uint32_t row_code;     // VS_ROW*: word offset of the row build's instruction words, their number << 16
+  uint32_t pad;          // (keeps the axis tables 16-byte aligned: the interpreter reads them as 128-bit words)
   VDim kdims[DVM_VEC_MAXR];
   VDim rdims[DVM_VEC_MAXR];
 } VVecHeader;            // 80 + 128 = 208 bytes

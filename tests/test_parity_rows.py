@@ -1,0 +1,81 @@
+"""GPU parity of the row build of the vector VM (dvm_vm_vec_row*): an output's whole reduced row lies in the registers of
+its team, one to eight slabs a lane. Row lengths sit at the edges of that layout (one element more or less than a whole
+number of slabs or lanes, the smallest and the longest rows, odd lengths whose rows start at every alignment), the row
+counts pick few and many slabs a lane. References are float64; tolerances are the 8-element fp32 sums' (2^-24 * 3 per
+sum, divided out) and the storage type's rounding."""
+import numpy as np
+import pytest
+
+from dvm_amd.tester import Tester
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"float32": 4e-6, "float16": 2e-3, "bfloat16": 1.6e-2}
+
+
+def _inputs(rows, cols, dtype, seed, scale=1.0):
+    x = np.random.default_rng(seed).standard_normal([rows, cols], dtype=np.float32) * np.float32(scale)
+    return Tester.convert_to_bf16(x) if dtype == "bfloat16" else x.astype(dtype)
+
+
+def _f64(a, dtype):
+    return (Tester.convert_from_bf16(a) if dtype == "bfloat16" else a).astype(np.float64)
+
+
+def _load(t, a, dtype):
+    op = t.load(a.shape, dtype)
+    t.input(op, a)
+    return op
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 264), (2, 257), (5, 511), (5, 513), (70, 1000), (300, 4095), (300, 4097), (2100, 4096), (2100, 4089), (2100, 4081),
+                                       (2100, 3073), (2100, 2569), (300, 12289), (9, 20001), (300, 32001), (4, 32768), (4, 32761)])
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+def test_softmax_rows(rows, cols, dtype):
+    x = _inputs(rows, cols, dtype, rows * 31 + cols, 2.0)
+    t = Tester("split")
+    v = _load(t, x, dtype)
+    v = t.cast(v, "float32") if dtype != "float32" else v
+    e = t.exp(t.sub(v, t.max(v, (1,), True)))
+    p = t.div(e, t.sum(e, (1,), True))
+    out = t.store(t.cast(p, dtype) if dtype != "float32" else p)
+    t.run()
+    assert " row=" in t.das(), t.das()
+    got, x64 = _f64(t.output(out), dtype), _f64(x, dtype)
+    want = np.exp(x64 - x64.max(1, keepdims=True))
+    want /= want.sum(1, keepdims=True)
+    # (values below 1 / 16384 of a softmax are subnormal or coarse in fp16)
+    assert np.allclose(got, want, rtol=EPS[dtype], atol=6e-8 if dtype == "float16" else 0)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4096), (37, 1003), (2100, 4096), (2100, 5120), (2100, 4091), (3, 16384), (6, 30000)])
+def test_residual_norm_rows_with_statistics_stored(rows, cols):
+    """Two 16-bit operands in one trip, a weight row, per-row outputs beside the row output."""
+    x, r = _inputs(rows, cols, "float16", 1), _inputs(rows, cols, "float16", 2)
+    w = np.random.default_rng(3).uniform(0.5, 1.5, [cols]).astype(np.float32)
+    t = Tester("split")
+    h = t.cast(t.add(_load(t, x, "float16"), _load(t, r, "float16")), "float32")
+    mean = t.mul(t.sum(h, (1,), True), 1.0 / cols)
+    c = t.sub(h, mean)
+    var = t.mul(t.sum(t.mul(c, c), (1,), True), 1.0 / cols)
+    outs = [t.store(t.mul(t.div(c, t.sqrt(t.add(var, 1e-5))), t.load(w))), t.store(mean), t.store(t.min(h, (1,), True))]
+    t.run()
+    assert " row=" in t.das(), t.das()
+    h64 = (x + r).astype(np.float64)
+    m64 = h64.mean(1, keepdims=True)
+    want = (h64 - m64) / np.sqrt(h64.var(1, keepdims=True) + 1e-5) * w
+    assert np.allclose(t.output(outs[0]), want, rtol=2e-5, atol=2e-6)
+    assert np.allclose(t.output(outs[1]), m64, rtol=1e-5, atol=1e-7)
+    assert np.array_equal(t.output(outs[2]), h64.min(1, keepdims=True).astype(np.float32))
+
+
+def test_nothing_is_written_past_a_ragged_row():
+    """Odd rows stored through strides into a wider buffer: what lies between them stays as it was."""
+    rows, cols, pitch = 65, 1021, 1024
+    x = _inputs(rows, cols, "float32", 5)
+    want = np.zeros([rows, pitch], np.float32)
+    want[:, :cols] = x - x.max(1, keepdims=True)
+    t = Tester("split")
+    v = t.load(x)
+    t.view_store_expect(t.sub(v, t.max(v, (1,), True)), (pitch, 1), want, 0)
+    assert t.run_check()
