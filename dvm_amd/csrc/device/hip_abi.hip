@@ -54,6 +54,12 @@ extern "C" __global__ void dvm_vm_attn_f16_d64(const VmParam p);
 extern "C" __global__ void dvm_vm_attn_bf16_d64(const VmParam p);
 extern "C" __global__ void dvm_vm_attn_f16_w8_d64(const VmParam p);
 extern "C" __global__ void dvm_vm_attn_bf16_w8_d64(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_keys_f16(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_keys_bf16(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_keys_f16_d64(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_keys_bf16_d64(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_merge_f16(const VmParam p);
+extern "C" __global__ void dvm_vm_attn_merge_bf16(const VmParam p);
 
 typedef void (*CubeKernel)(const VmParam);
 #define DVM_CUBE_ROW(prefix) {prefix##_nn, prefix##_nt, prefix##_tn, prefix##_tt}
@@ -173,7 +179,9 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
   for (const void *k : {reinterpret_cast<const void *>(dvm_vm_attn_f16), reinterpret_cast<const void *>(dvm_vm_attn_bf16),
                         reinterpret_cast<const void *>(dvm_vm_attn_f16_w8), reinterpret_cast<const void *>(dvm_vm_attn_bf16_w8),
                         reinterpret_cast<const void *>(dvm_vm_attn_f16_d64), reinterpret_cast<const void *>(dvm_vm_attn_bf16_d64),
-                        reinterpret_cast<const void *>(dvm_vm_attn_f16_w8_d64), reinterpret_cast<const void *>(dvm_vm_attn_bf16_w8_d64)})
+                        reinterpret_cast<const void *>(dvm_vm_attn_f16_w8_d64), reinterpret_cast<const void *>(dvm_vm_attn_bf16_w8_d64),
+                        reinterpret_cast<const void *>(dvm_vm_attn_keys_f16), reinterpret_cast<const void *>(dvm_vm_attn_keys_bf16),
+                        reinterpret_cast<const void *>(dvm_vm_attn_keys_f16_d64), reinterpret_cast<const void *>(dvm_vm_attn_keys_bf16_d64)})
     kernels.push_back(k);
   for (const void *k : kernels) {
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(g_dev.lds_per_cu)) ==
@@ -444,13 +452,26 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), lds_bytes, s, p);
   } else if (h->entry == VE_ATTN) {
     const VAttnHeader *a = reinterpret_cast<const VAttnHeader *>(p.w);
-    // the kernel has no guards of its own beyond the query tail: the header must fit it exactly
-    if (!DVM_ATTN_D_OK(a->d) || a->skv == 0 || !(a->scale > 0.0f) || a->sq == 0 || a->nb == 0 ||
-        a->q_blocks != (a->sq + DVM_ATTN_BQ - 1) / DVM_ATTN_BQ || static_cast<uint64_t>(a->nb) * a->q_blocks != block_dim || (threads != 256 && threads != 512) ||
-        lds_bytes < DVM_ATTN_LDS_BYTES_D(a->d) || a->q_addr == 0 || a->k_addr == 0 || a->v_addr == 0 || a->o_addr == 0 ||
+    // the kernels have no guards of their own beyond the query and key tails: the header must fit them exactly
+    const uint32_t bq = a->kv_parts != 0 ? DVM_ATTN_KEYS_BQ : DVM_ATTN_BQ;
+    if (!DVM_ATTN_D_OK(a->d) || a->skv == 0 || !(a->scale > 0.0f) || a->sq == 0 || a->nb == 0 || a->q_blocks != (a->sq - 1) / bq + 1 ||
+        a->q_addr == 0 || a->k_addr == 0 || a->v_addr == 0 || a->o_addr == 0 ||
         ((a->q_addr | a->k_addr | a->v_addr | a->o_addr) & 15u) != 0 || (a->dtype != VDT_F16 && a->dtype != VDT_BF16) ||
         a->nb_inner == 0 || a->nb % a->nb_inner != 0) {
       return static_cast<int>(hipErrorInvalidValue);
+    }
+    const uint64_t tiles = static_cast<uint64_t>(a->nb) * a->q_blocks;
+    if (a->kv_parts == 0) {
+      if (a->merge != 0 || tiles != block_dim || (threads != 256 && threads != 512) || lds_bytes < DVM_ATTN_LDS_BYTES_D(a->d)) return static_cast<int>(hipErrorInvalidValue);
+    } else {
+      const uint64_t blocks = (a->skv - 1) / DVM_ATTN_KEYS_BKV + 1;
+      const uint64_t merge_lanes = static_cast<uint64_t>(a->nb) * a->sq * (a->d / 4);
+      if (threads != 64u * DVM_ATTN_KEYS_WAVES || a->part_blocks == 0 || static_cast<uint64_t>(a->part_blocks) * a->kv_parts < blocks ||
+          static_cast<uint64_t>(a->part_blocks) * (a->kv_parts - 1) >= blocks || (a->kv_parts > 1 && (a->part_addr == 0 || (a->part_addr & 15u) != 0)) ||
+          (a->merge != 0 ? a->kv_parts == 1 || (merge_lanes + threads - 1) / threads != block_dim
+                         : tiles * a->kv_parts != block_dim || lds_bytes < DVM_ATTN_KEYS_LDS_BYTES_D(a->d))) {
+        return static_cast<int>(hipErrorInvalidValue);
+      }
     }
     for (int i = 0; i < 4; ++i) {  // rows of at least d elements, every stride on 16 bytes (the kernel has 128-bit accesses only)
       if (a->row_stride[i] < a->d || a->row_stride[i] >= (1u << 22) || ((a->row_stride[i] | a->outer_stride[i] | a->inner_stride[i]) & 7u) != 0) {
@@ -460,7 +481,12 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     // 256 lanes: four waves of 64 queries; 512 lanes: eight waves of 32 queries (same tile of 256 queries)
     const bool bf = a->dtype == VDT_BF16, narrow = a->d != DVM_ATTN_D;
     if (check_only) return 0;
-    if (threads == 512) {
+    if (a->merge != 0) {
+      hipLaunchKernelGGL(bf ? dvm_vm_attn_merge_bf16 : dvm_vm_attn_merge_f16, dim3(block_dim), dim3(threads), 0, s, p);
+    } else if (a->kv_parts != 0) {
+      hipLaunchKernelGGL(narrow ? (bf ? dvm_vm_attn_keys_bf16_d64 : dvm_vm_attn_keys_f16_d64) : (bf ? dvm_vm_attn_keys_bf16 : dvm_vm_attn_keys_f16),
+                         dim3(block_dim), dim3(threads), lds_bytes, s, p);
+    } else if (threads == 512) {
       hipLaunchKernelGGL(narrow ? (bf ? dvm_vm_attn_bf16_w8_d64 : dvm_vm_attn_f16_w8_d64) : (bf ? dvm_vm_attn_bf16_w8 : dvm_vm_attn_f16_w8),
                          dim3(block_dim), dim3(512), lds_bytes, s, p);
     } else {

@@ -32,6 +32,7 @@ namespace {
 
 typedef float vf16 __attribute__((ext_vector_type(16)));
 typedef float vf2 __attribute__((ext_vector_type(2)));
+typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
 typedef uint32_t vu2 __attribute__((ext_vector_type(2)));
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -351,7 +352,280 @@ __device__ __forceinline__ void vm_attn(const VmParam &p) {
   }
 }
 
+__device__ __forceinline__ uint32_t lds_offset(const uint16_t *ptr) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) uint16_t *)ptr));
+}
+
+// The transposing reads of one 16-key step for 64 or 128 values of d, as one block that ends with its own wait: behind
+// the builtin the compiler waits for every direct load in flight (it cannot tell their buffers apart), which would take
+// the next block's loads out of the loop's pipeline.
+template <int HT>
+__device__ __forceinline__ void read_tr(const uint32_t (&addr)[2][2], vu4 (&vf)[2 * HT]) {
+  vu2 r[2 * HT][2];
+  if constexpr (HT == 2) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %9 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %10\n\tds_read_b64_tr_b16 %3, %11 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %4, %8 offset:4096\n\tds_read_b64_tr_b16 %5, %9 offset:5120\n\t"
+        "ds_read_b64_tr_b16 %6, %10 offset:4096\n\tds_read_b64_tr_b16 %7, %11 offset:5120\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1]), "=&v"(r[2][0]), "=&v"(r[2][1]), "=&v"(r[3][0]), "=&v"(r[3][1])
+        : "v"(addr[0][0]), "v"(addr[0][1]), "v"(addr[1][0]), "v"(addr[1][1])
+        : "memory");
+  } else {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %5 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %6\n\tds_read_b64_tr_b16 %3, %7 offset:1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1])
+        : "v"(addr[0][0]), "v"(addr[0][1]), "v"(addr[1][0]), "v"(addr[1][1])
+        : "memory");
+  }
+#pragma unroll
+  for (int dt = 0; dt < 2 * HT; ++dt) vf[dt] = vu4{r[dt][0][0], r[dt][0][1], r[dt][1][0], r[dt][1][1]};
+}
+
+// Few queries: the waves of a workgroup share one tile of 32 queries and divide the keys (vm_attn divides the queries).
+// What bounds it: with one to 32 queries a pass is a read of K and V, and vm_attn spends its 256-query tile on them, one
+// block of 64 keys behind the other ([16,32] heads, 1 query, 1999 keys, D = 128 in bf16: 137 us for 524 MB); where the
+// products are larger but (head, tile) pairs are few, its 256-query workgroups leave most of the chip without work.
+// Here each of four waves walks 32-key blocks of its own (every fourth of the workgroup's part of the keys) through a
+// private piece of local memory, two blocks of K and V deep: no barrier in the loop, and 16 to 32 KB per wave in flight
+// (64 KB and more per compute unit, where the memory's latency asks for about 32). MFMA work is a tenth of the time of the
+// read at full bandwidth, so the padding of one query to 32 costs nothing. The waves' running maxima, sums and outputs
+// meet in local memory at the end (base-2 weights, fp32, wave 0 first: the same order on every run). With too few
+// (head, tile) pairs for the chip the keys are also divided between kv_parts workgroups, whose unscaled outputs, maxima
+// and sums go to part_addr in fp32 for dvm_vm_attn_merge. Measured, back to back: the shape above 145 -> 96 us (5.5 TB/s),
+// [1,4] heads, 1 query, 4096 keys 101 -> 14 us (16 parts), [1,4], 2000 x 2000 63 -> 29 us, [2,8], 500 x 1000, D = 64
+// 25 -> 11 us.
+template <bool IS_BF16, int D>
+__device__ __forceinline__ void vm_attn_keys(const VmParam &p) {
+  constexpr int HT = D / 64;
+  constexpr uint32_t kTile = DVM_ATTN_KEYS_BKV * ROW;  // elements of one half tile
+  constexpr uint32_t kBlock = 2 * HT * kTile;          // K block, V block
+  constexpr int kLoads = 2 * HT * 4;                   // direct loads of a block (8 keys of a half tile each)
+  constexpr uint32_t kOutRow = D + 4;                  // floats per query where the waves' outputs meet
+  extern __shared__ double lds_raw[];
+  const VAttnHeader *hp = reinterpret_cast<const VAttnHeader *>(p.w);
+  const uint32_t sq = hp->sq, skv = hp->skv, q_blocks = hp->q_blocks, parts = hp->kv_parts;
+  const uint32_t tid = threadIdx.x, wave = uni(tid >> 6), lane = tid & 63u;
+  const uint32_t lj = lane & 31u, lh = lane >> 5;
+  uint16_t *lds = reinterpret_cast<uint16_t *>(lds_raw) + wave * 2u * kBlock;
+  // Position (w % 8) * (grid / 8) + w / 8 of the (head, part, query tile) order, as in vm_attn: the query tiles of one
+  // part of a head's keys run on one XCD.
+  uint32_t pos = blockIdx.x;
+  if ((gridDim.x & 7u) == 0) pos = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t qb = pos % q_blocks, bp = pos / q_blocks, part = bp % parts, b = bp / parts;
+  const uint32_t b_out = b / hp->nb_inner, b_in = b % hp->nb_inner;
+  auto base_of = [&](uint64_t addr, int which) -> uint64_t {
+    return addr + (static_cast<uint64_t>(b_out) * hp->outer_stride[which] + static_cast<uint64_t>(b_in) * hp->inner_stride[which]) * 2;
+  };
+  const uint64_t q_base = base_of(hp->q_addr, 0), k_base = base_of(hp->k_addr, 1), v_base = base_of(hp->v_addr, 2), o_base = base_of(hp->o_addr, 3);
+  const uint32_t ldq = hp->row_stride[0], ldk = hp->row_stride[1], ldv = hp->row_stride[2], ldo = hp->row_stride[3];
+  const uint32_t q0 = qb * DVM_ATTN_KEYS_BQ;
+  const float c_log2 = hp->scale * 1.44269504088896340736f;
+
+  // lane (j, h): Q[q0 + j][16*kk + 8*h .. +7]; rows past the end repeat the last row (their results are never stored)
+  vu4 qf[D / 16];
+  {
+    const uint32_t row = q0 + lj < sq ? q0 + lj : sq - 1;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+      qf[kk] = *reinterpret_cast<const DVM_GLOBAL vu4 *>(q_base + (static_cast<uint64_t>(row) * ldq + 16 * kk + 8 * lh) * 2);
+  }
+
+  // One direct load moves 8 keys of a half tile (1 KB of local memory): lane l is key l / 8 of them, physical chunk l % 8.
+  // Keys past the end fetch the last key again; their scores are masked.
+  auto fetch = [&](uint32_t blk, uint32_t buf) {
+    const uint32_t key0 = blk * DVM_ATTN_KEYS_BKV, last_row = skv - 1u - key0;
+    const DVM_GLOBAL char *ksrc = reinterpret_cast<const DVM_GLOBAL char *>(k_base + static_cast<uint64_t>(key0) * ldk * 2);
+    const DVM_GLOBAL char *vsrc = reinterpret_cast<const DVM_GLOBAL char *>(v_base + static_cast<uint64_t>(key0) * ldv * 2);
+    uint16_t *dst = lds + buf * kBlock;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t row = 8u * i + (lane >> 3);
+      const uint32_t col = ((lane & 7u) ^ ((lane >> 3) ^ static_cast<uint32_t>(i))) << 4;  // bytes: the swizzle of tile_off
+      if (last_row < DVM_ATTN_KEYS_BKV - 1u) row = row > last_row ? last_row : row;
+#pragma unroll
+      for (int half = 0; half < HT; ++half) {
+        const uint32_t off = half * kTile + i * 8 * ROW;
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const DVM_GLOBAL void *>(ksrc + (row * ldk * 2u + half * 128u + col)), (__attribute__((address_space(3))) void *)(dst + off), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const DVM_GLOBAL void *>(vsrc + (row * ldv * 2u + half * 128u + col)), (__attribute__((address_space(3))) void *)(dst + HT * kTile + off), 16, 0, 0);
+      }
+    }
+  };
+
+  const uint32_t blocks = (skv + DVM_ATTN_KEYS_BKV - 1) / DVM_ATTN_KEYS_BKV;
+  const uint32_t first = part * hp->part_blocks;
+  const uint32_t last = first + hp->part_blocks < blocks ? first + hp->part_blocks : blocks;  // one past
+  vf16 o_acc[D / 32];
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt) o_acc[dt] = 0.0f;
+  float m_run = -1.0e30f, l_run = 0.0f;
+  const uint32_t k_x = (lh ^ ((lj ^ (lj >> 3)) & 7u)) << 3;
+  // (the transposing reads of V: see vm_attn)
+  const uint32_t tr_j = (lane & 15u) >> 2, tr_q = lane & 3u, tr_g = lane >> 4;
+  const uint32_t tr_key = 4u * (tr_g >> 1) + tr_j;
+  const uint32_t tr_chunk = 2u * (tr_g & 1u) + (tr_q >> 1);
+  const uint32_t tr_base = tr_key * ROW + 4u * (tr_q & 1u);
+  const uint32_t tr_x = (tr_chunk ^ tr_key) << 3;
+  uint32_t blk = first + wave, buf = 0;
+  if (blk < last) fetch(blk, 0);
+  if (blk + DVM_ATTN_KEYS_WAVES < last) fetch(blk + DVM_ATTN_KEYS_WAVES, 1);
+  for (; blk < last; blk += DVM_ATTN_KEYS_WAVES, buf ^= 1u) {
+    // this block has landed; the loads of the next one, the last kLoads issued, may still be in flight
+    if (blk + DVM_ATTN_KEYS_WAVES < last) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t *kbuf = lds + buf * kBlock, *vbuf = kbuf + HT * kTile;
+    vf16 s = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+      const vu4 kf = *reinterpret_cast<const vu4 *>(kbuf + (kk >> 2) * kTile + lj * ROW + (k_x ^ static_cast<uint32_t>(((kk & 3) * 2) << 3)));
+      s = mfma<IS_BF16>(kf, qf[kk], s);
+    }
+    if ((blk + 1u) * DVM_ATTN_KEYS_BKV > skv) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t key = blk * DVM_ATTN_KEYS_BKV + 8u * (r >> 2) + 4u * lh + (r & 3);
+        s[r] = key < skv ? s[r] : -__builtin_inff();
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx * c_log2);
+    const float alpha = exp2_neg(m_run - m_new);
+    m_run = m_new;
+    float sum = 0.0f;
+    vu4 pf[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = exp2_neg(s[r] * c_log2 - m_new);
+      sum += s[r];
+    }
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pf[st][e] = pack2<IS_BF16>(s[8 * st + 2 * e], s[8 * st + 2 * e + 1]);
+    l_run = l_run * alpha + sum;
+    if (!wave_all(alpha == 1.0f)) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) o_acc[dt] = o_acc[dt] * alpha;
+    }
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      vu4 vf[D / 32];
+      const uint32_t at = lds_offset(vbuf) + (st * 16 * ROW + tr_base) * 2;
+      uint32_t addr[2][2];  // [dt & 1][keys 16 * st + 8 * w ..]
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) addr[x][w] = at + ((tr_x ^ static_cast<uint32_t>(((4 * x) ^ (2 * st + w)) << 3)) << 1);
+      read_tr<HT>(addr, vf);
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) o_acc[dt] = mfma<IS_BF16>(vf[dt], pf[st], o_acc[dt]);
+    }
+    // every read of this buffer has returned before the loads that overwrite it are issued
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (blk + 2u * DVM_ATTN_KEYS_WAVES < last) fetch(blk + 2u * DVM_ATTN_KEYS_WAVES, buf);
+  }
+
+  // the waves meet: [wave][query][d] outputs relative to the common maximum, [wave][query] maxima and sums
+  float *out = reinterpret_cast<float *>(lds_raw);
+  float *ml = out + DVM_ATTN_KEYS_WAVES * DVM_ATTN_KEYS_BQ * kOutRow;
+  l_run += __shfl_xor(l_run, 32);
+  __syncthreads();  // (the last blocks have been read; no load is in flight)
+  if (lh == 0) {
+    ml[(wave * DVM_ATTN_KEYS_BQ + lj) * 2] = m_run;
+    ml[(wave * DVM_ATTN_KEYS_BQ + lj) * 2 + 1] = l_run;
+  }
+  __syncthreads();
+  float m_all = ml[lj * 2];
+#pragma unroll
+  for (int w = 1; w < DVM_ATTN_KEYS_WAVES; ++w) m_all = fmaxf(m_all, ml[(w * DVM_ATTN_KEYS_BQ + lj) * 2]);
+  const float own = exp2_neg(m_run - m_all);
+  const uint32_t rows = sq - q0 < DVM_ATTN_KEYS_BQ ? sq - q0 : DVM_ATTN_KEYS_BQ;
+  if (lj < rows) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float *dst = out + (wave * DVM_ATTN_KEYS_BQ + lj) * kOutRow + dt * 32 + 8 * g + 4 * lh;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e] = o_acc[dt][4 * g + e] * own;
+      }
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < rows * (D / 4); i += 64u * DVM_ATTN_KEYS_WAVES) {
+    const uint32_t q = i / (D / 4), d = (i % (D / 4)) * 4;
+    float m = ml[q * 2], l = 0.0f, v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 1; w < DVM_ATTN_KEYS_WAVES; ++w) m = fmaxf(m, ml[(w * DVM_ATTN_KEYS_BQ + q) * 2]);
+#pragma unroll
+    for (int w = 0; w < DVM_ATTN_KEYS_WAVES; ++w) {
+      const float *src = out + (w * DVM_ATTN_KEYS_BQ + q) * kOutRow + d;
+      l += ml[(w * DVM_ATTN_KEYS_BQ + q) * 2 + 1] * exp2_neg(ml[(w * DVM_ATTN_KEYS_BQ + q) * 2] - m);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += src[e];
+    }
+    if (parts > 1) {
+      const uint64_t at = (static_cast<uint64_t>(b) * parts + part) * sq + q0 + q;
+      *reinterpret_cast<DVM_GLOBAL vf4 *>(hp->part_addr + (at * D + d) * 4) = vf4{v[0], v[1], v[2], v[3]};
+      if (d == 0) *reinterpret_cast<DVM_GLOBAL vf2 *>(hp->part_addr + (static_cast<uint64_t>(hp->nb) * parts * sq * D + at * 2) * 4) = vf2{m, l};
+    } else {
+      const float inv = 1.0f / l;
+      const vu2 w = {pack2<IS_BF16>(v[0] * inv, v[1] * inv), pack2<IS_BF16>(v[2] * inv, v[3] * inv)};
+      *reinterpret_cast<DVM_GLOBAL vu2 *>(o_base + (static_cast<uint64_t>(q0 + q) * ldo + d) * 2) = w;
+    }
+  }
+}
+
+// Second launch of a division of the keys between workgroups: the parts' outputs meet as the waves' do, part 0 first. A
+// lane owns four consecutive d of one query; a few KB per (head, query), so what it costs is the launch.
+template <bool IS_BF16>
+__device__ __forceinline__ void vm_attn_merge(const VmParam &p) {
+  const VAttnHeader *hp = reinterpret_cast<const VAttnHeader *>(p.w);
+  const uint32_t D = hp->d, sq = hp->sq, parts = hp->kv_parts, per = D / 4;
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x, rows = static_cast<uint64_t>(hp->nb) * sq;
+  if (i >= rows * per) return;
+  const uint32_t d = static_cast<uint32_t>(i % per) * 4, q = static_cast<uint32_t>(i / per % sq), b = static_cast<uint32_t>(i / per / sq);
+  const DVM_GLOBAL vf4 *po = reinterpret_cast<const DVM_GLOBAL vf4 *>(hp->part_addr);
+  const DVM_GLOBAL vf2 *pm = reinterpret_cast<const DVM_GLOBAL vf2 *>(hp->part_addr + rows * parts * D * 4);
+  const uint64_t at = static_cast<uint64_t>(b) * parts * sq + q;
+  float m = -1.0e30f, l = 0.0f;
+#pragma unroll 8
+  for (uint32_t t = 0; t < parts; ++t) m = fmaxf(m, pm[at + static_cast<uint64_t>(t) * sq][0]);
+  vf4 v = 0.0f;
+#pragma unroll 8
+  for (uint32_t t = 0; t < parts; ++t) {
+    const uint64_t row = at + static_cast<uint64_t>(t) * sq;
+    const vf2 ml = pm[row];
+    const float w = exp2_neg(ml[0] - m);
+    const vf4 o = po[row * per + d / 4];
+    l += ml[1] * w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += o[e] * w;
+  }
+  const float inv = 1.0f / l;
+  const uint64_t o_base = hp->o_addr + (static_cast<uint64_t>(b / hp->nb_inner) * hp->outer_stride[3] + static_cast<uint64_t>(b % hp->nb_inner) * hp->inner_stride[3]) * 2;
+  const vu2 w = {pack2<IS_BF16>(v[0] * inv, v[1] * inv), pack2<IS_BF16>(v[2] * inv, v[3] * inv)};
+  *reinterpret_cast<DVM_GLOBAL vu2 *>(o_base + (static_cast<uint64_t>(q) * hp->row_stride[3] + d) * 2) = w;
+}
+
 }  // namespace
+
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_keys_f16(const VmParam p) { vm_attn_keys<false, 128>(p); }
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_keys_bf16(const VmParam p) { vm_attn_keys<true, 128>(p); }
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_keys_f16_d64(const VmParam p) { vm_attn_keys<false, 64>(p); }
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_keys_bf16_d64(const VmParam p) { vm_attn_keys<true, 64>(p); }
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_merge_f16(const VmParam p) { vm_attn_merge<false>(p); }
+extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_merge_bf16(const VmParam p) { vm_attn_merge<true>(p); }
 
 extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_f16(const VmParam p) { vm_attn<false, 2, 128>(p); }
 extern "C" __global__ void __launch_bounds__(256) dvm_vm_attn_bf16(const VmParam p) { vm_attn<true, 2, 128>(p); }

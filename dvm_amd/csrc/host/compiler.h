@@ -351,6 +351,7 @@ class Compiler {
   void CompileCube(int a);
   uint32_t FuseCubeEpilogue();
   void CompileAttn(int g);
+  void DivideKeys();
   void BuildNodes(int a);
   void UnifyAxes();
   void OrderAndMerge();

@@ -267,7 +267,9 @@ std::string &VKernel::DisAssemble() {
     } else if (h->entry == VE_ATTN) {
       const VAttnHeader *a = reinterpret_cast<const VAttnHeader *>(p.blob.w);
       os << "entry attention " << kMemTypes[a->dtype] << " batch=" << a->nb << " sq=" << a->sq << " skv=" << a->skv << " d=" << a->d
-         << " scale=" << a->scale << " blocks=" << p.grid << " lds=" << p.lds_bytes << "\n";
+         << " scale=" << a->scale << " blocks=" << p.grid << " lds=" << p.lds_bytes;
+      if (a->kv_parts != 0) os << " waves divide the keys, parts=" << a->kv_parts << (a->merge != 0 ? " merge" : "");
+      os << "\n";
       {
         static const char *names[4] = {"q", "k", "v", "o"};
         const uint32_t rows[4] = {a->sq, a->skv, a->skv, a->sq};
@@ -277,6 +279,10 @@ std::string &VKernel::DisAssemble() {
           if (!dense) os << "  " << names[i] << ": view, strides row=" << a->row_stride[i] << " batch=" << a->outer_stride[i] << "," << a->inner_stride[i]
                          << " (inner batch extent " << a->nb_inner << ")\n";
         }
+      }
+      if (a->merge != 0) {
+        os << "  merge o, partials\n  store o\n";
+        continue;
       }
       os << "  mmad s, K, Q^T\n  online_softmax p, s\n  mmad o, V^T, p\n  store o\n";
     } else {

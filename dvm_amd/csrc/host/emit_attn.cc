@@ -6,6 +6,7 @@
 #include <cstring>
 #include <stdexcept>
 
+#include "../../../include/dvm_hip.h"
 #include "compiler.h"
 
 namespace dvm {
@@ -92,5 +93,91 @@ void Compiler::CompileAttn(int gi) {
   if (k_->tuning_.attn_waves == 4) prog_->threads = 256;
   prog_->lds_bytes = DVM_ATTN_LDS_BYTES_D(h.d);
   prog_->grid = h.nb * h.q_blocks;
+  DivideKeys();
+}
+
+constexpr size_t kPartBytes = 8u << 20;
+
+// Hands an attention to the kernel whose waves divide the keys, where that is the faster one.
+void Compiler::DivideKeys() {
+  VAttnHeader *h = reinterpret_cast<VAttnHeader *>(prog_->blob.w);
+  const int forced = k_->tuning_.attn_keys;
+  if (forced == 0 || (forced < 0 && k_->tuning_.attn_waves >= 0)) return;
+  const uint64_t cus = g_system.core_num > 0 ? g_system.core_num : 256;
+  const uint64_t slots = h->d == DVM_ATTN_D ? cus : 2 * cus;  // 128 KB of local memory a workgroup, or 64
+  const uint32_t q_blocks = (h->sq - 1) / DVM_ATTN_KEYS_BQ + 1, blocks = (h->skv - 1) / DVM_ATTN_KEYS_BKV + 1;
+  const uint64_t tiles = static_cast<uint64_t>(h->nb) * q_blocks;
+  if (tiles >= (1u << 24)) return;
+  const bool wide = h->d == DVM_ATTN_D;
+  // Time of the kernel whose waves divide the queries, in us: one 64-key block behind the other, two workgroups share a
+  // compute unit when there are more than compute units, and together they fetch K and V at some 3.6 TB/s (a barrier
+  // ends every block).
+  const double q_rounds = prog_->grid <= cus ? 1.0 : 1.6 * std::ceil(static_cast<double>(prog_->grid) / static_cast<double>(2 * cus));
+  const double t_queries = std::max(3.5 + q_rounds * ((h->skv + DVM_ATTN_BKV - 1) / DVM_ATTN_BKV) * (wide ? 2.0 : 1.3),
+                                    static_cast<double>(h->nb) * h->skv * h->d * 4.0 / 3.6e6);
+  // Time of a division into `n` parts: rounds of workgroups, per round the steps of its waves (four blocks a step), a step
+  // bound by latency and compute (more with a full chip) or by what the workgroups of a round fetch together, 64 KB a step
+  // and compute unit at 5.5 TB/s, once for the query tiles of a head (L2); a merge costs its launch, a trip per part and the
+  // partial outputs' way through memory.
+  auto t_keys = [&](uint32_t n) {
+    const double steps = std::ceil(((blocks + n - 1) / n) / static_cast<double>(DVM_ATTN_KEYS_WAVES));
+    const uint64_t wgs = tiles * n;
+    auto round = [&](double fill) { return 3.2 + steps * std::max((wide ? 1.3 : 0.87) * (1.0 + 0.6 * fill), 3.05 * fill / q_blocks); };
+    double us = static_cast<double>(wgs / slots) * round(1.0);
+    if (wgs % slots != 0) us += round(static_cast<double>(wgs % slots) / static_cast<double>(slots));
+    if (n > 1) us += 6.0 + 0.35 * n + static_cast<double>(h->nb) * n * h->sq * (h->d + 2) * 8.0 / 3.0e6;
+    return us;
+  };
+  // What parts leave in memory stays a small share of the static workspace (DVM_HIP_STATIC_WS_BYTES), beside what the
+  // kernel's other values take: a kernel that fits it does so after the division too.
+  size_t taken = 0;
+  for (size_t bytes : k_->ws_sizes_) taken += (bytes + 255) & ~static_cast<size_t>(255);
+  auto part_bytes = [&](uint32_t n) { return static_cast<size_t>(h->nb) * n * h->sq * (h->d + 2) * 4; };
+  uint32_t parts = 1;
+  if (forced > 1) {
+    parts = std::min<uint32_t>(static_cast<uint32_t>(forced), (blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES);
+  } else if (forced < 0) {
+    double best = t_keys(1);
+    const uint32_t most = std::min<uint32_t>(32, (blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES);
+    for (uint32_t n = 2; n <= most; ++n) {
+      if (part_bytes(n) > kPartBytes || taken + part_bytes(n) > DVM_HIP_STATIC_WS_BYTES) break;
+      const double us = t_keys(n);
+      if (us < best) {
+        best = us;
+        parts = n;
+      }
+    }
+    // Where the estimates are close the query kernel stays: each key block is read from local memory once for 32 queries
+    // of a wave there, and for 32 queries of the workgroup here. Measured on MI355X in us, waves divide queries / keys
+    // (parts): [16,32] heads, 1 query, 1999 keys, D 128: 145 / 96 (1); [1,4], 1, 4096, 128: 101 / 14 (8); [1,32], 8, 4096,
+    // 64: 79 / 13 (8); [1,4], 2000, 2000, 128: 63 / 29 (1); [2,8], 500, 1000, 64: 25 / 11 (1); [4,16], 1000, 1000, 128:
+    // 46 / 121 (1); [8,32], 100, 200, 128: 15 / 28 (1).
+    if (best > 0.8 * t_queries) return;
+  }
+  uint32_t part_blocks = (blocks + parts - 1) / parts;
+  part_blocks = std::min<uint32_t>(blocks, (part_blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES * DVM_ATTN_KEYS_WAVES);
+  parts = (blocks + part_blocks - 1) / part_blocks;
+  h->q_blocks = q_blocks;
+  h->kv_parts = parts;
+  h->part_blocks = part_blocks;
+  prog_->threads = 64 * DVM_ATTN_KEYS_WAVES;
+  prog_->lds_bytes = DVM_ATTN_KEYS_LDS_BYTES_D(h->d);
+  prog_->grid = static_cast<uint32_t>(tiles * parts);
+  if (parts == 1) return;
+  Program::Patch pp;
+  pp.word = static_cast<uint32_t>(offsetof(VAttnHeader, part_addr) / 8);
+  pp.op_id = -1;
+  pp.ws_slot = static_cast<int>(k_->ws_sizes_.size());
+  pp.role = Program::kPatchPlain;
+  k_->ws_sizes_.push_back(part_bytes(parts));
+  prog_->patches.push_back(pp);
+  const Program first = *prog_;
+  k_->programs_.push_back(first);
+  prog_ = &k_->programs_.back();
+  h = reinterpret_cast<VAttnHeader *>(prog_->blob.w);
+  h->merge = 1;
+  prog_->lds_bytes = 0;
+  prog_->grid = static_cast<uint32_t>((static_cast<uint64_t>(h->nb) * h->sq * (h->d / 4) + prog_->threads - 1) / prog_->threads);
+  prog_->fills.clear();
 }
 }  // namespace dvm

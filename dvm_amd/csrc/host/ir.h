@@ -239,7 +239,8 @@ struct Tuning {
   int cube_dump16 = -1; // DVM_CUBE_DUMP16=0: the matmul epilogue always reads the tile back as fp32, half a tile per pass
   int cube_fuse_act = -1;  // DVM_CUBE_FUSE_ACT=0: x / (exp(x * c) + 1) and 1 / (exp(x * c) + 1) of a matmul epilogue stay separate instructions
   int cube_exact = -1;  // DVM_CUBE_EXACT=1: never the hardware approximations of exp, log, sqrt, division in a matmul epilogue
-  int attn_waves = -1;  // DVM_ATTN_WAVES=4
+  int attn_waves = -1;  // DVM_ATTN_WAVES=4 or 8: attention always by the kernels whose waves divide the queries
+  int attn_keys = -1;   // DVM_ATTN_KEYS=0: never by the kernel whose waves divide the keys, n: always, the keys in (up to) n parts
   bool debug = false;   // DVM_DEBUG: node dump in compile errors
   bool in_tuner = false;  // the kernel is a candidate the online tuner is timing: it is not tuned itself
   void Read();

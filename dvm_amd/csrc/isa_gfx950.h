@@ -371,6 +371,12 @@ enum { VCG_NONE = 0, VCG_M_BOUND = 1, VCG_M_SIZE = 2, VCG_K_BOUND = 3, VCG_K_SIZ
 #define DVM_ATTN_D_OK(d) ((d) == DVM_ATTN_D || (d) == DVM_ATTN_D / 2)
 #define DVM_ATTN_LDS_BYTES_D(d) (2u * 2u * DVM_ATTN_BKV * (d) * 2u)  // two buffers of a K block and a V block
 #define DVM_ATTN_LDS_BYTES DVM_ATTN_LDS_BYTES_D(DVM_ATTN_D)
+// The kernel whose waves divide the keys: queries per workgroup, keys per block, waves; per wave two buffers of a K and
+// a V block (where the waves' results meet, 32 x (d + 4) fp32 each and their maxima and sums, is smaller).
+#define DVM_ATTN_KEYS_BQ 32
+#define DVM_ATTN_KEYS_BKV 32
+#define DVM_ATTN_KEYS_WAVES 4
+#define DVM_ATTN_KEYS_LDS_BYTES_D(d) (DVM_ATTN_KEYS_WAVES * 2u * 2u * DVM_ATTN_KEYS_BKV * (d) * 2u)
 
 typedef struct {
   uint32_t entry;   // VE_ATTN
@@ -388,7 +394,11 @@ typedef struct {
   // row = heads * d, outer = seq * heads * d, inner = d with nb_inner = heads.
   uint32_t nb_inner;
   uint32_t row_stride[4], outer_stride[4], inner_stride[4];
-  uint32_t pad;
+  uint32_t kv_parts;     // 0: four or eight waves divide 256 queries. 1 and more: waves divide the keys of DVM_ATTN_KEYS_BQ
+                         // queries (q_blocks counts those), and kv_parts workgroups divide them per tile of queries
+  uint32_t part_blocks;  // key blocks (DVM_ATTN_KEYS_BKV) of one part; no part is empty
+  uint32_t merge;        // the second launch of a division into parts: reads part_addr, writes o_addr
+  uint64_t part_addr;    // kv_parts > 1: fp32 [nb][kv_parts][sq][d] unscaled outputs, then [nb][kv_parts][sq][2] maxima (base 2) and sums
 } VAttnHeader;
 
 typedef struct {
