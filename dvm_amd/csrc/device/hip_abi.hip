@@ -36,15 +36,9 @@ DVM_CUBE_DECL(dvm_vm_cube_bf16_small)
 DVM_CUBE_DECL(dvm_vm_cube_f16_small)
 DVM_CUBE_DECL(dvm_vm_cube_bf16_big8)
 DVM_CUBE_DECL(dvm_vm_cube_f16_big8)
-// the builds that sum the partial tiles of a split k axis (second launch), [tile][bf16] below
-extern "C" __global__ void dvm_vm_cube_f16_big_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_bf16_big_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_f16_mid_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_bf16_mid_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_f16_small_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_bf16_small_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_f16_big8_comb(const VmParam p);
-extern "C" __global__ void dvm_vm_cube_bf16_big8_comb(const VmParam p);
+// the builds that sum the partial tiles of a split k axis (second launch, tiles of any size)
+extern "C" __global__ void dvm_vm_cube_f16_comb(const VmParam p);
+extern "C" __global__ void dvm_vm_cube_bf16_comb(const VmParam p);
 
 extern "C" __global__ void dvm_vm_attn_f16(const VmParam p);
 extern "C" __global__ void dvm_vm_attn_bf16(const VmParam p);
@@ -69,10 +63,7 @@ static const CubeKernel kCubeKernels[4][2][4] = {
     {DVM_CUBE_ROW(dvm_vm_cube_f16_mid), DVM_CUBE_ROW(dvm_vm_cube_bf16_mid)},
     {DVM_CUBE_ROW(dvm_vm_cube_f16_small), DVM_CUBE_ROW(dvm_vm_cube_bf16_small)},
     {DVM_CUBE_ROW(dvm_vm_cube_f16_big8), DVM_CUBE_ROW(dvm_vm_cube_bf16_big8)}};
-static const CubeKernel kCubeCombKernels[4][2] = {{dvm_vm_cube_f16_big_comb, dvm_vm_cube_bf16_big_comb},
-                                                  {dvm_vm_cube_f16_mid_comb, dvm_vm_cube_bf16_mid_comb},
-                                                  {dvm_vm_cube_f16_small_comb, dvm_vm_cube_bf16_small_comb},
-                                                  {dvm_vm_cube_f16_big8_comb, dvm_vm_cube_bf16_big8_comb}};
+static const CubeKernel kCubeCombKernels[2] = {dvm_vm_cube_f16_comb, dvm_vm_cube_bf16_comb};
 
 // [slabs a lane]: the row build of the vector VM
 typedef void (*VecKernel)(const VmParam);
@@ -174,8 +165,7 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
   for (const auto &tile : kCubeKernels)
     for (const auto &dt : tile)
       for (CubeKernel k : dt) kernels.push_back(reinterpret_cast<const void *>(k));
-  for (const auto &tile : kCubeCombKernels)
-    for (CubeKernel k : tile) kernels.push_back(reinterpret_cast<const void *>(k));
+  for (CubeKernel k : kCubeCombKernels) kernels.push_back(reinterpret_cast<const void *>(k));
   for (const void *k : {reinterpret_cast<const void *>(dvm_vm_attn_f16), reinterpret_cast<const void *>(dvm_vm_attn_bf16),
                         reinterpret_cast<const void *>(dvm_vm_attn_f16_w8), reinterpret_cast<const void *>(dvm_vm_attn_bf16_w8),
                         reinterpret_cast<const void *>(dvm_vm_attn_f16_d64), reinterpret_cast<const void *>(dvm_vm_attn_bf16_d64),
@@ -412,12 +402,14 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const VCubeHeader *c = reinterpret_cast<const VCubeHeader *>(p.w);
     const uint64_t mem_end = static_cast<uint64_t>(c->mem_off) + static_cast<uint64_t>(c->n_mem) * (sizeof(VCubeMem) / 8);
     const uint64_t code_end = static_cast<uint64_t>(c->code_off) + c->n_code;
+    const bool comb = (c->epi_flags & VCF_SPLITK_COMBINE) != 0;
     const uint32_t bt = (c->tile == 0 || c->tile == 3) ? 256u : (c->tile == 1 ? 128u : 64u);
-    const uint32_t want_threads = c->tile == 3 ? 512u : 256u;  // tile 3: the 256x256 tile on eight waves
+    const uint32_t want_threads = c->tile == 3 && !comb ? 512u : 256u;  // tile 3: the 256x256 tile on eight waves
+    const uint32_t lds_tile = comb ? 64u : bt;
     // The tile loop trusts the header: check it describes the launch it gets.
     if (mem_end > DVM_PARAM_WORDS || code_end > DVM_PARAM_WORDS || c->n_code == 0 || VI_OP(p.w[code_end - 1]) != VOP_END ||
         c->tile > 3 || threads != want_threads || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
-        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < DVM_CUBE_LDS_BYTES(bt) ||
+        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < DVM_CUBE_LDS_BYTES(lds_tile) ||
         c->a_addr == 0 || c->b_addr == 0 || (c->dtype != VDT_F16 && c->dtype != VDT_BF16)) {
       return static_cast<int>(hipErrorInvalidValue);
     }
@@ -445,8 +437,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
         return static_cast<int>(hipErrorInvalidValue);
       }
     }
-    const CubeKernel kern = (c->epi_flags & VCF_SPLITK_COMBINE)
-                                ? kCubeCombKernels[c->tile][c->dtype == VDT_BF16 ? 1 : 0]
+    const CubeKernel kern = comb ? kCubeCombKernels[c->dtype == VDT_BF16 ? 1 : 0]
                                 : kCubeKernels[c->tile][c->dtype == VDT_BF16 ? 1 : 0][(c->trans_a ? 2 : 0) + (c->trans_b ? 1 : 0)];
     if (check_only) return 0;
     hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), lds_bytes, s, p);

@@ -1251,9 +1251,16 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
   const uint32_t n_tiles = g_rows ? tiles_per_batch : tiles_per_batch * h.nb0 * h.nb1;
   // Split k (VCF_SPLITK_*): the first launch has k_split workgroups per tile, each walks k_chunk of the k axis and
   // leaves its fp32 accumulators in the partials buffer, register by register as the lanes hold them; the second
-  // launch has one workgroup per tile, adds the partials in ascending k order and runs the epilogue.
+  // launch adds the partials in ascending k order and runs the epilogue. It takes the tiles of any size in pieces of
+  // 64 x 64: with a workgroup per tile as before a product of 128 tiles of 256 x 256 left half the chip idle there and
+  // the rest waiting for memory. Measured, a tile per workgroup / pieces: [4096,4096] x [4096,2048] in two parts
+  // 23.0 / 20.4 us (84 MB), [300,3000] x [3000,1000] 34.2 / 11.3 us, [1100,4096] x [4096,2056] 72.0 / 15.6 us,
+  // [8,8192] x [8192,8192] in four parts 8.3 / 7.4 us.
   const bool split_part = !COMB && (h.epi_flags & VCF_SPLITK_PARTIAL) != 0u;
-  const uint32_t n_work = split_part ? n_tiles * h.k_split : n_tiles;
+  const bool a_kc = COMB ? h.trans_a == 0u : A_KC;
+  const uint32_t part_bm = !COMB ? static_cast<uint32_t>(BM) : (h.tile == 1u ? 128u : (h.tile == 2u ? 64u : 256u));  // the tile the partials come from
+  const uint32_t side = part_bm / BM;  // pieces along its side
+  const uint32_t n_work = split_part ? n_tiles * h.k_split : n_tiles * side * side;
   constexpr uint32_t kPartVecs = TM * TN * 4;  // 16-byte vectors a lane holds of the tile
 
   // Fragment reads: fragment i of this wave is rows r0 + 32*i of the staged tile (r0 = the lane's row
@@ -1273,7 +1280,9 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     // order; the order itself walks 8-tile-wide column bands row by row, which makes the 32 tiles an XCD has
     // in flight a 4 x 8 block (12 operand panels to fetch instead of 18 for two full rows of 16).
     uint32_t t = t0;
-    if ((n_work & 7u) == 0 && gridDim.x >= n_work) t = (t0 & 7u) * (n_work >> 3) + (t0 >> 3);
+    if (!COMB && (n_work & 7u) == 0 && gridDim.x >= n_work) t = (t0 & 7u) * (n_work >> 3) + (t0 >> 3);
+    const uint32_t piece = t % (side * side);  // (0 of 1 unless the launch combines)
+    t /= side * side;
     const uint32_t ksplit = t / n_tiles;  // which part of the k axis (0 unless the launch writes partials)
     t -= ksplit * n_tiles;
     const uint32_t tile_id = t;
@@ -1303,7 +1312,7 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     // it can take the vector path like any full tile; its epilogue covers only the rows from m_lo and the columns
     // from n_lo on, the part no other tile writes. (Columns move in whole 8-element slabs only; an operand whose
     // rows are the contiguous axis needs the new origin 16-byte aligned.)
-    uint32_t m0 = tm * BM, n0 = tn * BN;
+    uint32_t m0 = tm * part_bm, n0 = tn * part_bm;
     uint32_t m_lo = m0, m_end = h.m;  // the rows of the output this tile stores
     const uint32_t n_lo = n0;
     bool k_fast = true;
@@ -1325,8 +1334,14 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       }
     }
     if (h.fast) {
-      if (m0 + BM > h.m && h.m >= BM && (A_KC || (h.m & 7u) == 0)) m0 = h.m - BM;
-      if (n0 + BN > h.n && h.n >= BN && (h.n & 7u) == 0) n0 = h.n - BN;
+      if (m0 + part_bm > h.m && h.m >= part_bm && (a_kc || (h.m & 7u) == 0)) m0 = h.m - part_bm;
+      if (n0 + part_bm > h.n && h.n >= part_bm && (h.n & 7u) == 0) n0 = h.n - part_bm;
+    }
+    const uint32_t piece_m = piece / side, piece_n = piece % side;
+    if constexpr (COMB) {
+      m0 += piece_m * BM;
+      n0 += piece_n * BN;
+      if (m0 >= h.m || n0 >= h.n || m0 + BM <= m_lo || n0 + BN <= n_lo) continue;
     }
     const uint64_t a_base = h.a_addr + (static_cast<uint64_t>(bi0) * h.a_sb0 + static_cast<uint64_t>(bi1) * h.a_sb1) * 2;
     const uint64_t b_base = h.b_addr + (static_cast<uint64_t>(bi0) * h.b_sb0 + static_cast<uint64_t>(bi1) * h.b_sb1) * 2;
@@ -1389,38 +1404,45 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     const uint64_t a_org = a_base + (A_KC ? static_cast<uint64_t>(m0) * h.lda + k_lo : static_cast<uint64_t>(k_lo) * h.lda + m0) * 2;
     const uint64_t b_org = b_base + (B_KC ? static_cast<uint64_t>(n0) * h.ldb + k_lo : static_cast<uint64_t>(k_lo) * h.ldb + n0) * 2;
     if constexpr (COMB) {
-      const DVM_GLOBAL vf4 *src = reinterpret_cast<const DVM_GLOBAL vf4 *>(h.part_addr) + static_cast<uint64_t>(tile_id) * kPartVecs * NTHR + tid;
-      const uint64_t split_stride = static_cast<uint64_t>(n_tiles) * kPartVecs * NTHR;
-      // One fragment (16 registers) at a time, its vectors of four or eight parts in flight together: a trip to memory
-      // per fragment and group of parts instead of several per part (a single workgroup per tile is latency bound);
-      // the parts are still added in ascending order.
-      constexpr int PC = TM * TN == 4 ? 8 : 4;  // (fewer where the accumulators take half the registers, or two workgroups share a compute unit)
-      for (uint32_t sp0 = 0; sp0 < h.k_split; sp0 += PC) {
-        const uint32_t n_here = h.k_split - sp0 < static_cast<uint32_t>(PC) ? h.k_split - sp0 : static_cast<uint32_t>(PC);
+      // The fragment of 32 x 32 this wave finishes, and where the wave that computed it (of two or four along the rows,
+      // two along the columns, TM x TN fragments each) left its lanes' registers.
+      static_assert(TM == 1 && TN == 1, "a piece is one fragment per wave");
+      const uint32_t w = uni(wave), fr = piece_m * 2u + (w >> 1), fc = piece_n * 2u + (w & 1u);
+      const uint32_t ptm = h.tile == 0u ? 4u : (h.tile == 2u ? 1u : 2u), ptn = h.tile == 1u ? 2u : (h.tile == 2u ? 1u : 4u);
+      const uint32_t plane = h.tile == 3u ? 512u : 256u;
+      const uint64_t tile_vecs = static_cast<uint64_t>(part_bm) * part_bm / 4u, split_stride = n_tiles * tile_vecs;
+      const DVM_GLOBAL vf4 *frag = reinterpret_cast<const DVM_GLOBAL vf4 *>(h.part_addr) + tile_id * tile_vecs +
+                                   ((fr % ptm) * ptn + fc % ptn) * 4u * plane + ((fr / ptm) * 2u + fc / ptn) * 64u + lane;
+      // groups of eight rows that hold rows of the output (what lies past its end was not written)
+      const uint32_t f_row = m0 + (w >> 1) * 32u;
+      const uint32_t groups = f_row >= h.m ? 0u : ((h.m - f_row + 7u) / 8u < 4u ? (h.m - f_row + 7u) / 8u : 4u);
+      // The vectors of four parts are in flight together; the parts are added in ascending order.
+      constexpr int PC = 4;
+      auto add_parts = [&](auto all) {
+        constexpr bool ALL = decltype(all)::value;
+        for (uint32_t sp0 = 0; sp0 < h.k_split; sp0 += PC) {
+          const uint32_t n_here = h.k_split - sp0 < static_cast<uint32_t>(PC) ? h.k_split - sp0 : static_cast<uint32_t>(PC);
+          vf4 v[PC][4];
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+          for (int pp = 0; pp < PC; ++pp)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            vf4 v[PC][4];
-            const DVM_GLOBAL vf4 *frag = src + sp0 * split_stride + static_cast<uint32_t>((i * TN + j) * 4) * NTHR;
-#pragma unroll
-            for (int pp = 0; pp < PC; ++pp) {
-              if (static_cast<uint32_t>(pp) < n_here) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[pp][q] = frag[pp * split_stride + static_cast<uint32_t>(q) * NTHR];
-              }
+            for (int q = 0; q < 4; ++q) {
+              v[pp][q] = 0.0f;
+              if (static_cast<uint32_t>(pp) < n_here && (ALL || static_cast<uint32_t>(q) < groups)) v[pp][q] = frag[(sp0 + pp) * split_stride + static_cast<uint32_t>(q) * plane];
             }
 #pragma unroll
-            for (int pp = 0; pp < PC; ++pp) {
-              if (static_cast<uint32_t>(pp) < n_here) {
+          for (int pp = 0; pp < PC; ++pp) {
+            if (static_cast<uint32_t>(pp) < n_here) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
+              for (int q = 0; q < 4; ++q)
 #pragma unroll
-                  for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += v[pp][q][e];
-              }
+                for (int e = 0; e < 4; ++e) acc[0][0][4 * q + e] += v[pp][q][e];
             }
           }
-      }
+        }
+      };
+      if (groups == 4u) add_parts(std::true_type{});
+      else add_parts(std::false_type{});
     } else {
     if (h.fast && k_fast && (m0 + BM <= h.m || a_clamps) && (n0 + BN <= h.n || b_clamps)) {
      if constexpr (RING) {
@@ -1579,12 +1601,14 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     if (split_part) {
       DVM_GLOBAL vf4 *dst = reinterpret_cast<DVM_GLOBAL vf4 *>(h.part_addr) +
                             (static_cast<uint64_t>(ksplit) * n_tiles + tile_id) * kPartVecs * NTHR + tid;
+      const uint32_t w_row = m0 + (uni(wave) >> 1) * TM * 32u;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
+            if (w_row + i * 32u + q * 8u >= h.m) continue;  // (rows past the end: the sum does not read them)
             const vf16 &c = acc[i][j];
             const vf4 v = {c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
             dst[static_cast<uint32_t>((i * TN + j) * 4 + q) * NTHR] = v;
@@ -1691,14 +1715,8 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
 
 #define DVM_CUBE_COMB(name, bf, tm, tn, wm, occ) \
   extern "C" __global__ void __launch_bounds__(wm * 128, occ) name(const VmParam p) { vm_cube<bf, tm, tn, true, false, wm, true>(p); }
-DVM_CUBE_COMB(dvm_vm_cube_bf16_big_comb, true, 4, 4, 2, 1)
-DVM_CUBE_COMB(dvm_vm_cube_f16_big_comb, false, 4, 4, 2, 1)
-DVM_CUBE_COMB(dvm_vm_cube_bf16_mid_comb, true, 2, 2, 2, 1)
-DVM_CUBE_COMB(dvm_vm_cube_f16_mid_comb, false, 2, 2, 2, 1)
-DVM_CUBE_COMB(dvm_vm_cube_bf16_small_comb, true, 1, 1, 2, 2)
-DVM_CUBE_COMB(dvm_vm_cube_f16_small_comb, false, 1, 1, 2, 2)
-DVM_CUBE_COMB(dvm_vm_cube_bf16_big8_comb, true, 2, 4, 4, 2)
-DVM_CUBE_COMB(dvm_vm_cube_f16_big8_comb, false, 2, 4, 4, 2)
+DVM_CUBE_COMB(dvm_vm_cube_bf16_comb, true, 1, 1, 2, 3)
+DVM_CUBE_COMB(dvm_vm_cube_f16_comb, false, 1, 1, 2, 3)
 DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_big, true, 4, 4, 2, 1)
 DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_big, false, 4, 4, 2, 1)
 DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_mid, true, 2, 2, 2, 1)

@@ -239,13 +239,14 @@ std::string &VKernel::DisAssemble() {
       const VCubeHeader *c = reinterpret_cast<const VCubeHeader *>(p.blob.w);
       static const int tile[] = {256, 128, 64, 256};
       os << "entry cube " << kMemTypes[c->dtype] << " m=" << c->m << " n=" << c->n << " k=" << c->k << " trans_a=" << c->trans_a
-         << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << tile[c->tile] << " blocks=" << p.grid
+         << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << tile[c->tile] << " blocks="
+         << ((c->epi_flags & VCF_SPLITK_COMBINE) ? static_cast<uint64_t>(c->tiles_m) * c->tiles_n * c->nb0 * c->nb1 : static_cast<uint64_t>(p.grid))
          << " lds=" << p.lds_bytes << (c->fast ? " fast" : " guarded") << (c->tile == 3 ? " eight-waves" : "");
       if (c->epi_flags & VCF_PLAIN_STORE) os << " plain-store";
       else if (c->epi_flags & VCF_SLIM) os << " slim-epilogue";
       if (c->epi_flags & VCF_DUMP16) os << " tile-as-16-bit";
       if (c->epi_flags & VCF_SPLITK_PARTIAL) os << " split-k partials " << c->k_split << " x " << c->k_chunk;
-      if (c->epi_flags & VCF_SPLITK_COMBINE) os << " split-k sum of " << c->k_split;
+      if (c->epi_flags & VCF_SPLITK_COMBINE) os << " split-k sum of " << c->k_split << " in pieces of 64x64, workgroups=" << p.grid;
       if (c->group_mode != VCG_NONE) {
         static const char *gm[] = {"", "rows by bounds", "rows by sizes", "k by bounds", "k by sizes"};
         os << " groups=" << c->nb1 << " (" << gm[c->group_mode <= VCG_K_SIZE ? c->group_mode : 0] << ", " << (c->group_i32 ? "int32" : "int64") << " list)";

@@ -122,7 +122,7 @@ void Compiler::DivideKeys() {
   auto t_keys = [&](uint32_t n) {
     const double steps = std::ceil(((blocks + n - 1) / n) / static_cast<double>(DVM_ATTN_KEYS_WAVES));
     const uint64_t wgs = tiles * n;
-    auto round = [&](double fill) { return 3.2 + steps * std::max((wide ? 1.3 : 0.87) * (1.0 + 0.6 * fill), 3.05 * fill / q_blocks); };
+    auto round = [&](double fill) { return std::max(3.2 + steps * (wide ? 1.3 : 0.87) * (1.0 + 0.6 * fill), 1.0 + steps * 3.05 * fill / q_blocks); };
     double us = static_cast<double>(wgs / slots) * round(1.0);
     if (wgs % slots != 0) us += round(static_cast<double>(wgs % slots) / static_cast<double>(slots));
     if (n > 1) us += 6.0 + 0.35 * n + static_cast<double>(h->nb) * n * h->sq * (h->d + 2) * 8.0 / 3.0e6;
@@ -147,12 +147,12 @@ void Compiler::DivideKeys() {
         parts = n;
       }
     }
-    // Where the estimates are close the query kernel stays: each key block is read from local memory once for 32 queries
+    // Where the estimates are within a fifth and a microsecond the query kernel stays: each key block is read from local memory once for 32 queries
     // of a wave there, and for 32 queries of the workgroup here. Measured on MI355X in us, waves divide queries / keys
     // (parts): [16,32] heads, 1 query, 1999 keys, D 128: 145 / 96 (1); [1,4], 1, 4096, 128: 101 / 14 (8); [1,32], 8, 4096,
     // 64: 79 / 13 (8); [1,4], 2000, 2000, 128: 63 / 29 (1); [2,8], 500, 1000, 64: 25 / 11 (1); [4,16], 1000, 1000, 128:
     // 46 / 121 (1); [8,32], 100, 200, 128: 15 / 28 (1).
-    if (best > 0.8 * t_queries) return;
+    if (best > 0.8 * t_queries - 1.0) return;
   }
   uint32_t part_blocks = (blocks + parts - 1) / parts;
   part_blocks = std::min<uint32_t>(blocks, (part_blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES * DVM_ATTN_KEYS_WAVES);

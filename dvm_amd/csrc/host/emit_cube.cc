@@ -570,7 +570,11 @@ void Compiler::CompileCube(int a) {
     k_->programs_.push_back(first);
     prog_ = &k_->programs_.back();
     reinterpret_cast<VCubeHeader *>(prog_->blob.w)->epi_flags = flags | VCF_SPLITK_COMBINE;
-    prog_->grid = static_cast<uint32_t>(tiles(bt));
+    // pieces of 64 x 64 whatever the tile, and no more workgroups than run at once (four per compute unit): what a
+    // piece costs beside its bytes is its workgroup's start
+    prog_->threads = 256;
+    prog_->lds_bytes = DVM_CUBE_LDS_BYTES(64u);
+    prog_->grid = static_cast<uint32_t>(std::min<uint64_t>(tiles(bt) * static_cast<uint64_t>(bt / 64) * (bt / 64), 4 * cus));
     prog_->fills.clear();
   }
 }
