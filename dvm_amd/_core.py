@@ -6,6 +6,7 @@ IntArrayRef, ScalarRef, Kernel (graph builder), PyKernel (builder + runner) and
 Device, with the same method names and argument meaning.
 """
 import ctypes
+import weakref
 import os
 
 import numpy as np
@@ -142,6 +143,16 @@ def _ptr(ret):
     if not ret:
         raise RuntimeError(_lib.dvm_c_last_error().decode())
     return ret
+
+
+_WS_PROTO = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p)
+
+
+def current_raw_stream(device):
+    """The hipStream_t of torch's current stream on `device` (what current_stream(device).cuda_stream is, without the
+    Stream object in between)."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 class DataType(int):
@@ -457,6 +468,7 @@ class PyKernel(Kernel):
         self._dyn = "dyn" in ker_type
         self._load_shape = {}   # load handle -> IntArrayRef
         self._inputs = {}
+        self._ws_torch = False  # the workspace allocator is torch_workspace's
 
     def __del__(self):
         rt, self._rt = getattr(self, "_rt", None), None
@@ -564,27 +576,47 @@ class PyKernel(Kernel):
     def bind_device(self, io, device_ptr, shape=None, strides=None):
         """Binds caller-owned device memory (e.g. a torch tensor's data_ptr()) to a load or store. `strides`
         (elements, one per dim) binds a load to memory that is not contiguous: it is then read through them."""
-        if shape is not None and io._h in self._load_shape:
-            self._load_shape[io._h].update(list(shape))
+        ref = self._load_shape.get(io._h)
+        if shape is not None and ref is not None and ref.shape() != shape:
+            ref.update(list(shape))
         if strides is not None:
             arr, n = _i64(strides)
-            _check(_lib.dvm_rt_bind_device_view(self._rt, io._h, ctypes.c_void_p(device_ptr), arr, n))
-        elif io._h in self._load_shape:  # (a load that was strided at an earlier call is dense again)
-            _check(_lib.dvm_rt_bind_device_view(self._rt, io._h, ctypes.c_void_p(device_ptr), None, 0))
+            _check(_lib.dvm_rt_bind_device_view(self._rt, io._h, device_ptr, arr, n))
+        elif ref is not None:  # (a load that was strided at an earlier call is dense again)
+            _check(_lib.dvm_rt_bind_device_view(self._rt, io._h, device_ptr, None, 0))
         else:
-            _check(_lib.dvm_rt_bind_device(self._rt, io._h, ctypes.c_void_p(device_ptr)))
+            _check(_lib.dvm_rt_bind_device(self._rt, io._h, device_ptr))
 
     def set_workspace_allocator(self, alloc):
         """`alloc(nbytes) -> device address` supplies the workspace of the launches from now on (a framework's
         caching allocator); None gives it back to the runner. The memory has to stay valid until the launches of
         the run that follows have finished."""
+        self._ws_torch = False
         if alloc is None:
             self._ws_callback = None
             _check(_lib.dvm_rt_set_workspace_allocator(self._rt, None, None))
             return
-        proto = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p)
-        self._ws_callback = proto(lambda nbytes, _user: int(alloc(int(nbytes))))  # kept alive with the kernel
+        self._ws_callback = _WS_PROTO(lambda nbytes, _user: int(alloc(int(nbytes))))  # kept alive with the kernel
         _check(_lib.dvm_rt_set_workspace_allocator(self._rt, ctypes.cast(self._ws_callback, ctypes.c_void_p), None))
+
+    def torch_workspace(self, device):
+        """The workspace of the launches from now on comes from torch's caching allocator. Returns the list that
+        receives the tensors behind it: new at every call, the caller keeps it until the launches have finished.
+        (The callback is made once per kernel: making one costs as much as a small kernel's code generation.)"""
+        scratch = []
+        self._ws_scratch, self._ws_device = scratch, device
+        if not self._ws_torch:
+            import torch
+            this = weakref.ref(self)  # (the callback lives as long as the kernel: no cycle)
+
+            def alloc(nbytes):
+                k = this()
+                k._ws_scratch.append(torch.empty(max(nbytes, 1), dtype=torch.uint8, device=k._ws_device))
+                return k._ws_scratch[-1].data_ptr()
+
+            self.set_workspace_allocator(alloc)
+            self._ws_torch = True
+        return scratch
 
     def normalize(self):
         """Shape inference only: store.shape() is valid afterwards."""
@@ -612,7 +644,7 @@ class PyKernel(Kernel):
         """Launches on the runner's own stream, or on `stream` (a hipStream_t as an integer). With on_given_stream
         the handle is taken as it is, 0 naming the device's default stream (what torch's default stream is)."""
         flags = (1 if sync else 0) | (2 if on_given_stream else 0)
-        _check(_lib.dvm_rt_run(self._rt, ctypes.c_void_p(stream) if stream else None, flags))
+        _check(_lib.dvm_rt_run(self._rt, stream or None, flags))
 
     def output(self, store, shape=None):
         """The stored tensor; `shape` (strided stores) reads back the whole buffer the store wrote into."""

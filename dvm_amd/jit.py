@@ -14,16 +14,19 @@ its workspace from torch's caching allocator.
 import inspect
 import os
 
-from ._core import PyKernel, DataType
+from ._core import PyKernel, DataType, current_raw_stream
 
 
 class _Slot:
     """What one positional argument of the traced function turned out to be."""
 
-    __slots__ = ("role", "handle")
+    __slots__ = ("role", "handle", "torch_dtype")
 
     def __init__(self, role, handle):
-        self.role, self.handle = role, handle  # role: "tensor", "scalar" or "ints"
+        self.role, self.handle, self.torch_dtype = role, handle, None  # role: "tensor", "scalar" or "ints"
+
+
+_TORCH_TYPES = {}  # DataType -> torch type, filled at the first call on torch tensors
 
 
 class JitKernel(PyKernel):
@@ -34,6 +37,7 @@ class JitKernel(PyKernel):
         PyKernel.__init__(self, spec, run_type, int(os.getenv("DEVICE_ID") or 0))
         self.dynamic = bool(dynamic)
         self._slots = []      # one _Slot per argument, filled while tracing
+        self._store_types = None  # torch types of the stores, from the first call on torch tensors
         self._results = None  # what the traced function returned: a store or a sequence of stores
 
     # ---- tracing ----
@@ -41,6 +45,7 @@ class JitKernel(PyKernel):
         positional = [p for p in inspect.signature(func).parameters.values()
                       if p.kind in (p.POSITIONAL_ONLY, p.POSITIONAL_OR_KEYWORD)]
         self._slots = [None] * (len(positional) - 1)  # the first parameter is the kernel itself
+        self._store_types = None
         self._results = func(self, *range(len(self._slots)))
         missing = [i for i, s in enumerate(self._slots) if s is None]
         if missing:
@@ -98,9 +103,11 @@ class _DeviceCall:
     def __init__(self, kern, args, out=None):
         import torch
         self.torch, self.kern, self.args, self.out = torch, kern, args, out
-        self.types = {int(DataType.bool): torch.bool, int(DataType.float16): torch.float16,
-                      int(DataType.bfloat16): torch.bfloat16, int(DataType.float32): torch.float32,
-                      int(DataType.int32): torch.int32, int(DataType.int64): torch.int64}
+        if not _TORCH_TYPES:
+            _TORCH_TYPES.update({int(DataType.bool): torch.bool, int(DataType.float16): torch.float16,
+                                 int(DataType.bfloat16): torch.bfloat16, int(DataType.float32): torch.float32,
+                                 int(DataType.int32): torch.int32, int(DataType.int64): torch.int64})
+        self.types = _TORCH_TYPES
 
     def _bind_inputs(self, in_place):
         """Binds the arguments; `in_place`: tensors that are not contiguous are read through their strides,
@@ -113,12 +120,15 @@ class _DeviceCall:
                     raise TypeError("tensor arguments have to live on the GPU, all of them")
                 k.input(slot.handle, value)
                 continue
-            want = self.types[int(slot.handle.dtype())]
+            want = slot.torch_dtype
+            if want is None:  # (the type of a load is fixed when the function is traced)
+                want = slot.torch_dtype = self.types[int(slot.handle.dtype())]
             if value.dtype != want:
                 raise TypeError("argument is %s, the kernel's load is %s" % (value.dtype, want))
             device = value.device
-            walkable = value.dim() > 0 and all(s >= 0 for s in value.stride()) and value.numel() > 0
-            if value.is_contiguous() or not (in_place and walkable):
+            if value.is_contiguous():
+                k.bind_device(slot.handle, value.data_ptr(), tuple(value.shape))
+            elif not (in_place and value.dim() > 0 and all(s >= 0 for s in value.stride()) and value.numel() > 0):
                 value = value.contiguous()
                 k.bind_device(slot.handle, value.data_ptr(), tuple(value.shape))
             else:
@@ -129,6 +139,8 @@ class _DeviceCall:
     def _bind_outputs(self, device):
         torch, k = self.torch, self.kern
         stores, many = k._stores()
+        if k._store_types is None:  # (fixed when the function is traced, like the shapes' ranks)
+            k._store_types = [self.types[int(st.dtype())] for st in stores]
         given = None
         if self.out is not None:
             given = list(self.out) if isinstance(self.out, (list, tuple)) else [self.out]
@@ -136,7 +148,7 @@ class _DeviceCall:
                 raise TypeError("the kernel has %d outputs, out= holds %d" % (len(stores), len(given)))
         outs = []
         for i, st in enumerate(stores):
-            shape, dtype = tuple(st.shape()), self.types[int(st.dtype())]
+            shape, dtype = st.shape(), k._store_types[i]
             if given is None:
                 o = torch.empty(shape, dtype=dtype, device=device)
             else:
@@ -154,13 +166,7 @@ class _DeviceCall:
             k.normalize()  # output shapes are known from here on
             outs, many = self._bind_outputs(device)
             # the workspace of the launches belongs to torch's caching allocator, like any temporary of an operator
-            scratch = []
-
-            def workspace(nbytes, scratch=scratch, device=device):
-                scratch.append(torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device))
-                return scratch[-1].data_ptr()
-
-            k.set_workspace_allocator(workspace)
+            scratch = k.torch_workspace(device)
             try:
                 k.codegen()  # addresses are part of the programs, so also for a kernel of fixed shapes
                 break
@@ -169,7 +175,7 @@ class _DeviceCall:
                 # once more on contiguous copies
                 if not in_place or not any(s in str(e) for s in ("not supported", "needs a Copy")):
                     raise
-        k.run(stream=torch.cuda.current_stream(device).cuda_stream, sync=False, on_given_stream=True)
+        k.run(stream=current_raw_stream(device), sync=False, on_given_stream=True)
         k._alive = held + outs + scratch  # until the next call: the launches may still be running
         return outs if many else outs[0]
 

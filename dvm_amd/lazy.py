@@ -26,7 +26,7 @@ import weakref
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from ._core import DataType, PyKernel
+from ._core import DataType, PyKernel, current_raw_stream
 
 aten = torch.ops.aten
 
@@ -111,7 +111,7 @@ class LazyFusion(TorchDispatchMode):
         out = torch.empty(tuple(shape), dtype=dtype, device=device)
         self._node_of[id(out)] = len(self._nodes)
         self._nodes.append(_Node(op, args, shape, dtype, out, const))
-        self._storages.add(out.untyped_storage().data_ptr())
+        self._storages.add(out.data_ptr())  # (a new tensor starts where its storage does)
         self.stats["captured"] += 1
         if len(self._nodes) >= _MAX_PENDING:
             self.flush()
@@ -265,15 +265,9 @@ class LazyFusion(TorchDispatchMode):
                     k.bind_device(ld, t.data_ptr(), shape, strides=tuple(t.stride()))
             for st, i in zip(stores, stored):
                 k.bind_device(st, outs[i].data_ptr())
-            scratch = []
-
-            def workspace(nbytes):
-                scratch.append(torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device))
-                return scratch[-1].data_ptr()
-
-            k.set_workspace_allocator(workspace)
+            scratch = k.torch_workspace(device)
             k.codegen()
-            k.run(stream=torch.cuda.current_stream(device).cuda_stream, sync=False, on_given_stream=True)
+            k.run(stream=current_raw_stream(device), sync=False, on_given_stream=True)
         self._alive = [inputs, outs, scratch]  # until the next segment has been queued behind this one
         self.stats["flushes"] += 1
         self.stats["launches"] += k.num_launches()
