@@ -472,7 +472,7 @@ class PyKernel(Kernel):
 
     def __del__(self):
         rt, self._rt = getattr(self, "_rt", None), None
-        if rt:
+        if rt and _lib is not None:  # (None: the interpreter is shutting down)
             _lib.dvm_rt_delete(rt)
 
     def load(self, shape, type):

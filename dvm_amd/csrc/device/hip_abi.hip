@@ -204,7 +204,11 @@ uint64_t dvm_hip_select_block_thread(uint64_t kind, uint64_t item_num, uint64_t 
   const uint64_t waves_per_wg = (threads + 63) / 64;
   uint64_t wg_per_cu = (4ull * kernel_waves_per_simd(kind)) / waves_per_wg;
   if (lds_bytes > 0) {
-    const uint64_t by_lds = g_dev.lds_per_cu / lds_bytes;
+    // (beside the launch's local memory every workgroup has its copy of the program. Without it in the sum, three
+    // workgroups of 51200 bytes counted as resident where two are, and a third of the grid ran as a pass of its own: the
+    // optimizer step over 2^24 weights, six V register planes, 135 us. At 49152 bytes, without the reduce scratch that
+    // pointwise programs had, three are: 99 us, 4.75 TB/s)
+    const uint64_t by_lds = g_dev.lds_per_cu / (lds_bytes + DVM_PARAM_BYTES);
     if (by_lds < wg_per_cu) wg_per_cu = by_lds;
   }
   if (wg_per_cu == 0) wg_per_cu = 1;

@@ -702,6 +702,8 @@ bool Compiler::FinishProgram() {
   std::memcpy(prog_->blob.w + hdr_.code_off, code_.data(), 8 * code_.size());
   std::memcpy(prog_->blob.w + (hdr_.row_code & 0xffffu), row_code_.data(), 8 * row_code_.size());
   prog_->lds_bytes = DVM_VEC_RED_SCRATCH_DOUBLES(hdr_.sched, prog_->threads) * 8 + static_cast<uint32_t>(max_vslot_) * u_ * 16 * prog_->threads;
+  // (pointwise programs without V registers keep the geometry they are exported with: a double per lane, which nothing reads)
+  prog_->lds_bytes = std::max<uint32_t>(prog_->lds_bytes, 8 * prog_->threads);
   const uint32_t lds_unparked = prog_->lds_bytes;
   PlanRereads();
   if (!row_code_.empty()) prog_->lds_bytes = lds_unparked;  // (the row build parks nothing)

@@ -80,8 +80,8 @@ enum {
 #define DVM_VEC_SWEEP_BODY 6
 // Local memory at the start of a vector program's segment, in doubles: what the lanes of a workgroup combine their
 // reduce partials through. One double per lane; eight (one per element of a lane's group) on the schedule that keeps
-// the innermost axis. The V registers lie behind it.
-#define DVM_VEC_RED_SCRATCH_DOUBLES(sched, threads) ((((sched) & 0xfu) == 2u ? 8u : 1u) * (threads))
+// the innermost axis; none for pointwise programs. The V registers lie behind it.
+#define DVM_VEC_RED_SCRATCH_DOUBLES(sched, threads) ((((sched) & 0xfu) == 2u ? 8u : (((sched) & 0xfu) == 0u ? 0u : 1u)) * (threads))
 
 // ---- opcodes ---------------------------------------------------------------
 // The interpreter is an accumulator machine. Per lane, `acc` holds U slabs of E
@@ -328,8 +328,9 @@ enum { VCG_NONE = 0, VCG_M_BOUND = 1, VCG_M_SIZE = 2, VCG_K_BOUND = 3, VCG_K_SIZ
 #define VCF_APPROX_MATH 1u
 // Split k, for products with fewer tiles than compute units and a long k axis: two launches of the same program.
 // VCF_SPLITK_PARTIAL: tiles * k_split workgroups; each multiplies one part of the k axis and writes its accumulators
-// to part_addr as the lanes hold them, no epilogue. VCF_SPLITK_COMBINE: one workgroup per tile adds the k_split
-// partials in ascending k order (fp32, the same order on every run) and runs the epilogue on the sum.
+// to part_addr as the lanes hold them (rows past the end of the output excepted), no epilogue. VCF_SPLITK_COMBINE: the
+// k_split partials are added in ascending k order (fp32, the same order on every run) and the epilogue runs on the sum,
+// in pieces of 64 x 64 of the tiles, 256 lanes each.
 // The epilogue is [add of a memory operand (a bias row)] [rounding to a float type] store: the kernel does it in
 // place, without walking the program through the interpreter (a dispatch costs more than this whole epilogue).
 #define VCF_PLAIN_STORE 8u
