@@ -409,10 +409,11 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const bool comb = (c->epi_flags & VCF_SPLITK_COMBINE) != 0;
     const uint32_t bt = (c->tile == 0 || c->tile == 3) ? 256u : (c->tile == 1 ? 128u : 64u);
     const uint32_t want_threads = c->tile == 3 && !comb ? 512u : 256u;  // tile 3: the 256x256 tile on eight waves
+    // (the sum of parts in pieces; a program exported with the geometry of the tile's own kernel is taken as well)
     const uint32_t lds_tile = comb ? 64u : bt;
     // The tile loop trusts the header: check it describes the launch it gets.
     if (mem_end > DVM_PARAM_WORDS || code_end > DVM_PARAM_WORDS || c->n_code == 0 || VI_OP(p.w[code_end - 1]) != VOP_END ||
-        c->tile > 3 || threads != want_threads || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
+        c->tile > 3 || (threads != want_threads && !(comb && c->tile == 3 && threads == 512u)) || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
         c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < DVM_CUBE_LDS_BYTES(lds_tile) ||
         c->a_addr == 0 || c->b_addr == 0 || (c->dtype != VDT_F16 && c->dtype != VDT_BF16)) {
       return static_cast<int>(hipErrorInvalidValue);
