@@ -787,15 +787,30 @@ void Compiler::CompileArea(int a) {
       if (!axes_[ax].reduced || fd) Fail("output smaller than the kernel domain");
     }
   }
-  EmitProgram();
-  if (!FinishProgram()) {  // laid out for the row build, and outside its vocabulary after all: once more without it
-    row_allowed_ = false;
-    for (int i = 0; i < nn_; ++i) {
-      nodes_[i].mem_idx = nodes_[i].reg = -1;
-      nodes_[i].slot_ready = false;
+  bool done = false;
+  if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0) {
+    // Laid out for the row build. Whatever keeps the program out of that layout (a word outside the build's vocabulary, V
+    // registers for up to twice the lanes the other builds would use) is settled here, with the layout of the other builds:
+    // thrown past this point it would make RunModes cut the graph.
+    std::string why = "a word outside the row build's vocabulary";
+    try {
+      EmitProgram();
+      done = FinishProgram();
+    } catch (const std::runtime_error &e) {
+      why = e.what();
     }
-    prog_->patches.clear();
-    ChooseSchedule();
+    if (!done) {
+      if (k_->tuning_.debug) std::fprintf(stderr, "dvm: sub-kernel %d leaves the row build: %s\n", a, why.c_str());
+      row_allowed_ = false;
+      for (int i = 0; i < nn_; ++i) {
+        nodes_[i].mem_idx = nodes_[i].reg = -1;
+        nodes_[i].slot_ready = false;
+      }
+      prog_->patches.clear();
+      ChooseSchedule();
+    }
+  }
+  if (!done) {
     EmitProgram();
     FinishProgram();
   }
