@@ -337,6 +337,7 @@ class Compiler {
   uint32_t vslot_used_ = 0;
   int max_vslot_ = 0;
   int vslot_limit_ = 0;
+  int VSlotLimit(uint32_t lanes) const;  // V register slots a lane has in a workgroup of so many
   int cur_sec_ = 0;
 
   int AddNode(AKind kind, NDObject *op, DataType t, const int64_t *dims, int rank);
@@ -391,9 +392,12 @@ class Compiler {
   void PlanRereads();
   bool FitsSweepBuild();
   bool RowCandidate() const;
+  uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;
   bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;
   bool BuildRowCode();
   bool row_allowed_ = true;             // (false: the program has turned out to be outside the row build's vocabulary)
+  uint64_t row_key_ = 0;                // RowKey of the layout being tried
+  std::vector<uint64_t> row_refused_;   // ... of layouts that did not fit: a dynamic kernel tries each once, not at every shape
   std::vector<uint64_t> row_code_;
   bool mem_is_view_[DVM_VEC_MAXMEM] = {false};  // memory operand i is a strided view
   int last_mem_ = -1;         // memory operand of the last memory instruction emitted in this round, or -1

@@ -580,6 +580,12 @@ void Compiler::EmitSection(int sec) {
   n_held_ = 0;
 }
 
+int Compiler::VSlotLimit(uint32_t lanes) const {
+  const uint32_t per_slot = static_cast<uint32_t>(u_) * 16u * lanes;
+  const uint32_t budget = g_system.lds_per_wg > 80 * 1024 ? 72 * 1024 : g_system.lds_per_wg - 8 * 1024;
+  return std::min<int>(DVM_VEC_NREG, static_cast<int>(budget / per_slot));
+}
+
 void Compiler::EmitProgram() {
   const int inner = n_dims_ - 1;
   const int inner_first = dims_[inner].first_axis, inner_last = dims_[inner].last_axis;
@@ -658,9 +664,7 @@ void Compiler::EmitProgram() {
     }
   }
   // local memory budget for V registers
-  const uint32_t per_slot = static_cast<uint32_t>(u_) * 16u * prog_->threads;
-  const uint32_t budget = g_system.lds_per_wg > 80 * 1024 ? 72 * 1024 : g_system.lds_per_wg - 8 * 1024;
-  vslot_limit_ = std::min<int>(DVM_VEC_NREG, static_cast<int>(budget / per_slot));
+  vslot_limit_ = VSlotLimit(prog_->threads);
   sreg_used_ = vslot_used_ = 0;
   max_vslot_ = 0;
   acc_node_ = -1;
@@ -801,6 +805,7 @@ void Compiler::CompileArea(int a) {
     }
     if (!done) {
       if (k_->tuning_.debug) std::fprintf(stderr, "dvm: sub-kernel %d leaves the row build: %s\n", a, why.c_str());
+      if (row_refused_.size() < 64) row_refused_.push_back(row_key_);
       row_allowed_ = false;
       for (int i = 0; i < nn_; ++i) {
         nodes_[i].mem_idx = nodes_[i].reg = -1;

@@ -474,14 +474,42 @@ bool Compiler::RowCandidate() const {
   for (int i = 0; i < nn_; ++i) {
     const ANode &n = nodes_[i];
     if (!is_float(n.dtype)) return false;
+    bool in_sweep = false;  // (varies along the reduced axis)
+    for (int d = 0; d < n.rank; ++d) {
+      if (n.axis[d] < 0 || !axes_[n.axis[d]].reduced) continue;
+      in_sweep = true;
+      if (n.view != nullptr && pos_[n.axis[d]] == dims_[n_dims_ - 1].last_axis && n.view->vstride_[d] != 1) return false;  // read element by element
+    }
     if (n.kind != AK_OP) continue;
     switch (n.op->kind) {
-      case kObjUnary: case kObjBinary: case kObjBinaryS: case kObjCast: break;
+      case kObjUnary:
+        if (in_sweep && n.op->op != kExp && n.op->op != kAbs) return false;  // (one value per row: all of them)
+        break;
+      case kObjBinary: case kObjBinaryS: case kObjCast: break;
       default: return false;
     }
     if ((n.op->kind == kObjBinary || n.op->kind == kObjBinaryS) && (n.op->op == kPow || n.op->op == kLogicalAnd || n.op->op == kLogicalOr)) return false;
   }
   return true;
+}
+
+// What the outcome of trying a row layout depends on: the operators, which of their values vary along the reduced axis,
+// whether a row is one round (up to two slabs a lane: values may wait in V registers there, and only there) and how many V
+// registers those lanes have. Two programs with the same key compile to the same instruction words but for their operands'
+// strides, so that a refusal holds for both and what a kernel is compiled to does not depend on the shapes before it.
+uint64_t Compiler::RowKey(uint32_t slabs, uint32_t lanes) const {
+  uint64_t h = 0xcbf29ce484222325ull;  // FNV-1a
+  auto add = [&h](uint64_t v) { h = (h ^ v) * 0x100000001b3ull; };
+  add(slabs > 2 ? 0 : static_cast<uint64_t>(VSlotLimit(lanes)) + 1);
+  for (int i = 0; i < nn_; ++i) {
+    const ANode &n = nodes_[i];
+    bool in_sweep = false;
+    for (int d = 0; d < n.rank; ++d) in_sweep = in_sweep || (n.axis[d] >= 0 && axes_[n.axis[d]].reduced);
+    add(static_cast<uint64_t>(n.kind) | static_cast<uint64_t>(n.dtype) << 8 | static_cast<uint64_t>(in_sweep) << 16 | static_cast<uint64_t>(n.view != nullptr) << 17);
+    if (n.op != nullptr) add(static_cast<uint64_t>(n.op->kind) | static_cast<uint64_t>(n.op->op) << 16 | static_cast<uint64_t>(n.op->scalar_left) << 32);
+    for (int j = 0; j < n.nin; ++j) add(static_cast<uint64_t>(static_cast<uint32_t>(n.in[j])));
+  }
+  return h;
 }
 
 // Slabs and lanes per row. More slabs a lane mean fewer waves per row: less scalar work between the sweeps, fewer
@@ -616,17 +644,23 @@ void Compiler::ChooseSchedule() {
       if (team > cap) team = cap;
     }
     // The row build, when the operators are in its vocabulary: a lane holds up to eight slabs and the row is one round.
-    uint32_t row_slabs = 0;
-    if (parts == 0 && !wide && RowCandidate() && ChooseRow(n_k, n_r, &row_slabs, &team)) hdr_.sched |= row_slabs << VS_ROW_SHIFT;
+    auto lanes_of = [n_k](uint32_t lanes) { return lanes > 64 ? lanes : (n_k * lanes >= 256 ? 256 : std::max<uint32_t>(64, Pow2Ceil(n_k * lanes))); };
+    uint32_t row_slabs = 0, row_team = 0;
+    if (parts == 0 && !wide && RowCandidate() && ChooseRow(n_k, n_r, &row_slabs, &row_team)) {
+      row_key_ = RowKey(row_slabs, lanes_of(row_team));
+      if (std::find(row_refused_.begin(), row_refused_.end(), row_key_) == row_refused_.end()) {
+        hdr_.sched |= row_slabs << VS_ROW_SHIFT;
+        team = row_team;
+      }
+    }
+    threads = lanes_of(team);
     if (team > 64) {
       hdr_.team_is_block = 1;
-      threads = team;
       hdr_.team_log2 = Log2(team);
       hdr_.n_items = static_cast<uint32_t>(n_k);
     } else {
       hdr_.team_is_block = 0;
       hdr_.team_log2 = Log2(team);
-      threads = n_k * team >= 256 ? 256 : std::max<uint32_t>(64, Pow2Ceil(n_k * team));
       const uint32_t per_wg = threads / team;
       hdr_.n_items = static_cast<uint32_t>((n_k + per_wg - 1) / per_wg);
     }

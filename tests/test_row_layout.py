@@ -1,6 +1,8 @@
 """Which layout a program that reduces the innermost axis is compiled to, without a GPU (disassembly mode): a program the
 row build (vm_vector_row.hip) cannot take is what it is with that build switched off (DVM_VEC_ROW=0), word for word, and is
 not cut into more launches on the way there."""
+import re
+
 import numpy as np
 import pytest
 
@@ -69,3 +71,48 @@ def test_values_held_across_a_reduce_use_the_row_build_where_its_registers_do(mo
     for graph, rows, cols in ((rms_backward, 64, 4096), (layer_norm_backward, 3, 512), (three_exponentials, 4096, 1000)):
         t = _compile(graph, rows, cols, "float32")
         assert t.num_launches() == 1 and " row=" in t.das(), t.das()
+
+
+def _dynamic(graph, shapes, dtype):
+    """The disassembly of each of `shapes` out of one dynamic kernel, code generated twice for each."""
+    t = Tester("split:dyn", run_mode="das")
+    x = t.load([-1, -1], dtype)
+    outs = [t.store(o) for o in graph(t, x)]
+    das = []
+    for shape in shapes:
+        t.input(x, np.zeros(shape, np.uint16 if dtype == "bfloat16" else dtype))
+        t.codegen()
+        t.codegen()
+        das.append(re.sub(r"@0x\w+", "@", t.das()))  # (the made-up addresses depend on what was bound before)
+    assert outs
+    return das
+
+
+def _held_over(t, x):  # eight slabs a lane have no V registers for the three values held across the reduce
+    h = t.cast(x, "float32")
+    a, b, c = t.exp(h), t.exp(t.mul(h, 0.5)), t.exp(t.mul(h, 0.25))
+    s = t.sum(t.mul(t.mul(a, b), c), (1,), True)
+    return [t.div(v, s) for v in (a, b, c)]
+
+
+def test_a_layout_that_does_not_fit_is_tried_once(monkeypatch, capfd):
+    monkeypatch.setenv("DVM_DEBUG", "1")
+    monkeypatch.delenv("DVM_VEC_ROW", raising=False)
+    shapes = [(4096, 4096), (3, 1000), (8192, 4096), (4000, 4104), (4096, 4096)]
+    many = _dynamic(_held_over, shapes, "bfloat16")
+    assert capfd.readouterr().err.count("leaves the row build") == 1
+    assert " row=" not in many[0] and " row=" in many[1] and " row=" not in many[2]
+    # ... and what a shape compiles to does not depend on the shapes before it
+    for shape, das in zip(shapes, many):
+        assert _dynamic(_held_over, [shape], "bfloat16") == [das]
+
+
+@pytest.mark.parametrize("op", ["sqrt", "log", "floor"])
+def test_reduces_over_operators_the_row_build_has_not_are_not_tried(monkeypatch, capfd, op):
+    monkeypatch.setenv("DVM_DEBUG", "1")
+    das = _dynamic(lambda t, x: [t.sum(getattr(t, op)(x), (1,), True)], [(4096, 4096), (200, 1000)], "float32")
+    assert "leaves the row build" not in capfd.readouterr().err
+    assert all("reduce-x" in d and " row=" not in d for d in das)
+    # (of one value per row they are the build's)
+    das = _dynamic(lambda t, x: [getattr(t, op)(t.sum(t.abs(x), (1,), True))], [(4096, 4096)], "float32")
+    assert " row=" in das[0]
