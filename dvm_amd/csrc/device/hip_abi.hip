@@ -258,13 +258,14 @@ static bool sweeps_flag_holds(const VmParam &p) {
   return true;
 }
 
-// The row build reads its words without looking for anything else, accesses rows without guards and holds exactly
-// `slabs` slabs a lane: a blob that carries VS_ROW_* must have that shape.
+// The row build reads its words without looking for anything else (what it has no arm for would run as the last arm of a
+// switch: a store, a maximum, a truncation), accesses rows without guards and holds exactly `slabs` slabs a lane: a blob
+// that carries VS_ROW_* must have that shape and hold nothing but that build's vocabulary.
 static bool row_words_hold(const VmParam &p, uint32_t threads) {
   const VVecHeader *h = reinterpret_cast<const VVecHeader *>(p.w);
   const uint32_t slabs = DVM_VEC_ROW_SLABS(h->sched), off = h->row_code & 0xffffu, n = h->row_code >> 16;
   if (!DVM_VEC_ROW_OK(slabs) || threads > DVM_VEC_ROW_LANES(slabs) || n == 0 || n > DVM_VEC_ROW_WORDS || off + n > DVM_PARAM_WORDS ||
-      off < h->code_off + h->n_code || VI_OP(p.w[off + n - 1]) != VOP_END) return false;
+      off < h->code_off + h->n_code || VI_OP(p.w[off + n - 1]) != VOP_END || h->mem_off + h->n_mem * (sizeof(VMemDesc) / 8) > off + n) return false;
   const uint64_t team = h->team_is_block ? threads : 64u;
   if (h->n_rdim != 1 || h->n_kdim > 2 || h->n_mem == 0 || h->n_mem > 64 || h->inner_extent < DVM_VEC_E || h->n_ridx != (h->inner_extent + DVM_VEC_E - 1) / DVM_VEC_E ||
       h->n_ridx > slabs * team || h->n_ridx <= (slabs - 1) * team || (h->n_kdim == 2 && h->kdims[0].extent == 0)) return false;
@@ -277,43 +278,66 @@ static bool row_words_hold(const VmParam &p, uint32_t threads) {
     if ((m.addr & (m.dtype == VDT_F32 ? 3u : 1u)) != 0) return false;
     return (m.flags & (VMF_VEC | VMF_GATHER)) == (row ? static_cast<uint32_t>(VMF_VEC) : 0u);
   };
+  auto sreg_ok = [](uint32_t s) { return s < DVM_VEC_NSREG; };
+  // second operation of a chained binary (VK_SREG2, VI_PRE_SREG): operator, S register and rounding in the immediate
+  auto chained_ok = [&](uint32_t imm) { return (imm & 0x3fu) <= VB_MAX && sreg_ok((imm >> 8) & 0xffu) && ((imm >> 16) & 3u) <= VRND_BF16; };
+  auto vregs_ok = [&](uint32_t a, uint32_t fmt) { return slabs <= 2 && a + (fmt == VF_F32 ? 2u : 1u) <= h->n_vslot; };
   bool in_sweep = false;
   for (uint32_t i = off; i < off + n; ++i) {
     const uint64_t w = p.w[i];
-    const uint32_t op = VI_OP(w), kind = VI_KIND(w), a = VI_A(w);
+    const uint32_t op = VI_OP(w), kind = VI_KIND(w), a = VI_A(w), sub = VI_SUB(w), imm = VI_IMM(w);
     const bool ends = (static_cast<uint32_t>(w) & VI_ENDS) != 0;
     if (op == VOP_END) {
       if (in_sweep || i != off + n - 1) return false;
       continue;
     }
     if (op == VOP_SWEEP) {
-      if (in_sweep) return false;
+      auto slot_ok = [](uint32_t k) { return k <= VR_MIN || k == VR_NONE; };
+      if (in_sweep || !slot_ok(imm & 0xfu) || !slot_ok((imm >> 4) & 0xfu)) return false;
       in_sweep = true;
       continue;
     }
     if (ends && !in_sweep) return false;
+    if (VI_RND(w) > VRND_BF16) return false;
     switch (op) {
       case VOP_LD: if (kind != VK_MEM || !mem_ok(a, in_sweep)) return false; break;
       case VOP_ST: if (!mem_ok(a, in_sweep)) return false; break;
       case VOP_BINF:
-        if (kind == VK_MEM && !mem_ok(a, in_sweep)) return false;
-        if (kind == VK_REG && (!in_sweep || slabs > 2 || a + 1 > h->n_vslot)) return false;
-        if (kind > VK_SREG2) return false;
+        if ((sub & 0x3fu) > VB_MAX) return false;
+        switch (kind) {
+          case VK_IMM: case VK_ACC: break;
+          case VK_MEM: if (!mem_ok(a, in_sweep) || ((imm & VI_PRE_SREG) != 0 && (!in_sweep || !chained_ok(imm)))) return false; break;
+          case VK_SREG: if (!sreg_ok(a)) return false; break;
+          case VK_SREG2: if (!sreg_ok(a) || !chained_ok(imm)) return false; break;
+          case VK_REG: if (!in_sweep || !vregs_ok(a, sub >> 6)) return false; break;
+          default: return false;
+        }
         break;
       case VOP_CMP: case VOP_MSK: case VOP_MOVM:
-        if (in_sweep || kind == VK_REG || (kind == VK_MEM && !mem_ok(a, false))) return false;
+        if (in_sweep || (op == VOP_CMP && (sub & 0x7fu) > VCMP_LE)) return false;  // (the top bit: VI_OFFS_ASIDE)
+        if (kind != VK_IMM && kind != VK_ACC && !(kind == VK_SREG && sreg_ok(a)) && !(kind == VK_MEM && mem_ok(a, false))) return false;
         break;
-      case VOP_LDR: case VOP_STR:
-        if (!in_sweep || slabs > 2 || a + ((VI_SUB(w) & 3u) == VF_F32 ? 2u : 1u) > h->n_vslot) return false;
+      case VOP_LDR: case VOP_STR: if (!in_sweep || !vregs_ok(a, sub & 3u)) return false; break;
+      case VOP_RED: {
+        const uint32_t rk = sub & 0xfu;
+        if (!in_sweep || a >= DVM_VEC_NSLOT || rk > VR_MIN || (sub & ~(0xfu | VRF_SQUARE | VRF_PAIR)) != 0) return false;
+        if ((sub & (VRF_SQUARE | VRF_PAIR)) != 0 && rk != VR_SUM) return false;
+        if ((sub & VRF_PAIR) != 0 && a != 0) return false;
         break;
-      case VOP_RED: case VOP_SPLAT: if (!in_sweep) return false; break;
-      case VOP_FIN: case VOP_STS: if (in_sweep) return false; break;
-      case VOP_LDS: case VOP_LDI: case VOP_UN: case VOP_CAST: case VOP_ENDSWEEP: break;
+      }
+      case VOP_FIN: if (in_sweep || a >= DVM_VEC_NSLOT || (sub & VRF_INT) != 0) return false; break;
+      case VOP_STS: if (in_sweep || !sreg_ok(a)) return false; break;
+      case VOP_LDS: if (!sreg_ok(a)) return false; break;
+      case VOP_UN: if (in_sweep ? sub != VU_EXP && sub != VU_ABS : sub > VU_TRUNC) return false; break;
+      case VOP_CAST: if (sub != VC_RND) return false; break;
+      case VOP_SPLAT: if (!in_sweep) return false; break;
+      case VOP_ENDSWEEP: if (!in_sweep || !ends) return false; break;
+      case VOP_LDI: break;
       default: return false;
     }
     if ((static_cast<uint32_t>(w) & VI_LD_PAIR) && op == VOP_LD) {
       const uint64_t w1 = i + 1 < off + n ? p.w[i + 1] : 0;
-      if (!in_sweep || ends || VI_OP(w1) != VOP_BINF || VI_KIND(w1) != VK_MEM || VI_A(w1) >= h->n_mem || mems[VI_A(w1)].dtype != mems[a].dtype ||
+      if (!in_sweep || ends || VI_OP(w1) != VOP_BINF || VI_KIND(w1) != VK_MEM || (VI_IMM(w1) & VI_PRE_SREG) != 0 || VI_A(w1) >= h->n_mem || mems[VI_A(w1)].dtype != mems[a].dtype ||
           mems[a].dtype == VDT_F32) return false;
     }
     if (ends) in_sweep = false;

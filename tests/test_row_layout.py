@@ -1,11 +1,15 @@
 """Which layout a program that reduces the innermost axis is compiled to, without a GPU (disassembly mode): a program the
 row build (vm_vector_row.hip) cannot take is what it is with that build switched off (DVM_VEC_ROW=0), word for word, and is
 not cut into more launches on the way there."""
+import ctypes
+import os
 import re
+import struct
 
 import numpy as np
 import pytest
 
+import dvm_amd
 from dvm_amd.tester import Tester
 
 
@@ -116,3 +120,67 @@ def test_reduces_over_operators_the_row_build_has_not_are_not_tried(monkeypatch,
     # (of one value per row they are the build's)
     das = _dynamic(lambda t, x: [getattr(t, op)(t.sum(t.abs(x), (1,), True))], [(4096, 4096)], "float32")
     assert " row=" in das[0]
+
+
+# ---- imported programs: the launch check takes the row build's vocabulary and nothing else ----
+
+END, LDS, LDI, STR, STS, ST, UN, CAST, RED, SWEEP, ENDSWEEP, FIN, LD, BINF, CMP = 0, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 16, 17, 19  # isa_gfx950.h
+IMM, MEM, SREG, SREG2, REG = 1, 2, 4, 5, 0
+PRE_SREG = 1 << 31
+
+
+def _word(op, sub=0, kind=0, rnd=0, a=0, imm=0, ends=False):
+    return op | (0x80 if ends else 0) | sub << 8 | kind << 16 | rnd << 20 | a << 24 | imm << 32
+
+
+def _launch_status(blob, geometry):
+    """What dvm_hip_launch_vm says of a blob on a machine without a GPU: 1 (hipErrorInvalidValue) if it refuses it, another
+    error where it would have launched it."""
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(dvm_amd.__file__), "lib", "libdvm_hip.so"))
+    return lib.dvm_hip_launch_vm(blob, *(ctypes.c_uint32(g) for g in geometry), None)
+
+
+def _row_program(graph, rows, cols):
+    (blob, geometry, _), = _compile(graph, rows, cols, "float32").programs()
+    row_code, = struct.unpack_from("<I", blob, 72)  # VVecHeader::row_code
+    off, n = row_code & 0xffff, row_code >> 16
+    assert n > 0 and geometry[2] <= 64 * 1024  # (the check knows the device's local memory only with a device)
+    return blob, geometry, list(struct.unpack_from("<%dQ" % n, blob, 8 * off)), off
+
+
+def _with_words(blob, off, words):
+    b = bytearray(blob)
+    struct.pack_into("<%dQ" % len(words), b, 8 * off, *words)
+    struct.pack_into("<I", b, 72, off | len(words) << 16)
+    return bytes(b)
+
+
+@pytest.mark.skipif(dvm_amd.Device.available(), reason="the made-up addresses of these programs must not reach a GPU")
+@pytest.mark.parametrize("graph,rows,cols", [(three_exponentials, 3, 512), (rms_backward, 3, 1000), (layer_norm_backward, 2100, 512)])
+def test_the_launch_check_takes_the_row_builds_vocabulary_and_nothing_else(monkeypatch, graph, rows, cols):
+    monkeypatch.delenv("DVM_VEC_ROW", raising=False)
+    blob, geometry, words, off = _row_program(graph, rows, cols)
+    assert _launch_status(blob, geometry) != 1 and _launch_status(_with_words(blob, off, words), geometry) != 1
+    n_vslot, = struct.unpack_from("<I", blob, 60)
+    first_sweep = next(i for i, w in enumerate(words) if w & 0x7f == SWEEP)
+
+    def status(in_sweep, *inserted):
+        at = first_sweep + 1 if in_sweep else first_sweep
+        return _launch_status(_with_words(blob, off, words[:at] + list(inserted) + words[at:]), geometry)
+
+    taken = [(True, _word(UN, 3)), (True, _word(UN, 1)), (False, _word(UN, 8)), (True, _word(CAST, 2, rnd=2)), (True, _word(BINF, 7, IMM)), (False, _word(CMP, 5, IMM)),
+             (True, _word(BINF, 0, SREG, a=7)), (False, _word(STS, a=7)), (True, _word(BINF, 3, SREG2, a=0, imm=7 | 7 << 8 | 2 << 16)),
+             (True, _word(BINF, 0, REG, a=n_vslot - 2)), (False, _word(LDI))]
+    for in_sweep, w in taken:
+        assert status(in_sweep, w) != 1, hex(w)
+    refused = [(True, _word(UN, 0)), (True, _word(UN, 2)), (True, _word(UN, 9)), (False, _word(UN, 9)),  # sqrt, log and int32 abs of a row
+               (True, _word(CAST, 0)), (False, _word(CAST, 3)), (True, _word(CAST, 2, rnd=3)),             # conversions, no such rounding
+               (True, _word(BINF, 8, IMM)), (False, _word(BINF, 10, IMM)), (True, _word(BINF, 0, 6)),      # logical, power, no such source
+               (True, _word(BINF, 0, SREG, a=8)), (False, _word(STS, a=8)), (True, _word(LDS, a=8)),
+               (True, _word(BINF, 3, SREG2, a=0, imm=8)), (True, _word(BINF, 3, SREG2, a=0, imm=8 << 8)), (True, _word(BINF, 0, REG, a=n_vslot - 1)),
+               (False, _word(CMP, 8, IMM)), (False, _word(CMP, 6, IMM)), (False, _word(ENDSWEEP)), (False, _word(ENDSWEEP, ends=True)), (True, _word(ENDSWEEP)),
+               (True, _word(RED, 3)), (True, _word(RED, 0x20)), (True, _word(RED, 0x11)), (True, _word(RED, 0x40, a=1)), (True, _word(RED, 0, a=2)),
+               (False, _word(FIN, a=2)), (False, _word(FIN, 0x20)), (False, _word(SWEEP, imm=3 | 15 << 4)),
+               (True, _word(BINF, 0, MEM, imm=PRE_SREG | 8)), (True, _word(BINF, 0, MEM, imm=PRE_SREG | 8 << 8))]
+    for in_sweep, w in refused:
+        assert status(in_sweep, w) == 1, hex(w)
