@@ -353,6 +353,8 @@ class Compiler {
   uint32_t FuseCubeEpilogue();
   void CompileAttn(int g);
   void DivideKeys();
+  size_t key_parts_bytes_ = 0;      // workspace of the attentions whose keys are divided between workgroups, in this attempt
+  bool key_parts_allowed_ = true;   // (false: with that workspace the kernel would no longer fit the static one)
   void BuildNodes(int a);
   void UnifyAxes();
   void OrderAndMerge();

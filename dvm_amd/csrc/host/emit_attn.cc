@@ -129,7 +129,8 @@ void Compiler::DivideKeys() {
     return us;
   };
   // What parts leave in memory stays a small share of the static workspace (DVM_HIP_STATIC_WS_BYTES), beside what the
-  // kernel's other values take: a kernel that fits it does so after the division too.
+  // sub-kernels before this one take. (Those behind it are not laid out yet: RunOnce compiles the kernel again without
+  // parts when it is they that no longer fit.)
   size_t taken = 0;
   for (size_t bytes : k_->ws_sizes_) taken += (bytes + 255) & ~static_cast<size_t>(255);
   auto part_bytes = [&](uint32_t n) { return static_cast<size_t>(h->nb) * n * h->sq * (h->d + 2) * 4; };
@@ -138,7 +139,7 @@ void Compiler::DivideKeys() {
     parts = std::min<uint32_t>(static_cast<uint32_t>(forced), (blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES);
   } else if (forced < 0) {
     double best = t_keys(1);
-    const uint32_t most = std::min<uint32_t>(32, (blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES);
+    const uint32_t most = key_parts_allowed_ ? std::min<uint32_t>(32, (blocks + DVM_ATTN_KEYS_WAVES - 1) / DVM_ATTN_KEYS_WAVES) : 1;
     for (uint32_t n = 2; n <= most; ++n) {
       if (part_bytes(n) > kPartBytes || taken + part_bytes(n) > DVM_HIP_STATIC_WS_BYTES) break;
       const double us = t_keys(n);
@@ -170,6 +171,7 @@ void Compiler::DivideKeys() {
   pp.ws_slot = static_cast<int>(k_->ws_sizes_.size());
   pp.role = Program::kPatchPlain;
   k_->ws_sizes_.push_back(part_bytes(parts));
+  key_parts_bytes_ += (part_bytes(parts) + 255) & ~static_cast<size_t>(255);
   prog_->patches.push_back(pp);
   const Program first = *prog_;
   k_->programs_.push_back(first);

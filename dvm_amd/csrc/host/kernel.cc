@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "../../../include/dvm_hip.h"
 #include "compiler.h"
 
 namespace dvm {
@@ -159,6 +160,7 @@ size_t Compiler::RunOnce(int mode) {
   k_->ws_sizes_.clear();
   k_->ws_offsets_.clear();
   PlanMaterialisation();
+  key_parts_bytes_ = 0;
   for (int a = 0; a < n_areas_; ++a) CompileArea(a);
   for (Program &p : k_->programs_)
     if (!p.skip) p.RememberBindDependent();
@@ -166,6 +168,17 @@ size_t Compiler::RunOnce(int mode) {
   for (size_t i = 0; i < k_->ws_sizes_.size(); ++i) {
     k_->ws_offsets_.push_back(total);
     total += (k_->ws_sizes_[i] + 255) & ~static_cast<size_t>(255);
+  }
+  // A kernel whose values fit the static workspace of the device library keeps fitting it: the keys of its attentions are
+  // then not divided between workgroups (unless the environment asks for the parts).
+  if (key_parts_allowed_ && key_parts_bytes_ > 0 && k_->tuning_.attn_keys < 0 && total > DVM_HIP_STATIC_WS_BYTES &&
+      total - key_parts_bytes_ <= DVM_HIP_STATIC_WS_BYTES) {
+    struct Restore {
+      bool &flag;
+      ~Restore() { flag = true; }
+    } restore{key_parts_allowed_};
+    key_parts_allowed_ = false;
+    return RunOnce(mode);
   }
   k_->ws_bytes_ = total;
   return total;

@@ -760,3 +760,28 @@ def test_a_wide_expression_tree_gets_more_registers_before_it_is_cut():
     t.store(acc)
     t.codegen()
     assert 1 < t.num_launches() <= 16, t.num_launches()
+
+
+def test_divided_keys_do_not_push_a_kernel_out_of_the_static_workspace():
+    # the partial outputs of an attention whose keys several workgroups divide are given up where, with the partial tiles of
+    # the products behind it, they would take the kernel past what dvm_hip_launch_vm_static_ws holds
+    limit = int(re.search(r"DVM_HIP_STATIC_WS_BYTES \((\d+)u \* 1024u \* 1024u\)", open(os.path.join(ROOT, "include", "dvm_hip.h")).read()).group(1)) << 20
+
+    def build(products):
+        t = Tester("mix", run_mode="das")
+        q, k, v = (t.load(np.zeros((16, n, 128), np.float16)) for n in (32, 2048, 2048))
+        x = t.cast(t.mul(t.matmul(q, k, False, True), 128 ** -0.5), "float32")
+        e = t.exp(t.sub(x, t.max(x, (2,), True)))
+        t.store(t.matmul(t.cast(t.div(e, t.sum(e, (2,), True)), "float16"), v, False, False))
+        for _ in range(products):  # 16 MiB of partial tiles each
+            t.store(t.matmul(t.load(np.zeros((1024, 4096), np.float16)), t.load(np.zeros((4096, 1024), np.float16)), False, False))
+        t.codegen()
+        return t
+
+    for products in (0, 1):
+        t = build(products)
+        assert "merge" in t.das() and t.workspace_bytes() <= limit and t.num_launches() == 2 + 2 * products, t.das()
+    t = build(2)
+    assert "waves divide the keys" in t.das() and "merge" not in t.das() and t.workspace_bytes() == limit and t.num_launches() == 5, t.das()
+    t = build(3)  # (past the limit with or without them)
+    assert "merge" in t.das() and t.num_launches() == 8, t.das()
