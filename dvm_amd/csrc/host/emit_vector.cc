@@ -708,9 +708,9 @@ bool Compiler::FinishProgram() {
   prog_->lds_bytes = DVM_VEC_RED_SCRATCH_DOUBLES(hdr_.sched, prog_->threads) * 8 + static_cast<uint32_t>(max_vslot_) * u_ * 16 * prog_->threads;
   // (pointwise programs without V registers keep the geometry they are exported with: a double per lane, which nothing reads)
   prog_->lds_bytes = std::max<uint32_t>(prog_->lds_bytes, 8 * prog_->threads);
-  const uint32_t lds_unparked = prog_->lds_bytes;
-  PlanRereads();
-  if (!row_code_.empty()) prog_->lds_bytes = lds_unparked;  // (the row build parks nothing)
+  // (the row build parks nothing; what the generic kernel runs in its place, where an operand does not even start on one of
+  // its elements, has its local memory)
+  if (row_code_.empty()) PlanRereads();
   uint64_t gt = (static_cast<uint64_t>(std::min<uint32_t>(hdr_.n_items, g_system.core_num * 4)) << 32) | prog_->threads;
   if (g_system.HasDevice()) {
     gt = g_system.Api().select_block_thread(hdr_.sched, hdr_.n_items, prog_->threads, prog_->lds_bytes);

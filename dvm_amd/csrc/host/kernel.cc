@@ -223,12 +223,16 @@ void VKernel::BindAddresses(const RelocEntry *relocs, size_t n, WsAllocator *all
       p.blob.w[pt.word] = addr;
       if ((addr & 15u) != 0) {
         if (pt.role == Program::kPatchVecMem) {
-          reinterpret_cast<VMemDesc *>(p.blob.w + pt.word)->flags &= ~static_cast<uint32_t>(VMF_ALIGNED);
-          // (the sweep build accesses the operands of its interior rounds without guards: the generic kernel runs instead)
+          VMemDesc *m = reinterpret_cast<VMemDesc *>(p.blob.w + pt.word);
+          m->flags &= ~static_cast<uint32_t>(VMF_ALIGNED);
+          // (the sweep build accesses the operands of its interior rounds without guards: the generic kernel runs instead;
+          // the row build takes rows that start at any element, but not inside one)
+          const uint64_t element = m->dtype == VDT_F32 ? 4 : 2;
           uint32_t sched;
           char *sched_at = reinterpret_cast<char *>(p.blob.w) + offsetof(VVecHeader, sched);
           std::memcpy(&sched, sched_at, sizeof(sched));
           sched &= ~static_cast<uint32_t>(VS_SWEEPS);
+          if ((addr & (element - 1)) != 0) sched &= ~static_cast<uint32_t>(VS_ROW_MASK);
           std::memcpy(sched_at, &sched, sizeof(sched));
         } else if (pt.role == Program::kPatchCubeOperand) {
           reinterpret_cast<VCubeHeader *>(p.blob.w)->fast = 0;

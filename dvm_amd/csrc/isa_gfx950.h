@@ -67,8 +67,8 @@ enum {
   // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.hip) may run the program from the words at
   // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space is one axis of n_ridx
   // groups, more than (slabs - 1) * team and at most slabs * team of them (team: the workgroup when team_is_block, else
-  // one wave), and holds at least eight elements. The words at code_off stay valid for the generic kernel at the same
-  // geometry, with the local memory the rounds they park need.
+  // one wave), and holds at least eight elements. The words at code_off are valid for the generic kernel at the same
+  // geometry: without these bits the blob runs there.
   VS_ROW_SHIFT = 8,
   VS_ROW_MASK = 0xf00,
 };

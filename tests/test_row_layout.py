@@ -184,3 +184,20 @@ def test_the_launch_check_takes_the_row_builds_vocabulary_and_nothing_else(monke
                (True, _word(BINF, 0, MEM, imm=PRE_SREG | 8)), (True, _word(BINF, 0, MEM, imm=PRE_SREG | 8 << 8))]
     for in_sweep, w in refused:
         assert status(in_sweep, w) == 1, hex(w)
+
+
+def test_rows_that_start_inside_an_element_keep_to_the_generic_kernel(monkeypatch):
+    """Packed memory with an operand at an odd byte: taken as before the row build existed, by the generic kernel at the same
+    geometry; bound to an element's address again, the kernel runs on the row build again."""
+    monkeypatch.delenv("DVM_VEC_ROW", raising=False)
+    t = Tester("split:dyn", run_mode="das")
+    x = t.load([-1, -1], "float32")
+    t.store(t.div(t.exp(x), t.sum(t.exp(x), (1,), True)))
+    for at, row in ((0x100000, True), (0x100004, True), (0x100002, False), (0x100001, False), (0x100004, True)):
+        t.bind_device(x, at, (2100, 1000))
+        t.codegen()
+        (blob, geometry, _), = t.programs()
+        sched, = struct.unpack_from("<I", blob, 4)
+        assert ((sched & 0xf00) != 0) == row == (" row=" in t.das()) and not (at & 15 and sched & 0x20), t.das()
+        if not dvm_amd.Device.available():
+            assert _launch_status(blob, geometry) != 1
