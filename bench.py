@@ -81,8 +81,12 @@ def bn_graph_two_pass(t, x, g, b, n_red, eps):
 
 def vector_kernel_name(das_text):
     """Name of the vector VM kernel a one-launch program runs on, from its disassembly header."""
+    import re
     head = das_text.split("\n")[1]
     if "sched=reduce-x" in head:
+        row = re.search(r" row=(\d+)", head)
+        if row:
+            return "dvm_vm_vec_row" + row.group(1)
         return "dvm_vm_vec_rx_sw" if " sweeps" in head else "dvm_vm_vec_rx"
     return "dvm_vm_vec_ry" if "sched=reduce-y" in head else "dvm_vm_vec_pw"
 

@@ -622,6 +622,11 @@ def test_sweep_build_is_chosen_from_the_instruction_words(monkeypatch):
     """Which programs carry VS_SWEEPS (isa_gfx950.h): those that reduce the innermost axis in sweeps of several
     rounds whose bodies are float chains behind one aligned, contiguous load."""
     monkeypatch.delenv("DVM_VEC_SWEEPS", raising=False)
+    # (rows that fit the row build's registers run there, and are called that)
+    monkeypatch.delenv("DVM_VEC_ROW", raising=False)
+    das = _row_norm(Tester("split", run_mode="das"), 8192, 4096)
+    assert "reduce-x row=" in das and "sweeps" not in das, das
+    monkeypatch.setenv("DVM_VEC_ROW", "0")
     assert "reduce-x sweeps" in _row_norm(Tester("split", run_mode="das"), 8192, 4096)
     assert "reduce-x sweeps" in _row_norm(Tester("split", run_mode="das"), 8192, 4096, "float16")
     assert "reduce-x sweeps" in _row_norm(Tester("split", run_mode="das"), 3, 100000)

@@ -5,7 +5,8 @@ accumulates per lane in the order of the rounds either way. Each graph is also c
 form. Shapes cover rows of one wave and of a whole workgroup, several rows per wave, ragged last rounds, rounds
 that are empty for some waves, two reduced axes (a channel of an NCHW tensor) and reduces shared between workgroups.
 
-The host's decision (which programs carry the flag) is checked without a GPU in test_host.py."""
+The row build is switched off throughout (DVM_VEC_ROW=0): rows that fit its registers would run there, on words of their
+own (test_parity_rows.py). The host's decision (which programs carry the flag) is checked without a GPU in test_host.py."""
 import numpy as np
 import pytest
 
@@ -15,6 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(monkeypatch, sweeps, build, ker="split"):
+    monkeypatch.setenv("DVM_VEC_ROW", "0")
     if sweeps:
         monkeypatch.delenv("DVM_VEC_SWEEPS", raising=False)
     else:
@@ -22,6 +24,7 @@ def _run(monkeypatch, sweeps, build, ker="split"):
     t = Tester(ker)
     outs = build(t)
     t.run()
+    assert " row=" not in t.das() and (sweeps or " sweeps" not in t.das()), t.das()
     return [t.output(o) for o in outs], t.das()
 
 
