@@ -493,7 +493,7 @@ bool Compiler::BuildRowCode() {
           return false;
       }
       uint64_t out = plain(b) | (static_cast<uint32_t>(b) & VI_ENDS);
-      if (bop == VOP_LD && j < last && VI_OP(code_[j + 1]) == VOP_BINF && VI_KIND(code_[j + 1]) == VK_MEM && !(VI_IMM(code_[j + 1]) & VI_PRE_SREG)) {
+      if (bop == VOP_LD && k_->tuning_.vec_pair != 0 && j < last && VI_OP(code_[j + 1]) == VOP_BINF && VI_KIND(code_[j + 1]) == VK_MEM && !(VI_IMM(code_[j + 1]) & VI_PRE_SREG)) {
         const VMemDesc &ma = mems_[VI_A(b)], &mb = mems_[VI_A(code_[j + 1])];
         if (ma.dtype == mb.dtype && ma.dtype != VDT_F32 && row_mem(VI_A(code_[j + 1]))) out |= VI_LD_PAIR;
       }

@@ -3,7 +3,8 @@ trip (VI_LD_PAIR), the load of a statistics sweep that fetches two rounds per tr
 and rounds parked behind the instruction two sweeps share (VI_LD_KEEP_* with a prefix). Each is an optimisation of
 the interpreter only: with DVM_VEC_PAIR=0 the same programs run instruction by instruction, and both must give
 the same bits (the reduce accumulates in the order of the rounds either way) and agree with the float64 closed
-forms. Shapes are chosen so that sweeps have one, two, odd and even numbers of rounds and ragged last rounds."""
+forms. Shapes are chosen so that sweeps have one, two, odd and even numbers of rounds and ragged last rounds.
+The row build is switched off (DVM_VEC_ROW=0): it runs words of its own in one round; its pairs are compared at the end."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ from dvm_amd.tester import Tester
 pytestmark = pytest.mark.gpu
 
 
-def _run(monkeypatch, pair, build):
+def _run(monkeypatch, pair, build, row="0"):
+    monkeypatch.setenv("DVM_VEC_ROW", row)
     if pair:
         monkeypatch.delenv("DVM_VEC_PAIR", raising=False)
     else:
@@ -20,6 +22,7 @@ def _run(monkeypatch, pair, build):
     t = Tester("split")
     outs = build(t)
     t.run()
+    assert (" row=" in t.das()) == (row != "0"), t.das()
     return [t.output(o) for o in outs], t.das()
 
 
@@ -138,10 +141,36 @@ def test_an_s_register_binary_in_front_of_a_memory_binary_is_one_instruction():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     res = {}
     for fuse in ("1", "0"):
-        env = dict(os.environ, DVM_VEC_FUSE=fuse, PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""))
+        env = dict(os.environ, DVM_VEC_FUSE=fuse, DVM_VEC_ROW="0", PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""))
         p = subprocess.run([sys.executable, "-c", _PRE_SREG_SCRIPT], env=env, cwd=root, capture_output=True, text=True, timeout=100)
         assert p.returncode == 0, p.stderr[-2000:]
         n, digest = p.stdout.split()
         res[fuse] = (int(n), digest)
     assert res["1"][0] >= 3 and res["0"][0] == 0, res  # (one of the four forms may come out with its operands the other way round)
     assert res["1"][1] == res["0"][1]
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 4096), (700, 4096), (4100, 4096), (33, 1000), (4, 24000), (300, 5001)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_row_build_pairs(monkeypatch, rows, cols, dtype):
+    # the row build's own pairs (two 16-bit rows in one trip; DVM_DEBUG prints the words it runs): the same bits as one
+    # after the other
+    monkeypatch.setenv("DVM_DEBUG", "1")
+    rng = np.random.default_rng(rows + cols)
+    xs, rs = (rng.standard_normal([rows, cols], dtype=np.float32) for _ in range(2))
+    xs, rs = (Tester.convert_to_bf16(v) if dtype == "bfloat16" else v.astype(dtype) for v in (xs, rs))
+
+    def build(t):
+        x, r = t.load(xs.shape, dtype), t.load(rs.shape, dtype)
+        t.input(x, xs)
+        t.input(r, rs)
+        hf = t.cast(t.add(x, r), "float32")
+        return [t.store(t.div(hf, t.sum(t.abs(hf), (1,), True)))]
+
+    (a,), das_on = _run(monkeypatch, True, build, row="8")
+    (b,), das_off = _run(monkeypatch, False, build, row="8")
+    on, off = (d.split("row build:")[1] for d in (das_on, das_off))
+    assert "in the same trip" in on and "in the same trip" not in off, das_on
+    assert np.array_equal(a, b)
+    h64 = (Tester.convert_from_bf16(Tester.convert_to_bf16(Tester.convert_from_bf16(xs) + Tester.convert_from_bf16(rs))) if dtype == "bfloat16" else xs + rs).astype(np.float64)
+    assert np.allclose(a, h64 / np.abs(h64).sum(1, keepdims=True), rtol=2e-6, atol=0)
