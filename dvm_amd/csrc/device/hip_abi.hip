@@ -117,12 +117,7 @@ __global__ void dvm_fill_u32_kernel(uint32_t *dst, uint32_t value, size_t n) {
 // registers). The grid is a multiple of what is resident: one workgroup too many per CU costs a whole extra pass.
 uint32_t kernel_waves_per_simd(uint64_t kind) {
   if (kind & VS_WIDE) return 2;
-  switch (DVM_VEC_ROW_SLABS(kind)) {  // (from the builds' register counts, as below)
-    case 0: break;
-    case 1: case 2: return 5;
-    case 3: case 4: return 4;
-    default: return 2;
-  }
+  if (const uint32_t slabs = DVM_VEC_ROW_SLABS(kind)) return DVM_VEC_ROW_WAVES(slabs);
   switch (kind & VS_KIND_MASK) {
     case VS_POINTWISE: return 5;
     case VS_REDX: return 4;
@@ -202,7 +197,7 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
 uint64_t dvm_hip_select_block_thread(uint64_t kind, uint64_t item_num, uint64_t threads, uint32_t lds_bytes) {
   if (threads == 0) threads = 256;
   const uint64_t waves_per_wg = (threads + 63) / 64;
-  uint64_t wg_per_cu = (4ull * kernel_waves_per_simd(kind)) / waves_per_wg;
+  uint64_t wg_per_cu = DVM_WG_PER_CU(kernel_waves_per_simd(kind), waves_per_wg);
   if (lds_bytes > 0) {
     // (beside the launch's local memory every workgroup has its copy of the program. Without it in the sum, three
     // workgroups of 51200 bytes counted as resident where two are, and a third of the grid ran as a pass of its own: the

@@ -394,6 +394,7 @@ class Compiler {
   void PlanRereads();
   bool FitsSweepBuild();
   bool RowCandidate() const;
+  bool ReadsAlignedRowsOnce() const;
   uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;
   bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;
   bool BuildRowCode();

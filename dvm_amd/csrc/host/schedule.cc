@@ -512,24 +512,60 @@ uint64_t Compiler::RowKey(uint32_t slabs, uint32_t lanes) const {
   return h;
 }
 
-// Slabs and lanes per row. More slabs a lane mean fewer waves per row: less scalar work between the sweeps, fewer
-// decodes per element, and from one wave per row on no barrier; but the chip wants some 2^17 lanes (two waves per SIMD)
-// in flight before it gives any up. Only the last slab of a row may be ragged. Measured on MI355X (times of a call, us;
-// without the row build / 2 / 4 / 8 slabs): residual RMSNorm bf16 [8192,4096] 63 / 57 / 54 / 51, [8192,8192] 116 / 120 /
-// 93 / 92, softmax fp32 [8192,4096] 87 / 76 / 72 / 68, [4096,16384] 192 / 179 / 139 / 137, [2048,32001] 535 / - / 152 /
-// 164; 37 rows of 4096 take the kernel 10.8 -> 7.7 us.
+// Whether nothing that varies along the reduced axis comes behind a reduce (a row sum: there is nothing to keep in
+// registers), and every row starts on 16 bytes (the other builds' fast paths).
+bool Compiler::ReadsAlignedRowsOnce() const {
+  bool behind[kMaxNodes];
+  for (int i = 0; i < nn_; ++i) {
+    const ANode &n = nodes_[i];
+    behind[i] = n.kind == AK_REDUCE;
+    bool in_sweep = false;
+    for (int j = 0; j < n.nin; ++j) {
+      if (n.in[j] < 0) continue;
+      behind[i] = behind[i] || behind[n.in[j]];
+      if (n.kind == AK_REDUCE && behind[n.in[j]]) return false;
+    }
+    for (int d = 0; d < n.rank; ++d) in_sweep = in_sweep || (n.axis[d] >= 0 && axes_[n.axis[d]].reduced);
+    if (!in_sweep) continue;
+    if (behind[i]) return false;
+    if (n.kind == AK_MEM && (n.view != nullptr || hdr_.inner_extent * DTypeSize(n.dtype) % 16 != 0)) return false;
+  }
+  return true;
+}
+
+// Slabs and lanes per row. A row's loads are in flight at once, so what counts is how many rows a compute unit holds at a
+// time: more slabs a lane (fewer waves a row) are taken where they raise it, and while there are rows for some 2^17 lanes
+// (two waves per SIMD) all the same. Where they do not raise it (their registers cost the waves they save, or the
+// workgroup's waves do not pack) the fewer slabs keep more lanes on the row; only eight slabs come before four at the same
+// number of rows from the fourth pass over the chip on (the build of four saves 19 registers a lane to scratch memory).
+// Only the last slab of a row may be ragged. Measured on MI355X (times of a launch, us; without the row build / with the
+// most slabs there are rows for / by this rule): log-sum-exp bf16 [1068,13440] 38 / 43 / 27, fp32 [2340,7168] 34 / 41 / 30,
+// softmax bf16 [1034,7680] 37 / 25 / 21, fp32 [2048,32001] 531 / 169 / 159, [8192,4096] 86 / 67 / 66, [4096,16384] 199 / 147
+// / 148, layer norm of a stored sum bf16 [2097,6272] 72 / 52 / 38, residual RMSNorm bf16 [8192,4096] 51 / 44 / 44, 37 rows
+// 12.1 / 9.3 / 9.2. Over 1336 drawn programs the rule is 0.4 % off the best number of slabs, the most slabs were 1.4 %. What
+// is left: at one row a unit and three to four passes a program that reads its row twice can be 5 to 13 % slower than in
+// rounds (log-sum-exp fp32 [840,19968] 35 / 36 / 40, RMSNorm bf16 [936,17920] 33 / 37 / 35), one that reads it three times
+// or computes more on it is up to twice as fast.
 bool Compiler::ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const {
   if (n_r <= 32) return false;  // (up to 256 elements: several rows share a wave on the other builds)
+  const uint64_t cus = g_system.core_num > 0 ? g_system.core_num : 256;
   uint32_t best = 0, best_team = 0;
+  uint64_t best_rows = 0;  // per compute unit
   for (uint32_t u = 1; u <= 8; ++u) {
     if (!DVM_VEC_ROW_OK(u) || (k_->tuning_.vec_row > 0 && u > static_cast<uint32_t>(k_->tuning_.vec_row))) continue;
     const uint64_t t = ((n_r + u - 1) / u + 63) / 64 * 64;
     if (t > DVM_VEC_ROW_LANES(u) || n_r <= t * (u - 1)) continue;
     if (best != 0 && n_k * t < (1ull << 17)) break;  // (more slabs would leave lanes idle)
+    const uint64_t rows = t > 64 ? DVM_WG_PER_CU(DVM_VEC_ROW_WAVES(u), t / 64) : 4ull * DVM_VEC_ROW_WAVES(u);
+    if (rows < best_rows || (rows == best_rows && !(u == 8 && best == 4 && rows > 1 && n_k > 3 * rows * cus))) continue;
     best = u;
     best_team = static_cast<uint32_t>(t);
+    best_rows = rows;
   }
   if (best == 0) return false;
+  // (one or two rows at a time are a trip to memory with nothing under it. Where rows are kept for a second sweep that still
+  // pays; a row sum at [1297,12928] in fp16 takes 17.0 us here and 14.6 in rounds, [589,28444] in fp32 22.2 and 19.2)
+  if (best_rows <= 2 && n_k > 2 * best_rows * cus && ReadsAlignedRowsOnce()) return false;
   *slabs = best;
   *team = best_team;
   return true;

@@ -77,6 +77,13 @@ enum {
 // slabs a lane the row build exists for, and the lanes a workgroup of that build may have
 #define DVM_VEC_ROW_OK(slabs) ((slabs) >= 1u && (slabs) <= 8u && (slabs) != 7u)
 #define DVM_VEC_ROW_LANES(slabs) ((slabs) <= 4u ? 1024u : 512u)
+// waves a SIMD that build's registers leave room for (79, 95, 128, 128, 167, 200 and 255 of 512)
+#define DVM_VEC_ROW_WAVES(slabs) ((slabs) <= 2u ? 5u : ((slabs) <= 4u ? 4u : ((slabs) == 5u ? 3u : 2u)))
+// Workgroups of `waves` waves a compute unit holds at `per_simd` waves on each of its four SIMDs. Up to four waves are
+// placed as they come; a larger workgroup is dealt out round robin and needs room for ceil(waves / 4) on one SIMD: five
+// waves to a workgroup leave room for two at four waves a SIMD, not for three, and for one at three. (Measured on MI355X
+// with workgroups that only wait: 1 to 16 waves at 2 to 5 waves a SIMD; only five at five hold one more.)
+#define DVM_WG_PER_CU(per_simd, waves) ((waves) <= 4u ? 4u * (per_simd) / (waves) : (per_simd) / (((waves) + 3u) / 4u))
 #define DVM_VEC_SWEEP_BODY 6
 // Local memory at the start of a vector program's segment, in doubles: what the lanes of a workgroup combine their
 // reduce partials through. One double per lane; eight (one per element of a lane's group) on the schedule that keeps

@@ -201,3 +201,38 @@ def test_rows_that_start_inside_an_element_keep_to_the_generic_kernel(monkeypatc
         assert ((sched & 0xf00) != 0) == row == (" row=" in t.das()) and not (at & 15 and sched & 0x20), t.das()
         if not dvm_amd.Device.available():
             assert _launch_status(blob, geometry) != 1
+
+
+def _softmax(t, rows, cols, dtype):
+    v = _wide(t, _load(t, (rows, cols), dtype), dtype)
+    e = t.exp(t.sub(v, t.max(v, (1,), True)))
+    return [t.div(e, t.sum(e, (1,), True))]
+
+
+def _row_sum(t, rows, cols, dtype):
+    return [t.sum(_wide(t, _load(t, (rows, cols), dtype), dtype), (1,), True)]
+
+
+@pytest.mark.parametrize("graph,rows,cols,dtype,slabs,lanes", [
+    (_softmax, 37, 4096, "float32", 1, 512), (_softmax, 1034, 7680, "bfloat16", 4, 256), (_softmax, 1068, 13440, "bfloat16", 4, 448),
+    (_softmax, 2340, 7168, "float32", 4, 256), (_softmax, 2048, 32001, "float32", 4, 1024), (_softmax, 8192, 4096, "float32", 8, 256),
+    (_softmax, 4096, 16384, "float32", 8, 256), (_softmax, 700, 17920, "float32", 3, 768), (_softmax, 5000, 2560, "float32", 5, 256),
+    # a row that is read once: in rounds where a compute unit would hold one or two rows, more than two passes over the chip
+    (_row_sum, 1297, 12928, "float16", 0, None), (_row_sum, 589, 28444, "float32", 0, None), (_row_sum, 500, 28444, "float32", 4, 896),
+    (_row_sum, 589, 28443, "float32", 4, 896), (_row_sum, 589, 28444, "float16", 4, 896), (_row_sum, 2692, 6232, "float32", 4, 256)])
+def test_slabs_and_lanes_of_a_row(monkeypatch, graph, rows, cols, dtype, slabs, lanes):
+    """The layout that keeps the most rows on a compute unit (ChooseRow in schedule.cc)."""
+    monkeypatch.delenv("DVM_VEC_ROW", raising=False)
+    das = _compile(graph, rows, cols, dtype).das()
+    assert (" row=%d " % slabs in das and " threads=%d " % lanes in das) if slabs else " row=" not in das, das
+
+
+@pytest.mark.parametrize("slabs,waves,groups", [(1, 2, 10), (1, 13, 1), (2, 3, 6), (2, 4, 5), (2, 7, 2), (3, 3, 5), (3, 5, 2), (3, 9, 1), (4, 4, 4), (4, 6, 2),
+                                                (4, 7, 2), (4, 8, 2), (4, 16, 1), (5, 2, 6), (5, 3, 4), (5, 4, 3), (5, 5, 1), (5, 6, 1), (6, 3, 2), (6, 5, 1), (8, 2, 4), (8, 4, 2), (8, 8, 1)])
+def test_workgroups_a_compute_unit_holds(slabs, waves, groups):
+    """The grid is what is resident at once: a workgroup of more than four waves needs ceil(waves / 4) of a SIMD's places."""
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(dvm_amd.__file__), "lib", "libdvm_hip.so"))
+    lib.dvm_hip_select_block_thread.restype = ctypes.c_uint64
+    lib.dvm_hip_select_block_thread.argtypes = [ctypes.c_uint64, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_uint32]
+    one = lib.dvm_hip_select_block_thread(1 | 8 << 8, 1 << 30, 512, 1024) >> 32  # (eight waves of eight slabs: one workgroup a unit)
+    assert lib.dvm_hip_select_block_thread(1 | slabs << 8, 1 << 30, 64 * waves, 512 * waves) >> 32 == groups * one
