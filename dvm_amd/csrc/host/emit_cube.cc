@@ -329,9 +329,9 @@ void Compiler::CompileCube(int a) {
   // from figures measured on MI355X (bf16, microseconds): a workgroup's time per 64 k (2.2 for the 256 tile, 1.3 for
   // 128, 0.71 for 64 alone on its compute unit and 0.9 when two share one; the guarded path of ragged or unaligned
   // tiles takes about two and a half times as long), rounds of workgroups over the chip, and for a split the second launch plus
-  // the time its one workgroup per tile needs per partial tile (3.2 / 0.8 / 0.2 with the vectors of several parts in
-  // flight together: a single workgroup streams at some 80 GB/s), which is what keeps deep splits of big tiles from
-  // paying, plus the time the first launch takes to write the partial tiles (some 4 TB/s over the whole chip).
+  // a time per part of a tile (3.2 / 0.8 / 0.2), plus the time the first launch takes to write the partial tiles (some
+  // 4 TB/s over the whole chip). The times per part were measured while one workgroup summed a tile (some 80 GB/s); the
+  // sum in pieces below costs less for the two larger tiles, so deep splits of those are chosen less often than would pay.
   uint32_t k_split = 1, k_chunk = 0;
   {
     const int forced = gmm != 0 ? 0 : k_->tuning_.cube_splitk;  // (the k axis of a grouped product is never shared)
@@ -570,8 +570,9 @@ void Compiler::CompileCube(int a) {
     k_->programs_.push_back(first);
     prog_ = &k_->programs_.back();
     reinterpret_cast<VCubeHeader *>(prog_->blob.w)->epi_flags = flags | VCF_SPLITK_COMBINE;
-    // pieces of 64 x 64 whatever the tile, and no more workgroups than run at once (four per compute unit): what a
-    // piece costs beside its bytes is its workgroup's start
+    // Pieces of 64 x 64 whatever the tile; a workgroup takes several where there are more than four per compute unit: what
+    // a piece costs beside its bytes is its workgroup's start. (Three run at once, 167 registers a lane: of a full grid
+    // every fourth starts when an earlier one ends.)
     prog_->threads = 256;
     prog_->lds_bytes = DVM_CUBE_LDS_BYTES(64u);
     prog_->grid = static_cast<uint32_t>(std::min<uint64_t>(tiles(bt) * static_cast<uint64_t>(bt / 64) * (bt / 64), 4 * cus));

@@ -49,3 +49,19 @@ def test_pieces_of_a_transposed_window(monkeypatch, tile, waves, parts):
     t.run()
     assert "split-k sum of " + parts in t.das() and "fast" in t.das(), t.das()
     assert np.array_equal(t.output(out).astype(np.float64), a[:, :m].T.astype(np.float64) @ b.astype(np.float64))
+
+
+@pytest.mark.parametrize("parts", [2, 3, 4, 5, 6, 7, 8, 11])
+@pytest.mark.parametrize("m", [8, 15, 17, 24, 25, 32, 40, 57])
+def test_pieces_by_number_of_parts_and_groups_of_rows(monkeypatch, m, parts):
+    # whole fours of parts and each remainder, one to four groups of eight rows in a fragment and none
+    monkeypatch.setenv("DVM_CUBE_TILE", "64")
+    monkeypatch.setenv("DVM_CUBE_SPLITK", str(parts))
+    k, n = 64 * parts, 136
+    rng = np.random.default_rng(m * 100 + parts)
+    a, b = _ints(rng, m, k), _ints(rng, k, n)
+    t = Tester("mix")
+    out = t.store(t.matmul(t.load(a), t.load(b), False, False))
+    t.run()
+    assert "split-k sum of %d " % parts in t.das(), t.das()
+    assert np.array_equal(t.output(out).astype(np.float64), a.astype(np.float64) @ b.astype(np.float64))
