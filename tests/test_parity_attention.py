@@ -41,12 +41,26 @@ def test_attention_example_small():  # examples/03_attention.py:52-63: too small
                golden=np_attention(q, k, v).astype(np.float16), eps=1e-2)
 
 
-def _fused(q, k, v, dt="float16"):
+@pytest.fixture(params=["0", "1"], ids=["waves divide the queries", "waves divide the keys"])
+def keys(request, monkeypatch):
+    """Runs a test on both kinds of attention kernel (few queries, or few heads, go to the one whose waves divide the keys)."""
+    monkeypatch.delenv("DVM_ATTN_WAVES", raising=False)
+    monkeypatch.setenv("DVM_ATTN_KEYS", request.param)
+    return request.param == "1"
+
+
+def _on(keys, t):
+    assert "entry attention" in t.das() and ("waves divide the keys" in t.das()) == keys, t.das()
+
+
+def _fused(q, k, v, dt="float16", keys=None):
     t = Tester("mix")
     dts = dt if dt == "bfloat16" else None
     out = t.store(attention_graph(t, t.load(q, dts), t.load(k, dts), t.load(v, dts), 1.0 / math.sqrt(q.shape[-1]), q.ndim, dt))
     t.run()
     assert "entry attention" in t.das() and t.num_launches() == 1, t.das()
+    if keys is not None:
+        _on(keys, t)
     o = t.output(out)
     return Tester.convert_from_bf16(o) if dt == "bfloat16" else o
 
@@ -68,29 +82,29 @@ def test_attention_fused(monkeypatch, shape, dt, waves):
 
 @pytest.mark.parametrize("dt", ["float16", "bfloat16"])
 @pytest.mark.parametrize("spread,d", [(20.0, 128), (20.0, 64), (0.0, 128), (6.0, 64)])
-def test_attention_sharp_and_flat_softmax(dt, spread, d):
+def test_attention_sharp_and_flat_softmax(keys, dt, spread, d):
     # scores hundreds apart (the weights of a row are one key's, the rest underflow) and scores all equal
     rng = np.random.default_rng(int(spread) + d)
     conv = (lambda x: x.astype(np.float16)) if dt == "float16" else _bf16
     q, k, v = (conv(rng.standard_normal((2, n, d)) * s) for n, s in ((300, spread), (520, spread), (520, 1.0)))
     if spread > 0:
         k[:, 7, :] = q[:, 0, :]  # query 0 has one key far above the rest
-    got, want = _fused(q, k, v, dt), np_attention(q, k, v)
+    got, want = _fused(q, k, v, dt, keys), np_attention(q, k, v)
     assert not np.isnan(got).any()
     assert np.allclose(got, want, rtol=2e-2, atol=2e-2), np.abs(got - want).max()
 
 
-def test_attention_fused_constant_values_and_key_order():
+def test_attention_fused_constant_values_and_key_order(keys):
     # softmax weights sum to one: with every row of V equal to c the output rows are c, at any size;
     # and the result does not depend on the order of the keys
     rng = np.random.default_rng(5)
     q, k = (rng.standard_normal((4, 512, 128)).astype(np.float16) for _ in range(2))
     c = rng.standard_normal(128).astype(np.float16)
-    got = _fused(q, k, np.broadcast_to(c, (4, 512, 128)).copy())
+    got = _fused(q, k, np.broadcast_to(c, (4, 512, 128)).copy(), keys=keys)
     assert np.allclose(got, c, rtol=2e-3, atol=2e-3)
     v = rng.standard_normal((4, 512, 128)).astype(np.float16)
     perm = rng.permutation(512)
-    a, b = _fused(q, k, v), _fused(q, k[:, perm], v[:, perm])
+    a, b = _fused(q, k, v, keys=keys), _fused(q, k[:, perm], v[:, perm], keys=keys)
     assert np.allclose(a, b, rtol=5e-3, atol=5e-3)
 
 
@@ -104,7 +118,7 @@ def test_attention_full_size_heads():  # BASELINE config 4 shape, three sampled 
 
 
 @pytest.mark.parametrize("dt", ["float16", "bfloat16"])
-def test_attention_fused_with_the_scale_behind_the_cast(dt):
+def test_attention_fused_with_the_scale_behind_the_cast(keys, dt):
     # the same graph with the scores scaled in fp32 (cast first, then the multiply): recognised as well
     rng = np.random.default_rng(77)
     conv = (lambda x: x.astype(np.float16)) if dt == "float16" else _bf16
@@ -117,6 +131,7 @@ def test_attention_fused_with_the_scale_behind_the_cast(dt):
     out = t.store(t.matmul(t.cast(t.div(e, t.sum(e, (2,), True)), dt), lv, False, False))
     t.run()
     assert "entry attention" in t.das() and t.num_launches() == 1, t.das()
+    _on(keys, t)
     got = t.output(out)
     got = Tester.convert_from_bf16(got) if dt == "bfloat16" else got
     want = np_attention(q, k, v)
@@ -139,16 +154,16 @@ def test_attention_fused_head_dimension_64(monkeypatch, shape, dt, waves):
     assert np.allclose(got, want, rtol=1e-2, atol=1e-2), np.abs(got - want).max()
 
 
-def test_attention_head_dimension_64_constant_values():
+def test_attention_head_dimension_64_constant_values(keys):
     # every row of V equal to c: the output rows are c whatever the scores; V = one-hot rows pick out softmax weights
     rng = np.random.default_rng(5)
     q, k = (rng.standard_normal((2, n, 64)).astype(np.float16) for n in (130, 192))
     v = np.tile(np.linspace(-1, 1, 64, dtype=np.float16), (2, 192, 1))
-    got = _fused(q, k, v)
+    got = _fused(q, k, v, keys=keys)
     assert np.allclose(got, v[:, :1, :].astype(np.float32), atol=2e-3), np.abs(got - v[:, :1, :]).max()
     v = np.zeros((2, 192, 64), np.float16)
     v[:, np.arange(64) * 3, np.arange(64)] = 1.0  # output column d = weight of key 3 d
-    got = _fused(q, k, v).astype(np.float64)
+    got = _fused(q, k, v, keys=keys).astype(np.float64)
     s = np.matmul(q.astype(np.float64), np.swapaxes(k.astype(np.float64), -1, -2)) / 8.0
     w = np.exp(s - s.max(-1, keepdims=True))
     w /= w.sum(-1, keepdims=True)
@@ -174,7 +189,7 @@ def test_attention_fused_with_a_short_last_block_of_keys(monkeypatch, waves, d, 
 
 @pytest.mark.parametrize("b,s,h,d", [(2, 320, 4, 128), (1, 200, 3, 64), (2, 512, 2, 128)])
 @pytest.mark.parametrize("how", ["view_load", "permute"])
-def test_attention_on_sequence_major_tensors_read_heads_first(b, s, h, d, how):
+def test_attention_on_sequence_major_tensors_read_heads_first(keys, b, s, h, d, how):
     # q, k, v stored [batch, seq, heads, d] and read as [batch, heads, seq, d]; the result is dense, heads first
     rng = np.random.default_rng(b * 1000 + s + h)
     q, k, v = (rng.standard_normal((b, s, h, d)).astype(np.float16) for _ in range(3))
@@ -187,11 +202,12 @@ def test_attention_on_sequence_major_tensors_read_heads_first(b, s, h, d, how):
     out = t.store(attention_graph(t, lq, lk, lv, 1.0 / math.sqrt(d), 4))
     t.run()
     assert "entry attention" in t.das() and "view, strides" in t.das() and t.num_launches() == 1, t.das()
+    _on(keys, t)
     want = np_attention(q.transpose(0, 2, 1, 3), k.transpose(0, 2, 1, 3), v.transpose(0, 2, 1, 3))
     assert np.allclose(t.output(out), want, rtol=1e-2, atol=1e-2)
 
 
-def test_attention_on_a_window_of_a_longer_key_value_cache():
+def test_attention_on_a_window_of_a_longer_key_value_cache(keys):
     # k, v are the first skv rows of a cache [heads, 1024, d]; q dense (a dense operand beside views)
     rng = np.random.default_rng(77)
     hds, sq, skv, d, cap = 6, 128, 333, 128, 1024
@@ -203,6 +219,7 @@ def test_attention_on_a_window_of_a_longer_key_value_cache():
     out = t.store(attention_graph(t, t.load(q), lk, lv, 1.0 / math.sqrt(d), 3))
     t.run()
     assert "entry attention" in t.das() and t.num_launches() == 1, t.das()
+    _on(keys, t)
     assert np.allclose(t.output(out), np_attention(q, kc[:, :skv], vc[:, 8:8 + skv]), rtol=1e-2, atol=1e-2)
 
 
@@ -225,7 +242,7 @@ def test_attention_views_the_kernel_cannot_walk_run_unfused():
 @pytest.mark.parametrize("b,s,h,d", [(2, 320, 4, 128), (1, 200, 3, 64), (2, 512, 2, 128)])
 @pytest.mark.parametrize("how", ["permute_store", "view_store"])
 @pytest.mark.parametrize("operands", ["dense", "views"])
-def test_attention_result_written_sequence_major(b, s, h, d, how, operands):
+def test_attention_result_written_sequence_major(keys, b, s, h, d, how, operands):
     # the result [batch, heads, seq, d] goes to memory as [batch, seq, heads, d] (what the projection behind an
     # attention reads), as the dense Store of a Permute or as a Store with a stride list: one launch either way
     rng = np.random.default_rng(b * 1000 + s + h + 5)
@@ -248,10 +265,11 @@ def test_attention_result_written_sequence_major(b, s, h, d, how, operands):
         t.run()
         got = t.output(out, (b, s, h, d))
     assert "entry attention" in t.das() and "o: view, strides row=%d" % (h * d) in t.das() and t.num_launches() == 1, t.das()
+    _on(keys, t)
     assert got.shape == (b, s, h, d) and np.allclose(got, want.transpose(0, 2, 1, 3), rtol=1e-2, atol=1e-2)
 
 
-def test_attention_result_into_a_padded_buffer_and_results_the_kernel_cannot_place():
+def test_attention_result_into_a_padded_buffer_and_results_the_kernel_cannot_place(keys):
     rng = np.random.default_rng(91)
     hds, s, d = 3, 200, 128
     q, k, v = (rng.standard_normal((hds, s, d)).astype(np.float16) for _ in range(3))
@@ -261,6 +279,7 @@ def test_attention_result_into_a_padded_buffer_and_results_the_kernel_cannot_pla
     out = t.view_store(attention_graph(t, t.load(q), t.load(k), t.load(v), 1.0 / math.sqrt(d), 3), [s * 160, 160, 1], hds * s * 160)
     t.run()
     assert t.num_launches() == 1 and "o: view, strides row=160" in t.das(), t.das()
+    _on(keys, t)
     got = t.output(out, (hds, s, 160))
     assert np.allclose(got[:, :, :d], want, rtol=1e-2, atol=1e-2) and not got[:, :, d:].any()
     # a transposing permute of the result (the head dimension no longer innermost) is a copy behind the kernel
