@@ -79,3 +79,45 @@ def test_nothing_is_written_past_a_ragged_row():
     v = t.load(x)
     t.view_store_expect(t.sub(v, t.max(v, (1,), True)), (pitch, 1), want, 0)
     assert t.run_check()
+
+
+@pytest.mark.parametrize("b,h,cols", [(3, 5, 264), (7, 3, 1003), (2, 9, 4096), (70, 31, 513), (61, 37, 4090), (1, 6, 12289), (257, 3, 300)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_two_kept_axes(b, h, cols, dtype):
+    """Rows numbered by two axes that do not merge: operands broadcast along either of them, one value per row of either, and
+    the result of every row stored."""
+    x, m = _inputs(b * h, cols, dtype, b * 7 + cols).reshape(b, h, cols), _inputs(b, cols, dtype, 3).reshape(b, 1, cols)
+    g = _inputs(h, cols, "float32", 4).reshape(1, h, cols)
+    rng = np.random.default_rng(h)
+    s, o = rng.uniform(0.5, 1.5, [1, h, 1]).astype(np.float32), rng.uniform(-1.0, 1.0, [b, 1, 1]).astype(np.float32)
+    t = Tester("split")
+    wide = (lambda v: v) if dtype == "float32" else (lambda v: t.cast(v, "float32"))
+    z = t.add(t.add(t.mul(wide(_load(t, x, dtype)), t.load(s)), wide(_load(t, m, dtype))), t.load(o))
+    top = t.max(z, (2,), True)
+    e = t.exp(t.sub(z, top))
+    p = t.mul(t.div(e, t.sum(e, (2,), True)), t.load(g))
+    outs = [t.store(p), t.store(top)]
+    t.run()
+    kdims = ("  kdims: %d %d" % (h, b)) if b > 1 else "  kdims: %d" % h
+    assert " row=" in t.das() and kdims in t.das(), t.das()
+    x64, m64 = _f64(x.reshape(b * h, cols), dtype).reshape(b, h, cols), _f64(m.reshape(b, cols), dtype).reshape(b, 1, cols)
+    z32 = ((x64.astype(np.float32) * s + m64.astype(np.float32)) + o)  # (rounded operator by operator, as the program does)
+    e64 = np.exp(z32.astype(np.float64) - z32.max(2, keepdims=True))
+    assert np.array_equal(t.output(outs[1]), z32.max(2, keepdims=True))
+    # (the difference inside exp is rounded to fp32: half a unit in the last place of at most 16)
+    assert np.allclose(t.output(outs[0]), e64 / e64.sum(2, keepdims=True) * g, rtol=4e-6, atol=0)
+
+
+@pytest.mark.parametrize("b,h,cols", [(5, 7, 1000), (3, 40, 1021), (50, 45, 2048)])
+def test_rows_read_and_written_through_strides(b, h, cols):
+    """[h, b, cols] in memory read as [b, h, cols] and the result written as [h, b, cols + 3]: both kept axes with strides of
+    their own, rows that start at any element, nothing written between them."""
+    x = _inputs(h * b, cols, "float32", 11).reshape(h, b, cols)
+    t = Tester("split")
+    v = t.view_load([b, h, cols], [cols, b * cols, 1], x)
+    d = t.sub(v, t.max(v, (2,), True))
+    pitch = cols + 3
+    want = np.zeros([h, b, pitch], np.float32)
+    want[:, :, :cols] = x - x.max(2, keepdims=True)
+    t.view_store_expect(d, (pitch, b * pitch, 1), want, 0)
+    assert t.run_check() and " row=" in t.das() and "  kdims: %d %d" % (h, b) in t.das(), t.das()
