@@ -387,7 +387,7 @@ __device__ __forceinline__ void read_tr(const uint32_t (&addr)[2][2], vu4 (&vf)[
 
 // Few queries: the waves of a workgroup share one tile of 32 queries and divide the keys (vm_attn divides the queries).
 // What bounds it: with one to 32 queries a pass is a read of K and V, and vm_attn spends its 256-query tile on them, one
-// block of 64 keys behind the other ([16,32] heads, 1 query, 1999 keys, D = 128 in bf16: 137 us for 524 MB); where the
+// block of 64 keys behind the other ([16,32] heads, 1 query, 1999 keys, D = 128 in bf16: 138 us for 524 MB); where the
 // products are larger but (head, tile) pairs are few, its 256-query workgroups leave most of the chip without work.
 // Here each of four waves walks 32-key blocks of its own (every fourth of the workgroup's part of the keys) through a
 // private piece of local memory, two blocks of K and V deep: no barrier in the loop, and 16 to 32 KB per wave in flight
@@ -395,9 +395,8 @@ __device__ __forceinline__ void read_tr(const uint32_t (&addr)[2][2], vu4 (&vf)[
 // read at full bandwidth, so the padding of one query to 32 costs nothing. The waves' running maxima, sums and outputs
 // meet in local memory at the end (base-2 weights, fp32, wave 0 first: the same order on every run). With too few
 // (head, tile) pairs for the chip the keys are also divided between kv_parts workgroups, whose unscaled outputs, maxima
-// and sums go to part_addr in fp32 for dvm_vm_attn_merge. Measured, back to back: the shape above 145 -> 96 us (5.5 TB/s),
-// [1,4] heads, 1 query, 4096 keys 101 -> 14 us (16 parts), [1,4], 2000 x 2000 63 -> 29 us, [2,8], 500 x 1000, D = 64
-// 25 -> 11 us.
+// and sums go to part_addr in fp32 for dvm_vm_attn_merge. The shape above takes 95 us (5.5 TB/s); both kernels at more
+// shapes stand beside the rule that chooses (Compiler::DivideKeys).
 template <bool IS_BF16, int D>
 __device__ __forceinline__ void vm_attn_keys(const VmParam &p) {
   constexpr int HT = D / 64;

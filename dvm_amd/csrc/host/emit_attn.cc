@@ -148,11 +148,12 @@ void Compiler::DivideKeys() {
         parts = n;
       }
     }
-    // Where the estimates are within a fifth and a microsecond the query kernel stays: each key block is read from local memory once for 32 queries
-    // of a wave there, and for 32 queries of the workgroup here. Measured on MI355X in us, waves divide queries / keys
-    // (parts): [16,32] heads, 1 query, 1999 keys, D 128: 145 / 96 (1); [1,4], 1, 4096, 128: 101 / 14 (8); [1,32], 8, 4096,
-    // 64: 79 / 13 (8); [1,4], 2000, 2000, 128: 63 / 29 (1); [2,8], 500, 1000, 64: 25 / 11 (1); [4,16], 1000, 1000, 128:
-    // 46 / 121 (1); [8,32], 100, 200, 128: 15 / 28 (1).
+    // Where the estimates are within a fifth and a microsecond the query kernel stays: each key block is read from local memory
+    // once for 32 queries of a wave there, and for 32 queries of the workgroup here. Measured on MI355X in us (all launches of
+    // a call, by events), waves divide queries / keys (the parts this rule picks): [16,32] heads, 1 query, 1999 keys, D 128:
+    // 138 / 95 (1); [1,4], 1, 4096, 128: 104 / 16 (11; undivided 40); [1,32], 8, 4096, 64: 80 / 15 (8; undivided 32); [1,4],
+    // 2000, 2000, 128: 65 / 32 (1); [2,8], 500, 1000, 64: 27 / 14 (1); and where the query kernel stays [4,16], 1000, 1000,
+    // 128: 49 / 133 (1); [8,32], 100, 200, 128: 17 / 31 (1).
     if (best > 0.8 * t_queries - 1.0) return;
   }
   uint32_t part_blocks = (blocks + parts - 1) / parts;

@@ -790,3 +790,19 @@ def test_divided_keys_do_not_push_a_kernel_out_of_the_static_workspace():
     assert "waves divide the keys" in t.das() and "merge" not in t.das() and t.workspace_bytes() == limit and t.num_launches() == 5, t.das()
     t = build(3)  # (past the limit with or without them)
     assert "merge" in t.das() and t.num_launches() == 8, t.das()
+
+
+@pytest.mark.parametrize("heads,sq,skv,d,parts", [(512, 1, 1999, 128, 1), (4, 1, 4096, 128, 11), (32, 8, 4096, 64, 8), (4, 2000, 2000, 128, 1), (16, 500, 1000, 64, 1),
+                                                  (64, 1000, 1000, 128, 0), (256, 100, 200, 128, 0)])
+def test_attention_kernel_and_parts_the_rule_picks(monkeypatch, heads, sq, skv, d, parts):
+    """The shapes whose times stand beside the rule (Compiler::DivideKeys), at the 256 compute units it assumes without a device."""
+    monkeypatch.delenv("DVM_ATTN_KEYS", raising=False)
+    monkeypatch.delenv("DVM_ATTN_WAVES", raising=False)
+    t = Tester("mix", run_mode="das")
+    q, k, v = (t.load(np.zeros((heads, n, d), np.float16)) for n in (sq, skv, skv))
+    x = t.cast(t.mul(t.matmul(q, k, False, True), d ** -0.5), "float32")
+    e = t.exp(t.sub(x, t.max(x, (2,), True)))
+    t.store(t.matmul(t.cast(t.div(e, t.sum(e, (2,), True)), "float16"), v, False, False))
+    t.codegen()
+    assert "entry attention" in t.das() and t.num_launches() == (2 if parts > 1 else 1), t.das()
+    assert ("waves divide the keys, parts=%d" % parts if parts else "entry attention") in t.das() and (parts > 0) == ("divide the keys" in t.das()), t.das()
