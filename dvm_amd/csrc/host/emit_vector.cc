@@ -704,7 +704,7 @@ bool Compiler::FinishProgram() {
   std::memcpy(prog_->blob.w, &hdr_, sizeof(hdr_));
   std::memcpy(prog_->blob.w + hdr_.mem_off, mems_, sizeof(VMemDesc) * n_mem_);
   std::memcpy(prog_->blob.w + hdr_.code_off, code_.data(), 8 * code_.size());
-  std::memcpy(prog_->blob.w + (hdr_.row_code & 0xffffu), row_code_.data(), 8 * row_code_.size());
+  if (!row_code_.empty()) std::memcpy(prog_->blob.w + (hdr_.row_code & 0xffffu), row_code_.data(), 8 * row_code_.size());
   prog_->lds_bytes = DVM_VEC_RED_SCRATCH_DOUBLES(hdr_.sched, prog_->threads) * 8 + static_cast<uint32_t>(max_vslot_) * u_ * 16 * prog_->threads;
   // (pointwise programs without V registers keep the geometry they are exported with: a double per lane, which nothing reads)
   prog_->lds_bytes = std::max<uint32_t>(prog_->lds_bytes, 8 * prog_->threads);
