@@ -1417,44 +1417,38 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       // groups of eight rows that hold rows of the output (what lies past its end was not written)
       const uint32_t f_row = m0 + (w >> 1) * 32u;
       const uint32_t groups = f_row >= h.m ? 0u : ((h.m - f_row + 7u) / 8u < 4u ? (h.m - f_row + 7u) / 8u : 4u);
-      // The vectors of four parts are in flight together; the parts are added in ascending order. (One loop per number of
-      // groups, whole fours of parts without a condition inside, the last parts with one each: a condition per vector was
-      // 16 branches and as many cleared registers a turn, 1.1 of 19.5 us at [64,9728] x [9728,64] in 31 parts.)
-      constexpr int PC = 4;
+      // The vectors of four parts, or of the last one to three, are in flight together; the parts are added in ascending
+      // order. (Straight code per number of parts and of groups: a condition per vector was 16 branches and as many cleared
+      // registers a turn, 2.1 of 19.3 us at [64,9728] x [9728,64] in 31 parts.)
       auto add_parts = [&](auto n_groups) {
         constexpr int G = decltype(n_groups)::value;
-        vf4 v[PC][G];
-        auto fetch = [&](int pp) {
+        auto together = [&](auto n_parts) {
+          constexpr int N = decltype(n_parts)::value;
+          vf4 v[N][G];
 #pragma unroll
-          for (int q = 0; q < G; ++q) {
-            v[pp][q] = *reinterpret_cast<const DVM_GLOBAL vf4 *>(reinterpret_cast<const DVM_GLOBAL char *>(frag + static_cast<uint32_t>(q) * plane * sizeof(vf4)) +
-                                                                 lane * static_cast<uint32_t>(sizeof(vf4)));
+          for (int pp = 0; pp < N; ++pp) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+              v[pp][q] = *reinterpret_cast<const DVM_GLOBAL vf4 *>(reinterpret_cast<const DVM_GLOBAL char *>(frag + static_cast<uint32_t>(q) * plane * sizeof(vf4)) +
+                                                                   lane * static_cast<uint32_t>(sizeof(vf4)));
+            }
+            frag += split_stride * sizeof(vf4);
           }
-          frag += split_stride * sizeof(vf4);
-        };
-        auto add = [&](int pp) {
+          // (Four: all of them on their way before the first is waited for. Fewer are left to the compiler, which is 1.2 of
+          // 213 us of a backward pass of [4096,4096] x [4096,2048] with its two sums of two parts.)
+          if constexpr (N == 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int q = 0; q < G; ++q)
+          for (int pp = 0; pp < N; ++pp)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[0][0][4 * q + e] += v[pp][q][e];
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[0][0][4 * q + e] += v[pp][q][e];
         };
         uint32_t left = h.k_split;
-        for (; left >= static_cast<uint32_t>(PC); left -= PC) {
-#pragma unroll
-          for (int pp = 0; pp < PC; ++pp) fetch(pp);
-          __builtin_amdgcn_sched_barrier(0);  // (all of them on their way before the first is waited for)
-#pragma unroll
-          for (int pp = 0; pp < PC; ++pp) add(pp);
-        }
-#pragma unroll
-        for (int pp = 0; pp < PC - 1; ++pp) {
-          if (static_cast<uint32_t>(pp) < left) fetch(pp);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int pp = 0; pp < PC - 1; ++pp) {
-          if (static_cast<uint32_t>(pp) < left) add(pp);
-        }
+        for (; left >= 4u; left -= 4u) together(std::integral_constant<int, 4>{});
+        if (left == 3u) together(std::integral_constant<int, 3>{});
+        else if (left == 2u) together(std::integral_constant<int, 2>{});
+        else if (left == 1u) together(std::integral_constant<int, 1>{});
       };
       if (groups == 4u) add_parts(std::integral_constant<int, 4>{});
       else if (groups == 3u) add_parts(std::integral_constant<int, 3>{});
