@@ -36,6 +36,8 @@ DVM_CUBE_DECL(dvm_vm_cube_bf16_small)
 DVM_CUBE_DECL(dvm_vm_cube_f16_small)
 DVM_CUBE_DECL(dvm_vm_cube_bf16_big8)
 DVM_CUBE_DECL(dvm_vm_cube_f16_big8)
+DVM_CUBE_DECL(dvm_vm_cube_bf16_deep)
+DVM_CUBE_DECL(dvm_vm_cube_f16_deep)
 // the builds that sum the partial tiles of a split k axis (second launch, tiles of any size)
 extern "C" __global__ void dvm_vm_cube_f16_comb(const VmParam p);
 extern "C" __global__ void dvm_vm_cube_bf16_comb(const VmParam p);
@@ -58,11 +60,12 @@ extern "C" __global__ void dvm_vm_attn_merge_bf16(const VmParam p);
 typedef void (*CubeKernel)(const VmParam);
 #define DVM_CUBE_ROW(prefix) {prefix##_nn, prefix##_nt, prefix##_tn, prefix##_tt}
 // [tile][bf16][trans_a * 2 + trans_b]
-static const CubeKernel kCubeKernels[4][2][4] = {
+static const CubeKernel kCubeKernels[DVM_CUBE_TILES][2][4] = {
     {DVM_CUBE_ROW(dvm_vm_cube_f16_big), DVM_CUBE_ROW(dvm_vm_cube_bf16_big)},
     {DVM_CUBE_ROW(dvm_vm_cube_f16_mid), DVM_CUBE_ROW(dvm_vm_cube_bf16_mid)},
     {DVM_CUBE_ROW(dvm_vm_cube_f16_small), DVM_CUBE_ROW(dvm_vm_cube_bf16_small)},
-    {DVM_CUBE_ROW(dvm_vm_cube_f16_big8), DVM_CUBE_ROW(dvm_vm_cube_bf16_big8)}};
+    {DVM_CUBE_ROW(dvm_vm_cube_f16_big8), DVM_CUBE_ROW(dvm_vm_cube_bf16_big8)},
+    {DVM_CUBE_ROW(dvm_vm_cube_f16_deep), DVM_CUBE_ROW(dvm_vm_cube_bf16_deep)}};
 static const CubeKernel kCubeCombKernels[2] = {dvm_vm_cube_f16_comb, dvm_vm_cube_bf16_comb};
 
 // [slabs a lane]: the row build of the vector VM
@@ -426,14 +429,14 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const uint64_t mem_end = static_cast<uint64_t>(c->mem_off) + static_cast<uint64_t>(c->n_mem) * (sizeof(VCubeMem) / 8);
     const uint64_t code_end = static_cast<uint64_t>(c->code_off) + c->n_code;
     const bool comb = (c->epi_flags & VCF_SPLITK_COMBINE) != 0;
-    const uint32_t bt = (c->tile == 0 || c->tile == 3) ? 256u : (c->tile == 1 ? 128u : 64u);
-    const uint32_t want_threads = c->tile == 3 && !comb ? 512u : 256u;  // tile 3: the 256x256 tile on eight waves
-    // (the sum of parts in pieces; a program exported with the geometry of the tile's own kernel is taken as well)
-    const uint32_t lds_tile = comb ? 64u : bt;
+    const uint32_t bt = DVM_CUBE_TILE_SIDE(c->tile);
+    const uint32_t want_threads = comb ? 256u : DVM_CUBE_TILE_LANES(c->tile);
+    // (the sum of parts in pieces of 64 x 64; a program exported with the geometry of the tile's own kernel is taken as well)
+    const uint32_t lds_need = comb ? DVM_CUBE_LDS_BYTES(2u) : DVM_CUBE_LDS_BYTES(c->tile);
     // The tile loop trusts the header: check it describes the launch it gets.
     if (mem_end > DVM_PARAM_WORDS || code_end > DVM_PARAM_WORDS || c->n_code == 0 || VI_OP(p.w[code_end - 1]) != VOP_END ||
-        c->tile > 3 || (threads != want_threads && !(comb && c->tile == 3 && threads == 512u)) || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
-        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < DVM_CUBE_LDS_BYTES(lds_tile) ||
+        c->tile >= DVM_CUBE_TILES || (threads != want_threads && !(comb && c->tile == 3 && threads == 512u)) || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
+        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < lds_need ||
         c->a_addr == 0 || c->b_addr == 0 || (c->dtype != VDT_F16 && c->dtype != VDT_BF16)) {
       return static_cast<int>(hipErrorInvalidValue);
     }
@@ -443,12 +446,13 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
       const bool rows = c->group_mode == VCG_M_BOUND || c->group_mode == VCG_M_SIZE;
       if (c->group_mode > VCG_K_SIZE || c->group_addr == 0 || (c->group_addr & (c->group_i32 ? 3u : 7u)) != 0 || c->nb0 != 1 ||
           c->nb1 > DVM_CUBE_MAX_GROUPS || (c->epi_flags & (VCF_SPLITK_PARTIAL | VCF_SPLITK_COMBINE)) != 0 ||
-          lds_bytes < DVM_CUBE_LDS_BYTES(bt) + 8u * c->nb1 || (rows && (c->a_sb0 != 0 || c->a_sb1 != 0))) {
+          lds_bytes < lds_need + 8u * c->nb1 || (rows && (c->a_sb0 != 0 || c->a_sb1 != 0))) {
         return static_cast<int>(hipErrorInvalidValue);
       }
     }
     const bool k_groups = c->group_mode == VCG_K_BOUND || c->group_mode == VCG_K_SIZE;
-    if (c->fast && (c->lda >= (1u << 22) || c->ldb >= (1u << 22) || (c->k % 64 != 0 && !k_groups) || c->k == 0 || c->lda % 8 != 0 || c->ldb % 8 != 0 ||
+    // (an operand with contiguous k: whole 16-byte chunks along k; a group's range along k is cut into whole chunks on the device)
+    if (c->fast && (c->lda >= (1u << 22) || c->ldb >= (1u << 22) || (c->k % 8 != 0 && !k_groups && (!c->trans_a || c->trans_b)) || c->k == 0 || c->lda % 8 != 0 || c->ldb % 8 != 0 ||
                     (c->a_addr & 15u) != 0 || (c->b_addr & 15u) != 0)) {
       return static_cast<int>(hipErrorInvalidValue);
     }

@@ -5,14 +5,14 @@
 // accumulation, one rounding to the operand type on write-out) plus the mix kernel's post-fusion
 // vector program (src/xkernel.cc:304-360). The reference's CUDA backend has no matmul at all
 // (src/system.cc:290-294); this kernel is specific to CDNA4:
-//  * v_mfma_f32_32x32x16 (bf16 / f16), 64-wide waves, WM x 2 waves per workgroup, each wave owning a
+//  * v_mfma_f32_32x32x16 (bf16 / f16), 64-wide waves, WM x WN waves per workgroup, each wave owning a
 //    (TM*32) x (TN*32) block of fp32 accumulators that stays in registers for the whole k loop;
-//  * the 256x256 tile (four or eight waves) walks k in stages of 32 through a ring of four stage buffers in
-//    local memory, every operand layout a straight direct-to-LDS copy (global_load_lds_dwordx4), the k-strided
-//    ones read back through ds_read_b64_tr_b16 (tile_loop_ring below);
-//  * the 128x128 and 64x64 tiles stage 64 k at a time, double buffered, k contiguous in local memory: rows of
-//    128 bytes whose eight 16-byte chunks are XOR-swizzled by the row number; operands whose k axis is strided in
-//    memory (B of an NN product, A of a TN product) are transposed in registers there, 8x8 elements per lane;
+//  * every tile (256x256 on eight or four waves, 128x128 and 64x64 on four) walks k in stages of 64 through a ring of
+//    stage buffers in local memory, every operand layout a straight direct-to-LDS copy (buffer_load_dwordx4 ... lds),
+//    the k-strided ones read back through ds_read_b64_tr_b16 (tile_loop_ring below). Stages of 64 k fetch whole 128-byte
+//    lines of an operand with contiguous k. Measured (bf16, stages of 32 / 64 k): 8192 x 4096 x 4096 with both operands
+//    k-contiguous 250 / 241 us, 4096 x 2048 x 4096 on the 128 tile 81 / 67 us;
+//  * operands that are not whole 16-byte chunks are staged element by element (stage_generic);
 //  * fragments are double buffered in registers: the reads of step s+1 are in flight while the MFMAs of step s run;
 //  * the epilogue runs in two passes over half tiles: accumulators go to local memory once, row
 //    major, and come back as slabs of 8 consecutive columns per lane, so every memory operand of the
@@ -71,113 +71,6 @@ __device__ __forceinline__ uint32_t tile_off(uint32_t row, uint32_t chunk) {
   return row * BK + ((chunk ^ ((row ^ (row >> 3)) & 7u)) << 3);
 }
 
-// ---- staging one operand tile: ROWS rows (m or n) x BK (k) ---------------------------------------------
-// KC source (k contiguous in memory: A when !trans_a, B when trans_b): the tile is a straight copy, so it
-// goes from memory to local memory directly (global_load_lds_dwordx4: a wave's 64 x 16 bytes land in 1 KB
-// of consecutive local memory, the swizzle is applied by choosing which chunk each lane fetches); no
-// registers, no ds_write, and the data may be in flight for a whole k tile.
-// KS source (k strided, the row index contiguous): 8x8 element blocks through registers, transposed on
-// the way (v_perm_b32), then written with ds_write_b128.
-struct LaneOffsets {
-  int32_t v[2];  // (signed: a row that is clamped back inside the operand lies before the row the loop would fetch)
-};
-
-template <int ROWS, bool KC, int NTHR>
-struct Stage;
-
-template <int ROWS, int NTHR>
-struct Stage<ROWS, true, NTHR> {
-  static constexpr int N = ROWS * BK / 8 / NTHR;  // 16-byte chunks per thread
-  static constexpr uint32_t RPS = NTHR / 8;        // rows one step of all threads covers
-  static constexpr int N_LOADS = N, N_WRITES = 0;
-
-  // Chunk position p = NTHR*i + tid of the tile holds row p/8, logical chunk (p%8) ^ swizzle(row): with
-  // row = RPS*i + tid/8 the swizzle depends at most on the parity of i (RPS = 32; not at all for 64), hence
-  // two byte offsets per lane.
-  // rows_valid < ROWS (a tile of which only the first rows lie inside the operand; tiles of at most two chunks per
-  // lane only): the rows past the end fetch the last valid row instead, so that no load leaves the operand; what
-  // they feed are accumulator rows the epilogue never stores.
-  static constexpr bool kCanClamp = N <= 2;
-  static __device__ __forceinline__ LaneOffsets lane_offset(uint32_t ld, uint32_t tid, uint32_t rows_valid = ROWS) {
-    LaneOffsets o;
-#pragma unroll
-    for (int par = 0; par < 2; ++par) {
-      const uint32_t row = RPS * par + (tid >> 3);
-      const uint32_t logical = (tid & 7u) ^ ((row ^ (row >> 3)) & 7u);
-      uint32_t from = tid >> 3;  // row fetched, relative to the first row of chunk `par`
-      int32_t back = 0;
-      if (kCanClamp && row >= rows_valid) back = static_cast<int32_t>(rows_valid - 1u) - static_cast<int32_t>(row);
-      o.v[par] = (static_cast<int32_t>(from) + back) * static_cast<int32_t>(ld * 2u) + static_cast<int32_t>((logical << 3) * 2u);
-    }
-    return o;
-  }
-
-  // origin: address of element (row0, k0) of the operand
-  __device__ __forceinline__ void fetch(uint64_t origin, uint32_t ld, const LaneOffsets &lane, uint32_t tid, uint16_t *tile) {
-    const DVM_GLOBAL char *base = reinterpret_cast<const DVM_GLOBAL char *>(origin);
-    const uint32_t wave_first = uni(tid >> 6) * 64u;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const DVM_GLOBAL char *src = base + (static_cast<int64_t>(static_cast<uint64_t>(i) * RPS * ld * 2u) + lane.v[i & 1]);
-      uint16_t *dst = tile + (static_cast<uint32_t>(i) * NTHR + wave_first) * 8u;
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const DVM_GLOBAL void *>(src), (__attribute__((address_space(3))) void *)(dst), 16, 0, 0);
-    }
-  }
-  __device__ __forceinline__ void commit(uint16_t *, uint32_t) const {}
-};
-
-template <int ROWS, int NTHR>
-struct Stage<ROWS, false, NTHR> {
-  static_assert(ROWS <= 256, "one 8x8 block per thread, the first ROWS threads");
-  // 8 (k) x 8 (rows) element blocks, ROWS of them per tile. With 256 lanes one lane takes a whole block; with 512
-  // lanes and 256 rows two lanes share one, each taking 4 of its rows (8-byte loads, half the registers).
-  static constexpr int TPB = (NTHR == 512 && ROWS == 256) ? 2 : 1;  // lanes per block
-  static constexpr int RPT = 8 / TPB;                               // rows of the block a lane owns
-  static constexpr int N = 8;
-  static constexpr int N_LOADS = 8, N_WRITES = RPT;
-  typedef uint32_t Row __attribute__((ext_vector_type(RPT / 2)));   // RPT 16-bit elements of one k
-  Row r[N];
-
-  static __device__ __forceinline__ bool active(uint32_t tid) { return (ROWS * TPB == NTHR) || tid < ROWS * TPB; }
-
-  static __device__ __forceinline__ LaneOffsets lane_offset(uint32_t ld, uint32_t tid) {
-    const uint32_t blk = tid / TPB, part = tid % TPB;
-    const uint32_t kb = blk / (ROWS / 8), rb = blk % (ROWS / 8);
-    LaneOffsets o;
-    o.v[0] = o.v[1] = static_cast<int32_t>((kb * 8u * ld + rb * 8u + part * RPT) * 2u);
-    return o;
-  }
-
-  __device__ __forceinline__ void fetch(uint64_t origin, uint32_t ld, const LaneOffsets &lane, uint32_t tid, uint16_t *) {
-    const DVM_GLOBAL char *base = reinterpret_cast<const DVM_GLOBAL char *>(origin);
-    if (active(tid)) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        r[j] = *reinterpret_cast<const DVM_GLOBAL Row *>(base + static_cast<uint64_t>(j) * ld * 2u + lane.v[0]);
-      }
-    }
-  }
-
-  __device__ __forceinline__ void commit(uint16_t *tile, uint32_t tid) const {
-    if (active(tid)) {
-      const uint32_t blk = tid / TPB, part = tid % TPB;
-      const uint32_t kb = blk / (ROWS / 8), rb = blk % (ROWS / 8);
-      // r[j] holds k = kb*8 + j, rows rb*8 + part*RPT .. +RPT-1; the tile wants, per row, k = kb*8 .. +7
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        vu4 o;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const uint32_t lo = r[2 * jj][i >> 1], hi = r[2 * jj + 1][i >> 1];
-          // bytes of the result, least significant first: (i odd ? upper : lower) half of lo, then of hi
-          o[jj] = __builtin_amdgcn_perm(hi, lo, (i & 1) ? 0x07060302u : 0x05040100u);
-        }
-        *reinterpret_cast<vu4 *>(tile + tile_off(rb * 8 + part * RPT + i, kb)) = o;
-      }
-    }
-  }
-};
-
 // Generic staging of one tile straight into local memory (edge tiles, odd leading dimensions, unaligned
 // operands, a k axis that is no multiple of 64). The unit is a run of 8 elements that are consecutive in memory:
 // 8 k of one row (k contiguous) or 8 rows at one k (rows contiguous); a run that lies inside the operand and is
@@ -232,52 +125,62 @@ __device__ __attribute__((noinline)) void stage_generic(uint16_t *tile, uint64_t
   }
 }
 
-// ---- the 256x256 tile on four waves: stages of 32 k, four of them in local memory ---------------------
-// A stage holds 256 rows x 32 k of each operand (16 KB + 16 KB); four stage buffers make a ring. While
-// stage s is multiplied, the direct loads of stages s+1 and s+2 are in flight and those of stage s+3 are
-// issued, a few at a time between the MFMAs, into the buffer stage s-1 has just left: every load has two
-// full stages (64 MFMAs per wave) to arrive before anyone waits for it, and the four waves never send
-// their loads in one burst. Both operand layouts are straight copies:
-//  * k contiguous in memory (A, or B of a product with trans_b): rows of 32 k = 64 bytes = four 16-byte
-//    chunks, chunk c of row r stored at chunk c ^ ((r >> 2) & 3): the 16 rows that one quarter of a fragment read
-//    touches (16 lanes x 16 bytes = all 64 banks once) then sit in 16 different bank groups; one ds_read_b128 per lane;
-//  * k strided (B, or A of a product with trans_a): the tile is stored as it lies in memory, 32 k rows of
-//    256 elements (512 bytes, 32 chunks), chunk c of k row kr stored at chunk c ^ kswz(kr & 3); a fragment is
-//    two ds_read_b64_tr_b16 per lane, which transpose 4 k x 16 rows inside each group of 16 lanes.
-// kswz = {0, 10, 4, 14}: the four k rows one transposing read touches land in four different 32-byte
-// columns of a 128-byte window, and the two 16-lane groups of a half-wave in different halves of 256 bytes.
-constexpr int SK = 32;                           // k extent of a stage
-constexpr uint32_t kStageOperand = 256 * SK;     // elements of one operand in a stage buffer
-constexpr uint32_t kStageBuf = 2 * kStageOperand;
+// ---- the tile loop: stages of 32 or 64 k in a ring of buffers in local memory ---------------------------
+// A stage holds BM rows x SK k of A and BN rows x SK k of B; NB stage buffers make a ring. While stage s is multiplied,
+// the direct loads of stages s+1 .. s+NB-2 are in flight and those of stage s+NB-1 are issued, a few at a time between
+// the MFMAs, into the buffer stage s-1 has just left. Both operand layouts are straight copies:
+//  * k contiguous in memory (A, or B of a product with trans_b): rows of SK k = four or eight 16-byte chunks, chunk c of
+//    row r stored at chunk c ^ kc_swz(r): the 16 rows that one quarter of a fragment read touches (16 lanes x 16 bytes =
+//    all 64 banks once) then sit in 16 different bank groups; one ds_read_b128 per lane;
+//  * k strided (B, or A of a product with trans_a): the tile is stored as it lies in memory, SK k rows of ROWS elements,
+//    chunk c of k row kr stored at chunk c ^ ks_swz(kr); a fragment is two ds_read_b64_tr_b16 per lane, which transpose
+//    4 k x 16 rows inside each group of 16 lanes. The swizzle puts the four k rows one transposing read touches, and the
+//    two 16-lane groups of a half-wave, into 16 different bank groups.
+// The loads go through a buffer descriptor whose range ends below the offset kOutside: a lane whose chunk lies outside
+// the operand (rows past m or n, k past the end of the k axis) asks for that offset, reads nothing and leaves zeros in
+// local memory. So a product with any m, n and k takes this loop (whole chunks only: the extent along the contiguous axis
+// is a multiple of 8), stages past the end of the k axis are loads of nothing, and the loop has one body: no prologue or
+// tail variants, no counts that depend on how many stages are left. Before, a k axis that is no multiple of 64 and tiles
+// larger than the output walked element by element: bf16 [5628,1816] x [1816,2016] 414 us.
+constexpr uint32_t kOutside = 0x80000000u;  // (every offset inside a stage is below: 256 rows of less than 2^22 elements)
 
-__device__ __forceinline__ uint32_t kc_swz(uint32_t row) { return (row >> 2) & 3u; }
-__device__ __forceinline__ uint32_t ks_swz(uint32_t krow) { return (((krow & 3u) + 4u * (krow & 1u)) << 1); }
+template <int SK>
+__device__ __forceinline__ uint32_t kc_swz(uint32_t row) {
+  static_assert(SK == 64, "rows of eight chunks");
+  return (row >> 1) & 7u;
+}
+template <int ROWS>
+__device__ __forceinline__ uint32_t ks_swz(uint32_t krow) {
+  return ROWS == 64 ? (krow & 2u) << 1 : (((krow & 3u) + 4u * (krow & 1u)) << 1);
+}
 
-template <bool KC, int NTHR>
-struct StageLoad {
-  static constexpr int N = 1024 / NTHR;  // 16-byte chunks per lane: 256 rows x 64 bytes over the workgroup
-  uint32_t lane_off;  // byte offset of the lane's first chunk from the tile's origin
-  uint32_t step;      // byte distance between the lane's chunks
+template <bool KC, int ROWS, int SK, int NTHR>
+struct RingLoad {
+  static constexpr int N = ROWS * SK / 8 / NTHR;                 // 16-byte chunks per lane and stage
+  static constexpr uint32_t CPR = (KC ? SK : ROWS) / 8;          // chunks per row (k contiguous) or per k row
+  static constexpr int kLines = static_cast<int>(NTHR / CPR);    // rows (k contiguous) or k rows from one chunk of a lane to its next
+  static_assert(kLines % (KC ? 16 : 4) == 0, "the swizzle of a lane's chunks is the same");
+  uint32_t off;     // byte offset of the lane's first chunk from the stage's origin
+  uint32_t step;    // bytes from one chunk of the lane to its next
+  int32_t k0, row;  // the first chunk's first k and row
+  int32_t rows;     // rows of the operand from the tile's first on
 
-  __device__ __forceinline__ void init(uint32_t ld, uint32_t tid) {
-    if constexpr (KC) {
-      // chunk position p = NTHR*i + tid: row p/4, physical chunk p%4 (NTHR/4 = 64 or 128 rows further do not change the swizzle)
-      const uint32_t row = tid >> 2;
-      lane_off = row * ld * 2u + (((tid & 3u) ^ kc_swz(row)) << 4);
-      step = (NTHR / 4u) * ld * 2u;
-    } else {
-      // chunk position p = NTHR*i + tid: k row p/32, physical chunk p%32
-      const uint32_t kr = tid >> 5;
-      lane_off = kr * ld * 2u + (((tid & 31u) ^ ks_swz(kr)) << 4);
-      step = (NTHR / 32u) * ld * 2u;
-    }
+  __device__ __forceinline__ void init(uint32_t ld, uint32_t rows_left, uint32_t tid) {
+    const uint32_t line = tid / CPR, chunk = (tid % CPR) ^ (KC ? kc_swz<SK>(line) : ks_swz<ROWS>(line));
+    off = line * ld * 2u + (chunk << 4);
+    step = static_cast<uint32_t>(kLines) * ld * 2u;
+    k0 = static_cast<int32_t>(KC ? chunk * 8u : line);
+    row = static_cast<int32_t>(KC ? line : chunk * 8u);
+    rows = static_cast<int32_t>(rows_left);
   }
-  // origin: address of element (row0, k0) of the operand; dst: the operand's part of a stage buffer
-  template <int I>
-  __device__ __forceinline__ void issue(uint64_t origin, uint32_t wave_first, uint16_t *dst) const {
-    const DVM_GLOBAL char *src = reinterpret_cast<const DVM_GLOBAL char *>(origin) + (lane_off + static_cast<uint32_t>(I) * step);
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const DVM_GLOBAL void *>(src),
-                                     (__attribute__((address_space(3))) void *)(dst + (static_cast<uint32_t>(I) * NTHR + wave_first) * 8u), 16, 0, 0);
+  // origin: address of element (row0, k0) of the operand; dst: the operand's part of a stage buffer; k_left: what the k
+  // axis has from the stage's first k on (zero or less: the stage lies past its end). The tests are made in every stage: a
+  // branch around them, taken for the last stages only, made the compiler copy accumulators from one block to the other.
+  __device__ __forceinline__ void issue(int i, uint64_t origin, int32_t k_left, uint32_t wave_first, uint16_t *dst) const {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(origin), 0, kOutside, 0x00027000);
+    const bool inside = KC ? (k0 < k_left) & (row < rows - i * kLines) : (k0 < k_left - i * kLines) & (row < rows);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(dst + (static_cast<uint32_t>(i) * NTHR + wave_first) * 8u), 16,
+                                             inside ? off : kOutside, static_cast<uint32_t>(i) * step, 0, 0);
   }
 };
 
@@ -290,175 +193,184 @@ __device__ __forceinline__ uint32_t lds_byte_address(const void *ptr) {
   return static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) const char *)(ptr)));
 }
 
-template <bool KC>
+template <bool KC, int ROWS, int SK>
 struct FragAddr {
-  uint32_t x[4];  // byte offsets inside the operand's part of a stage buffer
+  uint32_t x;  // byte offset of fragment 0 in step 0 inside the operand's part of a stage buffer
 
   __device__ __forceinline__ void init(uint32_t r0, uint32_t lane) {
     if constexpr (KC) {
-      // fragment f, step kk: row r0 + 32f + lane%32, chunk (2kk + lane/32) ^ swz(row); x[kk] for f = 0
+      // fragment f, step kk: row r0 + 32f + lane%32, chunk (2kk + lane/32) ^ swz(row)
       const uint32_t j = lane & 31u, hh = lane >> 5;
-      const uint32_t sw = kc_swz(j);  // r0 (a multiple of 64) and 32f do not change it
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) x[kk] = ((r0 + j) * SK + (((2u * kk + hh) ^ sw) << 3)) * 2u;
-      x[2] = x[3] = 0;
+      const uint32_t sw = kc_swz<SK>(j);  // r0 and 32f (multiples of 32) do not change it
+      x = ((r0 + j) * SK + ((hh ^ sw) << 3)) * 2u;
     } else {
       // fragment f, step kk, half w: the lane supplies k row 16kk + 8*(g>>1) + 4w + jj and the four elements
-      // r0 + 32f + 16*(g&1) + 4q .. +3, with g = lane/16, jj = (lane%16)/4, q = lane%4; x[f] for kk = w = 0
+      // r0 + 32f + 16*(g&1) + 4q .. +3, with g = lane/16, jj = (lane%16)/4, q = lane%4
       const uint32_t g = lane >> 4, jj = (lane & 15u) >> 2, q = lane & 3u;
       const uint32_t kr = 8u * (g >> 1) + jj;
-      const uint32_t sw = ks_swz(jj);
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const uint32_t chunk = (r0 >> 3) + 4u * f + 2u * (g & 1u) + (q >> 1);
-        x[f] = (kr * 256u + ((chunk ^ sw) << 3) + 4u * (q & 1u)) * 2u;
-      }
+      const uint32_t chunk = (r0 >> 3) + 2u * (g & 1u) + (q >> 1);
+      x = (kr * ROWS + ((chunk ^ ks_swz<ROWS>(jj)) << 3) + 4u * (q & 1u)) * 2u;
     }
   }
-  // base: byte address in local memory of the operand's part of the stage buffer
+  // base: byte address in local memory of the operand's part of the stage buffer (a multiple of 256: step kk, or fragment
+  // f of a k-strided operand, whose bits of the chunk number r0 / 8 are clear, flips address bits below that)
   template <int F, int KK>
   __device__ __forceinline__ vu4 read(uint32_t base) const {
     if constexpr (KC) {
       vu4 r;
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(base + x[KK]), "n"(F * 32 * SK * 2));
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"((base + x) ^ static_cast<uint32_t>(KK << 5)), "n"(F * 32 * SK * 2));
       return r;
     } else {
       vu2 lo, hi;
-      const uint32_t addr = base + x[F];
-      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(addr), "n"(KK * 16 * 512));
-      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(addr), "n"(KK * 16 * 512 + 4 * 512));
+      const uint32_t addr = (base + x) ^ static_cast<uint32_t>(F << 6);
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(addr), "n"(KK * 16 * ROWS * 2));
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(addr), "n"(KK * 16 * ROWS * 2 + 4 * ROWS * 2));
       return vu4{lo[0], lo[1], hi[0], hi[1]};
     }
   }
 };
 
-// The tile loop for WM x 2 waves (WM = 2: 128x128 accumulators per wave, one wave per SIMD; WM = 4: 64x128,
-// two per SIMD). a_org / b_org: address of element (m0, 0) of A and (n0, 0) of B; nks: stages (k / 32 >= 2).
-template <bool IS_BF16, bool A_KC, bool B_KC, int WM>
-__device__ __forceinline__ void tile_loop_ring(vf16 (&acc)[8 / WM][4], uint16_t *lds, uint64_t a_org, uint64_t b_org, uint32_t lda,
-                                               uint32_t ldb, uint32_t nks, uint32_t tid) {
-  constexpr int NTHR = WM * 128, TM = 8 / WM, TN = 4;
-  constexpr int NL = StageLoad<true, NTHR>::N;  // loads per lane, operand and stage
-  constexpr int BPG = TN / TM;                  // B fragments a group reads
-  static_assert(NL == TM && (NL == 2 || NL == 4), "one A or B load pair per group");
+// Waits until at most N of this wave's loads are outstanding and all its local-memory reads have returned, then meets
+// the other waves. One piece of assembly on purpose: behind __syncthreads() the compiler waits for every outstanding
+// load (the direct loads write local memory), which would drain the ring.
+template <int N>
+__device__ __forceinline__ void ring_meet() {
+  static_assert(N >= 0 && N <= 63, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <int N, typename F>
+__device__ __forceinline__ void for_index(F f) {
+  if constexpr (N > 0) {
+    for_index<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// The tile loop for WM x WN waves of TM x TN fragments. a_org / b_org: address of element (m0, k0) of A and (n0, k0) of
+// B; a_rows / b_rows: rows the operands have from there on; k: length of the k range (at least 1).
+template <bool IS_BF16, bool A_KC, bool B_KC, int TM, int TN, int WM, int WN, int NBUF>
+__device__ __forceinline__ void tile_loop_ring(vf16 (&acc)[TM][TN], uint16_t *lds, uint64_t a_org, uint64_t b_org, uint32_t lda,
+                                               uint32_t ldb, uint32_t a_rows, uint32_t b_rows, uint32_t k, uint32_t tid) {
+  constexpr int NTHR = WM * WN * 64, BM = WM * TM * 32, BN = WN * TN * 32;
+  constexpr int SK = DVM_CUBE_STAGE_K, NB = NBUF;
+  // A step is SUB * 16 k: with one fragment per wave and operand a step of 16 k is one MFMA, far less than the latency of
+  // the fragment reads it should hide.
+  constexpr int SUB = TM * TN == 1 ? 2 : 1, STEPS = SK / (16 * SUB);
+  constexpr uint32_t kStageA = BM * SK, kStageBuf = (BM + BN) * SK;  // elements
+  typedef RingLoad<A_KC, BM, SK, NTHR> LoadA;
+  typedef RingLoad<B_KC, BN, SK, NTHR> LoadB;
+  constexpr int NL = LoadA::N + LoadB::N;      // loads per lane and stage
+  constexpr int LPG = (NL + TM - 1) / TM;      // loads a group of MFMAs takes along
+  constexpr int BPG = (TN + TM - 1) / TM;      // B fragments a group reads
   const uint32_t wave = tid >> 6, lane = tid & 63u;
-  const uint32_t wm = wave >> 1, wn = wave & 1u;
+  const uint32_t wm = wave / WN, wn = wave % WN;
   const uint32_t wave_first = uni(wave) * 64u;
-  StageLoad<A_KC, NTHR> la;
-  StageLoad<B_KC, NTHR> lb;
-  la.init(lda, tid);
-  lb.init(ldb, tid);
-  FragAddr<A_KC> fa;
-  FragAddr<B_KC> fb;
+  LoadA la;
+  LoadB lb;
+  la.init(lda, a_rows, tid);
+  lb.init(ldb, b_rows, tid);
+  FragAddr<A_KC, BM, SK> fa;
+  FragAddr<B_KC, BN, SK> fb;
   fa.init(wm * (TM * 32u), lane);
-  fb.init(wn * 128u, lane);
+  fb.init(wn * (TN * 32u), lane);
   const uint64_t a_adv = (A_KC ? static_cast<uint64_t>(SK) : static_cast<uint64_t>(SK) * lda) * 2;
   const uint64_t b_adv = (B_KC ? static_cast<uint64_t>(SK) : static_cast<uint64_t>(SK) * ldb) * 2;
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
+  const uint32_t nks = (k + SK - 1) / SK;  // stages
 
-  // group g of a stage (TM groups) sends 2 * NL / TM = two of the lane's loads: the first half of the groups
-  // A's, the second half B's
-  auto issue_pair = [&](uint32_t st, auto group) {
-    constexpr int G = decltype(group)::value;
-    uint16_t *buf = lds + (st & 3u) * kStageBuf;
-    if constexpr (2 * G < TM) {
-      const uint64_t ao = a_org + st * a_adv;
-      la.template issue<2 * G>(ao, wave_first, buf);
-      la.template issue<2 * G + 1>(ao, wave_first, buf);
-    } else {
-      const uint64_t bo = b_org + st * b_adv;
-      lb.template issue<2 * G - TM>(bo, wave_first, buf + kStageOperand);
-      lb.template issue<2 * G - TM + 1>(bo, wave_first, buf + kStageOperand);
-    }
-  };
-  vu4 af[2][TM], bf[2][TN];
-  const uint32_t lds_base = lds_byte_address(lds);
-  auto read_group = [&](auto fbuf, uint32_t st, auto kk, auto group) {  // the fragments group g is in charge of
-    constexpr int FB = decltype(fbuf)::value, KK = decltype(kk)::value, G = decltype(group)::value;
-    const uint32_t buf = lds_base + (st & 3u) * (kStageBuf * 2u);
-    af[FB][G] = fa.template read<G, KK>(buf);
-    bf[FB][BPG * G] = fb.template read<BPG * G, KK>(buf + kStageOperand * 2u);
-    if constexpr (BPG == 2) bf[FB][2 * G + 1] = fb.template read<2 * G + 1, KK>(buf + kStageOperand * 2u);
-  };
-  // every read issued so far has returned; the fragments of buffer fbuf may be used from here on
-  auto reads_done = [&](int fbuf) {
-    if constexpr (TM == 4) {
-      asm volatile("s_waitcnt lgkmcnt(0)"
-                   : "+v"(af[fbuf][0]), "+v"(af[fbuf][1]), "+v"(af[fbuf][2]), "+v"(af[fbuf][3]), "+v"(bf[fbuf][0]), "+v"(bf[fbuf][1]),
-                     "+v"(bf[fbuf][2]), "+v"(bf[fbuf][3]));
-    } else {
-      asm volatile("s_waitcnt lgkmcnt(0)"
-                   : "+v"(af[fbuf][0]), "+v"(af[fbuf][1]), "+v"(bf[fbuf][0]), "+v"(bf[fbuf][1]), "+v"(bf[fbuf][2]), "+v"(bf[fbuf][3]));
-    }
-  };
-  auto mfma_row = [&](int fbuf, int i) {
+  // the next stage to load: the operands' addresses, what is left of the k axis, its buffer
+  int32_t ld_left = static_cast<int32_t>(k);
+  uint32_t ld_buf = 0;
+  auto load_some = [&](int from, int count) {  // loads [from, from + count) of the stage
+    uint16_t *buf = lds + ld_buf * kStageBuf;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = mfma<IS_BF16>(af[fbuf][i], bf[fbuf][j], acc[i][j]);
-  };
-  // Waits until at most `stages` stages of this wave's loads are outstanding and all its local-memory reads have
-  // returned, then meets the other waves. One piece of assembly on purpose: behind __syncthreads() the compiler
-  // waits for every outstanding load (the direct loads write local memory), which would drain the ring.
-  auto meet = [](auto stages) {
-    constexpr int N = decltype(stages)::value * 2 * NL;
-    static_assert(N == 0 || N == 4 || N == 8 || N == 16, "vmcnt values spelled out below");
-    if constexpr (N == 16) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else if constexpr (N == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  };
-  auto for_groups = [&](auto f) {
-    f(I0{});
-    f(I1{});
-    if constexpr (TM == 4) {
-      f(std::integral_constant<int, 2>{});
-      f(std::integral_constant<int, 3>{});
+    for (int i = from; i < from + count; ++i) {
+      if (i < LoadA::N) la.issue(i, a_org, ld_left, wave_first, buf);
+      else if (i < NL) lb.issue(i - LoadA::N, b_org, ld_left, wave_first, buf + kStageA);
     }
   };
+  auto load_end = [&]() {
+    a_org += a_adv;
+    b_org += b_adv;
+    ld_left -= SK;
+    ld_buf = ld_buf + 1u == NB ? 0u : ld_buf + 1u;
+  };
+  vu4 af[2][SUB * TM], bf[2][SUB * TN];
+  const uint32_t lds_base = lds_byte_address(lds);
+  uint32_t rd_base = lds_base;  // the stage buffer the fragments come from
+  auto read_group = [&](auto fbuf, auto step, auto group) {  // the fragments of a step that group g is in charge of
+    constexpr int FB = decltype(fbuf)::value, ST = decltype(step)::value, G = decltype(group)::value;
+    for_index<SUB>([&](auto sub) {
+      constexpr int S = decltype(sub)::value, KK = ST * SUB + S;
+      af[FB][S * TM + G] = fa.template read<G, KK>(rd_base);
+      for_index<BPG>([&](auto j) {
+        constexpr int J = G * BPG + decltype(j)::value;
+        if constexpr (J < TN) bf[FB][S * TN + J] = fb.template read<J, KK>(rd_base + kStageA * 2u);
+      });
+    });
+  };
+  // every read issued so far has returned; the fragments of buffer FB may be used from here on
+  auto reads_done = [&](auto fbuf) {
+    constexpr int FB = decltype(fbuf)::value;
+    vu4 &first = af[FB][0];
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(first));
+    for_index<SUB * TM - 1>([&](auto i) {
+      vu4 &f = af[FB][decltype(i)::value + 1];
+      asm volatile("" : "+v"(f));
+    });
+    for_index<SUB * TN>([&](auto j) {
+      vu4 &f = bf[FB][decltype(j)::value];
+      asm volatile("" : "+v"(f));
+    });
+  };
+  auto mfma_row = [&](auto fbuf, auto i) {
+    constexpr int FB = decltype(fbuf)::value, I = decltype(i)::value;
+#pragma unroll
+    for (int u = 0; u < SUB; ++u)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[I][j] = mfma<IS_BF16>(af[FB][u * TM + I], bf[FB][u * TN + j], acc[I][j]);
+  };
 
-  for_groups([&](auto g) { issue_pair(0, g); });
-  for_groups([&](auto g) { issue_pair(1, g); });
-  if (nks > 2) {
-    for_groups([&](auto g) { issue_pair(2, g); });
-    meet(std::integral_constant<int, 2>{});
-  } else {
-    meet(I1{});
+  for_index<NB>([&](auto) {
+    load_some(0, NL);
+    load_end();
+  });
+  ring_meet<(NB - 1) * NL>();
+  for_index<TM>([&](auto g) { read_group(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, g); });
+
+  // One stage = STEPS steps of 16 k, each TM groups of TN MFMAs (one row of accumulator tiles). Group g also reads its
+  // fragments of the next step. The last step first meets the other waves (stage st+1 has landed for everybody, and
+  // nobody reads stage st any more), reads the fragments of stage st+1 and sends the loads of stage st+NB into the buffer
+  // that stage st has left. The scheduler may not move anything across a group. (Behind the last stage there is one more
+  // set of fragments, which nothing multiplies.)
+  uint32_t rd_buf = 0;
+  for (uint32_t st = 0; st < nks; ++st) {
+    for_index<STEPS>([&](auto step) {
+      constexpr int S = decltype(step)::value;
+      constexpr bool LAST = S == STEPS - 1;
+      typedef std::integral_constant<int, S & 1> Cur;
+      typedef std::integral_constant<int, (S + 1) & 1> Nxt;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (LAST) {
+        rd_buf = rd_buf + 1u == NB ? 0u : rd_buf + 1u;
+        rd_base = lds_base + rd_buf * (kStageBuf * 2u);
+        ring_meet<(NB - 2) * NL>();
+      }
+      reads_done(Cur{});
+      __builtin_amdgcn_sched_barrier(0);
+      for_index<TM>([&](auto g) {
+        constexpr int G = decltype(g)::value;
+        read_group(Nxt{}, std::integral_constant<int, LAST ? 0 : S + 1>{}, g);
+        if constexpr (LAST) load_some(G * LPG, LPG);
+        mfma_row(Cur{}, g);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+    load_end();
   }
-  for_groups([&](auto g) { read_group(I0{}, 0, I0{}, g); });
-
-  // One stage = two steps of 16 k, each TM groups of four MFMAs (one row of accumulator tiles). Group g of
-  // step 0 also reads its fragments of step 1 and sends two of the loads of stage st+3; step 1 first meets the
-  // other waves (stage st+1 has landed for everybody, and nobody reads stage st any more, whose buffer the
-  // loads issued after the next meeting overwrite), then its group g reads its fragments of stage st+1. The
-  // scheduler may not move anything across a group.
-  auto stage = [&](uint32_t st, auto loads, auto next) {
-    constexpr bool LOADS = decltype(loads)::value, NEXT = decltype(next)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    reads_done(0);
-    __builtin_amdgcn_sched_barrier(0);
-    for_groups([&](auto g) {
-      read_group(I1{}, st, I1{}, g);
-      if constexpr (LOADS) issue_pair(st + 3, g);
-      mfma_row(0, decltype(g)::value);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    if constexpr (NEXT) {
-      if constexpr (LOADS) meet(std::integral_constant<int, 2>{});  // younger: the loads of stages st+2 and st+3
-      else meet(I0{});
-    }
-    reads_done(1);
-    __builtin_amdgcn_sched_barrier(0);
-    for_groups([&](auto g) {
-      if constexpr (NEXT) read_group(I0{}, st + 1, I0{}, g);
-      mfma_row(1, decltype(g)::value);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
-  uint32_t st = 0;
-  for (; st + 3 < nks; ++st) stage(st, std::true_type{}, std::true_type{});
-  for (; st + 1 < nks; ++st) stage(st, std::false_type{}, std::true_type{});
-  stage(st, std::false_type{}, std::false_type{});
-  __syncthreads();
+  static_assert(STEPS % 2 == 0, "the first step of a stage uses fragment buffer 0");
+  reads_done(std::integral_constant<int, 0>{});
+  ring_meet<0>();  // (the loads of nothing write zeros: they have landed before local memory is used for anything else)
 }
 
 // ---- epilogue ---------------------------------------------------------------------------------------
@@ -490,9 +402,22 @@ __device__ __forceinline__ uint32_t elem_size(uint32_t dtype) {
   return (dtype == VDT_F32 || dtype == VDT_I32) ? 4u : (dtype == VDT_BOOL ? 1u : 2u);
 }
 
-// One slab, element by element, with every guard: edges, strided or unaligned operands.
+// One slab with every guard (edges, strided or unaligned operands): 128-bit accesses for the lanes whose slab is whole,
+// contiguous and aligned (rows of a ragged tile), element by element for the others.
 __device__ __attribute__((noinline)) vf8 slab_load_slow(uint64_t addr, uint32_t dtype, uint32_t sn, uint64_t off, uint32_t ncol, uint32_t ok) {
   vf8 out;
+  const uint32_t esz = elem_size(dtype);
+  if (ok != 0 && ncol == 8 && sn == 1 && esz != 1 && ((addr + off * esz) & 15u) == 0) {
+    if (esz == 4) {
+      const DVM_GLOBAL vf4 *p = reinterpret_cast<const DVM_GLOBAL vf4 *>(addr + off * 4);
+      const vf4 a = p[0], b = p[1];
+      return vf8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    }
+    const vu4 a = *reinterpret_cast<const DVM_GLOBAL vu4 *>(addr + off * 2);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = cvt_in(dtype, (a[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+    return out;
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float v = 0.0f;
@@ -513,6 +438,19 @@ __device__ __attribute__((noinline)) vf8 slab_load_slow(uint64_t addr, uint32_t 
 
 __device__ __attribute__((noinline)) void slab_store_slow(uint64_t addr, uint32_t dtype, uint32_t sn, uint64_t off, uint32_t ncol, uint32_t ok, vf8 x) {
   if (ok == 0) return;
+  const uint32_t esz = elem_size(dtype);
+  if (ncol == 8 && sn == 1 && esz != 1 && ((addr + off * esz) & 15u) == 0) {
+    if (esz == 4) {
+      DVM_GLOBAL vf4 *p = reinterpret_cast<DVM_GLOBAL vf4 *>(addr + off * 4);
+      p[0] = vf4{x[0], x[1], x[2], x[3]};
+      p[1] = vf4{x[4], x[5], x[6], x[7]};
+    } else if (dtype == VDT_F16) {
+      *reinterpret_cast<DVM_GLOBAL vu4 *>(addr + off * 2) = vu4{pack_f16(x[0], x[1]), pack_f16(x[2], x[3]), pack_f16(x[4], x[5]), pack_f16(x[6], x[7])};
+    } else {
+      *reinterpret_cast<DVM_GLOBAL vu4 *>(addr + off * 2) = vu4{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7])};
+    }
+    return;
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     if (static_cast<uint32_t>(e) >= ncol) continue;
@@ -994,10 +932,9 @@ __device__ __forceinline__ void run_epilogue(typename SlabVec<SL>::type acc, con
 // returns true; otherwise the caller sends the slabs through epilogue_pass, which does the same with every guard.
 // A function of its own, and a small one: what a call costs is the registers the callee has to save (the interpreter's
 // pass saves and restores some hundred per lane through scratch memory, 12 us per tile and launch on MI355X).
-template <int ROWS, int BN, int TM, int WM, int D16>
+template <int ROWS, int BN, int TM, int WM, int NTHR, int D16>
 __device__ __attribute__((noinline)) bool epilogue_plain_pass(const void *dump, const uint32_t *prog32, EpiArgs ea, uint32_t m0, uint32_t n0,
                                                               uint32_t pass, uint32_t m, uint32_t n, uint32_t m_lo, uint32_t n_lo) {
-  constexpr int NTHR = WM * 2 * 64;
   constexpr int GROUPS = BN / 8;
   constexpr int PER_THREAD = ROWS * GROUPS / NTHR;
   constexpr int ROWS_PER_STEP = NTHR / GROUPS;
@@ -1104,21 +1041,20 @@ __device__ __attribute__((noinline)) bool epilogue_plain_pass(const void *dump, 
 
 // Second half of a pass: the half tile sits in local memory, row major with PITCH floats per row;
 // every lane takes slabs of 8 columns and walks the epilogue program over them.
-template <int ROWS, int BN, int TM, int WM, bool SLIM, int D16>
+template <int ROWS, int BN, int TM, int WM, int NTHR, bool SLIM, int D16>
 __device__ __forceinline__ void epilogue_pass_body(const void *dump, const uint32_t *prog32, EpiArgs ea, uint32_t m0, uint32_t n0,
                                                         uint32_t pass, uint32_t m, uint32_t n, uint32_t m_lo, uint32_t n_lo) {
-  constexpr int NTHR = WM * 2 * 64;
+  constexpr bool ALONE = NTHR == 256 && ROWS * BN * (D16 != 0 ? 1 : 2) == 256 * 256;  // the tile of four waves: one per SIMD
   constexpr int GROUPS = BN / 8;               // slabs per row
   constexpr int PER_THREAD = ROWS * GROUPS / NTHR;  // slabs per thread
   // four slabs per walk of the program where a wave may use all 512 registers; with two waves per SIMD two slabs
-  constexpr int SL = (PER_THREAD % 4 == 0 && (WM == 2 || SLIM)) ? 4 : 2;
+  constexpr int SL = (PER_THREAD % 4 == 0 && (ALONE || SLIM)) ? 4 : 2;
   static_assert(PER_THREAD % SL == 0, "slab count per thread");
   constexpr int ROWS_PER_STEP = NTHR / GROUPS;  // rows one step of all threads covers
   const uint32_t tid = threadIdx.x;
   const uint32_t g = tid % GROUPS, r0 = tid / GROUPS;
   constexpr int HALF = ROWS / WM;  // local rows [i * HALF, (i + 1) * HALF) belong to the i-th row of waves
   const uint32_t col = n0 + g * 8;
-  // (a tile moved back from the edge starts its columns a whole number of slabs before n_lo)
   const uint32_t ncol = (col >= n || col < n_lo) ? 0u : (n - col < 8u ? n - col : 8u);
   {
     const uint32_t *code32 = prog32 + 2 * ea.code_off;
@@ -1149,39 +1085,41 @@ __device__ __forceinline__ void epilogue_pass_body(const void *dump, const uint3
   }
 }
 
-template <int ROWS, int BN, int TM, int WM, bool SLIM, int D16>
+template <int ROWS, int BN, int TM, int WM, int NTHR, bool SLIM, int D16>
 __device__ __attribute__((noinline)) void epilogue_pass(const void *dump, const uint32_t *prog32, EpiArgs ea, uint32_t m0, uint32_t n0,
                                                         uint32_t pass, uint32_t m, uint32_t n, uint32_t m_lo, uint32_t n_lo) {
-  epilogue_pass_body<ROWS, BN, TM, WM, SLIM, D16>(dump, prog32, ea, m0, n0, pass, m, n, m_lo, n_lo);
+  epilogue_pass_body<ROWS, BN, TM, WM, NTHR, SLIM, D16>(dump, prog32, ea, m0, n0, pass, m, n, m_lo, n_lo);
 }
 
-// TM x TN 32x32 MFMA tiles per wave, 2 x 2 waves per workgroup; A_KC / B_KC: the operand's k axis is
+// TM x TN 32x32 MFMA tiles per wave, WM x WN waves per workgroup; A_KC / B_KC: the operand's k axis is
 // contiguous in memory.
 // COMB: the build for the second launch of a product with a split k axis (it sums the partial tiles and runs the
 // epilogue; no operand is read). A kernel of its own, so that the registers the sum holds in flight do not weigh on
 // the allocation of the tile loop (in one kernel with it the 256-tile product without a split lost 5 %).
-template <bool IS_BF16, int TM, int TN, bool A_KC, bool B_KC, int WM, bool COMB = false>
+template <bool IS_BF16, int TM, int TN, bool A_KC, bool B_KC, int WM, int WN, uint32_t TILE, bool COMB = false>
 __device__ __forceinline__ void vm_cube(const VmParam &p) {
-  constexpr int NTHR = WM * 2 * 64;  // WM x 2 waves
-  constexpr int BM = WM * TM * 32, BN = 2 * TN * 32;
+  constexpr int NTHR = WM * WN * 64;
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
   constexpr int PASSES = TM >= 2 ? 2 : 1;
+  static_assert(BM == DVM_CUBE_TILE_SIDE(TILE) && BN == BM && NTHR == (COMB ? 256 : DVM_CUBE_TILE_LANES(TILE)), "the tile's shape");
   constexpr int PROWS = BM / PASSES;  // rows of the tile one epilogue pass covers
   constexpr int PITCH = BN + 4;
-  extern __shared__ double lds_raw[];
+  extern __shared__ __align__(256) double lds_raw[];
   __shared__ uint32_t prog32[DVM_PARAM_BYTES / 4];
   {
-    // only the words the program occupies are read: the argument segment is far away
+    // only the words the program occupies are read (the argument segment is far away), the first of them without waiting
+    // for the header to say how many they are
     const uint32_t *src = reinterpret_cast<const uint32_t *>(p.w);
-    const VCubeHeader *hp = reinterpret_cast<const VCubeHeader *>(p.w);
-    uint32_t used = (hp->code_off + hp->n_code) * 2;
-    used = used < DVM_PARAM_BYTES / 4 ? used : DVM_PARAM_BYTES / 4;
-    const uint32_t trips = (used + NTHR - 1) / NTHR;
-    for (uint32_t t = 0; t < trips; ++t) {
-      uint32_t i = t * NTHR + threadIdx.x;
-      i = i < used ? i : used - 1;
-      prog32[i] = src[i];
-    }
+    static_assert(NTHR <= DVM_PARAM_BYTES / 4 && sizeof(VCubeHeader) <= NTHR * 4, "one word a lane holds the header");
+    prog32[threadIdx.x] = src[threadIdx.x];
     __syncthreads();
+    const VCubeHeader *hp = reinterpret_cast<const VCubeHeader *>(prog32);
+    uint32_t used = uni((hp->code_off + hp->n_code) * 2);
+    used = used < DVM_PARAM_BYTES / 4 ? used : DVM_PARAM_BYTES / 4;
+    if (used > NTHR) {
+      for (uint32_t i = NTHR + threadIdx.x; i < used; i += NTHR) prog32[i] = src[i];
+      __syncthreads();
+    }
   }
   VCubeHeader h;
   {
@@ -1195,7 +1133,7 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
   // summed up, every value clipped into the axis the groups split), behind the tile buffers in local memory. Groups of
   // rows get a second table behind the first: how many rows of tiles the groups up to and including g touch (a tile a
   // bound runs through counts for both sides), so that the work items are exactly the tiles that have rows to store.
-  uint32_t *gtab = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds_raw) + DVM_CUBE_LDS_BYTES(static_cast<uint32_t>(BM)));
+  uint32_t *gtab = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds_raw) + DVM_CUBE_LDS_BYTES(TILE));
   const uint32_t gmode = COMB ? static_cast<uint32_t>(VCG_NONE) : h.group_mode;
   const bool g_rows = gmode == VCG_M_BOUND || gmode == VCG_M_SIZE;
   uint32_t *gpre = gtab + h.nb1;
@@ -1239,12 +1177,11 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       __syncthreads();
     }
   }
-  // [A buffer 0 | A buffer 1 | B buffer 0 | B buffer 1], offsets in elements
-  constexpr uint32_t kABuf = BM * BK, kBBuf = BN * BK, kBBase = 2 * kABuf;
+  constexpr uint32_t kBBase = BM * BK;  // the guarded walk's staging: [A tile | B tile], offset in elements
 
   const uint32_t tid = threadIdx.x;
   const uint32_t wave = tid >> 6, lane = tid & 63u;
-  const uint32_t wm = wave >> 1, wn = wave & 1u;
+  const uint32_t wm = wave / WN, wn = wave % WN;
   // (groups of rows: the rows of tiles the groups touch, one after the other, stand in for the tile rows of one matrix)
   const uint32_t tile_rows = g_rows ? uni(gpre[h.nb1 - 1u]) : h.tiles_m;
   const uint32_t tiles_per_batch = tile_rows * h.tiles_n;
@@ -1257,9 +1194,8 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
   // 23.0 / 20.4 us (84 MB), [300,3000] x [3000,1000] 34.2 / 11.3 us, [1100,4096] x [4096,2056] 72.0 / 15.6 us,
   // [8,8192] x [8192,8192] in four parts 8.3 / 7.4 us.
   const bool split_part = !COMB && (h.epi_flags & VCF_SPLITK_PARTIAL) != 0u;
-  const bool a_kc = COMB ? h.trans_a == 0u : A_KC;
-  const uint32_t part_bm = !COMB ? static_cast<uint32_t>(BM) : (h.tile == 1u ? 128u : (h.tile == 2u ? 64u : 256u));  // the tile the partials come from
-  const uint32_t side_log2 = !COMB ? 0u : (h.tile == 1u ? 1u : (h.tile == 2u ? 0u : 2u));  // pieces along its side
+  const uint32_t part_bm = !COMB ? static_cast<uint32_t>(BM) : DVM_CUBE_TILE_SIDE(h.tile);  // the tile the partials come from
+  const uint32_t side_log2 = !COMB ? 0u : (DVM_CUBE_TILE_SIDE(h.tile) == 128u ? 1u : (h.tile == 2u ? 0u : 2u));  // pieces along its side
   const uint32_t n_work = split_part ? n_tiles * h.k_split : n_tiles << (2u * side_log2);
   constexpr uint32_t kPartVecs = TM * TN * 4;  // 16-byte vectors a lane holds of the tile
 
@@ -1275,12 +1211,14 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
   };
 
   for (uint32_t t0 = blockIdx.x; t0 < n_work; t0 += gridDim.x) {
-    // Tile order. Workgroups are dealt to the 8 XCDs round robin, each XCD has its own L2: workgroup w
-    // takes position (w % 8) * (n_tiles / 8) + w / 8, so an XCD works through one contiguous eighth of the
-    // order; the order itself walks 8-tile-wide column bands row by row, which makes the 32 tiles an XCD has
+    // Tile order. Workgroups are dealt to the 8 XCDs round robin, each XCD has its own L2: an XCD works through one
+    // contiguous eighth of the order (the first n_work % 8 of them through one more); the order itself walks 8-tile-wide column bands row by row, which makes the 32 tiles an XCD has
     // in flight a 4 x 8 block (12 operand panels to fetch instead of 18 for two full rows of 16).
     uint32_t t = t0;
-    if (!COMB && (n_work & 7u) == 0 && gridDim.x >= n_work) t = (t0 & 7u) * (n_work >> 3) + (t0 >> 3);
+    if (!COMB && gridDim.x >= n_work) {
+      const uint32_t xcd = t0 & 7u, more = n_work & 7u;
+      t = xcd * (n_work >> 3) + (xcd < more ? xcd : more) + (t0 >> 3);
+    }
     const uint32_t piece = t & ((1u << (2u * side_log2)) - 1u);  // (0 of 1 unless the launch combines)
     t >>= 2u * side_log2;
     const uint32_t ksplit = t / n_tiles;  // which part of the k axis (0 unless the launch writes partials)
@@ -1308,10 +1246,6 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       const uint32_t first_row = lo != 0u ? uni(gtab[lo - 1u]) : 0u;
       tm = first_row / BM + (tm - (lo != 0u ? uni(gpre[lo - 1u]) : 0u));
     }
-    // A ragged tile at the bottom or right edge is moved back inside the output (it overlaps its neighbour) so that
-    // it can take the vector path like any full tile; its epilogue covers only the rows from m_lo and the columns
-    // from n_lo on, the part no other tile writes. (Columns move in whole 8-element slabs only; an operand whose
-    // rows are the contiguous axis needs the new origin 16-byte aligned.)
     uint32_t m0 = tm * part_bm, n0 = tn * part_bm;
     uint32_t m_lo = m0, m_end = h.m;  // the rows of the output this tile stores
     const uint32_t n_lo = n0;
@@ -1333,15 +1267,11 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
         k_fast = (k_lo & 7u) == 0u && k_hi > k_lo && ((k_hi - k_lo) & 63u) == 0u;
       }
     }
-    if (h.fast) {
-      if (m0 + part_bm > h.m && h.m >= part_bm && (a_kc || (h.m & 7u) == 0)) m0 = h.m - part_bm;
-      if (n0 + part_bm > h.n && h.n >= part_bm && (h.n & 7u) == 0) n0 = h.n - part_bm;
-    }
     const uint32_t piece_m = piece >> side_log2, piece_n = piece & ((1u << side_log2) - 1u);
     if constexpr (COMB) {
       m0 += piece_m * BM;
       n0 += piece_n * BN;
-      if (m0 >= h.m || n0 >= h.n || m0 + BM <= m_lo || n0 + BN <= n_lo) continue;
+      if (m0 >= h.m || n0 >= h.n) continue;
     }
     const uint64_t a_base = h.a_addr + (static_cast<uint64_t>(bi0) * h.a_sb0 + static_cast<uint64_t>(bi1) * h.a_sb1) * 2;
     const uint64_t b_base = h.b_addr + (static_cast<uint64_t>(bi0) * h.b_sb0 + static_cast<uint64_t>(bi1) * h.b_sb1) * 2;
@@ -1352,12 +1282,11 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = 0.0f;
 
-    constexpr bool RING = BM == 256 && BN == 256;  // the ring of 32-deep stages
-    // The smallest tile also takes the vector path when an operand with contiguous k has fewer rows than the tile
-    // (one to 63 rows of A against a weight matrix): the rows past the end fetch the last valid row.
-    constexpr bool a_clamps = !RING && A_KC && (BM * BK / 8 / NTHR) <= 2, b_clamps = !RING && B_KC && (BN * BK / 8 / NTHR) <= 2;
     const uint32_t a_rows = h.m - m0 < static_cast<uint32_t>(BM) ? h.m - m0 : static_cast<uint32_t>(BM);
     const uint32_t b_rows = h.n - n0 < static_cast<uint32_t>(BN) ? h.n - n0 : static_cast<uint32_t>(BN);
+    // The ring takes whole 16-byte chunks: of an operand whose rows are the contiguous axis in memory (k strided), a last
+    // chunk that is not whole is in a ragged tile's way.
+    const bool ring_rows = (A_KC || m0 + BM <= h.m || (h.m & 7u) == 0u) && (B_KC || n0 + BN <= h.n || (h.n & 7u) == 0u);
     // The guarded walk over a part of the k axis: any start, any length, rows and columns past the edges read as zero.
     const uint32_t a_vec = ((h.lda & 7u) == 0u && (a_base & 15u) == 0u) ? 1u : 0u;
     const uint32_t b_vec = ((h.ldb & 7u) == 0u && (b_base & 15u) == 0u) ? 1u : 0u;
@@ -1385,7 +1314,7 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     // its middle, the guarded walk the few k in front (up to the next multiple of 8) and behind (less than a step).
     uint32_t tail_lo = 0, tail_hi = 0;
     if constexpr (!COMB) {
-      if (!g_rows && gmode != VCG_NONE && !k_fast && h.fast && k_hi > k_lo && (m0 + BM <= h.m || a_clamps) && (n0 + BN <= h.n || b_clamps)) {
+      if (!g_rows && gmode != VCG_NONE && !k_fast && h.fast && k_hi > k_lo && ring_rows) {
         const uint32_t up8 = (k_lo + 7u) & ~7u;
         const uint32_t f_lo = up8 < k_hi ? up8 : k_hi;
         const uint32_t f_hi = f_lo + ((k_hi - f_lo) & ~63u);
@@ -1399,7 +1328,6 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
         }
       }
     }
-    const uint32_t nk = (k_hi - k_lo + BK - 1) / BK;
     // address of element (row0, k_lo) of each operand
     const uint64_t a_org = a_base + (A_KC ? static_cast<uint64_t>(m0) * h.lda + k_lo : static_cast<uint64_t>(k_lo) * h.lda + m0) * 2;
     const uint64_t b_org = b_base + (B_KC ? static_cast<uint64_t>(n0) * h.ldb + k_lo : static_cast<uint64_t>(k_lo) * h.ldb + n0) * 2;
@@ -1408,11 +1336,15 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       // two along the columns, TM x TN fragments each) left its lanes' registers.
       static_assert(TM == 1 && TN == 1, "a piece is one fragment per wave");
       const uint32_t w = uni(wave), fr = piece_m * 2u + (w >> 1), fc = piece_n * 2u + (w & 1u);
-      const uint32_t ptm_log2 = h.tile == 0u ? 2u : (h.tile == 2u ? 0u : 1u), ptn_log2 = h.tile == 1u ? 1u : (h.tile == 2u ? 0u : 2u);
+      // (log2 of the fragments of a wave along m and n, and of the waves along n; lanes of the tile's kernel)
+      const bool wide_waves = DVM_CUBE_WAVES_2X4(h.tile, h.trans_b);
+      const uint32_t ptm_log2 = h.tile == 0u || wide_waves ? 2u : (h.tile == 2u ? 0u : 1u);
+      const uint32_t ptn_log2 = DVM_CUBE_TILE_SIDE(h.tile) == 128u || wide_waves ? 1u : (h.tile == 2u ? 0u : 2u);
+      const uint32_t pwn_log2 = wide_waves ? 2u : 1u;
       const uint32_t plane = h.tile == 3u ? 512u : 256u;
       const uint64_t tile_vecs = static_cast<uint64_t>(part_bm) * part_bm / 4u, split_stride = n_tiles * tile_vecs;
       const uint64_t at_vec = tile_id * tile_vecs + ((((fr & ((1u << ptm_log2) - 1u)) << ptn_log2) + (fc & ((1u << ptn_log2) - 1u))) * 4u) * plane +
-                              ((fr >> ptm_log2) * 2u + (fc >> ptn_log2)) * 64u;
+                              (((fr >> ptm_log2) << pwn_log2) + (fc >> ptn_log2)) * 64u;
       uint64_t frag = h.part_addr + at_vec * sizeof(vf4);  // the same in all lanes; lane l's vector is l further
       // groups of eight rows that hold rows of the output (what lies past its end was not written)
       const uint32_t f_row = m0 + (w >> 1) * 32u;
@@ -1455,154 +1387,8 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       else if (groups == 2u) add_parts(std::integral_constant<int, 2>{});
       else if (groups == 1u) add_parts(std::integral_constant<int, 1>{});
     } else {
-    if (h.fast && k_fast && (m0 + BM <= h.m || a_clamps) && (n0 + BN <= h.n || b_clamps)) {
-     if constexpr (RING) {
-      tile_loop_ring<IS_BF16, A_KC, B_KC, WM>(acc, lds, a_org, b_org, h.lda, h.ldb, (k_hi - k_lo) / SK, tid);
-     } else {
-      Stage<BM, A_KC, NTHR> sa;
-      Stage<BN, B_KC, NTHR> sb;
-      // k advances by BK per step
-      const uint64_t a_step = (A_KC ? static_cast<uint64_t>(BK) : static_cast<uint64_t>(BK) * h.lda) * 2;
-      const uint64_t b_step = (B_KC ? static_cast<uint64_t>(BK) : static_cast<uint64_t>(BK) * h.ldb) * 2;
-      LaneOffsets a_voff, b_voff;
-      if constexpr (A_KC) a_voff = Stage<BM, A_KC, NTHR>::lane_offset(h.lda, tid, a_rows);
-      else a_voff = Stage<BM, A_KC, NTHR>::lane_offset(h.lda, tid);
-      if constexpr (B_KC) b_voff = Stage<BN, B_KC, NTHR>::lane_offset(h.ldb, tid, b_rows);
-      else b_voff = Stage<BN, B_KC, NTHR>::lane_offset(h.ldb, tid);
-      sa.fetch(a_org, h.lda, a_voff, tid, lds);
-      sb.fetch(b_org, h.ldb, b_voff, tid, lds + kBBase);
-      sa.commit(lds, tid);
-      sb.commit(lds + kBBase, tid);
-      if (nk > 1) {
-        sa.fetch(a_org + a_step, h.lda, a_voff, tid, lds + kABuf);
-        sb.fetch(b_org + b_step, h.ldb, b_voff, tid, lds + kBBase + kBBuf);
-      }
-      __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): direct loads are not waited for by the barrier itself
-      __syncthreads();
-      vu4 af[2][TM], bf[2][TN];
-      auto read_frags = [&](int fb, uint32_t buf, int kk) {
-        const uint16_t *ab = lds + buf * kABuf, *bb = lds + buf * kBBuf;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) af[fb][i] = *reinterpret_cast<const vu4 *>(ab + frag_off(a_row, a_x, i, kk));
-#pragma unroll
-        for (int j = 0; j < TN; ++j) bf[fb][j] = *reinterpret_cast<const vu4 *>(bb + frag_off(b_row, b_x, j, kk));
-      };
-      auto mfmas = [&](int fb) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = mfma<IS_BF16>(af[fb][i], bf[fb][j], acc[i][j]);
-      };
-      // One k tile (4 steps of 16). Step s runs its MFMAs on fragment buffer s&1 while the reads of
-      // step s+1 land in the other one. A k-strided operand's tile kt+1 is written to the other
-      // local-memory buffer during step 1 (its global loads were issued three steps earlier) and the
-      // global loads of its tile kt+2 follow in step 2; the workgroup meets before step 3, which overlaps
-      // the first fragment reads of tile kt+1 and sends the direct loads of tile kt+2 of a k-contiguous
-      // operand into the buffer that has just been read for the last time (a whole tile of slack).
-      // The group barriers pin that interleaving: the scheduler would otherwise serialise each read
-      // against its use to save registers, and with one wave per SIMD nothing else hides the latency.
-      auto k_tile = [&](uint32_t kt, auto has_next, auto has_next2) {
-        constexpr bool NEXT = decltype(has_next)::value, NEXT2 = decltype(has_next2)::value;
-        constexpr int NF = TM + TN, NM = TM * TN;
-        const uint32_t cur = kt & 1u;
-        constexpr int NREST = NM - NF > 0 ? NM - NF : 1;  // MFMAs left in a step after the fragment reads
-        // staging instructions per such MFMA: ds_write of a k-strided operand (step 1), its global loads
-        // (step 2), direct-to-LDS loads of a k-contiguous operand (step 3)
-        constexpr int NW = ((A_KC ? 0 : Stage<BM, false, NTHR>::N_WRITES) + (B_KC ? 0 : Stage<BN, false, NTHR>::N_WRITES) + NREST - 1) / NREST;
-        constexpr int NL = ((A_KC ? 0 : 8) + (B_KC ? 0 : 8) + NREST - 1) / NREST;
-        constexpr int ND = ((A_KC ? Stage<BM, true, NTHR>::N : 0) + (B_KC ? Stage<BN, true, NTHR>::N : 0) + NREST - 1) / NREST;
-        // step 0
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(1, cur, 1);
-        mfmas(0);
-#pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, NM - NF > 0 ? NM - NF : 0, 0);
-        // step 1: tile kt+1 (loaded during the previous tile) goes to the other buffer
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(0, cur, 2);
-        if constexpr (NEXT) {
-          sa.commit(lds + (cur ^ 1u) * kABuf, tid);
-          sb.commit(lds + kBBase + (cur ^ 1u) * kBBuf, tid);
-        }
-        mfmas(1);
-#pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        if constexpr (NEXT && NW > 0) {
-#pragma unroll
-          for (int q = 0; q < NREST; ++q) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, NW, 0);
-          }
-        }
-        // step 2: the staging registers are free again: tile kt+2 starts its way from memory
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(1, cur, 3);
-        if constexpr (NEXT2 && !A_KC) sa.fetch(a_org + (kt + 2) * a_step, h.lda, a_voff, tid, lds);
-        if constexpr (NEXT2 && !B_KC) sb.fetch(b_org + (kt + 2) * b_step, h.ldb, b_voff, tid, lds);
-        mfmas(0);
-#pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        if constexpr (NEXT2 && NL > 0) {
-#pragma unroll
-          for (int q = 0; q < NREST; ++q) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, NL, 0);
-          }
-        }
-        // step 3: every wave has read its last fragments of this buffer and written its share of the
-        // next one a step ago; meet, then start on the next tile's fragments under the last MFMAs
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NEXT) {
-          // the direct loads of tile kt+1 (issued a tile ago) must have landed before anyone reads them; the
-          // only younger memory operations of this wave are the step-2 loads of a k-strided operand
-          if constexpr (A_KC || B_KC) {
-            constexpr int YOUNGER = (BM == 256 && BN == 256 && NEXT2) ? ((A_KC ? 0 : 8) + (B_KC ? 0 : 8)) : 0;
-            __builtin_amdgcn_s_waitcnt((YOUNGER & 0xf) | ((YOUNGER >> 4) << 14) | (7 << 4) | (15 << 8));
-          }
-          __syncthreads();
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NEXT) read_frags(0, cur ^ 1u, 0);
-        // this buffer has been read for the last time: tile kt+2 of a k-contiguous operand starts its way into it
-        if constexpr (NEXT2 && A_KC) sa.fetch(a_org + (kt + 2) * a_step, h.lda, a_voff, tid, lds + cur * kABuf);
-        if constexpr (NEXT2 && B_KC) sb.fetch(b_org + (kt + 2) * b_step, h.ldb, b_voff, tid, lds + kBBase + cur * kBBuf);
-        mfmas(1);
-        if constexpr (NEXT) {
-#pragma unroll
-          for (int q = 0; q < NF; ++q) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          }
-        }
-        if constexpr (NEXT2 && ND > 0) {
-#pragma unroll
-          for (int q = 0; q < NREST; ++q) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, ND, 0);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      read_frags(0, 0, 0);
-      uint32_t kt = 0;
-      for (; kt + 2 < nk; ++kt) k_tile(kt, std::true_type{}, std::true_type{});
-      if (kt + 1 < nk) {
-        k_tile(kt, std::true_type{}, std::false_type{});
-        ++kt;
-      }
-      k_tile(kt, std::false_type{}, std::false_type{});
-      __syncthreads();
-     }
+    if (h.fast && k_fast && ring_rows) {
+      tile_loop_ring<IS_BF16, A_KC, B_KC, TM, TN, WM, WN, DVM_CUBE_STAGES(TILE)>(acc, lds, a_org, b_org, h.lda, h.ldb, a_rows, b_rows, k_hi - k_lo, tid);
     } else {
       guarded_walk(k_lo, k_hi);
     }
@@ -1612,7 +1398,7 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
     if (split_part) {
       DVM_GLOBAL vf4 *dst = reinterpret_cast<DVM_GLOBAL vf4 *>(h.part_addr) +
                             (static_cast<uint64_t>(ksplit) * n_tiles + tile_id) * kPartVecs * NTHR + tid;
-      const uint32_t w_row = m0 + (uni(wave) >> 1) * TM * 32u;
+      const uint32_t w_row = m0 + (uni(wave) / WN) * TM * 32u;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -1675,11 +1461,11 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (!(h.epi_flags & VCF_PLAIN_STORE) || !epilogue_plain_pass<BM, BN, TM, WM, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo)) {
+      if (!(h.epi_flags & VCF_PLAIN_STORE) || !epilogue_plain_pass<BM, BN, TM, WM, NTHR, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo)) {
         if (h.epi_flags & VCF_SLIM) {
-          epilogue_pass_body<BM, BN, TM, WM, true, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo);
+          epilogue_pass_body<BM, BN, TM, WM, NTHR, true, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo);
         }
-        else epilogue_pass<BM, BN, TM, WM, false, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo);
+        else epilogue_pass<BM, BN, TM, WM, NTHR, false, D16K>(tile16, prog32, ea, m0, n0, 0, m_end, h.n, m_lo, n_lo);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       continue;
@@ -1703,9 +1489,9 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
       // before the next dump): they wait for this wave's local-memory operations and not, as __syncthreads() would,
       // for its stores to memory as well, which stay in flight under the next pass and the next tile's loop.
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (!(h.epi_flags & VCF_PLAIN_STORE) || !epilogue_plain_pass<PROWS, BN, TM, WM, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo)) {
-        if (h.epi_flags & VCF_SLIM) epilogue_pass<PROWS, BN, TM, WM, true, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo);
-        else epilogue_pass<PROWS, BN, TM, WM, false, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo);
+      if (!(h.epi_flags & VCF_PLAIN_STORE) || !epilogue_plain_pass<PROWS, BN, TM, WM, NTHR, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo)) {
+        if (h.epi_flags & VCF_SLIM) epilogue_pass<PROWS, BN, TM, WM, NTHR, true, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo);
+        else epilogue_pass<PROWS, BN, TM, WM, NTHR, false, 0>(dump, prog32, ea, m0, n0, ps, m_end, h.n, m_lo, n_lo);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -1714,26 +1500,34 @@ __device__ __forceinline__ void vm_cube(const VmParam &p) {
 
 }  // namespace
 
-// `occ` = waves per SIMD the register budget must leave room for (two workgroups of the 64x64 tile share a compute unit:
-// 256 registers a lane, vector and accumulation registers together)
-#define DVM_CUBE_KERNEL(name, bf, tm, tn, wm, occ, akc, bkc) \
-  extern "C" __global__ void __launch_bounds__(wm * 128, occ) name(const VmParam p) { vm_cube<bf, tm, tn, akc, bkc, wm>(p); }
-#define DVM_CUBE_LAYOUTS(prefix, bf, tm, tn, wm, occ)            \
-  DVM_CUBE_KERNEL(prefix##_nn, bf, tm, tn, wm, occ, true, false) \
-  DVM_CUBE_KERNEL(prefix##_nt, bf, tm, tn, wm, occ, true, true)  \
-  DVM_CUBE_KERNEL(prefix##_tn, bf, tm, tn, wm, occ, false, false) \
-  DVM_CUBE_KERNEL(prefix##_tt, bf, tm, tn, wm, occ, false, true)
+// `occ` = waves per SIMD the register budget must leave room for (two workgroups of the 64x64 and 128x128 tiles share a
+// compute unit: 256 registers a lane, vector and accumulation registers together)
+#define DVM_CUBE_KERNEL(name, tile, bf, tm, tn, wm, wn, occ, akc, bkc) \
+  extern "C" __global__ void __launch_bounds__(wm * wn * 64, occ) name(const VmParam p) { vm_cube<bf, tm, tn, akc, bkc, wm, wn, tile>(p); }
+#define DVM_CUBE_LAYOUTS(prefix, tile, bf, tm, tn, wm, wn, occ)            \
+  DVM_CUBE_KERNEL(prefix##_nn, tile, bf, tm, tn, wm, wn, occ, true, false) \
+  DVM_CUBE_KERNEL(prefix##_nt, tile, bf, tm, tn, wm, wn, occ, true, true)  \
+  DVM_CUBE_KERNEL(prefix##_tn, tile, bf, tm, tn, wm, wn, occ, false, false) \
+  DVM_CUBE_KERNEL(prefix##_tt, tile, bf, tm, tn, wm, wn, occ, false, true)
 
-#define DVM_CUBE_COMB(name, bf, tm, tn, wm, occ) \
-  extern "C" __global__ void __launch_bounds__(wm * 128, occ) name(const VmParam p) { vm_cube<bf, tm, tn, true, false, wm, true>(p); }
-DVM_CUBE_COMB(dvm_vm_cube_bf16_comb, true, 1, 1, 2, 3)
-DVM_CUBE_COMB(dvm_vm_cube_f16_comb, false, 1, 1, 2, 3)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_big, true, 4, 4, 2, 1)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_big, false, 4, 4, 2, 1)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_mid, true, 2, 2, 2, 1)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_mid, false, 2, 2, 2, 1)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_small, true, 1, 1, 2, 2)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_small, false, 1, 1, 2, 2)
-// the 256x256 tile on eight waves (4 x 2, 64x128 accumulators each): two waves per SIMD
-DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_big8, true, 2, 4, 4, 2)
-DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_big8, false, 2, 4, 4, 2)
+#define DVM_CUBE_COMB(name, bf, occ) \
+  extern "C" __global__ void __launch_bounds__(256, occ) name(const VmParam p) { vm_cube<bf, 1, 1, true, false, 2, 2, 2u, true>(p); }
+DVM_CUBE_COMB(dvm_vm_cube_bf16_comb, true, 3)
+DVM_CUBE_COMB(dvm_vm_cube_f16_comb, false, 3)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_big, 0u, true, 4, 4, 2, 2, 1)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_big, 0u, false, 4, 4, 2, 2, 1)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_mid, 1u, true, 2, 2, 2, 2, 2)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_mid, 1u, false, 2, 2, 2, 2, 2)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_deep, 4u, true, 2, 2, 2, 2, 2)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_deep, 4u, false, 2, 2, 2, 2, 2)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_bf16_small, 2u, true, 1, 1, 2, 2, 2)
+DVM_CUBE_LAYOUTS(dvm_vm_cube_f16_small, 2u, false, 1, 1, 2, 2, 2)
+// the 256x256 tile on eight waves: two waves per SIMD. 8192 x 4096 x 4096 with a k-strided B, waves 4 x 2 / 2 x 4:
+// 249 / 239 us with A k-contiguous, 254 / 239 us with A k-strided as well
+#define DVM_CUBE_BIG8(prefix, bf)                               \
+  DVM_CUBE_KERNEL(prefix##_nn, 3u, bf, 4, 2, 2, 4, 2, true, false)  \
+  DVM_CUBE_KERNEL(prefix##_nt, 3u, bf, 2, 4, 4, 2, 2, true, true)   \
+  DVM_CUBE_KERNEL(prefix##_tn, 3u, bf, 4, 2, 2, 4, 2, false, false) \
+  DVM_CUBE_KERNEL(prefix##_tt, 3u, bf, 2, 4, 4, 2, 2, false, true)
+DVM_CUBE_BIG8(dvm_vm_cube_bf16_big8, true)
+DVM_CUBE_BIG8(dvm_vm_cube_f16_big8, false)

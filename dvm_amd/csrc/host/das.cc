@@ -237,11 +237,10 @@ std::string &VKernel::DisAssemble() {
       }
     } else if (h->entry == VE_CUBE) {
       const VCubeHeader *c = reinterpret_cast<const VCubeHeader *>(p.blob.w);
-      static const int tile[] = {256, 128, 64, 256};
       os << "entry cube " << kMemTypes[c->dtype] << " m=" << c->m << " n=" << c->n << " k=" << c->k << " trans_a=" << c->trans_a
-         << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << tile[c->tile] << " blocks="
+         << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << DVM_CUBE_TILE_SIDE(c->tile) << " blocks="
          << ((c->epi_flags & VCF_SPLITK_COMBINE) ? static_cast<uint64_t>(c->tiles_m) * c->tiles_n * c->nb0 * c->nb1 : static_cast<uint64_t>(p.grid))
-         << " lds=" << p.lds_bytes << (c->fast ? " fast" : " guarded") << (c->tile == 3 ? " eight-waves" : "");
+         << " lds=" << p.lds_bytes << (c->fast ? (c->k % 64 != 0 ? " fast guarded-k-end" : " fast") : " guarded") << (c->tile == 3 ? " eight-waves" : "");
       if (c->epi_flags & VCF_PLAIN_STORE) os << " plain-store";
       else if (c->epi_flags & VCF_SLIM) os << " slim-epilogue";
       if (c->epi_flags & VCF_DUMP16) os << " tile-as-16-bit";

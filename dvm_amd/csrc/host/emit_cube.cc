@@ -283,122 +283,114 @@ void Compiler::CompileCube(int a) {
       k_->tuning_.cube_splitk = c.split <= 1 ? 0 : c.split;
     }
   }
-  // block tile: the largest that still gives most compute units a tile
   // (groups of rows: a tile is computed once per group that owns rows of it, so about once: the groups do not multiply the work)
   const uint64_t batch = gmm == 1 ? 1 : static_cast<uint64_t>(h.nb0) * h.nb1;
-  auto tiles = [&](int64_t t) { return static_cast<uint64_t>((M + t - 1) / t) * static_cast<uint64_t>((N + t - 1) / t) * batch; };
+  auto tiles = [&](uint32_t tile) {
+    const int64_t t = DVM_CUBE_TILE_SIDE(tile);
+    return static_cast<uint64_t>((M + t - 1) / t) * static_cast<uint64_t>((N + t - 1) / t) * batch;
+  };
   const uint64_t cus = g_system.core_num;
-  int64_t bt;
-  if (tiles(256) * 4 >= cus * 3) {
-    h.tile = 0;
-    bt = 256;
-  } else if (tiles(128) * 2 >= cus) {
-    h.tile = 1;
-    bt = 128;
-  } else {
-    h.tile = 2;
-    bt = 64;
-  }
-  // ... unless most of such a tile would lie outside the output (batches of small matrices, an output narrower than
-  // the tile): a tile half the size that covers half the area or less wins. Measured on MI355X, fp16 P x V of an
-  // unfused attention, [128,1024,1024] x [128,1024,64]: 299 us on the 256 tile, 416 on 128, 88 on 64;
-  // [256,2048,2048] x [256,2048,128]: 1976 / 858 / 1186 us; [64,512,512] x [64,512,32]: 82 / 56 / 31 us.
-  {
-    auto padded = [&](int64_t t) { return static_cast<double>(tiles(t)) * static_cast<double>(t * t); };
-    while (bt > 64 && padded(bt) >= 2.0 * padded(bt / 2)) {
-      bt /= 2;
-      ++h.tile;
-    }
-  }
-  {  // tuning override: 256, 128 or 64
-    const int v = k_->tuning_.cube_tile;
-    if (v == 256 || v == 128 || v == 64) {
-      bt = v;
-      h.tile = v == 256 ? 0 : (v == 128 ? 1 : 2);
-    }
-  }
-  // The 256x256 tile runs on eight waves (two per SIMD, 64x128 accumulators each) unless DVM_CUBE_WAVES=4 asks for
-  // four (one per SIMD, 128x128): the second wave of a SIMD fills the stalls of the first in the prologue and in
-  // the interpreted epilogue. Measured on MI355X, bf16 8192x4096xk, row-major operands, four -> eight waves:
-  // k = 64: 60 -> 54 us (with bias + SiLU 106 -> 87 us), k = 512: 82 -> 76 us, k = 4096: 296-301 us either way for
-  // the plain product (the sustained rate is set by the power cap there), 338-342 -> 334-339 us with bias + SiLU.
-  // Split k: with fewer tiles than compute units and a long k axis, k_split workgroups share a tile's k axis and a
-  // second launch adds their fp32 partial tiles in a fixed order and runs the epilogue (the reference splits k into
-  // consecutive matmuls accumulating in fp32 when the operands exceed its L2, src/ops_m.cc:240-264,
-  // src/xkernel.cc:1511-1547; here the reason is to fill the chip). Every candidate (tile, parts) gets an estimate
-  // from figures measured on MI355X (bf16, microseconds): a workgroup's time per 64 k (2.2 for the 256 tile, 1.3 for
-  // 128, 0.71 for 64 alone on its compute unit and 0.9 when two share one; the guarded path of ragged or unaligned
-  // tiles takes about two and a half times as long), rounds of workgroups over the chip, and for a split the second launch plus
-  // a time per part of a tile (3.2 / 0.8 / 0.2), plus the time the first launch takes to write the partial tiles (some
-  // 4 TB/s over the whole chip). The times per part were measured while one workgroup summed a tile (some 80 GB/s); the
-  // sum in pieces below costs less for the two larger tiles, so deep splits of those are chosen less often than would pay.
+  // the ring of direct loads takes operands that are whole 16-byte chunks along their contiguous axis; anything else is
+  // staged element by element
+  // (groups along k: every group's range is cut into whole chunks on the device)
+  h.fast = (K > 0 && (gmm == 2 || ((trans_a || K % 8 == 0) && (!trans_b || K % 8 == 0))) && h.lda < (1u << 22) && h.ldb < (1u << 22) &&
+            h.lda % 8 == 0 && h.ldb % 8 == 0 && h.a_sb0 % 8 == 0 && h.a_sb1 % 8 == 0 && h.b_sb0 % 8 == 0 && h.b_sb1 % 8 == 0)
+               ? 1
+               : 0;
   uint32_t k_split = 1, k_chunk = 0;
   {
+    int forced_tile = -1;
+    switch (k_->tuning_.cube_tile) {  // tuning override
+      case 256: forced_tile = 0; break;
+      case 128: forced_tile = 1; break;
+      case 64: forced_tile = 2; break;
+      default: break;
+    }
     const int forced = gmm != 0 ? 0 : k_->tuning_.cube_splitk;  // (the k axis of a grouped product is never shared)
-    const bool user_tile = k_->tuning_.cube_tile == 256 || k_->tuning_.cube_tile == 128 || k_->tuning_.cube_tile == 64;
     auto parts_of = [&](uint32_t want, uint32_t *chunk) -> uint32_t {  // parts actually made when `want` are asked for
       if (want < 2 || K < 128) return 1;
       const int64_t c = ((K + want - 1) / want + 63) / 64 * 64;
       *chunk = static_cast<uint32_t>(c);
       return static_cast<uint32_t>((K + c - 1) / c);
     };
-    if (forced >= 2) {
-      k_split = parts_of(static_cast<uint32_t>(forced), &k_chunk);
-    } else if (forced != 0 && forced != 1) {
-      static const int64_t kTiles[3] = {256, 128, 64};
-      static const double kStepUs[3] = {2.2, 1.3, 0.71}, kPartUs[3] = {3.2, 0.8, 0.2};
-      const bool aligned = K % 64 == 0 && h.lda % 8 == 0 && h.ldb % 8 == 0;
-      double best = 0.0;
-      int best_tile = -1;
-      uint32_t best_split = 1, best_chunk = 0;
-      for (int ti = 0; ti < 3; ++ti) {
-        const int64_t t = kTiles[ti];
-        if (user_tile && t != bt) continue;
-        const uint64_t nt = tiles(t);
-        const uint64_t slots = ti == 2 ? 2 * cus : cus;  // two 64x64 workgroups fit a compute unit
-        const uint32_t max_split = nt >= slots ? 1u : static_cast<uint32_t>(std::min<uint64_t>(slots / nt, 32));
-        // (ragged edge tiles of an aligned product are moved back inside the output and stay on the vector path)
-        // (and the 64 tile fetches the rows of a short operand with contiguous k through clamped addresses)
-        const bool m_fast = M % t == 0 || (M >= t && (!trans_a || M % 8 == 0)) || (t == 64 && !trans_a);
-        const bool n_fast = N % t == 0 || (N >= t && N % 8 == 0) || (t == 64 && trans_b);
-        const double slow = (aligned && m_fast && n_fast) ? 1.0 : 2.5;
-        for (uint32_t want = 1; want <= max_split; want = want < 2 ? 2 : want * 2) {
-          uint32_t chunk = 0;
-          const uint32_t parts = parts_of(want, &chunk);
-          if (want > 1 && (parts < 2 || chunk < 256)) break;
-          const double steps = (parts > 1 ? static_cast<double>(chunk) : static_cast<double>(K)) / 64.0;
-          const uint64_t wgs = nt * parts;
-          const double rounds = std::ceil(static_cast<double>(wgs) / static_cast<double>(slots));
-          const double step_us = (ti == 2 && wgs > cus) ? 0.9 : kStepUs[ti];
-          double us = rounds * steps * step_us * slow + 3.0;
-          if (parts > 1) us += 5.0 + parts * kPartUs[ti] + static_cast<double>(wgs) * static_cast<double>(t * t) * 4.0 / 4.0e6;
-          if (parts > 1 && static_cast<double>(wgs) * static_cast<double>(t * t) * 4.0 > 512.0 * 1024 * 1024) continue;
-          if (best_tile < 0 || us < best) {
-            best = us;
-            best_tile = ti;
-            best_split = parts;
-            best_chunk = chunk;
-          }
+    // Every candidate (tile, parts of the k axis) gets an estimate in microseconds from figures measured on an MI355X (bf16):
+    //  * a workgroup's time per stage of 64 k: alone on its compute unit, and for the two workgroups that share one
+    //    (64 and 128) or on a chip that is more than half full (256: power and the L2s). 4096 x 2048 x 4096: 85-90 us on
+    //    the 256 tile (128 workgroups), 66-69 on 128 (512); 4096 x 4096 x 2048: 64-66 and 73; 1000 x 2000 x 1800: the 64
+    //    tile 22 us (512); 2530 x 920 x 1320: 21.5 on 128 (160 workgroups), 23.9 on 64; 142 x 1576 x 3608: 21 on 64 (75).
+    //    A long k axis brings its operands out of memory rather than the L2s, which the tile that reads them most often
+    //    feels first: 1024 x 1024 x 4096 from operands in no cache, 64 tile 24.5, 128 tile in four parts 23.8 us;
+    //  * operands that are staged element by element (guarded) take several times as long;
+    //  * what a workgroup costs beside its stages (program, first loads, epilogue), and once per launch;
+    //  * a sum of parts: its launch, a trip per part, the partial tiles written and read (4 bytes an element and part).
+    //    812 x 1840 x 3440 on the 128 tile: 49 us in one part, 34 in two, 30 in four (27 MB), 36 in eight;
+    //  * the operands cannot arrive faster than memory delivers them.
+    // Over 42 drawn products the choice is within 1 % of the fastest candidate on average, 5 % at worst.
+    static const double kStage[3][2] = {{1.28, 1.82}, {0.63, 1.08}, {0.26, 0.60}};
+    static const double kGuarded[3] = {8.0, 6.0, 3.0}, kEnds[3][2] = {{4.5, 4.5}, {2.5, 3.5}, {1.5, 2.0}};
+    const bool guarded = h.fast == 0 || (trans_a && M % 8 != 0) || (!trans_b && N % 8 != 0);
+    auto estimate = [&](int ti, uint32_t parts, uint32_t chunk) {
+      const uint64_t side = DVM_CUBE_TILE_SIDE(static_cast<uint32_t>(ti)), wgs = tiles(static_cast<uint32_t>(ti)) * parts;
+      const uint64_t slots = ti == 0 ? cus : 2 * cus;  // (two workgroups of the smaller tiles share a compute unit)
+      const double stages = static_cast<double>(((parts > 1 ? static_cast<int64_t>(chunk) : K) + 63) / 64);
+      auto round = [&](bool crowded) {
+        const double stage = guarded ? kGuarded[ti] : (ti == 2 && !crowded && stages > 48.0 ? 0.32 : kStage[ti][crowded]);
+        return kEnds[ti][crowded] + stages * stage;
+      };
+      const uint64_t rest = wgs % slots;
+      double us = 3.0 + static_cast<double>(wgs / slots) * round(true);
+      if (rest != 0) us += round(wgs > slots || rest > (ti == 0 ? cus / 2 : cus));  // (behind a full round the rest share compute units too)
+      const double a_bytes = static_cast<double>(M) * K * 2 * batch, b_bytes = static_cast<double>(N) * K * 2 * batch;
+      us = std::max(us, 5.0 + (a_bytes + b_bytes) / 5.5e6);
+      const double part_mb = static_cast<double>(wgs) * static_cast<double>(side * side) * 4e-6;
+      if (parts > 1) us += 4.8 + 0.25 * parts + 0.16 * part_mb + 0.2 * std::max(0.0, part_mb - 32.0);
+      return us;
+    };
+    // A call with one launch takes the host some 12 us, with two 18: a product that one launch does in that time is not
+    // split (27 x 1752 x 1736: 18.9 us a call in two launches, 12.6 in one).
+    uint32_t best_tile = 0, best_chunk = 0, one_launch_tile = 0;
+    double best = -1.0, one_launch = -1.0;
+    for (int ti = 0; ti < 3; ++ti) {
+      if (forced_tile >= 0 && ti != forced_tile) continue;
+      const uint64_t side = DVM_CUBE_TILE_SIDE(static_cast<uint32_t>(ti)), nt = tiles(static_cast<uint32_t>(ti));
+      const uint64_t slots = ti == 0 ? cus : 2 * cus;
+      uint32_t max_split = nt >= slots ? 1u : static_cast<uint32_t>(std::min<uint64_t>(slots / nt, 32));
+      if (gmm != 0 || forced == 0 || forced == 1) max_split = 1;
+      for (uint32_t want = 1; want <= max_split || (forced >= 2 && want == 1); ++want) {
+        uint32_t chunk = 0;
+        const uint32_t parts = parts_of(forced >= 2 ? static_cast<uint32_t>(forced) : want, &chunk);
+        if (forced < 2 && want > 1) {
+          if (chunk < (guarded ? 256u : 128u)) break;
+          if (parts < want) continue;  // (whole stages: the same parts as for fewer)
+        }
+        if (forced < 2 && parts > 1 && static_cast<double>(nt) * parts * static_cast<double>(side * side) * 4.0 > 512.0 * 1024 * 1024) continue;
+        const double us = estimate(ti, parts, chunk);
+        if (parts == 1 && (one_launch < 0.0 || us < one_launch)) {
+          one_launch = us;
+          one_launch_tile = static_cast<uint32_t>(ti);
+        }
+        if (best < 0.0 || us < best) {
+          best = us;
+          best_tile = static_cast<uint32_t>(ti);
+          k_split = parts;
+          best_chunk = chunk;
         }
       }
-      // without a split the tile stays the one chosen above
-      if (best_tile >= 0 && best_split > 1) {
-        bt = kTiles[best_tile];
-        h.tile = static_cast<uint32_t>(best_tile);
-        k_split = best_split;
-        k_chunk = best_chunk;
-      }
     }
+    if (k_split > 1 && forced < 2 && one_launch >= 0.0 && one_launch <= 18.0) {
+      best_tile = one_launch_tile;
+      k_split = 1;
+    }
+    h.tile = best_tile;
+    if (k_split > 1) k_chunk = best_chunk;
   }
   if (h.tile == 0 && k_->tuning_.cube_waves != 4) h.tile = 3;
+  // a 128 tile alone on its compute unit has the local memory for four stage buffers: DEEP
+  if (h.tile == 1 && tiles(1) * k_split <= cus) h.tile = 4;
+  const uint32_t bt = DVM_CUBE_TILE_SIDE(h.tile);
   h.tiles_m = static_cast<uint32_t>((M + bt - 1) / bt);
   h.tiles_n = static_cast<uint32_t>((N + bt - 1) / bt);
-  if (tiles(bt) * (gmm == 1 ? h.nb1 : 1) >= (1ull << 31)) Fail("too many matmul tiles");
-  // (groups along k: every group's range decides for itself on the device whether it is whole 64-steps from an aligned start)
-  h.fast = ((K % 64 == 0 || gmm == 2) && K > 0 && h.lda < (1u << 22) && h.ldb < (1u << 22) && h.lda % 8 == 0 && h.ldb % 8 == 0 && h.a_sb0 % 8 == 0 &&
-            h.a_sb1 % 8 == 0 && h.b_sb0 % 8 == 0 && h.b_sb1 % 8 == 0)
-               ? 1
-               : 0;
+  if (tiles(h.tile) * (gmm == 1 ? h.nb1 : 1) >= (1ull << 31)) Fail("too many matmul tiles");
   // operand addresses
   for (int which = 0; which < 2; ++which) {
     const ANode &x = which == 0 ? an : bn;
@@ -535,9 +527,9 @@ void Compiler::CompileCube(int a) {
   std::memcpy(prog_->blob.w, &h, sizeof(h));
   std::memcpy(prog_->blob.w + h.mem_off, cmems_, sizeof(VCubeMem) * n_mem_);
   std::memcpy(prog_->blob.w + h.code_off, code_.data(), 8 * code_.size());
-  prog_->threads = h.tile == 3 ? 512 : 256;
-  prog_->lds_bytes = DVM_CUBE_LDS_BYTES(static_cast<uint32_t>(bt)) + (gmm != 0 ? 8u * h.nb1 : 0u);
-  prog_->grid = static_cast<uint32_t>(tiles(bt));
+  prog_->threads = DVM_CUBE_TILE_LANES(h.tile);
+  prog_->lds_bytes = DVM_CUBE_LDS_BYTES(h.tile) + (gmm != 0 ? 8u * h.nb1 : 0u);
+  prog_->grid = static_cast<uint32_t>(tiles(h.tile));
   if (gmm == 1) {
     // The work items are the tiles that have rows of a group to store, counted on the device from the list: at most
     // one row of tiles more per group than the matrix has (a tile a bound runs through is computed for both sides).
@@ -553,7 +545,7 @@ void Compiler::CompileCube(int a) {
   if (k_split > 1) {
     // two launches of the same program: partial products per part of the k axis, then their sum and the epilogue
     const int slot = static_cast<int>(k_->ws_sizes_.size());
-    k_->ws_sizes_.push_back(static_cast<size_t>(k_split) * tiles(bt) * static_cast<size_t>(bt * bt) * 4);
+    k_->ws_sizes_.push_back(static_cast<size_t>(k_split) * tiles(h.tile) * static_cast<size_t>(bt * bt) * 4);
     Program::Patch pp;
     pp.word = static_cast<uint32_t>(offsetof(VCubeHeader, part_addr) / 8);
     pp.op_id = -1;
@@ -565,7 +557,7 @@ void Compiler::CompileCube(int a) {
     ph->k_chunk = k_chunk;
     const uint32_t flags = ph->epi_flags;
     ph->epi_flags = flags | VCF_SPLITK_PARTIAL;
-    prog_->grid = static_cast<uint32_t>(tiles(bt) * k_split);
+    prog_->grid = static_cast<uint32_t>(tiles(h.tile) * k_split);
     const Program first = *prog_;
     k_->programs_.push_back(first);
     prog_ = &k_->programs_.back();
@@ -574,8 +566,8 @@ void Compiler::CompileCube(int a) {
     // a piece costs beside its bytes is its workgroup's start. (Three run at once, 167 registers a lane: of a full grid
     // every fourth starts when an earlier one ends.)
     prog_->threads = 256;
-    prog_->lds_bytes = DVM_CUBE_LDS_BYTES(64u);
-    prog_->grid = static_cast<uint32_t>(std::min<uint64_t>(tiles(bt) * static_cast<uint64_t>(bt / 64) * (bt / 64), 4 * cus));
+    prog_->lds_bytes = DVM_CUBE_LDS_BYTES(2u);
+    prog_->grid = static_cast<uint32_t>(std::min<uint64_t>(tiles(h.tile) * static_cast<uint64_t>(bt / 64) * (bt / 64), 4 * cus));
     prog_->fills.clear();
   }
 }

@@ -305,11 +305,11 @@ typedef struct {
   uint32_t lda, ldb;   // leading dimensions in elements
   uint32_t nb0, nb1;   // batch extents (outer, inner); 1 when absent
   uint32_t a_sb0, a_sb1, b_sb0, b_sb1;  // batch strides in elements (0 = broadcast)
-  uint32_t tile;       // block tile: 0 = 256x256, 1 = 128x128, 2 = 64x64 (four waves), 3 = 256x256 on eight waves (512 lanes)
+  uint32_t tile;       // block tile: 0 = 256x256, 1 = 128x128, 2 = 64x64 (four waves), 4 = 128x128 with four stage buffers instead of two (one workgroup per compute unit), 3 = 256x256 on eight waves (512 lanes)
   uint32_t tiles_m, tiles_n;
   uint32_t n_mem, n_code;
   uint32_t mem_off, code_off;  // word offsets
-  uint32_t fast;       // k is a multiple of 64 and every 8-element operand chunk is 16-byte aligned: full tiles take the vector path
+  uint32_t fast;       // the operands are whole 16-byte chunks along their contiguous axes: the ring of direct loads takes them
   uint32_t epi_flags;  // VCF_*
   uint64_t a_addr, b_addr;
   uint32_t k_split;    // VCF_SPLITK_*: parts the k axis is cut into (>= 2), each k_chunk long (a multiple of 64; the last
@@ -357,15 +357,26 @@ enum { VCG_NONE = 0, VCG_M_BOUND = 1, VCG_M_SIZE = 2, VCG_K_BOUND = 3, VCG_K_SIZ
 #define VCF_SPLITK_PARTIAL 2u
 #define VCF_SPLITK_COMBINE 4u
 
-// Dynamic local memory a VE_CUBE launch needs for block tile `bt` (256, 128 or 64): the operand tiles of the k
-// loop (two buffers of 64 k per operand; for the 256 tile the same bytes as four stage buffers of 32 k), or what
-// the epilogue reads back: half the tile as fp32 accumulators, or the whole tile as 16-bit values (VCF_DUMP16).
-#define DVM_CUBE_LDS_LOOP_BYTES(bt) (2u * (2u * (bt)) * 64u * 2u)
+// Block tiles (VCubeHeader::tile), square: rows and columns of the output per workgroup.
+#define DVM_CUBE_TILES 5u
+#define DVM_CUBE_TILE_SIDE(tile) ((tile) == 1u || (tile) == 4u ? 128u : ((tile) == 2u ? 64u : 256u))
+#define DVM_CUBE_TILE_LANES(tile) ((tile) == 3u ? 512u : 256u)
+// The eight waves of tile 3 stand 2 x 4 (128 x 64 accumulators each) instead of 4 x 2 where B is read through the
+// transposing reads, which run at half the rate: a wave then reads less of B.
+#define DVM_CUBE_WAVES_2X4(tile, trans_b) ((tile) == 3u && !(trans_b))
+// The ring of the tile loop: k extent of a stage and number of stage buffers.
+#define DVM_CUBE_STAGE_K 64
+#define DVM_CUBE_STAGES(tile) ((tile) == 2u || (tile) == 4u ? 4u : 2u)
+// Dynamic local memory a VE_CUBE launch needs for a block tile: the stages of the tile loop, or what
+// the epilogue reads back: half the tile (a tile of 64 rows: all of it) as fp32 accumulators, or the whole tile as 16-bit
+// values (VCF_DUMP16).
+#define DVM_CUBE_LDS_LOOP_BYTES(tile) (DVM_CUBE_STAGES(tile) * DVM_CUBE_STAGE_K * (2u * DVM_CUBE_TILE_SIDE(tile)) * 2u)
 #define DVM_CUBE_LDS_DUMP32_BYTES(bt) (((bt) >= 128u ? (bt) / 2u : (bt)) * ((bt) + 4u) * 4u)
 #define DVM_CUBE_LDS_DUMP16_BYTES(bt) ((bt) * ((bt) + 8u) * 2u)
 #define DVM_CUBE_MAX2(a, b) ((a) > (b) ? (a) : (b))
-#define DVM_CUBE_LDS_BYTES(bt) \
-  DVM_CUBE_MAX2(DVM_CUBE_LDS_LOOP_BYTES(bt), DVM_CUBE_MAX2(DVM_CUBE_LDS_DUMP32_BYTES(bt), DVM_CUBE_LDS_DUMP16_BYTES(bt)))
+#define DVM_CUBE_LDS_BYTES(tile) \
+  DVM_CUBE_MAX2(DVM_CUBE_LDS_LOOP_BYTES(tile), \
+                DVM_CUBE_MAX2(DVM_CUBE_LDS_DUMP32_BYTES(DVM_CUBE_TILE_SIDE(tile)), DVM_CUBE_LDS_DUMP16_BYTES(DVM_CUBE_TILE_SIDE(tile))))
 // (a grouped product keeps its tables behind that: 8 bytes per group)
 
 // ---- fused attention programs (VE_ATTN) -------------------------------------------
