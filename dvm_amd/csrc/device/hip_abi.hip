@@ -19,6 +19,7 @@ extern "C" __global__ void dvm_vm_vec_ry_parts(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_sw(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_sw_parts(const VmParam p);
 #define DVM_ROW_DECL(slabs) extern "C" __global__ void dvm_vm_vec_row##slabs(const VmParam p);
+extern "C" __global__ void dvm_vm_vec_col(const VmParam p);
 DVM_ROW_DECL(1) DVM_ROW_DECL(2) DVM_ROW_DECL(3) DVM_ROW_DECL(4) DVM_ROW_DECL(5) DVM_ROW_DECL(6) DVM_ROW_DECL(8)
 extern "C" __global__ void dvm_vm_vec_pw_u4(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_u4(const VmParam p);
@@ -156,6 +157,7 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
                                        reinterpret_cast<const void *>(dvm_vm_vec_ry), reinterpret_cast<const void *>(dvm_vm_vec_rx_parts),
                                        reinterpret_cast<const void *>(dvm_vm_vec_ry_parts),
                                        reinterpret_cast<const void *>(dvm_vm_vec_rx_sw), reinterpret_cast<const void *>(dvm_vm_vec_rx_sw_parts),
+                                       reinterpret_cast<const void *>(dvm_vm_vec_col),
                                        reinterpret_cast<const void *>(dvm_vm_vec_pw_u4), reinterpret_cast<const void *>(dvm_vm_vec_rx_u4),
                                        reinterpret_cast<const void *>(dvm_vm_vec_ry_u4)};
   for (VecKernel k : kRowKernels)
@@ -344,6 +346,47 @@ static bool row_words_hold(const VmParam &p, uint32_t threads) {
 }
 
 // Checks one program blob against the launch it is to get and launches the interpreter kernel its entry type names.
+// The column build trusts its flag: the program is what VS_COLS says, the teams cover the kept index space, and the operands
+// lie where 128-bit accesses to whole elements reach them.
+static bool col_words_hold(const VmParam &p, uint32_t threads) {
+  const VVecHeader *h = reinterpret_cast<const VVecHeader *>(p.w);
+  const uint64_t *code = p.w + h->code_off;
+  const VMemDesc *mems = reinterpret_cast<const VMemDesc *>(p.w + h->mem_off);
+  if (threads < 64 || threads > 512 || h->n_rdim != 1 || h->n_kdim == 0 || h->inner_reduced != 0 || h->inner_extent < DVM_VEC_E || h->n_mem == 0 ||
+      h->n_kidx == 0 || h->n_ridx == 0 || h->team_log2 > 6 || (threads & (threads - 1)) != 0 || h->kdims[0].extent != (h->inner_extent + DVM_VEC_E - 1) / DVM_VEC_E ||
+      h->n_items != ((h->n_kidx - 1) >> h->team_log2) + 1 || h->n_code < 4) return false;
+  auto mem_ok = [&](uint32_t a, bool strided) {
+    if (a >= h->n_mem) return false;
+    const VMemDesc &m = mems[a];
+    if (m.dtype != VDT_F32 && m.dtype != VDT_F16 && m.dtype != VDT_BF16) return false;
+    if ((m.addr & (m.dtype == VDT_F32 ? 3u : 1u)) != 0) return false;
+    const uint32_t walk = m.flags & (VMF_VEC | VMF_GATHER);
+    return walk == VMF_VEC || (strided && walk == VMF_GATHER);
+  };
+  if (VI_OP(code[0]) != VOP_SWEEP || VI_OP(code[1]) != VOP_LD || VI_KIND(code[1]) != VK_MEM || !mem_ok(VI_A(code[1]), false)) return false;
+  uint32_t i = 2;
+  for (bool ends = false; !ends; ++i) {
+    if (i >= h->n_code || i > 4) return false;
+    const uint32_t sub = VI_SUB(code[i]), kind = sub & 0xfu;
+    ends = (static_cast<uint32_t>(code[i]) & VI_ENDS) != 0;
+    if (VI_OP(code[i]) == VOP_ENDSWEEP) continue;
+    if (VI_OP(code[i]) != VOP_RED || VI_A(code[i]) >= DVM_VEC_NSLOT || kind > VR_MIN || (sub & ~(0xfu | VRF_SQUARE | VRF_PAIR)) != 0 ||
+        ((sub & (VRF_SQUARE | VRF_PAIR)) != 0 && kind != VR_SUM) || ((sub & VRF_PAIR) != 0 && (VI_A(code[i]) != 0 || (sub & VRF_SQUARE) != 0))) return false;
+  }
+  for (; i < h->n_code; ++i) {
+    const uint64_t w = code[i];
+    switch (VI_OP(w)) {
+      case VOP_END: return i + 1 == h->n_code;
+      case VOP_FIN: if (VI_A(w) >= DVM_VEC_NSLOT || (VI_SUB(w) & VRF_INT) != 0) return false; break;
+      case VOP_BINF: if ((VI_SUB(w) & 0x3fu) > VB_MAX || (VI_KIND(w) != VK_IMM && VI_KIND(w) != VK_ACC)) return false; break;
+      case VOP_CAST: if (VI_SUB(w) != VC_RND) return false; break;
+      case VOP_ST: if (!mem_ok(VI_A(w), true)) return false; break;
+      default: return false;
+    }
+  }
+  return false;
+}
+
 static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads, uint32_t lds_bytes, void *stream, bool check_only = false) {
   if (block_dim == 0 || threads == 0 || threads > 1024 || (threads & 63u) != 0) {
     return static_cast<int>(hipErrorInvalidValue);
@@ -376,6 +419,8 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const uint32_t row = DVM_VEC_ROW_SLABS(h->sched);
     if (row != 0 && (wide || h->r_chunk != 0 || (h->sched & VS_KIND_MASK) != VS_REDX || !row_words_hold(p, threads))) return static_cast<int>(hipErrorInvalidValue);
     if (row == 0 && sweeps && (wide || (h->sched & VS_KIND_MASK) != VS_REDX || !sweeps_flag_holds(p))) return static_cast<int>(hipErrorInvalidValue);
+    const bool cols = (h->sched & VS_COLS) != 0;
+    if (cols && (wide || (h->sched & VS_KIND_MASK) != VS_REDY || !col_words_hold(p, threads))) return static_cast<int>(hipErrorInvalidValue);
     // a reduce shared between workgroups: its parts are the outermost kept axis and cover the reduced index space
     const bool parts = h->r_chunk != 0;
     if (parts) {
@@ -419,7 +464,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
         }
         break;
       case VS_REDY:
-        hipLaunchKernelGGL(parts ? dvm_vm_vec_ry_parts : (wide ? dvm_vm_vec_ry_u4 : dvm_vm_vec_ry), dim3(block_dim), dim3(threads), lds_bytes, s, p);
+        hipLaunchKernelGGL(cols ? dvm_vm_vec_col : parts ? dvm_vm_vec_ry_parts : (wide ? dvm_vm_vec_ry_u4 : dvm_vm_vec_ry), dim3(block_dim), dim3(threads), lds_bytes, s, p);
         break;
       default:
         return static_cast<int>(hipErrorInvalidValue);

@@ -394,6 +394,10 @@ class Compiler {
   void PlanRereads();
   bool FitsSweepBuild();
   bool RowCandidate() const;
+  bool ColCandidate(uint32_t *elem_size) const;
+  bool FitsColBuild() const;
+  bool ReducesColumnsOfALoad(const NDObject *r, const NDObject **load) const;
+  bool col_allowed_ = true;             // (false: the program has turned out to be outside the column build's vocabulary)
   bool ReadsAlignedRowsOnce() const;
   uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;
   bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;

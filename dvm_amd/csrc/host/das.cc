@@ -208,6 +208,7 @@ std::string &VKernel::DisAssemble() {
       static const char *sched[] = {"pointwise", "reduce-x", "reduce-y"};
       os << "entry vector sched=" << sched[h->sched & VS_KIND_MASK] << ((h->sched & VS_WIDE) ? " wide" : "") << ((h->sched & VS_SWEEPS) && DVM_VEC_ROW_SLABS(h->sched) == 0 ? " sweeps" : "");
       if (DVM_VEC_ROW_SLABS(h->sched) != 0) os << " row=" << DVM_VEC_ROW_SLABS(h->sched);  // (the build that runs, whatever others could)
+      if (h->sched & VS_COLS) os << " columns";
       os << " blocks=" << p.grid << " threads=" << p.threads
          << " lds=" << p.lds_bytes << " items=" << h->n_items << " kept=" << h->n_kidx << " red=" << h->n_ridx
          << " inner=" << h->inner_extent << " team=" << (h->team_is_block ? p.threads : (1u << h->team_log2))

@@ -689,6 +689,7 @@ bool Compiler::FinishProgram() {
   if (k_->tuning_.vec_sweeps != 0 && FitsSweepBuild()) hdr_.sched |= VS_SWEEPS;
   row_code_.clear();
   if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && !BuildRowCode()) return false;
+  if ((hdr_.sched & VS_COLS) != 0 && !FitsColBuild()) return false;
   hdr_.n_mem = n_mem_;
   hdr_.n_code = static_cast<uint32_t>(code_.size());
   hdr_.mem_off = sizeof(VVecHeader) / 8;
@@ -764,7 +765,7 @@ void Compiler::CompileArea(int a) {
   }
   UnifyAxes();
   OrderAndMerge();
-  row_allowed_ = true;
+  row_allowed_ = col_allowed_ = true;
   ChooseSchedule();
   // a stored value must span the index space it is stored from, or it would be written several times. (The axis
   // that numbers the parts of a shared reduce is the exception: a value stored inside the sweep over the reduced space
@@ -792,11 +793,12 @@ void Compiler::CompileArea(int a) {
     }
   }
   bool done = false;
-  if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0) {
-    // Laid out for the row build. Whatever keeps the program out of that layout (a word outside the build's vocabulary, V
+  if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 || (hdr_.sched & VS_COLS) != 0) {
+    // Laid out for the row build (or, likewise, the column build). Whatever keeps the program out of that layout (a word outside the build's vocabulary, V
     // registers for up to twice the lanes the other builds would use) is settled here, with the layout of the other builds:
     // thrown past this point it would make RunModes cut the graph.
-    std::string why = "a word outside the row build's vocabulary";
+    const bool columns = (hdr_.sched & VS_COLS) != 0;
+    std::string why = columns ? "a word outside the column build's vocabulary" : "a word outside the row build's vocabulary";
     try {
       EmitProgram();
       done = FinishProgram();
@@ -804,9 +806,13 @@ void Compiler::CompileArea(int a) {
       why = e.what();
     }
     if (!done) {
-      if (k_->tuning_.debug) std::fprintf(stderr, "dvm: sub-kernel %d leaves the row build: %s\n", a, why.c_str());
-      if (row_refused_.size() < 64) row_refused_.push_back(row_key_);
-      row_allowed_ = false;
+      if (k_->tuning_.debug) std::fprintf(stderr, "dvm: sub-kernel %d leaves the %s build: %s\n", a, columns ? "column" : "row", why.c_str());
+      if (columns) {
+        col_allowed_ = false;
+      } else {
+        if (row_refused_.size() < 64) row_refused_.push_back(row_key_);
+        row_allowed_ = false;
+      }
       for (int i = 0; i < nn_; ++i) {
         nodes_[i].mem_idx = nodes_[i].reg = -1;
         nodes_[i].slot_ready = false;

@@ -231,6 +231,7 @@ struct Tuning {
   int vec_sweeps = -1;  // DVM_VEC_SWEEPS=0: never the sweep build of the vector VM
   int vec_row = -1;     // DVM_VEC_ROW=0: never the row build of the vector VM; n: at most n slabs a lane there
   int vec_gather_tile = -1;  // DVM_VEC_GATHER_TILE=0: pointwise programs with a gathered operand keep the plain slab order
+  int vec_col = -1;     // DVM_VEC_COL=0: never the column build of the vector VM
   int cube_tile = -1;   // DVM_CUBE_TILE=256|128|64
   int cube_waves = -1;  // DVM_CUBE_WAVES=4|8
   int red_split_turn = -1;  // DVM_RED_SPLIT_TURN=0: the reduce over the parts of a shared reduce walks them outermost, as they lie in memory

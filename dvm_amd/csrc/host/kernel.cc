@@ -35,6 +35,7 @@ void Tuning::Read() {
   vec_reread = num("DVM_VEC_REREAD");
   vec_sweeps = num("DVM_VEC_SWEEPS");
   vec_row = num("DVM_VEC_ROW");
+  vec_col = num("DVM_VEC_COL");
   vec_gather_tile = num("DVM_VEC_GATHER_TILE");
   cube_tile = num("DVM_CUBE_TILE");
   cube_waves = num("DVM_CUBE_WAVES");
@@ -226,13 +227,13 @@ void VKernel::BindAddresses(const RelocEntry *relocs, size_t n, WsAllocator *all
           VMemDesc *m = reinterpret_cast<VMemDesc *>(p.blob.w + pt.word);
           m->flags &= ~static_cast<uint32_t>(VMF_ALIGNED);
           // (the sweep build accesses the operands of its interior rounds without guards: the generic kernel runs instead;
-          // the row build takes rows that start at any element, but not inside one)
+          // the row and column builds take rows that start at any element, but not inside one)
           const uint64_t element = m->dtype == VDT_F32 ? 4 : 2;
           uint32_t sched;
           char *sched_at = reinterpret_cast<char *>(p.blob.w) + offsetof(VVecHeader, sched);
           std::memcpy(&sched, sched_at, sizeof(sched));
           sched &= ~static_cast<uint32_t>(VS_SWEEPS);
-          if ((addr & (element - 1)) != 0) sched &= ~static_cast<uint32_t>(VS_ROW_MASK);
+          if ((addr & (element - 1)) != 0) sched &= ~static_cast<uint32_t>(VS_ROW_MASK | VS_COLS);
           std::memcpy(sched_at, &sched, sizeof(sched));
         } else if (pt.role == Program::kPatchCubeOperand) {
           reinterpret_cast<VCubeHeader *>(p.blob.w)->fast = 0;

@@ -247,6 +247,48 @@ void Compiler::MarkUniformRuns() {
   code_.swap(out);
 }
 
+// Whether the finished instruction stream is in the vocabulary of the column build (VS_COLS in isa_gfx950.h).
+bool Compiler::FitsColBuild() const {
+  auto is_float = [](uint32_t dt) { return dt == VDT_F32 || dt == VDT_F16 || dt == VDT_BF16; };
+  if (code_.size() < 4 || VI_OP(code_[0]) != VOP_SWEEP || VI_OP(code_[1]) != VOP_LD || VI_KIND(code_[1]) != VK_MEM) return false;
+  const VMemDesc &m = mems_[VI_A(code_[1])];
+  if ((m.flags & (VMF_VEC | VMF_GATHER)) != VMF_VEC || !is_float(m.dtype) || (static_cast<uint32_t>(code_[1]) & (VI_ENDS | VI_UNIFORM))) return false;
+  size_t i = 2;
+  for (bool ends = false; !ends; ++i) {
+    if (i >= code_.size() || i > 4) return false;
+    const uint64_t w = code_[i];
+    ends = (static_cast<uint32_t>(w) & VI_ENDS) != 0;
+    if (VI_OP(w) == VOP_ENDSWEEP) continue;
+    const uint32_t kind = VI_SUB(w) & 0xfu;
+    if (VI_OP(w) != VOP_RED || VI_A(w) >= DVM_VEC_NSLOT || kind > VR_MIN || (VI_SUB(w) & ~(0xfu | VRF_SQUARE | VRF_PAIR)) != 0) return false;
+    if ((VI_SUB(w) & (VRF_SQUARE | VRF_PAIR)) != 0 && kind != VR_SUM) return false;
+    if ((VI_SUB(w) & VRF_PAIR) != 0 && (VI_A(w) != 0 || (VI_SUB(w) & VRF_SQUARE) != 0)) return false;
+  }
+  for (; i < code_.size(); ++i) {
+    const uint64_t w = code_[i];
+    switch (VI_OP(w)) {
+      case VOP_END:
+        if (i + 1 != code_.size()) return false;
+        break;
+      case VOP_FIN:
+        if (VI_A(w) >= DVM_VEC_NSLOT || (VI_SUB(w) & VRF_INT) != 0) return false;
+        break;
+      case VOP_BINF:
+        if ((VI_SUB(w) & 0x3fu) > VB_MAX || (VI_KIND(w) != VK_IMM && VI_KIND(w) != VK_ACC)) return false;
+        break;
+      case VOP_CAST:
+        if (VI_SUB(w) != VC_RND) return false;
+        break;
+      case VOP_ST:
+        if ((mems_[VI_A(w)].flags & (VMF_VEC | VMF_GATHER)) == 0 || !is_float(mems_[VI_A(w)].dtype)) return false;
+        break;
+      default:
+        return false;
+    }
+  }
+  return true;
+}
+
 // Whether the finished instruction stream fits the sweep build of the device VM (VS_SWEEPS in isa_gfx950.h spells
 // out the vocabulary). Everything is decided from the instruction words and the operand descriptors: shapes,
 // alignment and ragged ends are the device's business on either build.

@@ -493,6 +493,29 @@ bool Compiler::RowCandidate() const {
   return true;
 }
 
+// The column build: everything that varies along the one reduced axis is a load, its casts and its square.
+bool Compiler::ColCandidate(uint32_t *elem_size) const {
+  if (!col_allowed_ || k_->tuning_.vec_col == 0 || k_->tuning_.vec_pair == 0 || k_->tuning_.vec_fuse == 0) return false;
+  if (nr_ != 1 || n_peel_ > 0 || hdr_.inner_extent < static_cast<uint32_t>(E)) return false;
+  int loads = 0;
+  for (int i = 0; i < nn_; ++i) {
+    const ANode &n = nodes_[i];
+    if (n.dtype != kFloat32 && n.dtype != kFloat16 && n.dtype != kBFloat16) return false;
+    bool in_sweep = false;
+    for (int d = 0; d < n.rank; ++d) in_sweep = in_sweep || (n.axis[d] >= 0 && axes_[n.axis[d]].reduced);
+    if (n.kind == AK_MEM) {
+      if (!in_sweep || ++loads > 1) return false;
+      *elem_size = static_cast<uint32_t>(DTypeSize(n.dtype));
+    } else if (in_sweep && n.kind == AK_OP) {
+      const bool square = n.op->kind == kObjBinary && n.op->op == kMul && n.nin == 2 && n.in[0] == n.in[1];
+      if (n.op->kind != kObjCast && !square) return false;
+    } else if (in_sweep && n.kind == AK_OUT) {
+      return false;
+    }
+  }
+  return loads == 1;
+}
+
 // What the outcome of trying a row layout depends on: the operators, which of their values vary along the reduced axis,
 // whether a row is one round (up to two slabs a lane: values may wait in V registers there, and only there) and how many V
 // registers those lanes have. Two programs with the same key compile to the same instruction words but for their operands'
@@ -708,14 +731,31 @@ void Compiler::ChooseSchedule() {
     const uint64_t n_k_part = parts != 0 ? std::max<uint64_t>(n_k / parts, 1) : n_k;
     uint32_t tx = n_k_part >= 64 ? 64 : Pow2Ceil(n_k_part);
     uint32_t ty = 256 / tx;
-    const uint64_t items = (n_k + tx - 1) / tx;
+    uint64_t items = (n_k + tx - 1) / tx;
+    uint32_t elem_size = 0;
+    const bool columns = !wide && ColCandidate(&elem_size);
+    if (columns) {
+      // One 128-byte line of columns per workgroup, half of one where that leaves fewer than 64 workgroups of 16-bit elements,
+      // more while there are four workgroups per compute unit all the same; as many lanes along the rows as there are rows,
+      // 512 in all. Measured on MI355X, bf16 sums over axis 0, us on the generic kernel / here: [489,824] 100 / 7.0,
+      // [282,584] 60 / 6.6, [1473,3848] 30 (two launches) / 11, [4096,4096] 26 (two) / 17; with 16 / 8 / 4 lanes along the
+      // columns [4096,4096] 26 / 17 / 20, [4096,512] 23 / 14 / 10, [4000,600] 26 / 18 / 14.
+      tx = std::min<uint32_t>(16u / elem_size, Pow2Ceil(n_k_part));
+      if (tx == 8 && n_k < 8 * 64) tx = 4;
+      while (tx < 64 && n_k / (2 * tx) >= 4ull * g_system.core_num && 2 * tx <= Pow2Ceil(n_k_part)) tx *= 2;
+      items = (n_k + tx - 1) / tx;
+      ty = 512 / tx;
+      while (ty > 1 && ty / 2 >= n_r && tx * ty > 64) ty >>= 1;
+      hdr_.sched |= VS_COLS;
+    } else
     if (items < 128 && n_r > 256) ty = 512 / tx;  // few outputs: give each more lanes along the reduce space (the kernel's limit is 512)
     else if (items < 128 && n_r >= 64) ty = 512 / tx;     // (the launch that reduces over the parts of a shared reduce, mostly)
     // (the parts of a shared reduce: with fewer than two workgroups per compute unit, 512 lanes each put twice the
     // loads in flight. Measured on MI355X, fp32 sums over axis 0: [8192,1024] 57 -> 47 us, [65536,768] 136 -> 97 us,
     // [32,3136,256] over its first two axes 86 -> 70 us; 1024 lanes are slower again, 54 / 120 / 79 us)
-    if (parts != 0 && items < 2ull * g_system.core_num && n_r >= 32) ty = 512 / tx;
-    while (ty > 1 && static_cast<uint64_t>(ty) * U > 2 * n_r) ty >>= 1;
+    if (!columns && parts != 0 && items < 2ull * g_system.core_num && n_r >= 32) ty = 512 / tx;
+    if (!columns)
+      while (ty > 1 && static_cast<uint64_t>(ty) * U > 2 * n_r) ty >>= 1;
     threads = std::max<uint32_t>(64, tx * ty);
     ty = threads / tx;
     hdr_.team_log2 = Log2(tx);

@@ -64,6 +64,11 @@ enum {
   // (dvm_vm_vec_rx_sw), which decodes a sweep's body once per sweep instead of once per instruction and round; the
   // generic kernel runs it as well and gives the same bits.
   VS_SWEEPS = 0x20,
+  // flag (VS_REDY only): the column build (vm_vector_col.hip) may run the program. One reduced axis and at least eight
+  // elements along the innermost one; the words are a sweep of one load (innermost stride 1) and one or two float reduces
+  // of what it loads, then reduce results, float binaries (add .. max) on immediates or the accumulator, roundings and
+  // stores. The generic kernel runs the same words at the same geometry.
+  VS_COLS = 0x40,
   // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.hip) may run the program from the words at
   // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space is one axis of n_ridx
   // groups, more than (slabs - 1) * team and at most slabs * team of them (team: the workgroup when team_is_block, else
