@@ -1,5 +1,6 @@
 # make-style entry for the native libraries (the same commands as `python -m dvm_amd.build`):
-#   make                 dvm_amd/lib/libdvm_hip.so (device layer, hipcc, gfx950) and dvm_amd/lib/libdvm.so (host library, g++)
+#   make                 dvm_amd/lib/libdvm_hip.so (device layer, hipcc, gfx950), dvm_amd/lib/libdvm.so (host library, g++) and
+#                        dvm_amd/lib/_torch_call.so (repeated calls on torch tensors)
 #   make consumers       the C++ programs of tests/cc against include/*.h and the two libraries
 #   make oracle          the CPU oracle of the tests (oracle/libdvm_oracle.so)
 #   make asan=1          the host library again with AddressSanitizer and UndefinedBehaviorSanitizer, into dvm_amd/lib/asan/
@@ -43,7 +44,7 @@ HOST_OBJ := $(patsubst $(CSRC)/host/%.cc,$(OBJ)$(SAN_DIR)/%.cc.o,$(HOST_SRC))
 ifneq ($(asan),)
 all: $(LIB)/asan/libdvm.so
 else
-all: $(LIB)/libdvm_hip.so $(LIB)/libdvm.so
+all: $(LIB)/libdvm_hip.so $(LIB)/libdvm.so $(LIB)/_torch_call.so
 endif
 
 $(OBJ):
@@ -67,6 +68,10 @@ $(LIB)$(SAN_DIR)/libdvm.so: $(HOST_OBJ)
 	@mkdir -p $(dir $@)
 	$(CXX) -shared -fPIC $(SAN_FLAGS) $(HOST_OBJ) -o $@ -ldl -lpthread
 
+# the extension behind repeated calls on torch tensors (nothing where torch or the interpreter's headers are missing)
+$(LIB)/_torch_call.so: $(CSRC)/torch/torch_call.cc | $(OBJ)
+	python3 -c "import subprocess, sys; from dvm_amd import build; c = build.torch_call_command(); sys.exit(subprocess.call(c[2]) if c else 0)"
+
 # the CPU tests (the device layer is not needed for them) and the random graphs of tests/random_graphs.py, compiled in
 # disassembly mode, against the sanitizer build; any report ends the run with an error
 asan-check:
@@ -89,4 +94,4 @@ oracle:
 	$(MAKE) -C oracle
 
 clean:
-	rm -rf $(OBJ) $(LIB)/libdvm_hip.so $(LIB)/libdvm.so $(LIB)/tests
+	rm -rf $(OBJ) $(LIB)/libdvm_hip.so $(LIB)/libdvm.so $(LIB)/_torch_call.so $(LIB)/tests

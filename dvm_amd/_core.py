@@ -89,6 +89,8 @@ def _load():
         "dvm_rt_codegen": (ci, [vp]),
         "dvm_rt_jit_us": (ctypes.c_double, [vp]),
         "dvm_rt_run": (ci, [vp, vp, ci]),
+        "dvm_rt_plan_stamp": (ctypes.c_uint64, [vp]),
+        "dvm_rt_rebind_run": (ci, [vp, ctypes.c_uint64, ctypes.POINTER(vp), ctypes.POINTER(vp), cs, vp, vp]),
         "dvm_rt_output": (ci, [vp, vp, vp, cs]),
         "dvm_rt_device_ptr": (vp, [vp, vp]),
         "dvm_rt_perf": (ci, [vp, ci, ci, ctypes.POINTER(ctypes.c_double)]),
@@ -115,6 +117,29 @@ def _load():
         fn.restype = res
         fn.argtypes = args
     return lib
+
+
+def new_call_plan(rt):
+    """A native plan for repeated calls of the runner `rt` on torch tensors (csrc/torch/torch_call.cc), or None where the
+    extension has not been built: calls then bind, generate code and launch from Python every time."""
+    global _call_plans
+    if _call_plans is None:
+        import importlib.machinery
+        import importlib.util
+        path = os.path.join(_LIB_DIR, "_torch_call.so")
+        if not os.path.exists(path):
+            _call_plans = False
+            return None
+        import torch  # noqa: F401  (the extension's symbols come from it)
+        loader = importlib.machinery.ExtensionFileLoader("_torch_call", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_call", loader))
+        loader.exec_module(module)
+        address = lambda name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value
+        _call_plans = (module.Plan, address("dvm_rt_rebind_run"), address("dvm_rt_plan_stamp"), address("dvm_c_last_error"))
+    return _call_plans[0](*_call_plans[1:], rt) if _call_plans else None
+
+
+_call_plans = None
 
 
 class _LazyLib:

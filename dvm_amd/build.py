@@ -53,6 +53,21 @@ def _run(cmd):
     return err
 
 
+def torch_call_command():
+    """g++ line for the extension that makes repeated calls on torch tensors (csrc/torch/torch_call.cc): source, target, command;
+    None where torch or the interpreter's headers are missing (calls then stay in Python)."""
+    import importlib.util
+    import sysconfig
+    spec = importlib.util.find_spec("torch")
+    inc = sysconfig.get_paths()["include"]
+    if spec is None or not os.path.exists(os.path.join(inc, "Python.h")):
+        return None
+    torch = list(spec.submodule_search_locations)[0]
+    src, out = os.path.join(CSRC, "torch", "torch_call.cc"), os.path.join(LIB, "_torch_call.so")
+    return src, out, ["g++"] + HOST_FLAGS + ["-D_GLIBCXX_USE_CXX11_ABI=1", "-I" + inc, "-isystem", os.path.join(torch, "include"), "-shared", src, "-o", out,
+                                             "-L" + os.path.join(torch, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(force=False, verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     deps = _deps()
@@ -74,6 +89,9 @@ def build(force=False, verbose=False):
         host_objs.append(obj)
         if force or _stale(obj, [src] + deps):
             jobs.append(["g++"] + HOST_FLAGS + ["-c", src, "-o", obj])
+    call = torch_call_command()
+    if call is not None and (force or _stale(call[1], [call[0]])):
+        jobs.append(call[2])
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for msg in ex.map(_run, jobs):
             if verbose and msg:

@@ -2,6 +2,7 @@
 #include "../../../include/dvm_c.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <map>
@@ -64,6 +65,7 @@ struct dvm_rt {
   void *ws_user = nullptr;
   std::map<NDObject *, std::unique_ptr<dvm_shape>> view_strides;  // loads bound through strides (dvm_rt_bind_device_view)
   uint64_t fake_addr = 0x1000;
+  uint64_t changes = 0;  // counts what may change the compiled programs or the walk of a load (dvm_rt_plan_stamp)
   double jit_us = 0.0;
   WsAlloc ws_alloc;
 
@@ -259,6 +261,7 @@ void dvm_rt_delete(dvm_rt *rt) {
 int dvm_rt_reset(dvm_rt *rt) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->FreeAll();
         rt->fake_addr = 0x1000;  // dry runs hand out the same placeholder addresses after every reset
         rt->store_extent.clear();
@@ -729,11 +732,13 @@ int dvm_rt_bind_device_view(dvm_rt *rt, dvm_obj *load, void *device_ptr, const i
         if (o->kind != kObjLoad || o->full_shape_ref != nullptr) throw std::runtime_error("DVM EXCEPTION. reason: only a plain load takes a strided binding");
         if (strides == nullptr) {
           if (rt->view_strides.erase(o) != 0) {
+            ++rt->changes;
             o->strided = false;
             o->stride_ref = nullptr;
           }
         } else {
           if (rank != static_cast<size_t>(o->shape_ref_->size)) throw std::runtime_error("DVM EXCEPTION. reason: one stride per dim of the load");
+          ++rt->changes;
           std::unique_ptr<dvm_shape> &st = rt->view_strides[o];
           if (!st) st.reset(new dvm_shape());
           st->Set(strides, rank);
@@ -765,6 +770,7 @@ int dvm_rt_set_workspace_allocator(dvm_rt *rt, dvm_ws_alloc_fn alloc, void *user
 int dvm_rt_unbind_device(dvm_rt *rt) {
   return Guard(
       [&]() {
+        ++rt->changes;
         for (auto &kv : rt->view_strides) {
           kv.first->strided = false;
           kv.first->stride_ref = nullptr;
@@ -786,6 +792,7 @@ int dvm_rt_unbind_device(dvm_rt *rt) {
 int dvm_rt_normalize(dvm_rt *rt) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.Normalize();
         return 0;
       },
@@ -795,6 +802,7 @@ int dvm_rt_normalize(dvm_rt *rt) {
 int dvm_rt_codegen(dvm_rt *rt) {
   return Guard(
       [&]() {
+        ++rt->changes;
         const auto t0 = std::chrono::steady_clock::now();
         rt->kernel.Normalize();
         const auto t1 = std::chrono::steady_clock::now();
@@ -854,6 +862,35 @@ int dvm_rt_run(dvm_rt *rt, void *stream, int flags) {
           rc = rt->Api().synchronize_stream(s);
           if (rc != 0) throw std::runtime_error(std::string("kernel execution failed: ") + rt->Api().error_string(rc));
         }
+        return 0;
+      },
+      -1);
+}
+
+namespace {
+std::atomic<uint64_t> g_tuner_changes{0};  // the tuner's switches decide what a code generation of an unchanged kernel gives
+}
+
+uint64_t dvm_rt_plan_stamp(dvm_rt *rt) {
+  return (rt->changes << 24) + (static_cast<uint64_t>(rt->kernel.GetImpl()->ops_.size()) << 8) + (g_tuner_changes.load(std::memory_order_relaxed) & 0xffu);
+}
+
+int dvm_rt_rebind_run(dvm_rt *rt, uint64_t stamp, dvm_obj *const *ios, void *const *ptrs, size_t n, void *workspace, void *stream) {
+  return Guard(
+      [&]() {
+        VKernel *k = rt->kernel.GetImpl();
+        if (rt->das_mode || dvm_rt_plan_stamp(rt) != stamp || n > 64) return 1;
+        RelocEntry relocs[64];
+        for (size_t i = 0; i < n; ++i) {
+          NDObject *o = Obj(ios[i]);
+          Buffer &b = rt->buffers[o];
+          rt->Release(b);
+          b.ptr = ptrs[i];
+          relocs[i] = RelocEntry(o, ptrs[i]);
+        }
+        k->BindAddresses(relocs, n, nullptr, workspace);
+        const int rc = rt->kernel.Launch(stream);
+        if (rc != 0) throw std::runtime_error(std::string("launch failed: ") + rt->Api().error_string(rc));
         return 0;
       },
       -1);
@@ -934,17 +971,22 @@ int dvm_rt_perf(dvm_rt *rt, int warmup, int iters, double out[3]) {
 }
 
 void dvm_set_online_tuner(int enable) {
+  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
   g_system.Init();
   if (enable) g_system.SetOnlineTuner();
   else g_system.UnsetOnlineTuner();
 }
 void dvm_set_lazy_tuner(int enable) {
+  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
   g_system.Init();
   if (enable) g_system.SetLazyTuner();
   else g_system.UnsetLazyTuner();
 }
 void dvm_tuner_stats(uint64_t *shapes_measured, uint64_t *table_size) { CubeTunerStats(shapes_measured, table_size); }
-void dvm_tuner_clear(void) { CubeTunerClear(); }
+void dvm_tuner_clear(void) {
+  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
+  CubeTunerClear();
+}
 
 int dvm_rt_perf_samples(dvm_rt *rt, int warmup, int iters, double *samples) {
   return Guard(

@@ -14,7 +14,7 @@ its workspace from torch's caching allocator.
 import inspect
 import os
 
-from ._core import PyKernel, DataType, current_raw_stream
+from ._core import PyKernel, DataType, current_raw_stream, new_call_plan
 
 
 class _Slot:
@@ -27,6 +27,7 @@ class _Slot:
 
 
 _TORCH_TYPES = {}  # DataType -> torch type, filled at the first call on torch tensors
+_raw_stream_of = None  # device index -> torch's current stream there, from the first call on torch tensors
 
 
 class JitKernel(PyKernel):
@@ -39,6 +40,8 @@ class JitKernel(PyKernel):
         self._slots = []      # one _Slot per argument, filled while tracing
         self._store_types = None  # torch types of the stores, from the first call on torch tensors
         self._results = None  # what the traced function returned: a store or a sequence of stores
+        self._plan = None     # the last call on torch tensors, to be made again natively (False: never)
+        self._last_shapes = None
 
     # ---- tracing ----
     def build(self, func):
@@ -75,6 +78,10 @@ class JitKernel(PyKernel):
         return (list(self._results) if many else [self._results]), many
 
     def __call__(self, *args, out=None):
+        if self._plan and out is None:
+            result = self._plan.call(self, args, _raw_stream_of)
+            if result is not None:
+                return result
         if len(args) != len(self._slots):
             raise TypeError("kernel takes %d arguments, %d given" % (len(self._slots), len(args)))
         if any(_on_gpu(a) for a in args):
@@ -177,7 +184,27 @@ class _DeviceCall:
                     raise
         k.run(stream=current_raw_stream(device), sync=False, on_given_stream=True)
         k._alive = held + outs + scratch  # until the next call: the launches may still be running
+        if self.out is None and in_place and k._plan is not False:
+            self._plan_next(outs, many)
         return outs if many else outs[0]
+
+
+    def _plan_next(self, outs, many):
+        """Records this call, the second with these shapes, as the plan of the next one."""
+        global _raw_stream_of
+        k = self.kern
+        shapes = [a.shape for a, s in zip(self.args, k._slots) if s.role == "tensor"]
+        if shapes != k._last_shapes:
+            k._last_shapes = shapes
+            return
+        if k._plan is None:
+            k._plan = new_call_plan(k._rt) if all(s.role in ("tensor", "scalar") for s in k._slots) else None
+            if k._plan is None:
+                k._plan = False
+                return
+            _raw_stream_of = self.torch._C._cuda_getCurrentRawStream
+        k._plan.record(tuple(self.args), [s.handle._h for s in k._slots if s.role == "tensor"], outs, [st._h for st in k._stores()[0]], many,
+                       k.workspace_bytes())
 
 
 def _on_gpu(value):

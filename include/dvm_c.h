@@ -149,6 +149,12 @@ double dvm_rt_jit_us(const dvm_rt *rt);
 #define DVM_RUN_WAIT 1
 #define DVM_RUN_ON_GIVEN_STREAM 2
 int dvm_rt_run(dvm_rt *rt, void *stream, int flags);
+/* What was compiled, once more on other memory: `ios[n]` are all loads and stores of the kernel, `ptrs[n]` where they lie
+ * now, `workspace` dvm_rt_workspace_bytes of device memory (or NULL when that is 0); the launches go to `stream`. Shapes,
+ * strides and scalars are those of the last dvm_rt_codegen. `stamp` is what dvm_rt_plan_stamp said after it: 1 is returned,
+ * and nothing done, when anything that decides the programs has changed since. */
+uint64_t dvm_rt_plan_stamp(dvm_rt *rt);
+int dvm_rt_rebind_run(dvm_rt *rt, uint64_t stamp, dvm_obj *const *ios, void *const *ptrs, size_t n, void *workspace, void *stream);
 int dvm_rt_output(dvm_rt *rt, dvm_obj *store, void *host, size_t bytes);
 void *dvm_rt_device_ptr(dvm_rt *rt, dvm_obj *io);
 /* warmup + iters timed launches with events: out = {min, max, mean} microseconds (src/pybind_api.cc:751-767). */

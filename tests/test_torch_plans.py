@@ -1,0 +1,124 @@
+"""GPU: repeated calls of `@kernel` functions on torch tensors, which are made natively from the plan of the second one: new
+tensors, other addresses, shapes, strides, numbers and streams from call to call, and whatever else changes the kernel in
+between, against torch. Runs in a process of its own that imports torch first (see tests/test_torch_adapter.py for why)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+_SCRIPT = r'''
+import numpy as np
+import torch
+import dvm_amd as dvm
+from dvm_amd import _core
+
+gen = torch.Generator(device="cuda").manual_seed(5)
+def rnd(*shape):
+    return torch.randn(shape, device="cuda", generator=gen)
+
+@dvm.kernel(ktype="split", dynamic=True)
+def axpy(k, x, y, a):
+    x, y = k.load(x, dvm.float32), k.load(y, dvm.float32)
+    s = k.add(k.mul(x, k.scalar(a)), y)
+    return k.store(s), k.store(k.sub(s, y))
+
+def check(x, y, a):
+    s, d = axpy(x, y, a)
+    want = x * a + y
+    assert s.shape == want.shape and s.is_contiguous() and torch.allclose(s, want, rtol=1e-6, atol=1e-6)
+    assert torch.allclose(d, want - y, rtol=1e-6, atol=1e-6)
+    return s, d
+
+def natively():  # whether a call like the last one would go through the plan
+    return bool(axpy._plan)
+
+for n in (1000, 1000, 1000, 37, 37, 1000, 1000, 1000):
+    for a in (2.0, 2.0, -3.5, -3.5):
+        check(rnd(n, 24), rnd(n, 24), a)
+assert natively()
+# what the plan recorded is told apart from everything else
+p = axpy._plan
+x, y = rnd(1000, 24), rnd(1000, 24)
+check(x, y, -3.5); check(x, y, -3.5)
+call = lambda *args: p.call(axpy, args, torch._C._cuda_getCurrentRawStream)
+assert call(x, y, -3.5) is not None
+for other in ((x, y, 2.0), (x, y, -3), (x[:999], y[:999], -3.5), (x.double(), y, -3.5), (x.cpu(), y, -3.5), (x, y), (x, y.t().contiguous().t(), -3.5)):
+    assert call(*other) is None, other
+keep = [check(x + i, y, -3.5) for i in range(4)]  # results of earlier calls stay
+for i, (s, d) in enumerate(keep):
+    assert torch.allclose(s, (x + i) * -3.5 + y, rtol=1e-6, atol=1e-6)
+# tensors that start inside a line, on 4 and on 16 bytes
+big = rnd(2, 1000 * 24 + 64)
+for off in (0, 1, 4, 3, 0):
+    check(big[0, off:off + 24000].view(1000, 24), big[1, off:off + 24000].view(1000, 24), -3.5)
+# strided views, then dense ones of the same shape
+wide = rnd(1000, 48)
+for _ in range(3):
+    check(wide[:, :24], y, -3.5)
+for _ in range(3):
+    check(x, y, -3.5)
+# numpy in between, a kernel whose bindings were taken away, out=, an error
+s = axpy(x.cpu().numpy(), y.cpu().numpy(), -3.5)[0]
+assert np.allclose(s, (x * -3.5 + y).cpu().numpy(), rtol=1e-6, atol=1e-6)
+for _ in range(3):
+    check(x, y, -3.5)
+axpy.release_device_bindings()
+check(x, y, -3.5)
+outs = [torch.empty_like(x), torch.empty_like(x)]
+axpy(x, y, -3.5, out=outs)
+assert torch.allclose(outs[0], x * -3.5 + y, rtol=1e-6, atol=1e-6)
+try:
+    axpy(x.double(), y, -3.5)
+    raise SystemExit("a double went through")
+except TypeError as e:
+    assert "float64" in str(e)
+try:
+    torch.vmap(lambda v: axpy(v, y, -3.5)[0])(x.expand(2, 1000, 24))
+    raise SystemExit("a batched tensor went through")
+except RuntimeError:
+    pass
+check(x, y, -3.5)
+# a workspace and two streams: every call has memory of its own
+@dvm.kernel(ktype="mix", dynamic=True)
+def product(k, x, w):
+    return k.store(k.matmul(k.load(x, dvm.float16), k.load(w, dvm.float16), False, False))
+
+def ints(*shape):
+    return torch.randint(-1, 2, shape, device="cuda", generator=gen).half()
+pairs = [(ints(64, 8192), ints(8192, 128)) for _ in range(6)]
+side = torch.cuda.Stream()
+side.wait_stream(torch.cuda.current_stream())
+got = []
+for i, (a, b) in enumerate(pairs):
+    with torch.cuda.stream(side if i % 2 else torch.cuda.current_stream()):
+        got.append(product(a, b))
+torch.cuda.synchronize()
+assert product.workspace_bytes() > 0 and bool(product._plan)
+for (a, b), c in zip(pairs, got):
+    assert torch.equal(c.double(), a.double() @ b.double())
+# captured into a graph and replayed on new inputs
+a, b = pairs[0]
+static = a.clone()
+g = torch.cuda.CUDAGraph()
+product(static, b); product(static, b)
+torch.cuda.synchronize()
+with torch.cuda.graph(g):
+    c = product(static, b)
+for src, _ in pairs:
+    static.copy_(src)
+    g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(c.double(), src.double() @ b.double())
+    assert torch.equal(product(src, b), c)
+print("plans: ok")
+'''
+
+
+def test_plans():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""))
+    r = subprocess.run([sys.executable, "-c", _SCRIPT], cwd=root, env=env, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and "plans: ok" in r.stdout, r.stdout + r.stderr
