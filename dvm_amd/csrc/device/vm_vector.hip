@@ -23,7 +23,7 @@
 namespace {
 
 // the program, copied from the kernel argument once per workgroup
-__shared__ uint32_t prog32[DVM_PARAM_BYTES / 4];
+__shared__ __align__(16) uint32_t prog32[DVM_PARAM_BYTES / 4];
 
 // PARTS: the program's reduce is shared between workgroups (VVecHeader::r_chunk); a build of its own, so that the
 // programs without one pay nothing for the part bounds.
@@ -37,20 +37,10 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
   // The blob arrives as a kernel argument; decoding from there would cost a
   // dependent scalar-memory round trip per access, so each workgroup copies it
   // into local memory once and decodes from there.
-  {
-    // uniform trip count and clamped indices: no per-lane branch (lanes past the end rewrite the last word)
-    // only the words the program occupies are read: the argument segment is far away
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(p.w);
-    const VVecHeader *hp = reinterpret_cast<const VVecHeader *>(p.w);
-    uint32_t used = (hp->code_off + hp->n_code) * 2;
-    used = used < DVM_PARAM_BYTES / 4 ? used : DVM_PARAM_BYTES / 4;
-    const uint32_t trips = (used + blockDim.x - 1) / blockDim.x;
-    for (uint32_t t = 0; t < trips; ++t) {
-      uint32_t i = t * blockDim.x + threadIdx.x;
-      i = i < used ? i : used - 1;
-      prog32[i] = src[i];
-    }
-    __syncthreads();
+  if constexpr (SCHED == VS_POINTWISE) {
+    fetch_program(prog32, p.w, [&]() { return (prog32[offsetof(VVecHeader, code_off) / 4] + prog32[offsetof(VVecHeader, n_code) / 4]) * 2; });
+  } else {  // (the reduce kernels are 1 % slower with it: their registers are given out another way)
+    fetch_used_words(prog32, p.w, (reinterpret_cast<const VVecHeader *>(p.w)->code_off + reinterpret_cast<const VVecHeader *>(p.w)->n_code) * 2);
   }
   STAMP();
   // the scalar fields of the header live in scalar registers; the axis tables stay in local memory

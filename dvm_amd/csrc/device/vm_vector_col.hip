@@ -14,7 +14,7 @@
 
 namespace {
 
-__shared__ uint32_t prog_lds[DVM_PARAM_BYTES / 4];
+__shared__ __align__(16) uint32_t prog_lds[DVM_PARAM_BYTES / 4];
 
 typedef uint32_t vu4_any __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes at any address of a 16- or 32-bit element
 
@@ -122,15 +122,7 @@ __device__ __forceinline__ void col_store(const VMemDesc &m, uint64_t off, const
 
 extern "C" __global__ void __launch_bounds__(512) dvm_vm_vec_col(const VmParam p) {
   const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
-  {
-    // the words the program occupies, once per workgroup (the argument segment is far away)
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(p.w);
-    const VVecHeader *hp = reinterpret_cast<const VVecHeader *>(p.w);
-    uint32_t used = (hp->code_off + hp->n_code) * 2;
-    used = used < DVM_PARAM_BYTES / 4 ? used : DVM_PARAM_BYTES / 4;
-    for (uint32_t i = tid; i < used; i += nthreads) prog_lds[i] = src[i];
-    __syncthreads();
-  }
+  fetch_program(prog_lds, p.w, [&]() { return (prog_lds[offsetof(VVecHeader, code_off) / 4] + prog_lds[offsetof(VVecHeader, n_code) / 4]) * 2; });
 #define HDR(field) uni(prog_lds[offsetof(VVecHeader, field) / 4])
   const VDim *kdims = reinterpret_cast<const VDim *>(prog_lds + offsetof(VVecHeader, kdims) / 4);
   const uint32_t n_kdim = HDR(n_kdim), n_kidx = HDR(n_kidx), n_items = HDR(n_items), mem_off = HDR(mem_off);

@@ -27,7 +27,7 @@
 namespace {
 
 // the program, copied from the kernel argument once per workgroup
-__shared__ uint32_t prog_lds[DVM_PARAM_BYTES / 4];
+__shared__ __align__(16) uint32_t prog_lds[DVM_PARAM_BYTES / 4];
 
 #define FOR_R _Pragma("unroll") for (int u = 0; u < UR; ++u)
 // One slab after the other, as written: the scheduler would otherwise interleave all of a lane's elements through a
@@ -300,19 +300,14 @@ __device__ __forceinline__ float row_one_unary(uint32_t sub, float x) {
 
 template <int UR>
 __device__ __forceinline__ void vm_vector_row(const VmParam &p) {
-  // the words the program occupies, once per workgroup (the argument segment is far away)
-  {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(p.w);
-    const VVecHeader *hp = reinterpret_cast<const VVecHeader *>(p.w);
-    uint32_t used = ((hp->row_code & 0xffffu) + (hp->row_code >> 16)) * 2;
-    used = used < DVM_PARAM_BYTES / 4 ? used : DVM_PARAM_BYTES / 4;
-    const uint32_t trips = (used + blockDim.x - 1) / blockDim.x;
-    for (uint32_t t = 0; t < trips; ++t) {
-      uint32_t i = t * blockDim.x + threadIdx.x;
-      i = i < used ? i : used - 1;
-      prog_lds[i] = src[i];
-    }
-    __syncthreads();
+  if constexpr (UR == 4) {  // (residual RMSNorm bf16 [4490,1648] 14.9 us this way, 16.6 the other)
+    const uint32_t rc = reinterpret_cast<const VVecHeader *>(p.w)->row_code;
+    fetch_used_words(prog_lds, p.w, ((rc & 0xffffu) + (rc >> 16)) * 2);
+  } else {
+    fetch_program(prog_lds, p.w, [&]() {
+      const uint32_t rc = prog_lds[offsetof(VVecHeader, row_code) / 4];
+      return ((rc & 0xffffu) + (rc >> 16)) * 2;
+    });
   }
   auto word32 = [&](uint32_t i) -> uint32_t { return uni(prog_lds[i]); };
 #define HDR(field) word32(static_cast<uint32_t>(offsetof(VVecHeader, field) / 4))

@@ -346,10 +346,8 @@ void Compiler::CompileCube(int a) {
       if (parts > 1) us += 4.8 + 0.25 * parts + 0.16 * part_mb + 0.2 * std::max(0.0, part_mb - 32.0);
       return us;
     };
-    // A call with one launch takes the host some 12 us, with two 18: a product that one launch does in that time is not
-    // split (27 x 1752 x 1736: 18.9 us a call in two launches, 12.6 in one).
-    uint32_t best_tile = 0, best_chunk = 0, one_launch_tile = 0;
-    double best = -1.0, one_launch = -1.0;
+    uint32_t best_tile = 0, best_chunk = 0;
+    double best = -1.0;
     for (int ti = 0; ti < 3; ++ti) {
       if (forced_tile >= 0 && ti != forced_tile) continue;
       const uint64_t side = DVM_CUBE_TILE_SIDE(static_cast<uint32_t>(ti)), nt = tiles(static_cast<uint32_t>(ti));
@@ -365,10 +363,6 @@ void Compiler::CompileCube(int a) {
         }
         if (forced < 2 && parts > 1 && static_cast<double>(nt) * parts * static_cast<double>(side * side) * 4.0 > 512.0 * 1024 * 1024) continue;
         const double us = estimate(ti, parts, chunk);
-        if (parts == 1 && (one_launch < 0.0 || us < one_launch)) {
-          one_launch = us;
-          one_launch_tile = static_cast<uint32_t>(ti);
-        }
         if (best < 0.0 || us < best) {
           best = us;
           best_tile = static_cast<uint32_t>(ti);
@@ -376,10 +370,6 @@ void Compiler::CompileCube(int a) {
           best_chunk = chunk;
         }
       }
-    }
-    if (k_split > 1 && forced < 2 && one_launch >= 0.0 && one_launch <= 18.0) {
-      best_tile = one_launch_tile;
-      k_split = 1;
     }
     h.tile = best_tile;
     if (k_split > 1) k_chunk = best_chunk;
