@@ -21,6 +21,8 @@ extern "C" __global__ void dvm_vm_vec_rx_sw_parts(const VmParam p);
 #define DVM_ROW_DECL(slabs) extern "C" __global__ void dvm_vm_vec_row##slabs(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_col(const VmParam p);
 DVM_ROW_DECL(1) DVM_ROW_DECL(2) DVM_ROW_DECL(3) DVM_ROW_DECL(4) DVM_ROW_DECL(5) DVM_ROW_DECL(6) DVM_ROW_DECL(8)
+#define DVM_PLANES_DECL(slabs) extern "C" __global__ void dvm_vm_vec_planes##slabs(const VmParam p);
+DVM_PLANES_DECL(1) DVM_PLANES_DECL(2) DVM_PLANES_DECL(3) DVM_PLANES_DECL(5) DVM_PLANES_DECL(6) DVM_PLANES_DECL(8)
 extern "C" __global__ void dvm_vm_vec_pw_u4(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_rx_u4(const VmParam p);
 extern "C" __global__ void dvm_vm_vec_ry_u4(const VmParam p);
@@ -69,10 +71,12 @@ static const CubeKernel kCubeKernels[DVM_CUBE_TILES][2][4] = {
     {DVM_CUBE_ROW(dvm_vm_cube_f16_deep), DVM_CUBE_ROW(dvm_vm_cube_bf16_deep)}};
 static const CubeKernel kCubeCombKernels[2] = {dvm_vm_cube_f16_comb, dvm_vm_cube_bf16_comb};
 
-// [slabs a lane]: the row build of the vector VM
+// [two reduced axes][slabs a lane]: the row build of the vector VM
 typedef void (*VecKernel)(const VmParam);
-static const VecKernel kRowKernels[9] = {nullptr, dvm_vm_vec_row1, dvm_vm_vec_row2, dvm_vm_vec_row3, dvm_vm_vec_row4,
-                                         dvm_vm_vec_row5, dvm_vm_vec_row6, nullptr, dvm_vm_vec_row8};
+static const VecKernel kRowKernels[2][9] = {
+    {nullptr, dvm_vm_vec_row1, dvm_vm_vec_row2, dvm_vm_vec_row3, dvm_vm_vec_row4, dvm_vm_vec_row5, dvm_vm_vec_row6, nullptr, dvm_vm_vec_row8},
+    {nullptr, dvm_vm_vec_planes1, dvm_vm_vec_planes2, dvm_vm_vec_planes3, nullptr, dvm_vm_vec_planes5, dvm_vm_vec_planes6, nullptr,
+     dvm_vm_vec_planes8}};
 
 // The workspace of dvm_hip_launch_vm_static_ws: device memory that belongs to the library's code object, one copy
 // per device. Host code never uses this name as an address: it asks the runtime for the array's address on the
@@ -160,8 +164,9 @@ int dvm_hip_init_vm(int dev_id, dvm_hip_sysconfig *conf) {
                                        reinterpret_cast<const void *>(dvm_vm_vec_col),
                                        reinterpret_cast<const void *>(dvm_vm_vec_pw_u4), reinterpret_cast<const void *>(dvm_vm_vec_rx_u4),
                                        reinterpret_cast<const void *>(dvm_vm_vec_ry_u4)};
-  for (VecKernel k : kRowKernels)
-    if (k != nullptr) kernels.push_back(reinterpret_cast<const void *>(k));
+  for (const auto &axes : kRowKernels)
+    for (VecKernel k : axes)
+      if (k != nullptr) kernels.push_back(reinterpret_cast<const void *>(k));
   for (const auto &tile : kCubeKernels)
     for (const auto &dt : tile)
       for (CubeKernel k : dt) kernels.push_back(reinterpret_cast<const void *>(k));
@@ -267,13 +272,21 @@ static bool row_words_hold(const VmParam &p, uint32_t threads) {
   if (!DVM_VEC_ROW_OK(slabs) || threads > DVM_VEC_ROW_LANES(slabs) || n == 0 || n > DVM_VEC_ROW_WORDS || off + n > DVM_PARAM_WORDS ||
       off < h->code_off + h->n_code || VI_OP(p.w[off + n - 1]) != VOP_END || h->mem_off + h->n_mem * (sizeof(VMemDesc) / 8) > off + n) return false;
   const uint64_t team = h->team_is_block ? threads : 64u;
-  if (h->n_rdim != 1 || h->n_kdim > 2 || h->n_mem == 0 || h->n_mem > 64 || h->inner_extent < DVM_VEC_E || h->n_ridx != (h->inner_extent + DVM_VEC_E - 1) / DVM_VEC_E ||
-      h->n_ridx > slabs * team || h->n_ridx <= (slabs - 1) * team || (h->n_kdim == 2 && h->kdims[0].extent == 0)) return false;
+  const bool planes = h->n_rdim == 2;
+  const uint64_t groups = (static_cast<uint64_t>(h->inner_extent) + DVM_VEC_E - 1) / DVM_VEC_E;
+  if ((h->n_rdim != 1 && !planes) || h->n_kdim > 2 || h->n_mem == 0 || h->n_mem > 64 || h->inner_extent < DVM_VEC_E || h->n_ridx != groups * (planes ? h->rdims[1].extent : 1u) ||
+      h->n_ridx > slabs * team || (!planes && h->n_ridx <= (slabs - 1) * team) || (planes && !DVM_VEC_PLANES_OK(slabs)) || (h->n_kdim == 2 && h->kdims[0].extent == 0)) return false;
   if (h->team_is_block ? h->n_items > h->n_kidx : static_cast<uint64_t>(h->n_items) * (threads / 64u) >= static_cast<uint64_t>(h->n_kidx) + threads / 64u) return false;
+  if (planes) {  // (the kernel divides by the groups of a plane, and its offsets have 32 bits)
+    auto divides = [](const VDim &d) { return d.shift < 32u && ((((static_cast<uint64_t>(d.extent) * d.magic) >> 32) + d.extent) >> d.shift) == 1u; };
+    if (h->rdims[0].extent != groups || h->rdims[1].extent == 0 || !divides(h->rdims[0]) ||
+        static_cast<uint64_t>(h->rdims[1].extent - 1) * h->plane_stride + h->inner_extent > DVM_VEC_PLANES_SPAN) return false;
+  }
   const VMemDesc *mems = reinterpret_cast<const VMemDesc *>(p.w + h->mem_off);
   auto mem_ok = [&](uint32_t a, bool row) {
     if (a >= h->n_mem) return false;
     const VMemDesc &m = mems[a];
+    if (planes && row && m.rstride[1] != h->plane_stride) return false;
     if (m.dtype != VDT_F32 && m.dtype != VDT_F16 && m.dtype != VDT_BF16) return false;
     if ((m.addr & (m.dtype == VDT_F32 ? 3u : 1u)) != 0) return false;
     return (m.flags & (VMF_VEC | VMF_GATHER)) == (row ? static_cast<uint32_t>(VMF_VEC) : 0u);
@@ -456,7 +469,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
         break;
       case VS_REDX:
         if (row != 0) {
-          hipLaunchKernelGGL(kRowKernels[row], dim3(block_dim), dim3(threads), lds_bytes, s, p);
+          hipLaunchKernelGGL(kRowKernels[h->n_rdim == 2 ? 1 : 0][row], dim3(block_dim), dim3(threads), lds_bytes, s, p);
         } else if (sweeps) {
           hipLaunchKernelGGL(parts ? dvm_vm_vec_rx_sw_parts : dvm_vm_vec_rx_sw, dim3(block_dim), dim3(threads), lds_bytes, s, p);
         } else {

@@ -402,6 +402,8 @@ class Compiler {
   uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;
   bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;
   bool BuildRowCode();
+  int64_t PlaneStride(const ANode &n) const;
+  bool RowsStartAligned() const;
   bool row_allowed_ = true;             // (false: the program has turned out to be outside the row build's vocabulary)
   uint64_t row_key_ = 0;                // RowKey of the layout being tried
   std::vector<uint64_t> row_refused_;   // ... of layouts that did not fit: a dynamic kernel tries each once, not at every shape

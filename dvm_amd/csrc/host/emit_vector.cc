@@ -689,6 +689,13 @@ bool Compiler::FinishProgram() {
   if (k_->tuning_.vec_sweeps != 0 && FitsSweepBuild()) hdr_.sched |= VS_SWEEPS;
   row_code_.clear();
   if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && !BuildRowCode()) return false;
+  if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && nr_ == 2) {
+    for (int i = 0; i < n_mem_; ++i)
+      if ((mems_[i].flags & VMF_VEC) != 0) {
+        if (hdr_.plane_stride != 0 && hdr_.plane_stride != mems_[i].rstride[1]) return false;
+        hdr_.plane_stride = mems_[i].rstride[1];
+      }
+  }
   if ((hdr_.sched & VS_COLS) != 0 && !FitsColBuild()) return false;
   hdr_.n_mem = n_mem_;
   hdr_.n_code = static_cast<uint32_t>(code_.size());

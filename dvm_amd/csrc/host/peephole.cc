@@ -379,7 +379,7 @@ bool Compiler::FitsSweepBuild() {
   return true;
 }
 
-// The row build's instruction words (vm_vector_row.hip), from the finished words of the program: per-output runs lose
+// The row build's instruction words (vm_vector_row.h), from the finished words of the program: per-output runs lose
 // their brackets (every wave computes them), loads lose what concerns rounds, and a sweep that begins with the very
 // words whose result the accumulator still holds from the sweep before begins behind them. False: a word outside the
 // build's vocabulary.

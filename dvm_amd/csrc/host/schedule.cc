@@ -464,12 +464,13 @@ uint32_t Log2(uint32_t v) {
   return l;
 }
 
-// Whether a sub-kernel's operators are worth trying on the row build (vm_vector_row.hip): values that vary along the
-// reduced axis are floats from contiguous rows, combined by the arithmetic that build knows. BuildRowCode has the last
+// Whether a sub-kernel's operators are worth trying on the row build (vm_vector_row.h): values that vary along the
+// reduced axis, or along either of two, are floats from contiguous rows, combined by the arithmetic that build knows. BuildRowCode has the last
 // word; this only keeps code generation from laying a program out for a build that will refuse it.
 bool Compiler::RowCandidate() const {
   if (!row_allowed_ || k_->tuning_.vec_sweeps == 0 || k_->tuning_.vec_row == 0 || k_->tuning_.vec_team >= 1) return false;
-  if (nr_ != 1 || nk_ > 2 || n_peel_ > 0 || hdr_.inner_extent < static_cast<uint32_t>(E)) return false;
+  if (nr_ > 2 || nk_ > 2 || n_peel_ > 0 || hdr_.inner_extent < static_cast<uint32_t>(E)) return false;
+  int64_t plane_stride = -1;
   auto is_float = [](DataType t) { return t == kFloat32 || t == kFloat16 || t == kBFloat16; };
   for (int i = 0; i < nn_; ++i) {
     const ANode &n = nodes_[i];
@@ -479,6 +480,11 @@ bool Compiler::RowCandidate() const {
       if (n.axis[d] < 0 || !axes_[n.axis[d]].reduced) continue;
       in_sweep = true;
       if (n.view != nullptr && pos_[n.axis[d]] == dims_[n_dims_ - 1].last_axis && n.view->vstride_[d] != 1) return false;  // read element by element
+    }
+    if (in_sweep && nr_ == 2 && (n.kind == AK_MEM || n.kind == AK_OUT)) {  // (planes: one stride between them, and every operand has both axes)
+      const int64_t stride = PlaneStride(n);
+      if (stride <= 0 || (plane_stride >= 0 && stride != plane_stride)) return false;
+      plane_stride = stride;
     }
     if (n.kind != AK_OP) continue;
     switch (n.op->kind) {
@@ -490,7 +496,22 @@ bool Compiler::RowCandidate() const {
     }
     if ((n.op->kind == kObjBinary || n.op->kind == kObjBinaryS) && (n.op->op == kPow || n.op->op == kLogicalAnd || n.op->op == kLogicalOr)) return false;
   }
-  return true;
+  return nr_ == 1 || (plane_stride > 0 && (dims_[rlist_[1]].extent - 1) * plane_stride + dims_[rlist_[0]].extent <= static_cast<int64_t>(DVM_VEC_PLANES_SPAN));
+}
+
+// Elements between two steps of the outer one of two reduced axes in an operand that has both, or -1.
+int64_t Compiler::PlaneStride(const ANode &n) const {
+  int64_t stride = 1, plane = -1;
+  bool inner = false;
+  for (int d = n.rank - 1; d >= 0; --d) {
+    if (n.axis[d] >= 0) {
+      const int p = pos_[n.axis[d]], md = dim_of_axis_[p];
+      inner = inner || md == rlist_[0];
+      if (md == rlist_[1] && p == dims_[md].last_axis) plane = n.view != nullptr ? n.view->vstride_[d] : stride;
+    }
+    stride *= n.dims[d];
+  }
+  return inner ? plane : -1;
 }
 
 // The column build: everything that varies along the one reduced axis is a load, its casts and its square.
@@ -556,12 +577,34 @@ bool Compiler::ReadsAlignedRowsOnce() const {
   return true;
 }
 
+// Whether every row (every plane) of every operand starts on 16 bytes when its tensor does.
+bool Compiler::RowsStartAligned() const {
+  for (int i = 0; i < nn_; ++i) {
+    const ANode &n = nodes_[i];
+    if (n.kind != AK_MEM && n.kind != AK_OUT) continue;
+    int64_t dense = 1;
+    bool in_sweep = false, aligned = true;
+    for (int d = n.rank - 1; d >= 0; --d) {
+      if (n.axis[d] >= 0) {
+        const int p = pos_[n.axis[d]], md = dim_of_axis_[p];
+        in_sweep = in_sweep || axes_[n.axis[d]].reduced;
+        const int64_t stride = n.view != nullptr ? n.view->vstride_[d] : dense;
+        if (md != n_dims_ - 1 && p == dims_[md].last_axis) aligned = aligned && stride * static_cast<int64_t>(DTypeSize(n.dtype)) % 16 == 0;
+      }
+      dense *= n.dims[d];
+    }
+    if (in_sweep && !aligned) return false;
+  }
+  return true;
+}
+
 // Slabs and lanes per row. A row's loads are in flight at once, so what counts is how many rows a compute unit holds at a
 // time: more slabs a lane (fewer waves a row) are taken where they raise it, and while there are rows for some 2^17 lanes
 // (two waves per SIMD) all the same. Where they do not raise it (their registers cost the waves they save, or the
 // workgroup's waves do not pack) the fewer slabs keep more lanes on the row; only eight slabs come before four at the same
 // number of rows from the fourth pass over the chip on (the build of four saves 19 registers a lane to scratch memory).
-// Only the last slab of a row may be ragged. Measured on MI355X (times of a launch, us; without the row build / with the
+// Only the last slab of a row may be ragged (over planes any may be: there eight slabs also take rows of six to seven, which
+// has no build of its own). Measured on MI355X (times of a launch, us; without the row build / with the
 // most slabs there are rows for / by this rule): log-sum-exp bf16 [1068,13440] 38 / 43 / 27, fp32 [2340,7168] 34 / 41 / 30,
 // softmax bf16 [1034,7680] 37 / 25 / 21, fp32 [2048,32001] 531 / 169 / 159, [8192,4096] 86 / 67 / 66, [4096,16384] 199 / 147
 // / 148, layer norm of a stored sum bf16 [2097,6272] 72 / 52 / 38, residual RMSNorm bf16 [8192,4096] 51 / 44 / 44, 37 rows
@@ -570,14 +613,20 @@ bool Compiler::ReadsAlignedRowsOnce() const {
 // rounds (log-sum-exp fp32 [840,19968] 35 / 36 / 40, RMSNorm bf16 [936,17920] 33 / 37 / 35), one that reads it three times
 // or computes more on it is up to twice as fast.
 bool Compiler::ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const {
-  if (n_r <= 32) return false;  // (up to 256 elements: several rows share a wave on the other builds)
+  const bool planes = nr_ == 2;
+  // Up to 256 elements several rows share a wave on the other builds. A wave for each row is faster until the rows of such waves
+  // are more than the chip holds a few times over, and where rows do not start on 16 bytes for twice as many. Measured on MI355X
+  // (us, rows sharing waves / a wave for each): softmax fp16 [32,64] 9.5 / 6.7, [32,100] 16.9 / 6.7, [2048,128] 10.4 / 7.5,
+  // [4096,128] 10.4 / 8.7, [8192,128] 10.6 / 13.7, [8192,100] 18.0 / 13.7, [16384,100] 20.5 / 24.8; RMSNorm fp16 [256,200]
+  // 13.9 / 6.3; fp32 row sums [1024,64] 5.6 / 4.1, [8192,64] 5.8 / 6.9.
+  if (n_r <= 32 && (n_k > 8192 || (n_k >= 4096 && RowsStartAligned()))) return false;
   const uint64_t cus = g_system.core_num > 0 ? g_system.core_num : 256;
   uint32_t best = 0, best_team = 0;
   uint64_t best_rows = 0;  // per compute unit
   for (uint32_t u = 1; u <= 8; ++u) {
-    if (!DVM_VEC_ROW_OK(u) || (k_->tuning_.vec_row > 0 && u > static_cast<uint32_t>(k_->tuning_.vec_row))) continue;
+    if (!(planes ? DVM_VEC_PLANES_OK(u) : DVM_VEC_ROW_OK(u)) || (k_->tuning_.vec_row > 0 && u > static_cast<uint32_t>(k_->tuning_.vec_row))) continue;
     const uint64_t t = ((n_r + u - 1) / u + 63) / 64 * 64;
-    if (t > DVM_VEC_ROW_LANES(u) || n_r <= t * (u - 1)) continue;
+    if (t > DVM_VEC_ROW_LANES(u) || n_r <= t * (planes && u == 8 ? 6 : u - 1)) continue;
     if (best != 0 && n_k * t < (1ull << 17)) break;  // (more slabs would leave lanes idle)
     const uint64_t rows = t > 64 ? DVM_WG_PER_CU(DVM_VEC_ROW_WAVES(u), t / 64) : 4ull * DVM_VEC_ROW_WAVES(u);
     if (rows < best_rows || (rows == best_rows && !(u == 8 && best == 4 && rows > 1 && n_k > 3 * rows * cus))) continue;
@@ -589,6 +638,10 @@ bool Compiler::ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *
   // (one or two rows at a time are a trip to memory with nothing under it. Where rows are kept for a second sweep that still
   // pays; a row sum at [1297,12928] in fp16 takes 17.0 us here and 14.6 in rounds, [589,28444] in fp32 22.2 and 19.2)
   if (best_rows <= 2 && n_k > 2 * best_rows * cus && ReadsAlignedRowsOnce()) return false;
+  // (planes that start on 16 bytes: from the second pass over the chip on the rounds are as fast, since their loads and stores
+  // overlap and one row a unit leaves nothing to. Batch-norm, us in rounds / here: [24,256,28,28] 22.3 / 17.3, [24,512,28,28]
+  // 28.7 / 29.8, [20,1024,28,28] 39.2 / 52.4; planes that do not, [30,1024,27,27] 134 / 68)
+  if (planes && n_k > best_rows * cus && RowsStartAligned()) return false;
   *slabs = best;
   *team = best_team;
   return true;

@@ -69,10 +69,12 @@ enum {
   // of what it loads, then reduce results, float binaries (add .. max) on immediates or the accumulator, roundings and
   // stores. The generic kernel runs the same words at the same geometry.
   VS_COLS = 0x40,
-  // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.hip) may run the program from the words at
-  // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space is one axis of n_ridx
-  // groups, more than (slabs - 1) * team and at most slabs * team of them (team: the workgroup when team_is_block, else
-  // one wave), and holds at least eight elements. The words at code_off are valid for the generic kernel at the same
+  // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.h) may run the program from the words at
+  // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space has n_ridx groups, at most
+  // slabs * team of them (team: the workgroup when team_is_block, else one wave), and at least eight elements along its inner
+  // axis. It is one axis and more than (slabs - 1) * team groups (dvm_vm_vec_row*), or planes of inner_extent elements
+  // that lie VVecHeader::plane_stride elements apart in every operand that varies along them (dvm_vm_vec_planes*), at
+  // most DVM_VEC_PLANES_SPAN elements from the first to the last. The words at code_off are valid for the generic kernel at the same
   // geometry: without these bits the blob runs there.
   VS_ROW_SHIFT = 8,
   VS_ROW_MASK = 0xf00,
@@ -81,7 +83,12 @@ enum {
 #define DVM_VEC_ROW_WORDS 64  // instruction words of a row program at most (one per lane of a wave)
 // slabs a lane the row build exists for, and the lanes a workgroup of that build may have
 #define DVM_VEC_ROW_OK(slabs) ((slabs) >= 1u && (slabs) <= 8u && (slabs) != 7u)
+// (over planes: not four, whose kernel would save 37 registers a lane to scratch memory and was the slowest of all that hold a
+// row, 22.9 us against 17.3 with three and 19.4 with eight at [24,256,28,28]; eight take a row of six to eight slabs there)
+#define DVM_VEC_PLANES_OK(slabs) (DVM_VEC_ROW_OK(slabs) && (slabs) != 4u)
 #define DVM_VEC_ROW_LANES(slabs) ((slabs) <= 4u ? 1024u : 512u)
+// elements from the first of a row's first plane to behind the last of its last one (byte offsets in 32 bits)
+#define DVM_VEC_PLANES_SPAN 0x3fff0000u
 // waves a SIMD that build's registers leave room for (79, 95, 128, 128, 167, 200 and 255 of 512)
 #define DVM_VEC_ROW_WAVES(slabs) ((slabs) <= 2u ? 5u : ((slabs) <= 4u ? 4u : ((slabs) == 5u ? 3u : 2u)))
 // Workgroups of `waves` waves a compute unit holds at `per_simd` waves on each of its four SIMDs. Up to four waves are
@@ -276,7 +283,8 @@ typedef struct {
   uint32_t r_chunk;
   uint32_t k_per_chunk;
   uint32_t row_code;     // VS_ROW*: word offset of the row build's instruction words, their number << 16
-  uint32_t pad;          // (keeps the axis tables 16-byte aligned: the interpreter reads them as 128-bit words)
+  uint32_t plane_stride; // VS_ROW* with two reduced axes: elements from one plane to the next (the field also keeps the axis
+                         // tables 16-byte aligned: the interpreter reads them as 128-bit words)
   VDim kdims[DVM_VEC_MAXR];
   VDim rdims[DVM_VEC_MAXR];
 } VVecHeader;            // 80 + 128 = 208 bytes
