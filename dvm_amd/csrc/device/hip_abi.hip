@@ -491,10 +491,14 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const uint32_t want_threads = comb ? 256u : DVM_CUBE_TILE_LANES(c->tile);
     // (the sum of parts in pieces of 64 x 64; a program exported with the geometry of the tile's own kernel is taken as well)
     const uint32_t lds_need = comb ? DVM_CUBE_LDS_BYTES(2u) : DVM_CUBE_LDS_BYTES(c->tile);
+    // (programs of the 64 tile and sums of parts are also taken with two stage buffers, as they were exported when that tile had
+    // no more, and run with what the kernel uses)
+    const uint32_t lds_exported = (comb || c->tile == 2) ? DVM_CUBE_LDS_TWO_STAGES : lds_need;
+    const uint32_t lds_groups = c->group_mode != VCG_NONE ? 8u * c->nb1 : 0u;
     // The tile loop trusts the header: check it describes the launch it gets.
     if (mem_end > DVM_PARAM_WORDS || code_end > DVM_PARAM_WORDS || c->n_code == 0 || VI_OP(p.w[code_end - 1]) != VOP_END ||
         c->tile >= DVM_CUBE_TILES || (threads != want_threads && !(comb && c->tile == 3 && threads == 512u)) || c->m == 0 || c->n == 0 || c->nb0 == 0 || c->nb1 == 0 ||
-        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < lds_need ||
+        c->tiles_m != (c->m + bt - 1) / bt || c->tiles_n != (c->n + bt - 1) / bt || lds_bytes < lds_exported ||
         c->a_addr == 0 || c->b_addr == 0 || (c->dtype != VDT_F16 && c->dtype != VDT_BF16)) {
       return static_cast<int>(hipErrorInvalidValue);
     }
@@ -504,7 +508,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
       const bool rows = c->group_mode == VCG_M_BOUND || c->group_mode == VCG_M_SIZE;
       if (c->group_mode > VCG_K_SIZE || c->group_addr == 0 || (c->group_addr & (c->group_i32 ? 3u : 7u)) != 0 || c->nb0 != 1 ||
           c->nb1 > DVM_CUBE_MAX_GROUPS || (c->epi_flags & (VCF_SPLITK_PARTIAL | VCF_SPLITK_COMBINE)) != 0 ||
-          lds_bytes < lds_need + 8u * c->nb1 || (rows && (c->a_sb0 != 0 || c->a_sb1 != 0))) {
+          lds_bytes < lds_exported + lds_groups || (rows && (c->a_sb0 != 0 || c->a_sb1 != 0))) {
         return static_cast<int>(hipErrorInvalidValue);
       }
     }
@@ -526,7 +530,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const CubeKernel kern = comb ? kCubeCombKernels[c->dtype == VDT_BF16 ? 1 : 0]
                                 : kCubeKernels[c->tile][c->dtype == VDT_BF16 ? 1 : 0][(c->trans_a ? 2 : 0) + (c->trans_b ? 1 : 0)];
     if (check_only) return 0;
-    hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), lds_bytes, s, p);
+    hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), lds_bytes < lds_need + lds_groups ? lds_need + lds_groups : lds_bytes, s, p);
   } else if (h->entry == VE_ATTN) {
     const VAttnHeader *a = reinterpret_cast<const VAttnHeader *>(p.w);
     // the kernels have no guards of their own beyond the query and key tails: the header must fit them exactly

@@ -387,6 +387,7 @@ enum { VCG_NONE = 0, VCG_M_BOUND = 1, VCG_M_SIZE = 2, VCG_K_BOUND = 3, VCG_K_SIZ
 #define DVM_CUBE_LDS_DUMP32_BYTES(bt) (((bt) >= 128u ? (bt) / 2u : (bt)) * ((bt) + 4u) * 4u)
 #define DVM_CUBE_LDS_DUMP16_BYTES(bt) ((bt) * ((bt) + 8u) * 2u)
 #define DVM_CUBE_MAX2(a, b) ((a) > (b) ? (a) : (b))
+#define DVM_CUBE_LDS_TWO_STAGES (2u * DVM_CUBE_STAGE_K * (2u * 64u) * 2u)  // the 64 tile with two stage buffers
 #define DVM_CUBE_LDS_BYTES(tile) \
   DVM_CUBE_MAX2(DVM_CUBE_LDS_LOOP_BYTES(tile), \
                 DVM_CUBE_MAX2(DVM_CUBE_LDS_DUMP32_BYTES(DVM_CUBE_TILE_SIDE(tile)), DVM_CUBE_LDS_DUMP16_BYTES(DVM_CUBE_TILE_SIDE(tile))))

@@ -63,3 +63,32 @@ def test_batches_end_inside_a_stage(monkeypatch):
     # the row behind the last of one matrix is the first of the next: it must not be read for it
     _run(40, 72, 88, False, True, batch=(3,))
     _run(40, 72, 88, True, False, batch=(3,))
+
+
+def test_a_program_of_the_64_tile_exported_with_two_stage_buffers_still_runs():
+    import ctypes
+    import os
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "dvm_amd", "lib", "libdvm_hip.so"))
+    lib.dvm_hip_launch_vm_static_ws.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_uint32),
+                                                ctypes.c_uint32, ctypes.c_size_t, ctypes.c_void_p]
+    lib.dvm_hip_memset.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+    lib.dvm_hip_synchronize_stream.argtypes = [ctypes.c_void_p]
+    rng = np.random.default_rng(2)
+    for m, n, k, launches in ((100, 200, 320, 1), (64, 64, 8192, 2)):
+        a, b = (rng.standard_normal(s).astype(np.float16) / 16 for s in ((m, k), (k, n)))
+        t = Tester("mix")
+        out = t.store(t.matmul(t.load(a), t.load(b), False, False))
+        t.run()
+        want = t.output(out).copy()
+        programs = t.programs()
+        assert len(programs) == launches, t.das()
+        blobs = b"".join(p[0] for p in programs)
+        pairs = [v for i, p in enumerate(programs) for w in p[2] for v in (i, w)]
+        words = (ctypes.c_uint32 * max(1, len(pairs)))(*pairs)
+        for lds, rc in ((32768, 0), (32768 - 16, 1)):  # (1: hipErrorInvalidValue, before anything is launched)
+            geo = (ctypes.c_uint32 * (3 * len(programs)))(*[v for p in programs for v in (p[1][0], p[1][1], lds)])
+            assert lib.dvm_hip_memset(t.device_ptr(out), 0, want.nbytes) == 0
+            got_rc = lib.dvm_hip_launch_vm_static_ws(ctypes.create_string_buffer(blobs, len(blobs)), len(programs), geo, words, len(pairs) // 2, t.workspace_bytes(), None)
+            assert got_rc == rc and lib.dvm_hip_synchronize_stream(None) == 0
+            got = t.output(out)
+            assert np.array_equal(got.view(np.uint16), want.view(np.uint16)) if rc == 0 else not got.any()
