@@ -358,6 +358,20 @@ static bool row_words_hold(const VmParam &p, uint32_t threads) {
   return true;
 }
 
+// VS_RUNS32 changes which elements a lane holds: only programs in which that is the same for every operand.
+static bool runs_hold(const VmParam &p) {
+  const VVecHeader *h = reinterpret_cast<const VVecHeader *>(p.w);
+  const VMemDesc *mems = reinterpret_cast<const VMemDesc *>(p.w + h->mem_off);
+  if ((h->sched & (VS_KIND_MASK | VS_WIDE)) != VS_POINTWISE || h->n_kdim != 1) return false;
+  for (uint32_t i = 0; i < h->n_mem; ++i) {
+    if (mems[i].dtype != VDT_F32 || (mems[i].flags & VMF_GATHER) != 0) return false;
+    if ((mems[i].flags & VMF_VEC) != 0 ? (mems[i].flags & VMF_ALIGNED) == 0 || mems[i].kstride[0] != 1 : mems[i].kstride[0] != 0) return false;
+  }
+  for (uint32_t i = h->code_off; i < h->code_off + h->n_code; ++i)
+    if (VI_OP(p.w[i]) == VOP_LDX) return false;
+  return true;
+}
+
 // Checks one program blob against the launch it is to get and launches the interpreter kernel its entry type names.
 // The column build trusts its flag: the program is what VS_COLS says, the teams cover the kept index space, and the operands
 // lie where 128-bit accesses to whole elements reach them.
@@ -432,6 +446,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const uint32_t row = DVM_VEC_ROW_SLABS(h->sched);
     if (row != 0 && (wide || h->r_chunk != 0 || (h->sched & VS_KIND_MASK) != VS_REDX || !row_words_hold(p, threads))) return static_cast<int>(hipErrorInvalidValue);
     if (row == 0 && sweeps && (wide || (h->sched & VS_KIND_MASK) != VS_REDX || !sweeps_flag_holds(p))) return static_cast<int>(hipErrorInvalidValue);
+    if ((h->sched & VS_RUNS32) != 0 && !runs_hold(p)) return static_cast<int>(hipErrorInvalidValue);
     const bool cols = (h->sched & VS_COLS) != 0;
     if (cols && (wide || (h->sched & VS_KIND_MASK) != VS_REDY || !col_words_hold(p, threads))) return static_cast<int>(hipErrorInvalidValue);
     // a reduce shared between workgroups: its parts are the outermost kept axis and cover the reduced index space

@@ -308,7 +308,8 @@ __device__ __forceinline__ Slabs slab_state(uint32_t nvp) {
 
 // Wide path of a load: the slabs in `full` are full and aligned in every lane of the wave (the others are empty
 // in every lane and read as zero). All loads are issued before any use.
-__device__ __forceinline__ void mem_load_wide(const VMemDesc &m, const Offs &off, uint32_t full, Acc &out) {
+// (half: from the first half of a 32-bit slab to the second, in units of 16 bytes; see VS_RUNS32)
+__device__ __forceinline__ void mem_load_wide(const VMemDesc &m, const Offs &off, uint32_t full, Acc &out, uint32_t half = 1u) {
   const uint32_t dtype = m.dtype;
   if (dtype == VDT_F32 || dtype == VDT_I32) {
     vf4 a[U], b[U];
@@ -318,7 +319,7 @@ __device__ __forceinline__ void mem_load_wide(const VMemDesc &m, const Offs &off
       if ((full >> u) & 1u) {
         const DVM_GLOBAL vf4 *p = reinterpret_cast<const DVM_GLOBAL vf4 *>(m.addr + off.v[u] * 4);
         a[u] = p[0];
-        b[u] = p[1];
+        b[u] = p[half];
       }
     }
     FOR_U out.v[u] = __builtin_shufflevector(a[u], b[u], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -360,7 +361,7 @@ __device__ __forceinline__ void mem_load_wide(const VMemDesc &m, const Offs &off
 
 // Two operands that walk memory identically (same element offsets), both on the wide path: every load of both is
 // issued before anything is used, so the pair costs one trip to memory instead of two.
-__device__ __forceinline__ void mem_load2_wide(const VMemDesc &m, const VMemDesc &mb, const Offs &off, uint32_t full, Acc &x, Acc &y) {
+__device__ __forceinline__ void mem_load2_wide(const VMemDesc &m, const VMemDesc &mb, const Offs &off, uint32_t full, Acc &x, Acc &y, uint32_t half = 1u) {
   if (m.dtype == VDT_BF16 && mb.dtype == VDT_BF16) {
     vu4 a[U], b[U];
     FOR_U {
@@ -402,9 +403,9 @@ __device__ __forceinline__ void mem_load2_wide(const VMemDesc &m, const VMemDesc
         const DVM_GLOBAL vf4 *pa = reinterpret_cast<const DVM_GLOBAL vf4 *>(m.addr + off.v[u] * 4);
         const DVM_GLOBAL vf4 *pb = reinterpret_cast<const DVM_GLOBAL vf4 *>(mb.addr + off.v[u] * 4);
         a0[u] = pa[0];
-        a1[u] = pa[1];
+        a1[u] = pa[half];
         b0[u] = pb[0];
-        b1[u] = pb[1];
+        b1[u] = pb[half];
       }
     }
     FOR_U {
@@ -475,14 +476,14 @@ __device__ __forceinline__ void mem_load_wide_2rounds(const VMemDesc &m, const O
   }
 }
 
-__device__ __forceinline__ void mem_store_wide(const VMemDesc &m, const Offs &off, uint32_t full, const Acc &in) {
+__device__ __forceinline__ void mem_store_wide(const VMemDesc &m, const Offs &off, uint32_t full, const Acc &in, uint32_t half = 1u) {
   const uint32_t dtype = m.dtype;
   FOR_U {
     if (!((full >> u) & 1u)) continue;
     if (dtype == VDT_F32 || dtype == VDT_I32) {
       DVM_GLOBAL vf4 *p = reinterpret_cast<DVM_GLOBAL vf4 *>(m.addr + off.v[u] * 4);
       p[0] = __builtin_shufflevector(in.v[u], in.v[u], 0, 1, 2, 3);
-      p[1] = __builtin_shufflevector(in.v[u], in.v[u], 4, 5, 6, 7);
+      p[half] = __builtin_shufflevector(in.v[u], in.v[u], 4, 5, 6, 7);
     } else if (dtype == VDT_BF16) {
       vu4 a;
 #pragma unroll
@@ -503,11 +504,11 @@ __device__ __forceinline__ void mem_store_wide(const VMemDesc &m, const Offs &of
   }
 }
 
-__device__ __forceinline__ void mem_load(const VMemDesc &m, const Offs &off, const Slabs &sl, Acc &out) {
+__device__ __forceinline__ void mem_load(const VMemDesc &m, const Offs &off, const Slabs &sl, Acc &out, uint32_t half = 1u) {
   const uint32_t nvp = sl.nvp;
   const bool fast = (m.flags & (VMF_VEC | VMF_ALIGNED)) == (VMF_VEC | VMF_ALIGNED);
   if (fast && sl.uniform) {
-    mem_load_wide(m, off, sl.full, out);
+    mem_load_wide(m, off, sl.full, out, half);
   } else if (!(m.flags & (VMF_VEC | VMF_GATHER)) && (m.dtype == VDT_F32 || m.dtype == VDT_I32)) {
     // one 32-bit element per slab, replicated (an operand broadcast along the innermost axis: a per-channel
     // scale, a per-row statistic); lanes without a valid slab read the base element and get zero, like the
@@ -522,10 +523,10 @@ __device__ __forceinline__ void mem_load(const VMemDesc &m, const Offs &off, con
   }
 }
 
-__device__ __forceinline__ void mem_store(const VMemDesc &m, const Offs &off, const Slabs &sl, const Acc &in) {
+__device__ __forceinline__ void mem_store(const VMemDesc &m, const Offs &off, const Slabs &sl, const Acc &in, uint32_t half = 1u) {
   const bool fast = (m.flags & (VMF_VEC | VMF_ALIGNED)) == (VMF_VEC | VMF_ALIGNED);
   if (fast && sl.uniform) {
-    mem_store_wide(m, off, sl.full, in);
+    mem_store_wide(m, off, sl.full, in, half);
   } else {
     mem_store_slow(m.addr, m.dtype, m.flags, off, sl.nvp, in);
   }

@@ -45,13 +45,14 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
   STAMP();
   // the scalar fields of the header live in scalar registers; the axis tables stay in local memory
   struct {
-    uint32_t n_kdim, n_rdim, team_log2, team_is_block, n_kidx, n_ridx, inner_extent, n_items, mem_off, code_off, n_vslot, r_chunk, k_per_chunk;
+    uint32_t n_kdim, n_rdim, sched, team_log2, team_is_block, n_kidx, n_ridx, inner_extent, n_items, mem_off, code_off, n_vslot, r_chunk, k_per_chunk;
     const VDim *kdims, *rdims;
   } h;
   {
     const VVecHeader *hp = reinterpret_cast<const VVecHeader *>(prog32);
     h.n_kdim = uni(hp->n_kdim);
     h.n_rdim = uni(hp->n_rdim);
+    h.sched = uni(hp->sched);
     h.team_log2 = uni(hp->team_log2);
     h.team_is_block = uni(hp->team_is_block);
     h.n_kidx = uni(hp->n_kidx);
@@ -134,6 +135,9 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
     }
 
     const Slabs sl_out = slab_state(nvp_out);
+    // VS_RUNS32: a wave whose slabs are full holds them in two runs of four elements a lane
+    const bool runs = SCHED == VS_POINTWISE && (h.sched & VS_RUNS32) != 0u && sl_out.uniform;
+    const uint32_t half = runs ? 64u : 1u;
     bool in_sweep = false;
     Slabs sl = sl_out;  // valid counts of the current round's slabs (outside sweeps: of the lane's output)
     uint32_t round = 0, sweep_pc = 0, slot_kinds = 0;
@@ -212,7 +216,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
           const uint32_t wb = uni(fetched[0]);
           const VMemDesc mb = load_desc(prog32, mem_off, wb >> 24);
           if ((mb.flags & kFast) == kFast) {
-            mem_load2_wide(m, mb, off, s2.full, x, y);
+            mem_load2_wide(m, mb, off, s2.full, x, y, half);
             w0 = wb;
             op = wb & 0x7fu;
             sub = (wb >> 8) & 0xffu;
@@ -221,7 +225,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
             return true;
           }
         }
-        mem_load(m, off, s2, x);
+        mem_load(m, off, s2, x, half);
         return false;
       };
 
@@ -378,6 +382,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
               FOR_U {
                 const uint32_t ku = kidx + u * nthreads;
                 off.v[u] = space_offset(ku < h.n_kidx ? ku : 0u, h.kdims, h.n_kdim, m.kstride, true);
+                if (runs && (m.flags & VMF_VEC) != 0u) off.v[u] -= (tid & 63u) * 4u;
               }
             } else {
               const uint64_t koff = space_offset(kvalid ? kidx : 0u, h.kdims, h.n_kdim, m.kstride, !inner_red);
@@ -545,7 +550,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
             acc = mem_gather(m.addr, m.dtype, m.flags, off, sl.nvp, acc);
             continue;
           } else {
-            mem_load(m, off, sl, src);
+            mem_load(m, off, sl, src, half);
             if (op == VOP_BINF && (imm & VI_PRE_SREG)) {  // an S-register binary in front, while the operand is on its way
               const float pv = sreg_read(sr, (imm >> 8) & 0xffu);
               switch (imm & 0x3fu) {
@@ -689,6 +694,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
               FOR_U {
                 const uint32_t ku = kidx + u * nthreads;
                 off.v[u] = space_offset(ku < h.n_kidx ? ku : 0u, h.kdims, h.n_kdim, m.kstride, true);
+                if (runs && (m.flags & VMF_VEC) != 0u) off.v[u] -= (tid & 63u) * 4u;
               }
             } else {
               const uint64_t koff = space_offset(kvalid ? kidx : 0u, h.kdims, h.n_kdim, m.kstride, !inner_red);
@@ -708,7 +714,7 @@ __device__ __forceinline__ void vm_vector(const VmParam &p) {
               st.uniform = false;
             }
           }
-          mem_store(m, off, st, acc);
+          mem_store(m, off, st, acc, half);
           break;
         }
         case VOP_UN: {

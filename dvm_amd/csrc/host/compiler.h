@@ -402,6 +402,7 @@ class Compiler {
   uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;
   bool ChooseRow(uint64_t n_k, uint64_t n_r, uint32_t *slabs, uint32_t *team) const;
   bool BuildRowCode();
+  bool HoldsRuns() const;
   int64_t PlaneStride(const ANode &n) const;
   bool RowsStartAligned() const;
   bool row_allowed_ = true;             // (false: the program has turned out to be outside the row build's vocabulary)

@@ -209,6 +209,7 @@ std::string &VKernel::DisAssemble() {
       os << "entry vector sched=" << sched[h->sched & VS_KIND_MASK] << ((h->sched & VS_WIDE) ? " wide" : "") << ((h->sched & VS_SWEEPS) && DVM_VEC_ROW_SLABS(h->sched) == 0 ? " sweeps" : "");
       if (DVM_VEC_ROW_SLABS(h->sched) != 0) os << " row=" << DVM_VEC_ROW_SLABS(h->sched);  // (the build that runs, whatever others could)
       if (h->sched & VS_COLS) os << " columns";
+      if (h->sched & VS_RUNS32) os << " runs";
       os << " blocks=" << p.grid << " threads=" << p.threads
          << " lds=" << p.lds_bytes << " items=" << h->n_items << " kept=" << h->n_kidx << " red=" << h->n_ridx
          << " inner=" << h->inner_extent << " team=" << (h->team_is_block ? p.threads : (1u << h->team_log2))

@@ -687,6 +687,7 @@ bool Compiler::FinishProgram() {
   if (k_->tuning_.vec_unirun != 0) MarkUniformRuns();
   if (k_->tuning_.vec_pair != 0) PairLoads();
   if (k_->tuning_.vec_sweeps != 0 && FitsSweepBuild()) hdr_.sched |= VS_SWEEPS;
+  if (k_->tuning_.vec_runs32 != 0 && HoldsRuns()) hdr_.sched |= VS_RUNS32;
   row_code_.clear();
   if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && !BuildRowCode()) return false;
   if (DVM_VEC_ROW_SLABS(hdr_.sched) != 0 && nr_ == 2) {

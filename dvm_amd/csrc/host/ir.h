@@ -230,6 +230,7 @@ struct Tuning {
   int vec_reread = -1;  // DVM_VEC_REREAD=0: nothing parked, no reversed sweeps; 2: parked rounds only; 3: reversed sweeps only
   int vec_sweeps = -1;  // DVM_VEC_SWEEPS=0: never the sweep build of the vector VM
   int vec_row = -1;     // DVM_VEC_ROW=0: never the row build of the vector VM; n: at most n slabs a lane there
+  int vec_runs32 = -1;  // DVM_VEC_RUNS32=0: fp32 pointwise programs keep a lane's eight elements side by side
   int vec_gather_tile = -1;  // DVM_VEC_GATHER_TILE=0: pointwise programs with a gathered operand keep the plain slab order
   int vec_col = -1;     // DVM_VEC_COL=0: never the column build of the vector VM
   int cube_tile = -1;   // DVM_CUBE_TILE=256|128|64

@@ -35,6 +35,7 @@ void Tuning::Read() {
   vec_reread = num("DVM_VEC_REREAD");
   vec_sweeps = num("DVM_VEC_SWEEPS");
   vec_row = num("DVM_VEC_ROW");
+  vec_runs32 = num("DVM_VEC_RUNS32");
   vec_col = num("DVM_VEC_COL");
   vec_gather_tile = num("DVM_VEC_GATHER_TILE");
   cube_tile = num("DVM_CUBE_TILE");
@@ -233,6 +234,7 @@ void VKernel::BindAddresses(const RelocEntry *relocs, size_t n, WsAllocator *all
           char *sched_at = reinterpret_cast<char *>(p.blob.w) + offsetof(VVecHeader, sched);
           std::memcpy(&sched, sched_at, sizeof(sched));
           sched &= ~static_cast<uint32_t>(VS_SWEEPS);
+          if ((m->flags & VMF_VEC) != 0) sched &= ~static_cast<uint32_t>(VS_RUNS32);
           if ((addr & (element - 1)) != 0) sched &= ~static_cast<uint32_t>(VS_ROW_MASK | VS_COLS);
           std::memcpy(sched_at, &sched, sizeof(sched));
         } else if (pt.role == Program::kPatchCubeOperand) {

@@ -69,6 +69,10 @@ enum {
   // of what it loads, then reduce results, float binaries (add .. max) on immediates or the accumulator, roundings and
   // stores. The generic kernel runs the same words at the same geometry.
   VS_COLS = 0x40,
+  // flag (VS_POINTWISE only, not VS_WIDE): one kept axis, and every operand is fp32: contiguous and 16-byte aligned, or one element for
+  // all. A wave's elements may then be spread over its lanes in any way that is the same for every operand, and the wave
+  // of 512 elements takes lane i's eight as [4i, 4i + 4) and [256 + 4i, 256 + 4i + 4): an access instruction moves whole lines.
+  VS_RUNS32 = 0x80,
   // bits [11:8] (VS_REDX only, 0: none): the row build (vm_vector_row.h) may run the program from the words at
   // VVecHeader::row_code with this many slabs of eight elements a lane. The reduced index space has n_ridx groups, at most
   // slabs * team of them (team: the workgroup when team_is_block, else one wave), and at least eight elements along its inner
