@@ -186,6 +186,7 @@ class Compiler {
   // Only reduces whose consumers work on the reduce's own output shape qualify (a consumer that walks x again would
   // be as short of workgroups in the second launch). SplitLongReduces rewrites the operator list and returns true
   // if it changed anything; UndoSplitReduces restores it and renumbers the operators the programs refer to.
+  size_t RunShared();
   bool SplitLongReduces();
   void UndoSplitReduces(bool keep_programs);
   struct SplitRecord {
@@ -397,6 +398,11 @@ class Compiler {
   bool ColCandidate(uint32_t *elem_size) const;
   bool FitsColBuild() const;
   bool ReducesColumnsOfALoad(const NDObject *r, const NDObject **load) const;
+  bool WalkedBesideItsReduces(const NDObject *load) const;
+  uint64_t GraphKey() const;
+  std::vector<const NDObject *> unshared_;  // reduces left in one launch because the column build is to take them ...
+  bool unshared_refused_ = false;           // ... and whether one of them ended on another build
+  std::vector<uint64_t> unshared_not_;      // GraphKey of the graphs where that happened: shared there from then on
   bool col_allowed_ = true;             // (false: the program has turned out to be outside the column build's vocabulary)
   bool ReadsAlignedRowsOnce() const;
   uint64_t RowKey(uint32_t slabs, uint32_t lanes) const;

@@ -833,6 +833,10 @@ void Compiler::CompileArea(int a) {
     EmitProgram();
     FinishProgram();
   }
+  if ((hdr_.sched & VS_COLS) == 0 && !unshared_.empty()) {
+    for (int i = 0; i < nn_; ++i)
+      if (nodes_[i].kind == AK_REDUCE && std::find(unshared_.begin(), unshared_.end(), nodes_[i].op) != unshared_.end()) unshared_refused_ = true;
+  }
   if (n_peel_ > 0) ReplicatePeeled();
 }
 

@@ -56,6 +56,28 @@ void Tuning::Read() {
 // shapes, 2 additionally ends a sub-kernel after every reduce (the reference's rule), 3 gives
 // every operator its own sub-kernel.
 size_t Compiler::Run() {
+  const int mode_before = k_->part_mode_, limit_before = k_->ops_limit_;
+  const uint32_t cap_before = k_->pw_cap_;
+  unshared_.clear();
+  try {
+    const size_t ws = RunShared();
+    if (!unshared_refused_) return ws;
+  } catch (...) {
+    if (unshared_.empty()) throw;
+  }
+  // A reduce was left in one launch for the column build, and its sub-kernel did not end there: on any other build that is
+  // a handful of workgroups (fp32 [4096,2048], its column sum beside its exponential: 664 us, 30 shared), so once more with
+  // every long reduce shared.
+  if (unshared_not_.size() >= 256) unshared_not_.clear();
+  unshared_not_.push_back(GraphKey());
+  unshared_.clear();
+  k_->part_mode_ = mode_before;
+  k_->ops_limit_ = limit_before;
+  k_->pw_cap_ = cap_before;
+  return RunShared();
+}
+
+size_t Compiler::RunShared() {
   // Reduces with few outputs and a long reduced extent are rewritten, for this code generation only, into a reduce
   // per part of the reduced index space and a reduce over the parts; should that graph not compile, the kernel
   // is compiled as it was built.
@@ -163,6 +185,7 @@ size_t Compiler::RunOnce(int mode) {
   k_->ws_offsets_.clear();
   PlanMaterialisation();
   key_parts_bytes_ = 0;
+  unshared_refused_ = false;
   for (int a = 0; a < n_areas_; ++a) CompileArea(a);
   for (Program &p : k_->programs_)
     if (!p.skip) p.RememberBindDependent();

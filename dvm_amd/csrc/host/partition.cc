@@ -252,6 +252,46 @@ bool Compiler::ReducesColumnsOfALoad(const NDObject *r, const NDObject **load) c
   return true;
 }
 
+// Whether something other than a reduce certainly walks a load (or what is computed from it) in the launch of its reduces:
+// operators of loads alone, over the same elements, that end in a store.
+bool Compiler::WalkedBesideItsReduces(const NDObject *load) const {
+  std::vector<char> of_loads(k_->ops_.size(), 0);
+  for (const NDObject *c : k_->ops_) {
+    bool from_loads = c->kind == kObjLoad || (IsPointwiseKind(c->kind) && c->nin > 0);
+    for (int j = 0; from_loads && j < c->nin; ++j) from_loads = c->in[j] != nullptr && c->in[j]->id < c->id && of_loads[static_cast<size_t>(c->in[j]->id)] != 0;
+    of_loads[static_cast<size_t>(c->id)] = from_loads;
+  }
+  std::vector<const NDObject *> walk = {load};
+  for (size_t i = 0; i < walk.size(); ++i) {
+    for (const NDObject *c : k_->ops_) {
+      bool uses = false;
+      for (int j = 0; j < c->nin; ++j) uses = uses || c->in[j] == walk[i];
+      if (!uses || !of_loads[static_cast<size_t>(c->id)]) continue;
+      if (IsStoreLike(c)) return true;
+      if (c->numel() == load->numel() && std::find(walk.begin(), walk.end(), c) == walk.end()) walk.push_back(c);
+    }
+  }
+  return false;
+}
+
+// What decides how the operators are grouped and laid out: the graph, its shapes and the strides of its loads.
+uint64_t Compiler::GraphKey() const {
+  uint64_t h = 0xcbf29ce484222325ull;  // FNV-1a
+  auto add = [&h](uint64_t v) { h = (h ^ v) * 0x100000001b3ull; };
+  for (const NDObject *o : k_->ops_) {
+    add(static_cast<uint64_t>(o->kind) | static_cast<uint64_t>(o->op) << 16 | static_cast<uint64_t>(o->type_id_) << 24 | static_cast<uint64_t>(o->strided) << 32 |
+        static_cast<uint64_t>(o->rank()) << 40);
+    for (int d = 0; d < o->rank(); ++d) {
+      add(static_cast<uint64_t>(o->dim(d)));
+      if (o->strided) add(static_cast<uint64_t>(o->vstride_[d]));
+    }
+    for (int j = 0; j < o->nin; ++j) add(o->in[j] != nullptr ? static_cast<uint64_t>(o->in[j]->id) + 1 : 0);
+    if (o->kind == kObjReduce && o->aux_ref != nullptr)
+      for (size_t j = 0; j < o->aux_ref->size; ++j) add(static_cast<uint64_t>(o->aux_ref->data[j]));
+  }
+  return h;
+}
+
 bool Compiler::SplitLongReduces() {
   const int forced = k_->tuning_.red_split;
   if (forced == 0 || forced == 1) return false;
@@ -295,28 +335,8 @@ bool Compiler::SplitLongReduces() {
     } else {
       // workgroups the schedules would give it: one per output when the innermost axis is reduced, else one per
       // 64 lanes of 8 outputs along the innermost axis
-      uint64_t wgs = red[last] ? n_out : (n_out + 511) / 512;
+      const uint64_t wgs = red[last] ? n_out : (n_out + 511) / 512;
       if (wgs >= cus) continue;
-      const NDObject *load = nullptr;
-      if (!red[last] && k_->tuning_.vec_col != 0 && ReducesColumnsOfALoad(r, &load)) {
-        // The column build gives a workgroup one 128-byte line of columns. In one launch: while the whole operand is at most
-        // 40 MB and a workgroup's share half a megabyte, and every reduce beside this one goes the same way. bf16 [4096,4096]
-        // over axis 0: 26 us in two launches, 17 in one; [4096,512] 17 and 10.
-        bool leading = true, seen_kept = false;
-        for (int d = 0; d < xr; ++d) {
-          if (x->dim(d) == 1) continue;
-          if (!red[d]) seen_kept = true;
-          else if (seen_kept) leading = false;
-        }
-        bool alike = leading;
-        for (const NDObject *q : ops) {
-          const NDObject *other = nullptr;
-          if (q == r || q->kind != kObjReduce || q->in[0] == nullptr || q->aux_ref == nullptr || !SameReduce(r, q)) continue;
-          if (!ReducesColumnsOfALoad(q, &other) || other != load) alike = false;
-        }
-        const uint64_t bytes = n_red * n_out * DTypeSize(load->type_id_);
-        if (alike && n_red <= 4096 && bytes <= (40ull << 20)) continue;
-      }
       // worth a second launch only when a workgroup would have a quarter of a million elements to itself (measured:
       // [32, 65536] summed along its rows takes 18 us in one launch and 24-29 us in two)
       const uint64_t outs_per_wg = red[last] ? 1 : std::min<uint64_t>(n_out, 512);
@@ -340,7 +360,33 @@ bool Compiler::SplitLongReduces() {
       for (const NDObject *part : c->parts)
         if (part == r) split = 0;
     }
-    if (ok && split >= 2) cands.push_back({r, split});
+    if (!ok || split < 2) continue;
+    const NDObject *load = nullptr;
+    if (forced < 2 && !red[last] && k_->tuning_.vec_col != 0 && ReducesColumnsOfALoad(r, &load)) {
+      // The column build gives a workgroup one 128-byte line of columns. In one launch: while the whole operand is at most
+      // 40 MB and a workgroup's share half a megabyte, and every reduce beside this one goes the same way. bf16 [4096,4096]
+      // over axis 0: 26 us in two launches, 17 in one; [4096,512] 17 and 10.
+      bool alike = !load->strided || load->vstride_[load->rank() - 1] == 1, seen_kept = false;
+      for (int d = 0; d < xr; ++d) {
+        if (x->dim(d) == 1) continue;
+        if (!red[d]) seen_kept = true;
+        else if (seen_kept) alike = false;
+      }
+      int reduces = 0;
+      for (const NDObject *q : ops) {
+        const NDObject *other = nullptr;
+        if (q->kind != kObjReduce || q->in[0] == nullptr || q->aux_ref == nullptr || !SameReduce(r, q)) continue;
+        if (!ReducesColumnsOfALoad(q, &other) || other != load) alike = false;
+        ++reduces;
+      }
+      const uint64_t bytes = n_red * n_out * DTypeSize(load->type_id_);
+      if (alike && reduces <= DVM_VEC_NSLOT && n_red <= 4096 && bytes <= (40ull << 20) && !WalkedBesideItsReduces(load) &&
+          (unshared_not_.empty() || std::find(unshared_not_.begin(), unshared_not_.end(), GraphKey()) == unshared_not_.end())) {
+        unshared_.push_back(r);
+        continue;
+      }
+    }
+    cands.push_back({r, split});
   }
   // reduces that would share a launch are shared alike or not at all
   for (size_t i = 0; i < cands.size(); ++i) {
