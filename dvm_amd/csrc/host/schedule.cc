@@ -789,13 +789,15 @@ void Compiler::ChooseSchedule() {
     const bool columns = !wide && ColCandidate(&elem_size);
     if (columns) {
       // One 128-byte line of columns per workgroup, half of one where that leaves fewer than 64 workgroups of 16-bit elements,
-      // more while there are four workgroups per compute unit all the same; as many lanes along the rows as there are rows,
+      // more where they would be well above the four per compute unit that are resident; as many lanes along the rows as there are rows,
       // 512 in all. Measured on MI355X, bf16 sums over axis 0, us on the generic kernel / here: [489,824] 100 / 7.0,
       // [282,584] 60 / 6.6, [1473,3848] 30 (two launches) / 11, [4096,4096] 26 (two) / 17; with 16 / 8 / 4 lanes along the
-      // columns [4096,4096] 26 / 17 / 20, [4096,512] 23 / 14 / 10, [4000,600] 26 / 18 / 14.
+      // columns [4096,4096] 26 / 17 / 20, [4096,512] 23 / 14 / 10, [4000,600] 26 / 18 / 14. Lanes along the columns / twice
+      // as many, workgroups in parentheses: fp32 [6000,1000] 27.0 (2000) / 17.2, [5000,1000] 26.7 (2000) / 17.2, bf16
+      // [4096,12000] 34.3 (1500) / 30.7, [5000,9000] 33.8 (1125) / 36.3.
       tx = std::min<uint32_t>(16u / elem_size, Pow2Ceil(n_k_part));
       if (tx == 8 && n_k < 8 * 64) tx = 4;
-      while (tx < 64 && n_k / (2 * tx) >= 4ull * g_system.core_num && 2 * tx <= Pow2Ceil(n_k_part)) tx *= 2;
+      while (tx < 64 && (n_k + tx - 1) / tx > 5ull * g_system.core_num && 2 * tx <= Pow2Ceil(n_k_part)) tx *= 2;
       items = (n_k + tx - 1) / tx;
       ty = 512 / tx;
       while (ty > 1 && ty / 2 >= n_r && tx * ty > 64) ty >>= 1;

@@ -86,6 +86,12 @@ def test_columns_that_are_no_line_of_memory(graph, monkeypatch):
     assert blocks == blocks_before, (entries, before)
 
 
+@pytest.mark.parametrize("shape", [(6000, 1000), (5000, 1000), (9000, 1000), (4096, 12000), (300, 33000)])
+def test_no_more_workgroups_than_the_chip_takes_at_once(shape, monkeypatch):
+    entries, _ = _launches(plain, shape, monkeypatch)
+    assert " columns " in entries[0] and int(re.search(r"items=(\d+)", entries[0]).group(1)) <= 1280, entries
+
+
 def test_a_kernel_of_many_shapes(monkeypatch):
     # the refusal of one shape says nothing about another one of the same kernel
     monkeypatch.delenv("DVM_VEC_COL", raising=False)
