@@ -505,9 +505,10 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const uint32_t bt = DVM_CUBE_TILE_SIDE(c->tile);
     const uint32_t want_threads = comb ? 256u : DVM_CUBE_TILE_LANES(c->tile);
     // (the sum of parts in pieces of 64 x 64; a program exported with the geometry of the tile's own kernel is taken as well)
-    const uint32_t lds_need = comb ? DVM_CUBE_LDS_BYTES(2u) : DVM_CUBE_LDS_BYTES(c->tile);
-    // (programs of the 64 tile and sums of parts are also taken with two stage buffers, as they were exported when that tile had
-    // no more, and run with what the kernel uses)
+    const uint32_t lds_need = comb ? DVM_CUBE_LDS_SUM_BYTES : DVM_CUBE_LDS_BYTES(c->tile);
+    // (programs of the 64 tile are also taken with two stage buffers, as they were exported when that tile had no more, and run
+    // with what the kernel uses; sums of parts carry that much or more and always run with what theirs uses, so that as many
+    // workgroups share a compute unit as their registers allow)
     const uint32_t lds_exported = (comb || c->tile == 2) ? DVM_CUBE_LDS_TWO_STAGES : lds_need;
     const uint32_t lds_groups = c->group_mode != VCG_NONE ? 8u * c->nb1 : 0u;
     // The tile loop trusts the header: check it describes the launch it gets.
@@ -545,7 +546,7 @@ static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads
     const CubeKernel kern = comb ? kCubeCombKernels[c->dtype == VDT_BF16 ? 1 : 0]
                                 : kCubeKernels[c->tile][c->dtype == VDT_BF16 ? 1 : 0][(c->trans_a ? 2 : 0) + (c->trans_b ? 1 : 0)];
     if (check_only) return 0;
-    hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), lds_bytes < lds_need + lds_groups ? lds_need + lds_groups : lds_bytes, s, p);
+    hipLaunchKernelGGL(kern, dim3(block_dim), dim3(want_threads), comb || lds_bytes < lds_need + lds_groups ? lds_need + lds_groups : lds_bytes, s, p);
   } else if (h->entry == VE_ATTN) {
     const VAttnHeader *a = reinterpret_cast<const VAttnHeader *>(p.w);
     // the kernels have no guards of their own beyond the query and key tails: the header must fit them exactly

@@ -554,9 +554,10 @@ void Compiler::CompileCube(int a) {
     reinterpret_cast<VCubeHeader *>(prog_->blob.w)->epi_flags = flags | VCF_SPLITK_COMBINE;
     // Pieces of 64 x 64 whatever the tile; a workgroup takes several where there are more than four per compute unit: what
     // a piece costs beside its bytes is its workgroup's start. (Three run at once, 167 registers a lane: of a full grid
-    // every fourth starts when an earlier one ends.)
+    // every fourth starts when an earlier one ends. With the local memory of the 64 tile's four stage buffers two would:
+    // bf16 [1100,4096] x [4096,2056], 612 pieces, 37.7 us, 35.6 with three.)
     prog_->threads = 256;
-    prog_->lds_bytes = DVM_CUBE_LDS_BYTES(2u);
+    prog_->lds_bytes = DVM_CUBE_LDS_TWO_STAGES;
     prog_->grid = static_cast<uint32_t>(std::min<uint64_t>(tiles(h.tile) * static_cast<uint64_t>(bt / 64) * (bt / 64), 4 * cus));
     prog_->fills.clear();
   }

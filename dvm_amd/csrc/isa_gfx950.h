@@ -395,6 +395,9 @@ enum { VCG_NONE = 0, VCG_M_BOUND = 1, VCG_M_SIZE = 2, VCG_K_BOUND = 3, VCG_K_SIZ
 #define DVM_CUBE_LDS_BYTES(tile) \
   DVM_CUBE_MAX2(DVM_CUBE_LDS_LOOP_BYTES(tile), \
                 DVM_CUBE_MAX2(DVM_CUBE_LDS_DUMP32_BYTES(DVM_CUBE_TILE_SIDE(tile)), DVM_CUBE_LDS_DUMP16_BYTES(DVM_CUBE_TILE_SIDE(tile))))
+// What the launch that sums the parts of a split k axis uses: a 64 x 64 piece as the epilogue reads it back. (Its programs
+// carry DVM_CUBE_LDS_TWO_STAGES, what the 64 tile's kernel had when they were first exported.)
+#define DVM_CUBE_LDS_SUM_BYTES DVM_CUBE_MAX2(DVM_CUBE_LDS_DUMP32_BYTES(64u), DVM_CUBE_LDS_DUMP16_BYTES(64u))
 // (a grouped product keeps its tables behind that: 8 bytes per group)
 
 // ---- fused attention programs (VE_ATTN) -------------------------------------------
