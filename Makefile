@@ -44,7 +44,7 @@ HOST_OBJ := $(patsubst $(CSRC)/host/%.cc,$(OBJ)$(SAN_DIR)/%.cc.o,$(HOST_SRC))
 ifneq ($(asan),)
 all: $(LIB)/asan/libdvm.so
 else
-all: $(LIB)/libdvm_hip.so $(LIB)/libdvm.so $(LIB)/_torch_call.so
+all: $(LIB)/libdvm_hip.so $(LIB)/libdvm.so torch-call
 endif
 
 $(OBJ):
@@ -68,9 +68,11 @@ $(LIB)$(SAN_DIR)/libdvm.so: $(HOST_OBJ)
 	@mkdir -p $(dir $@)
 	$(CXX) -shared -fPIC $(SAN_FLAGS) $(HOST_OBJ) -o $@ -ldl -lpthread
 
-# the extension behind repeated calls on torch tensors (nothing where torch or the interpreter's headers are missing)
-$(LIB)/_torch_call.so: $(CSRC)/torch/torch_call.cc | $(OBJ)
-	python3 -c "import subprocess, sys; from dvm_amd import build; c = build.torch_call_command(); sys.exit(subprocess.call(c[2]) if c else 0)"
+# the extension behind repeated calls on torch tensors (nothing where torch or the interpreter's headers are missing); whether it
+# is out of date depends on both of those too: dvm_amd/build.py knows
+.PHONY: torch-call
+torch-call: | $(OBJ)
+	@python3 -c "import subprocess, sys; from dvm_amd import build; c = build.torch_call_job(); sys.exit(subprocess.call(c) if c else 0)"
 
 # the CPU tests (the device layer is not needed for them) and the random graphs of tests/random_graphs.py, compiled in
 # disassembly mode, against the sanitizer build; any report ends the run with an error

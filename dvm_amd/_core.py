@@ -121,22 +121,37 @@ def _load():
 
 def new_call_plan(rt):
     """A native plan for repeated calls of the runner `rt` on torch tensors (csrc/torch/torch_call.cc), or None where the
-    extension has not been built: calls then bind, generate code and launch from Python every time."""
+    extension has not been built or was built for another torch or interpreter: calls then bind, generate code and launch from
+    Python every time."""
     global _call_plans
     if _call_plans is None:
-        import importlib.machinery
-        import importlib.util
-        path = os.path.join(_LIB_DIR, "_torch_call.so")
-        if not os.path.exists(path):
-            _call_plans = False
-            return None
-        import torch  # noqa: F401  (the extension's symbols come from it)
+        module = _call_module()
+        address = lambda name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value
+        _call_plans = (module.Plan, address("dvm_rt_rebind_run"), address("dvm_rt_plan_stamp"), address("dvm_c_last_error")) if module else False
+    return _call_plans[0](*_call_plans[1:], rt) if _call_plans else None
+
+
+def _call_module():
+    import importlib.machinery
+    import importlib.util
+    import logging
+    import sysconfig
+    import torch  # (the extension's symbols come from it)
+    path = os.path.join(_LIB_DIR, "_torch_call.so")
+    if not os.path.exists(path):
+        return None
+    try:
         loader = importlib.machinery.ExtensionFileLoader("_torch_call", path)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_call", loader))
         loader.exec_module(module)
-        address = lambda name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value
-        _call_plans = (module.Plan, address("dvm_rt_rebind_run"), address("dvm_rt_plan_stamp"), address("dvm_c_last_error"))
-    return _call_plans[0](*_call_plans[1:], rt) if _call_plans else None
+        here = "torch %s, %s" % (torch.__version__, sysconfig.get_config_var("SOABI"))
+        if module.built_for == here:
+            return module
+        why = "it was built for %s, this is %s" % (module.built_for, here)
+    except (ImportError, OSError, SystemError, AttributeError) as e:
+        why = str(e)
+    logging.getLogger("dvm_amd").warning("%s is not used, repeated calls on torch tensors stay in Python: %s (python -m dvm_amd.build)", path, why)
+    return None
 
 
 _call_plans = None

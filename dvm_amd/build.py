@@ -53,19 +53,43 @@ def _run(cmd):
     return err
 
 
-def torch_call_command():
-    """g++ line for the extension that makes repeated calls on torch tensors (csrc/torch/torch_call.cc): source, target, command;
-    None where torch or the interpreter's headers are missing (calls then stay in Python)."""
+def torch_call_tag():
+    """What the extension below is compiled for: torch's version and the interpreter's ABI (dvm_amd/_core.py compares it with what
+    runs). None where torch or the interpreter's headers are missing."""
     import importlib.util
+    import re
     import sysconfig
     spec = importlib.util.find_spec("torch")
-    inc = sysconfig.get_paths()["include"]
-    if spec is None or not os.path.exists(os.path.join(inc, "Python.h")):
+    if spec is None or not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
         return None
-    torch = list(spec.submodule_search_locations)[0]
-    src, out = os.path.join(CSRC, "torch", "torch_call.cc"), os.path.join(LIB, "_torch_call.so")
-    return src, out, ["g++"] + HOST_FLAGS + ["-D_GLIBCXX_USE_CXX11_ABI=1", "-I" + inc, "-isystem", os.path.join(torch, "include"), "-shared", src, "-o", out,
-                                             "-L" + os.path.join(torch, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    with open(os.path.join(list(spec.submodule_search_locations)[0], "version.py")) as f:
+        version = re.search(r"__version__ = '([^']*)'", f.read())
+    return "torch %s, %s" % (version.group(1), sysconfig.get_config_var("SOABI")) if version else None
+
+
+def torch_call_job(force=False):
+    """The g++ line for the extension that makes repeated calls on torch tensors (csrc/torch/torch_call.cc), or None where it is
+    up to date: compiled from this source, for this torch and interpreter, by this file; or where it cannot be compiled (calls
+    then stay in Python)."""
+    import sysconfig
+    tag = torch_call_tag()
+    src, out, record = os.path.join(CSRC, "torch", "torch_call.cc"), os.path.join(LIB, "_torch_call.so"), os.path.join(OBJ, "_torch_call.tag")
+    if tag is None:
+        return None
+    if not force and not _stale(out, [src, os.path.abspath(__file__)]) and os.path.exists(record):
+        with open(record) as f:
+            if f.read() == tag:
+                return None
+    import torch
+    where = os.path.dirname(torch.__file__)
+    os.makedirs(OBJ, exist_ok=True)
+    with open(record, "w") as f:  # (a compilation that fails leaves no library behind, and the next build tries again)
+        f.write(tag)
+    if os.path.exists(out):
+        os.remove(out)
+    return ["g++"] + HOST_FLAGS + ["-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), '-DDVM_TORCH_CALL_TAG="%s"' % tag,
+                                   "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(where, "include"), "-shared", src, "-o", out,
+                                   "-L" + os.path.join(where, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
 
 
 def build(force=False, verbose=False):
@@ -89,9 +113,9 @@ def build(force=False, verbose=False):
         host_objs.append(obj)
         if force or _stale(obj, [src] + deps):
             jobs.append(["g++"] + HOST_FLAGS + ["-c", src, "-o", obj])
-    call = torch_call_command()
-    if call is not None and (force or _stale(call[1], [call[0]])):
-        jobs.append(call[2])
+    call = torch_call_job(force)
+    if call is not None:
+        jobs.append(call)
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for msg in ex.map(_run, jobs):
             if verbose and msg:

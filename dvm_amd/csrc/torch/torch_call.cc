@@ -266,6 +266,10 @@ PyMODINIT_FUNC __attribute__((visibility("default"))) PyInit__torch_call(void) {
   if (PyType_Ready(&plan_type) < 0) return nullptr;
   PyObject *m = PyModule_Create(&module_def);
   if (m == nullptr) return nullptr;
+  if (PyModule_AddStringConstant(m, "built_for", DVM_TORCH_CALL_TAG) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
   Py_INCREF(&plan_type);
   if (PyModule_AddObject(m, "Plan", reinterpret_cast<PyObject *>(&plan_type)) < 0) {
     Py_DECREF(&plan_type);
