@@ -18,6 +18,7 @@
 using namespace dvm;
 
 struct dvm_shape {
+  uint64_t *changes = nullptr;  // of the runner it belongs to (dvm_rt::changes)
   std::vector<int64_t> dims;
   IntArrayRef ref;
   void Set(const int64_t *d, size_t n) {
@@ -29,12 +30,17 @@ struct dvm_shape {
 };
 
 struct dvm_scalar {
+  uint64_t *changes = nullptr;
   ScalarRef ref;
 };
 
 namespace {
 
 thread_local std::string g_last_error;
+
+// counts changes that no runner hears of: the tuner's switches, which decide what a code generation of an unchanged kernel
+// gives, and the offset of a view
+std::atomic<uint64_t> g_changes{0};
 
 struct Buffer {
   void *ptr = nullptr;
@@ -65,7 +71,11 @@ struct dvm_rt {
   void *ws_user = nullptr;
   std::map<NDObject *, std::unique_ptr<dvm_shape>> view_strides;  // loads bound through strides (dvm_rt_bind_device_view)
   uint64_t fake_addr = 0x1000;
-  uint64_t changes = 0;  // counts what may change the compiled programs or the walk of a load (dvm_rt_plan_stamp)
+  // dvm_rt_plan_stamp: counts everything that may change what the next code generation of the kernel, or a launch of it with
+  // the loads and stores of one plan bound anew, gives
+  uint64_t changes = 0;
+  size_t ops_seen = 0;      // what `changes` does not hear of: operators added, what concerns all runners
+  uint64_t global_seen = 0;
   double jit_us = 0.0;
   WsAlloc ws_alloc;
 
@@ -277,6 +287,7 @@ dvm_shape *dvm_rt_new_shape(dvm_rt *rt, const int64_t *dims, size_t n) {
   return Guard(
       [&]() {
         rt->shapes.emplace_back(new dvm_shape());
+        rt->shapes.back()->changes = &rt->changes;
         rt->shapes.back()->dims.reserve(kMaxRank);
         rt->shapes.back()->Set(dims, n);
         return rt->shapes.back().get();
@@ -285,6 +296,7 @@ dvm_shape *dvm_rt_new_shape(dvm_rt *rt, const int64_t *dims, size_t n) {
 }
 
 int dvm_shape_update(dvm_shape *s, const int64_t *dims, size_t n) {
+  ++*s->changes;
   s->Set(dims, n);
   return 0;
 }
@@ -294,6 +306,7 @@ dvm_scalar *dvm_rt_new_scalar(dvm_rt *rt, int dtype) {
       [&]() {
         rt->scalars.emplace_back(new dvm_scalar());
         dvm_scalar *s = rt->scalars.back().get();
+        s->changes = &rt->changes;
         if (dtype == kInt32) {
           s->ref = 0;
         } else if (dtype == kInt64) {
@@ -307,6 +320,7 @@ dvm_scalar *dvm_rt_new_scalar(dvm_rt *rt, int dtype) {
 }
 
 int dvm_scalar_update_f(dvm_scalar *s, double v) {
+  ++*s->changes;
   if (s->ref.type == kInt32) {
     s->ref = static_cast<int32_t>(v);
   } else if (s->ref.type == kInt64) {
@@ -318,6 +332,7 @@ int dvm_scalar_update_f(dvm_scalar *s, double v) {
 }
 
 int dvm_scalar_update_i(dvm_scalar *s, int64_t v) {
+  ++*s->changes;
   if (s->ref.type == kInt32) {
     s->ref = static_cast<int32_t>(v);
   } else if (s->ref.type == kInt64) {
@@ -475,6 +490,7 @@ int dvm_rt_clone(dvm_rt *rt, dvm_rt *base, const int *kinds, void *const *items,
           std::map<ScalarRef *, ScalarRef *> scalars;
           std::map<NDObject *, NDObject *> ops;
         } helper;
+        ++rt->changes;
         rt->FreeAll();
         rt->loads.clear();
         rt->stores.clear();
@@ -482,6 +498,7 @@ int dvm_rt_clone(dvm_rt *rt, dvm_rt *base, const int *kinds, void *const *items,
         std::map<const dvm_scalar *, dvm_scalar *> scalar_of;
         for (const auto &sh : base->shapes) {
           rt->shapes.emplace_back(new dvm_shape());
+          rt->shapes.back()->changes = &rt->changes;
           rt->shapes.back()->dims.reserve(kMaxRank);
           rt->shapes.back()->Set(sh->dims.data(), sh->dims.size());
           helper.shapes[&sh->ref] = &rt->shapes.back()->ref;
@@ -489,6 +506,7 @@ int dvm_rt_clone(dvm_rt *rt, dvm_rt *base, const int *kinds, void *const *items,
         }
         for (const auto &sc : base->scalars) {
           rt->scalars.emplace_back(new dvm_scalar());
+          rt->scalars.back()->changes = &rt->changes;
           rt->scalars.back()->ref = sc->ref;
           helper.scalars[&sc->ref] = &rt->scalars.back()->ref;
           scalar_of[sc.get()] = rt->scalars.back().get();
@@ -514,6 +532,7 @@ int dvm_rt_clone(dvm_rt *rt, dvm_rt *base, const int *kinds, void *const *items,
 int dvm_rt_seq_add(dvm_rt *rt, int ktype, unsigned flags) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.SequenceAdd(static_cast<KernelType>(ktype), flags);
         return 0;
       },
@@ -523,6 +542,7 @@ int dvm_rt_seq_add(dvm_rt *rt, int ktype, unsigned flags) {
 int dvm_rt_parallel_add(dvm_rt *rt, int ktype, unsigned flags, size_t core_limit) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.ParallelAdd(static_cast<KernelType>(ktype), flags, core_limit);
         return 0;
       },
@@ -644,6 +664,7 @@ int dvm_rt_split(dvm_rt *rt, dvm_obj *x, int dim, long long chunk, size_t num, d
 }
 
 int dvm_obj_set_view_offset(dvm_obj *io, long long elems) {
+  if (Obj(io)->view_offset != elems) g_changes.fetch_add(1, std::memory_order_relaxed);
   Obj(io)->view_offset = elems;
   return 0;
 }
@@ -651,6 +672,7 @@ int dvm_obj_set_view_offset(dvm_obj *io, long long elems) {
 int dvm_rt_set_store_inplace(dvm_rt *rt, dvm_obj *store) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.SetStoreInplace(Obj(store));
         return 0;
       },
@@ -660,6 +682,7 @@ int dvm_rt_set_store_inplace(dvm_rt *rt, dvm_obj *store) {
 int dvm_rt_set_store_temp(dvm_rt *rt, dvm_obj *store) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.SetStoreTemp(Obj(store));
         return 0;
       },
@@ -669,6 +692,7 @@ int dvm_rt_set_store_temp(dvm_rt *rt, dvm_obj *store) {
 int dvm_rt_set_load_bind(dvm_rt *rt, dvm_obj *load, dvm_obj *store) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.SetLoadBind(Obj(load), Obj(store));
         return 0;
       },
@@ -678,6 +702,7 @@ int dvm_rt_set_load_bind(dvm_rt *rt, dvm_obj *load, dvm_obj *store) {
 int dvm_rt_spec_next(dvm_rt *rt) {
   return Guard(
       [&]() {
+        ++rt->changes;
         rt->kernel.SpecNext();
         return 0;
       },
@@ -698,6 +723,7 @@ int dvm_obj_dtype(const dvm_obj *o) { return reinterpret_cast<const NDObject *>(
 int dvm_rt_input(dvm_rt *rt, dvm_obj *load, const void *host, size_t bytes) {
   return Guard(
       [&]() {
+        ++rt->changes;
         NDObject *o = Obj(load);
         // memory the caller bound earlier (dvm_rt_bind_device) is the caller's: host data never goes there
         auto bound = rt->buffers.find(o);
@@ -715,6 +741,7 @@ int dvm_rt_input(dvm_rt *rt, dvm_obj *load, const void *host, size_t bytes) {
 int dvm_rt_bind_device(dvm_rt *rt, dvm_obj *io, void *device_ptr) {
   return Guard(
       [&]() {
+        ++rt->changes;
         Buffer &b = rt->buffers[Obj(io)];
         rt->Release(b);
         b.ptr = device_ptr;
@@ -728,17 +755,16 @@ int dvm_rt_bind_device(dvm_rt *rt, dvm_obj *io, void *device_ptr) {
 int dvm_rt_bind_device_view(dvm_rt *rt, dvm_obj *load, void *device_ptr, const int64_t *strides, size_t rank) {
   return Guard(
       [&]() {
+        ++rt->changes;
         NDObject *o = Obj(load);
         if (o->kind != kObjLoad || o->full_shape_ref != nullptr) throw std::runtime_error("DVM EXCEPTION. reason: only a plain load takes a strided binding");
         if (strides == nullptr) {
           if (rt->view_strides.erase(o) != 0) {
-            ++rt->changes;
             o->strided = false;
             o->stride_ref = nullptr;
           }
         } else {
           if (rank != static_cast<size_t>(o->shape_ref_->size)) throw std::runtime_error("DVM EXCEPTION. reason: one stride per dim of the load");
-          ++rt->changes;
           std::unique_ptr<dvm_shape> &st = rt->view_strides[o];
           if (!st) st.reset(new dvm_shape());
           st->Set(strides, rank);
@@ -867,12 +893,13 @@ int dvm_rt_run(dvm_rt *rt, void *stream, int flags) {
       -1);
 }
 
-namespace {
-std::atomic<uint64_t> g_tuner_changes{0};  // the tuner's switches decide what a code generation of an unchanged kernel gives
-}
-
 uint64_t dvm_rt_plan_stamp(dvm_rt *rt) {
-  return (rt->changes << 24) + (static_cast<uint64_t>(rt->kernel.GetImpl()->ops_.size()) << 8) + (g_tuner_changes.load(std::memory_order_relaxed) & 0xffu);
+  const size_t ops = rt->kernel.GetImpl()->ops_.size();
+  const uint64_t global = g_changes.load(std::memory_order_relaxed);
+  if (ops != rt->ops_seen || global != rt->global_seen) ++rt->changes;
+  rt->ops_seen = ops;
+  rt->global_seen = global;
+  return rt->changes;
 }
 
 int dvm_rt_rebind_run(dvm_rt *rt, uint64_t stamp, dvm_obj *const *ios, void *const *ptrs, size_t n, void *workspace, void *stream) {
@@ -971,20 +998,20 @@ int dvm_rt_perf(dvm_rt *rt, int warmup, int iters, double out[3]) {
 }
 
 void dvm_set_online_tuner(int enable) {
-  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
+  g_changes.fetch_add(1, std::memory_order_relaxed);
   g_system.Init();
   if (enable) g_system.SetOnlineTuner();
   else g_system.UnsetOnlineTuner();
 }
 void dvm_set_lazy_tuner(int enable) {
-  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
+  g_changes.fetch_add(1, std::memory_order_relaxed);
   g_system.Init();
   if (enable) g_system.SetLazyTuner();
   else g_system.UnsetLazyTuner();
 }
 void dvm_tuner_stats(uint64_t *shapes_measured, uint64_t *table_size) { CubeTunerStats(shapes_measured, table_size); }
 void dvm_tuner_clear(void) {
-  g_tuner_changes.fetch_add(1, std::memory_order_relaxed);
+  g_changes.fetch_add(1, std::memory_order_relaxed);
   CubeTunerClear();
 }
 

@@ -149,10 +149,11 @@ double dvm_rt_jit_us(const dvm_rt *rt);
 #define DVM_RUN_WAIT 1
 #define DVM_RUN_ON_GIVEN_STREAM 2
 int dvm_rt_run(dvm_rt *rt, void *stream, int flags);
-/* What was compiled, once more on other memory: `ios[n]` are all loads and stores of the kernel, `ptrs[n]` where they lie
- * now, `workspace` dvm_rt_workspace_bytes of device memory (or NULL when that is 0); the launches go to `stream`. Shapes,
- * strides and scalars are those of the last dvm_rt_codegen. `stamp` is what dvm_rt_plan_stamp said after it: 1 is returned,
- * and nothing done, when anything that decides the programs has changed since. */
+/* What was compiled, once more on other memory: `ios[n]` (at most 64) are loads and stores of the kernel, `ptrs[n]` where they
+ * lie now (the others stay where they were bound), `workspace` dvm_rt_workspace_bytes of device memory (or NULL when that is 0);
+ * the launches go to `stream`. Shapes, strides and scalars are those of the last dvm_rt_codegen. `stamp` is what
+ * dvm_rt_plan_stamp said after it: 1 is returned, and nothing done, when anything has changed since that decides the programs
+ * or where a load or store lies, whether or not the next code generation would give others. */
 uint64_t dvm_rt_plan_stamp(dvm_rt *rt);
 int dvm_rt_rebind_run(dvm_rt *rt, uint64_t stamp, dvm_obj *const *ios, void *const *ptrs, size_t n, void *workspace, void *stream);
 int dvm_rt_output(dvm_rt *rt, dvm_obj *store, void *host, size_t bytes);

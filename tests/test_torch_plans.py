@@ -116,6 +116,56 @@ for src, _ in pairs:
 print("plans: ok")
 '''
 
+_CHANGES = r'''
+import torch
+import dvm_amd as dvm
+from dvm_amd import _core
+
+gen = torch.Generator(device="cuda").manual_seed(6)
+def rnd(*shape):
+    return torch.randn(shape, device="cuda", generator=gen)
+
+# a store that is no result, bound by the caller, and a number that is no argument
+held = {}
+@dvm.kernel(ktype="split", dynamic=True)
+def scaled(k, x):
+    held["factor"] = _core.Kernel.scalar(k)
+    held["factor"].update(2.0)
+    y = k.mul(k.load(x, dvm.float32), held["factor"])
+    held["side"] = k.store(k.add(y, 1.0))
+    return k.store(y)
+
+sides = [torch.zeros(40, 16, device="cuda") for _ in range(3)]
+expect = [torch.zeros(40, 16) for _ in range(3)]
+for turn, (side, factor) in enumerate([(0, 2.0), (0, 2.0), (0, 2.0), (0, 2.0), (1, 2.0), (1, 2.0), (1, 2.0), (1, 5.0), (1, 5.0), (1, 5.0), (2, 3.0), (0, 3.0)]):
+    scaled.bind_device(held["side"], sides[side].data_ptr())
+    held["factor"].update(factor)
+    x = rnd(40, 16)
+    got = scaled(x)
+    expect[side] = (x * factor + 1.0).cpu()
+    assert torch.equal(got, x * factor), turn
+    for s, e in zip(sides, expect):
+        assert torch.allclose(s.cpu(), e, rtol=1e-6, atol=1e-6), turn
+# the same without touching anything in between: the plan makes the calls
+for turn in range(4):
+    x = rnd(40, 16)
+    assert torch.equal(scaled(x), x * 3.0)
+    assert torch.allclose(sides[0], x * 3.0 + 1.0, rtol=1e-6, atol=1e-6)
+assert bool(scaled._plan)
+print("changes: ok")
+'''
+
+
+def _run(script, said):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""))
+    r = subprocess.run([sys.executable, "-c", script], cwd=root, env=env, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and said in r.stdout, r.stdout + r.stderr
+
+
+def test_what_changes_the_kernel_between_two_calls():
+    _run(_CHANGES, "changes: ok")
+
 
 def test_plans():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
