@@ -15,7 +15,7 @@
 
 #include <cstdint>
 #include <cstring>
-#include <string>
+#include <memory>
 #include <vector>
 
 namespace {
@@ -37,19 +37,24 @@ struct ArgSpec {
   int64_t i = 0;
 };
 
+struct Recorded {  // what a call is compared with and made from; never changed once it stands
+  std::vector<ArgSpec> args;
+  std::vector<TensorSpec> outs;
+  std::vector<void *> ios;  // the loads behind the tensor arguments, then the stores
+  bool many = false;
+  uint64_t stamp = 0;
+  int64_t ws_bytes = 0;
+  c10::DeviceIndex device = -1;
+};
+
 struct Plan {
   PyObject_HEAD
   RebindRunFn rebind_run;
   StampFn stamp_of;
   LastErrorFn last_error;
   void *rt;
-  std::vector<void *> *ios;  // the loads behind the tensor arguments, then the stores
-  std::vector<ArgSpec> *args;
-  std::vector<TensorSpec> *outs;
-  bool valid, many;
-  uint64_t stamp;
-  int64_t ws_bytes;
-  c10::DeviceIndex device;
+  std::shared_ptr<const Recorded> *now;  // (empty: nothing recorded, or stale)
+  std::vector<ArgSpec> *seen;            // arguments of the last call made from Python (empty: none that can be recorded)
 };
 
 bool IsPlainTensor(PyObject *o) { return THPVariable_CheckExact(o); }
@@ -87,74 +92,121 @@ PyObject *PlanNew(PyTypeObject *type, PyObject *args, PyObject *) {
   p->stamp_of = reinterpret_cast<StampFn>(stamp_of);
   p->last_error = reinterpret_cast<LastErrorFn>(last_error);
   p->rt = reinterpret_cast<void *>(rt);
-  p->ios = new std::vector<void *>();
-  p->args = new std::vector<ArgSpec>();
-  p->outs = new std::vector<TensorSpec>();
-  p->valid = false;
+  p->now = new std::shared_ptr<const Recorded>();
+  p->seen = new std::vector<ArgSpec>();
   return reinterpret_cast<PyObject *>(p);
 }
 
 void PlanDealloc(PyObject *self) {
   Plan *p = reinterpret_cast<Plan *>(self);
-  delete p->ios;
-  delete p->args;
-  delete p->outs;
+  delete p->now;
+  delete p->seen;
   Py_TYPE(self)->tp_free(self);
 }
 
-// record(args, load handles, outputs, store handles, many, workspace bytes): what the call that has just been made was.
-// False when calls like it cannot go this way.
+// Whether the arguments of a call are those of `specs`; ptrs: where the tensors among them lie.
+bool Matches(const std::vector<ArgSpec> &specs, c10::DeviceIndex device, PyObject *args, void **ptrs) {
+  const size_t n = specs.size();
+  if (static_cast<size_t>(PyTuple_GET_SIZE(args)) != n) return false;
+  for (size_t i = 0; i < n; ++i) {
+    PyObject *o = PyTuple_GET_ITEM(args, static_cast<Py_ssize_t>(i));
+    const ArgSpec &a = specs[i];
+    if (!a.tensor) {
+      ArgSpec now;
+      if (!ReadNumber(o, &now) || !SameNumber(a, now)) return false;
+      continue;
+    }
+    if (!IsPlainTensor(o)) return false;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    if (!Readable(t, device) || t.scalar_type() != a.spec.type || t.sizes() != at::IntArrayRef(a.spec.sizes) ||
+        t.strides() != at::IntArrayRef(a.spec.strides)) return false;
+    if (ptrs != nullptr) *ptrs++ = t.data_ptr();
+  }
+  return true;
+}
+
+c10::DeviceIndex DeviceOf(PyObject *args) {
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args); ++i) {
+    PyObject *o = PyTuple_GET_ITEM(args, i);
+    if (!IsPlainTensor(o)) continue;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    return t.is_cuda() ? t.device().index() : static_cast<c10::DeviceIndex>(-1);
+  }
+  return -1;
+}
+
+// repeats(args): whether the call from Python that has just been made was like the one before it. Only then is a plan worth its
+// recording: where a number or a shape is another one at every call, what is added to the call is this comparison.
+PyObject *PlanRepeats(PyObject *self, PyObject *args) {
+  HANDLE_TH_ERRORS
+  Plan *p = reinterpret_cast<Plan *>(self);
+  if (!PyTuple_Check(args)) {
+    PyErr_SetString(PyExc_TypeError, "repeats(args)");
+    return nullptr;
+  }
+  const c10::DeviceIndex device = DeviceOf(args);
+  if (!p->seen->empty() && device >= 0 && Matches(*p->seen, device, args, nullptr)) Py_RETURN_TRUE;
+  std::vector<ArgSpec> &seen = *p->seen;
+  const size_t n = static_cast<size_t>(PyTuple_GET_SIZE(args));
+  seen.resize(device >= 0 ? n : 0);
+  for (size_t i = 0; i < seen.size(); ++i) {
+    PyObject *o = PyTuple_GET_ITEM(args, static_cast<Py_ssize_t>(i));
+    ArgSpec &a = seen[i];
+    a.tensor = IsPlainTensor(o);
+    if (a.tensor) {
+      const at::Tensor &t = THPVariable_Unpack(o);
+      if (Readable(t, device)) {
+        a.spec.type = t.scalar_type();
+        a.spec.sizes.assign(t.sizes().begin(), t.sizes().end());
+        a.spec.strides.assign(t.strides().begin(), t.strides().end());
+        continue;
+      }
+    } else {
+      a.is_float = false;
+      if (ReadNumber(o, &a)) continue;
+    }
+    seen.clear();
+    break;
+  }
+  Py_RETURN_FALSE;
+  END_HANDLE_TH_ERRORS
+}
+
+// record(load handles, outputs, store handles, many, workspace bytes): the call that `repeats` has just been asked about becomes
+// the plan. False when calls like it cannot go this way.
 PyObject *PlanRecord(PyObject *self, PyObject *pyargs) {
   HANDLE_TH_ERRORS
   Plan *p = reinterpret_cast<Plan *>(self);
-  PyObject *args, *loads, *outs, *stores;
+  PyObject *loads, *outs, *stores;
   int many = 0;
   long long ws_bytes = 0;
-  if (!PyArg_ParseTuple(pyargs, "O!O!O!O!pL", &PyTuple_Type, &args, &PyList_Type, &loads, &PyList_Type, &outs, &PyList_Type, &stores, &many, &ws_bytes)) return nullptr;
-  p->valid = false;
-  p->ios->clear();
-  p->args->clear();
-  p->outs->clear();
-  c10::DeviceIndex device = -1;
-  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args); ++i) {
-    PyObject *o = PyTuple_GET_ITEM(args, i);
-    ArgSpec a;
-    if (IsPlainTensor(o)) {
-      const at::Tensor &t = THPVariable_Unpack(o);
-      if (!t.is_cuda()) Py_RETURN_FALSE;
-      if (device < 0) device = t.device().index();
-      if (!Readable(t, device)) Py_RETURN_FALSE;
-      a.tensor = true;
-      a.spec.type = t.scalar_type();
-      a.spec.sizes = t.sizes().vec();
-      a.spec.strides = t.strides().vec();
-    } else if (!ReadNumber(o, &a)) {
-      Py_RETURN_FALSE;
-    }
-    p->args->push_back(std::move(a));
-  }
+  if (!PyArg_ParseTuple(pyargs, "O!O!O!pL", &PyList_Type, &loads, &PyList_Type, &outs, &PyList_Type, &stores, &many, &ws_bytes)) return nullptr;
+  p->now->reset();
+  auto r = std::make_shared<Recorded>();
+  r->args = *p->seen;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(outs); ++i) {
     PyObject *o = PyList_GET_ITEM(outs, i);
     if (!IsPlainTensor(o)) Py_RETURN_FALSE;
     const at::Tensor &t = THPVariable_Unpack(o);
-    if (!Readable(t, device) || !t.is_contiguous()) Py_RETURN_FALSE;
-    p->outs->push_back({t.scalar_type(), t.sizes().vec(), {}});
+    if (!t.is_cuda()) Py_RETURN_FALSE;
+    if (r->device < 0) r->device = t.device().index();
+    if (!Readable(t, r->device) || !t.is_contiguous()) Py_RETURN_FALSE;
+    r->outs.push_back({t.scalar_type(), t.sizes().vec(), {}});
   }
   for (PyObject *list : {loads, stores}) {
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
       void *h = PyLong_AsVoidPtr(PyList_GET_ITEM(list, i));
       if (h == nullptr) return PyErr_Occurred() ? nullptr : (Py_INCREF(Py_False), Py_False);
-      p->ios->push_back(h);
+      r->ios.push_back(h);
     }
   }
-  size_t tensors = p->outs->size();
-  for (const ArgSpec &a : *p->args) tensors += a.tensor;
-  if (tensors != p->ios->size() || device < 0) Py_RETURN_FALSE;
-  p->device = device;
-  p->many = many != 0;
-  p->ws_bytes = ws_bytes;
-  p->stamp = p->stamp_of(p->rt);
-  p->valid = true;
+  size_t tensors = r->outs.size();
+  for (const ArgSpec &a : r->args) tensors += a.tensor;
+  if (tensors != r->ios.size() || tensors > 64 || r->device < 0) Py_RETURN_FALSE;
+  r->many = many != 0;
+  r->ws_bytes = ws_bytes;
+  r->stamp = p->stamp_of(p->rt);
+  *p->now = r;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -169,44 +221,14 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
     return nullptr;
   }
   PyObject *kernel = argv[0], *args = argv[1];
-  const size_t n = p->args->size();
-  if (!p->valid || static_cast<size_t>(PyTuple_GET_SIZE(args)) != n) Py_RETURN_NONE;
+  const std::shared_ptr<const Recorded> r = *p->now;  // (a callback of the allocation may lead to another plan)
   void *ptrs[64];
-  size_t np = 0;
-  if (p->ios->size() > 64) Py_RETURN_NONE;
-  for (size_t i = 0; i < n; ++i) {
-    PyObject *o = PyTuple_GET_ITEM(args, static_cast<Py_ssize_t>(i));
-    const ArgSpec &a = (*p->args)[i];
-    if (!a.tensor) {
-      ArgSpec now;
-      if (!ReadNumber(o, &now) || !SameNumber(a, now)) Py_RETURN_NONE;
-      continue;
-    }
-    if (!IsPlainTensor(o)) Py_RETURN_NONE;
-    const at::Tensor &t = THPVariable_Unpack(o);
-    if (!Readable(t, p->device) || t.scalar_type() != a.spec.type || t.sizes() != at::IntArrayRef(a.spec.sizes) ||
-        t.strides() != at::IntArrayRef(a.spec.strides)) Py_RETURN_NONE;
-    ptrs[np++] = t.data_ptr();
-  }
-  if (p->stamp_of(p->rt) != p->stamp) {
-    p->valid = false;
+  if (!r || !Matches(r->args, r->device, args, ptrs)) Py_RETURN_NONE;
+  if (p->stamp_of(p->rt) != r->stamp) {
+    p->now->reset();
     Py_RETURN_NONE;
   }
-  const c10::Device device(c10::kCUDA, p->device);
-  std::vector<at::Tensor> made;
-  made.reserve(p->outs->size() + 1);
-  for (const TensorSpec &s : *p->outs) {
-    made.push_back(at::empty(s.sizes, at::TensorOptions().dtype(s.type).device(device)));
-    if (!made.back().has_storage()) Py_RETURN_NONE;  // (a mode that makes something else of an allocation)
-    ptrs[np++] = made.back().data_ptr();
-  }
-  void *workspace = nullptr;
-  if (p->ws_bytes > 0) {
-    made.push_back(at::empty({p->ws_bytes}, at::TensorOptions().dtype(at::kByte).device(device)));
-    if (!made.back().has_storage()) Py_RETURN_NONE;
-    workspace = made.back().data_ptr();
-  }
-  PyObject *index = PyLong_FromLong(p->device);
+  PyObject *index = PyLong_FromLong(r->device);
   if (index == nullptr) return nullptr;
   PyObject *stream = PyObject_CallOneArg(argv[2], index);
   Py_DECREF(index);
@@ -214,21 +236,40 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
   void *raw = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (raw == nullptr && PyErr_Occurred()) return nullptr;
-  const int rc = p->rebind_run(p->rt, p->stamp, p->ios->data(), ptrs, np, workspace, raw);
+  std::vector<at::Tensor> made;
+  made.reserve(r->outs.size() + 1);
+  int rc = 1;
+  {
+    const c10::Device device(c10::kCUDA, r->device);
+    size_t np = r->ios.size() - r->outs.size();
+    void *workspace = nullptr;
+    bool memory = true;  // (false: a mode makes something else of an allocation)
+    for (const TensorSpec &s : r->outs) {
+      made.push_back(at::empty(s.sizes, at::TensorOptions().dtype(s.type).device(device)));
+      memory = memory && made.back().has_storage();
+      if (memory) ptrs[np++] = made.back().data_ptr();
+    }
+    if (memory && r->ws_bytes > 0) {
+      made.push_back(at::empty({r->ws_bytes}, at::TensorOptions().dtype(at::kByte).device(device)));
+      memory = made.back().has_storage();
+      if (memory) workspace = made.back().data_ptr();
+    }
+    if (memory) rc = p->rebind_run(p->rt, r->stamp, r->ios.data(), ptrs, np, workspace, raw);
+  }
   if (rc != 0) {
-    p->valid = false;
+    p->now->reset();
     if (rc > 0) Py_RETURN_NONE;
     PyErr_SetString(PyExc_RuntimeError, p->last_error());
     return nullptr;
   }
-  const Py_ssize_t n_out = static_cast<Py_ssize_t>(p->outs->size()), n_made = static_cast<Py_ssize_t>(made.size());
+  const Py_ssize_t n_out = static_cast<Py_ssize_t>(r->outs.size()), n_made = static_cast<Py_ssize_t>(made.size());
   PyObject *alive = PyList_New(static_cast<Py_ssize_t>(1) + n_made);
   if (alive == nullptr) return nullptr;
   Py_INCREF(args);
   PyList_SET_ITEM(alive, 0, args);
   for (Py_ssize_t i = 0; i < n_made; ++i) PyList_SET_ITEM(alive, 1 + i, THPVariable_Wrap(made[static_cast<size_t>(i)]));
   PyObject *result;
-  if (p->many) {
+  if (r->many) {
     result = PyList_New(n_out);
     for (Py_ssize_t i = 0; result != nullptr && i < n_out; ++i) {
       PyObject *o = PyList_GET_ITEM(alive, 1 + i);
@@ -247,6 +288,7 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
 }
 
 PyMethodDef plan_methods[] = {
+    {"repeats", PlanRepeats, METH_O, nullptr},
     {"record", PlanRecord, METH_VARARGS, nullptr},
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(PlanCall)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

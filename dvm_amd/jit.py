@@ -41,7 +41,6 @@ class JitKernel(PyKernel):
         self._store_types = None  # torch types of the stores, from the first call on torch tensors
         self._results = None  # what the traced function returned: a store or a sequence of stores
         self._plan = None     # the last call on torch tensors, to be made again natively (False: never)
-        self._last_shapes = None
 
     # ---- tracing ----
     def build(self, func):
@@ -188,23 +187,20 @@ class _DeviceCall:
             self._plan_next(outs, many)
         return outs if many else outs[0]
 
-
     def _plan_next(self, outs, many):
-        """Records this call, the second with these shapes, as the plan of the next one."""
+        """Records this call, when it was like the one before it, as the plan of the next one."""
         global _raw_stream_of
         k = self.kern
-        shapes = [a.shape for a, s in zip(self.args, k._slots) if s.role == "tensor"]
-        if shapes != k._last_shapes:
-            k._last_shapes = shapes
-            return
         if k._plan is None:
             k._plan = new_call_plan(k._rt) if all(s.role in ("tensor", "scalar") for s in k._slots) else None
             if k._plan is None:
                 k._plan = False
                 return
             _raw_stream_of = self.torch._C._cuda_getCurrentRawStream
-        k._plan.record(tuple(self.args), [s.handle._h for s in k._slots if s.role == "tensor"], outs, [st._h for st in k._stores()[0]], many,
-                       k.workspace_bytes())
+        if not k._plan.repeats(tuple(self.args)):
+            return
+        if not k._plan.record([s.handle._h for s in k._slots if s.role == "tensor"], outs, [st._h for st in k._stores()[0]], many, k.workspace_bytes()):
+            k._plan = False
 
 
 def _on_gpu(value):

@@ -155,6 +155,59 @@ assert bool(scaled._plan)
 print("changes: ok")
 '''
 
+_NUMBERS = r'''
+import numpy as np
+import torch
+import dvm_amd as dvm
+
+@dvm.kernel(ktype="split", dynamic=True)
+def step(k, p, g, lr):
+    return k.store(k.sub(k.load(p, dvm.float32), k.mul(k.load(g, dvm.float32), k.scalar(lr))))
+
+class Counting:  # the plan, and how often it is recorded and makes a call
+    def __init__(self, plan):
+        self.plan, self.recorded, self.called = plan, 0, 0
+    def repeats(self, args):
+        return self.plan.repeats(args)
+    def record(self, *args):
+        self.recorded += 1
+        return self.plan.record(*args)
+    def call(self, *args):
+        r = self.plan.call(*args)
+        self.called += r is not None
+        return r
+
+p, g = torch.randn(100, 8, device="cuda"), torch.randn(100, 8, device="cuda")
+def go(lr):
+    assert torch.allclose(step(p, g, lr), p - g * float(lr), rtol=1e-6, atol=1e-6)
+go(0.5)
+step._plan = Counting(step._plan)
+# another number at every call, a number of another type, NaN among them: nothing is recorded
+for i in range(20):
+    go(1.0 / (1 + i))
+for lr in (np.float32(0.25), np.float32(0.25), np.float64(0.25), True, True, 1, True, 0.25):
+    go(lr)
+assert step._plan.recorded == 0 and step._plan.called == 0
+# a number that stays: recorded at its second call, made from the plan from the third on
+for i in range(5):
+    go(0.125)
+assert step._plan.recorded == 1 and step._plan.called == 3
+# and when it changes once more
+go(0.25); go(0.25); go(0.25)
+assert step._plan.recorded == 2 and step._plan.called == 4
+# two shapes in turn: nothing is recorded, nothing is mixed up
+q, h = torch.randn(7, 8, device="cuda"), torch.randn(7, 8, device="cuda")
+for i in range(6):
+    a, b = ((p, g), (q, h))[i % 2]
+    assert torch.allclose(step(a, b, 0.25), a - b * 0.25, rtol=1e-6, atol=1e-6)
+assert step._plan.recorded <= 3
+print("numbers: ok")
+'''
+
+
+def test_numbers_that_change_are_not_recorded():
+    _run(_NUMBERS, "numbers: ok")
+
 
 def _run(script, said):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
