@@ -12,10 +12,12 @@
 #include <ATen/ATen.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <pybind11/gil.h>
 
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 namespace {
@@ -55,6 +57,7 @@ struct Plan {
   void *rt;
   std::shared_ptr<const Recorded> *now;  // (empty: nothing recorded, or stale)
   std::vector<ArgSpec> *seen;            // arguments of the last call made from Python (empty: none that can be recorded)
+  std::mutex *launch;                    // one thread at a time writes addresses into the programs and launches them
 };
 
 bool IsPlainTensor(PyObject *o) { return THPVariable_CheckExact(o); }
@@ -94,6 +97,7 @@ PyObject *PlanNew(PyTypeObject *type, PyObject *args, PyObject *) {
   p->rt = reinterpret_cast<void *>(rt);
   p->now = new std::shared_ptr<const Recorded>();
   p->seen = new std::vector<ArgSpec>();
+  p->launch = new std::mutex();
   return reinterpret_cast<PyObject *>(p);
 }
 
@@ -101,6 +105,7 @@ void PlanDealloc(PyObject *self) {
   Plan *p = reinterpret_cast<Plan *>(self);
   delete p->now;
   delete p->seen;
+  delete p->launch;
   Py_TYPE(self)->tp_free(self);
 }
 
@@ -221,7 +226,7 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
     return nullptr;
   }
   PyObject *kernel = argv[0], *args = argv[1];
-  const std::shared_ptr<const Recorded> r = *p->now;  // (a callback of the allocation may lead to another plan)
+  const std::shared_ptr<const Recorded> r = *p->now;  // (another thread may record a plan while this one is at work)
   void *ptrs[64];
   if (!r || !Matches(r->args, r->device, args, ptrs)) Py_RETURN_NONE;
   if (p->stamp_of(p->rt) != r->stamp) {
@@ -240,6 +245,9 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
   made.reserve(r->outs.size() + 1);
   int rc = 1;
   {
+    // Other threads run meanwhile: an allocation may have to free memory and wait for the GPU, a launch waits while the
+    // stream's queue is full.
+    pybind11::gil_scoped_release no_gil;
     const c10::Device device(c10::kCUDA, r->device);
     size_t np = r->ios.size() - r->outs.size();
     void *workspace = nullptr;
@@ -254,7 +262,10 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
       memory = made.back().has_storage();
       if (memory) workspace = made.back().data_ptr();
     }
-    if (memory) rc = p->rebind_run(p->rt, r->stamp, r->ios.data(), ptrs, np, workspace, raw);
+    if (memory) {
+      const std::lock_guard<std::mutex> one(*p->launch);
+      rc = p->rebind_run(p->rt, r->stamp, r->ios.data(), ptrs, np, workspace, raw);
+    }
   }
   if (rc != 0) {
     p->now->reset();

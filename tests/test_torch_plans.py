@@ -208,6 +208,83 @@ print("numbers: ok")
 def test_numbers_that_change_are_not_recorded():
     _run(_NUMBERS, "numbers: ok")
 
+_THREADS = r'''
+import ctypes
+import threading
+import time
+import torch
+import dvm_amd as dvm
+
+@dvm.kernel(ktype="split", dynamic=True)
+def scale(k, x, a):
+    return k.store(k.mul(k.load(x, dvm.float32), k.scalar(a)))
+
+@dvm.kernel(ktype="mix", dynamic=True)
+def product(k, x, w):  # (a workspace per call)
+    return k.store(k.matmul(k.load(x, dvm.float16), k.load(w, dvm.float16), False, False))
+
+x = torch.arange(4096.0, device="cuda").view(64, 64)
+a = torch.randint(-1, 2, (64, 8192), device="cuda").half()
+b = torch.randint(-1, 2, (8192, 128), device="cuda").half()
+want = a.double() @ b.double()
+for _ in range(4):
+    scale(x, 2.0); product(a, b)
+torch.cuda.synchronize()
+assert bool(scale._plan) and product.workspace_bytes() > 0
+
+# other threads run while a plan allocates and launches: a plan whose launch is a sleep of the C library
+beats, stop = [0], threading.Event()
+def beat():
+    while not stop.is_set():
+        beats[0] += 1
+t = threading.Thread(target=beat)
+t.start()
+libc = ctypes.CDLL(None)
+address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+class Kernel:
+    pass
+slow = type(scale._plan)(address(libc.usleep), address(libc.abs), 0, 300000)
+args = (x, 2.0)
+assert not slow.repeats(args) and slow.repeats(args) and slow.record([1], [x], [2], False, 0)
+before = beats[0]
+time.sleep(0.3)
+free = beats[0] - before
+before = beats[0]
+assert slow.call(Kernel(), args, lambda device: 0).shape == x.shape
+ran = beats[0] - before
+stop.set(); t.join()
+assert ran > free / 3, (ran, free)
+
+# the same kernels from several threads, a stream each: every call reads and writes its own tensors
+failed = []
+def work(n):
+    try:
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            for i in range(200):
+                y = x + float(n * 1000 + i)
+                got = scale(y, 2.0)
+                c = product(a, b) if i % 8 == 0 else None
+                stream.synchronize()
+                if not torch.equal(got, y * 2.0):
+                    failed.append((n, i))
+                if c is not None and not torch.equal(c.double(), want):
+                    failed.append((n, i, "product"))
+    except Exception as e:
+        failed.append(repr(e))
+threads = [threading.Thread(target=work, args=(n,)) for n in range(4)]
+[w.start() for w in threads]
+[w.join(90) for w in threads]
+assert not any(w.is_alive() for w in threads)
+assert not failed, failed[:5]
+print("threads: ok")
+'''
+
+
+def test_several_threads_call_the_same_kernel():
+    _run(_THREADS, "threads: ok")
+
 
 def _run(script, said):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
