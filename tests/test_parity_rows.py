@@ -121,3 +121,64 @@ def test_rows_read_and_written_through_strides(b, h, cols):
     want[:, :, :cols] = x - x.max(2, keepdims=True)
     t.view_store_expect(d, (pitch, b * pitch, 1), want, 0)
     assert t.run_check() and " row=" in t.das() and "  kdims: %d %d" % (h, b) in t.das(), t.das()
+
+
+def _held_cases():
+    # two slabs a lane: the first in whole lines, the last (ragged but for 1024) side by side; the values held across the reduce
+    # lie in V registers
+    return [(2100, 520), (2100, 777), (2100, 1000), (2100, 1017), (2100, 1024), (1100, 1031), (1100, 2047)]
+
+
+def _assert_held(t):
+    das = t.das()
+    assert " row=2 " in das and "vslots=0" not in das and t.num_launches() == 1, das
+
+
+@pytest.mark.parametrize("rows,cols", _held_cases())
+def test_fp32_rows_with_exponentials_held_across_the_reduce(rows, cols):
+    xs = [_inputs(rows, cols, "float32", 100 * cols + i, 0.5) for i in range(3)]
+    t = Tester("split")
+    e = [t.exp(t.load(x)) for x in xs]
+    s = t.sum(t.mul(t.mul(e[0], e[1]), e[2]), (1,), True)
+    outs = [t.store(t.div(v, s)) for v in e]
+    t.run()
+    _assert_held(t)
+    e64 = [np.exp(x.astype(np.float64)) for x in xs]
+    s64 = (e64[0] * e64[1] * e64[2]).sum(1, keepdims=True)
+    # units in the last place: an exponential 1.2, three of them and two products 4.6, eight elements' sum 1.5, the sum's and
+    # the quotient's rounding 1
+    for o, v in zip(outs, e64):
+        assert np.allclose(t.output(o), v / s64, rtol=8.3 * 2.0 ** -23, atol=0)
+
+
+@pytest.mark.parametrize("rows,cols", _held_cases())
+@pytest.mark.parametrize("centred", [False, True])
+def test_fp32_rows_of_a_norms_backward(rows, cols, centred):
+    x, dy = (_inputs(rows, cols, "float32", 100 * cols + i) for i in range(2))
+    w = np.random.default_rng(3).uniform(0.5, 1.5, [cols]).astype(np.float32)
+    x64, dy64, w64 = (a.astype(np.float64) for a in (x, dy, w))
+    mean = x64.mean(1, keepdims=True).astype(np.float32) if centred else np.zeros((rows, 1), np.float32)
+    rstd = (1.0 / np.sqrt(((x64 - mean) ** 2).mean(1, keepdims=True) + 1e-6)).astype(np.float32)
+    t = Tester("split")
+    vx, vdy, vw = t.load(x), t.load(dy), t.load(w)
+    if centred:
+        r = t.load(rstd)
+        xh = t.mul(t.sub(vx, t.load(mean)), r)
+    else:
+        r = t.div(1.0, t.sqrt(t.add(t.mul(t.sum(t.mul(vx, vx), (1,), True), 1.0 / cols), 1e-6)))
+        xh = t.mul(vx, r)
+    g = t.mul(vdy, vw)
+    b = t.mul(t.sum(t.mul(g, xh), (1,), True), 1.0 / cols)
+    inner = t.sub(t.sub(g, t.mul(t.sum(g, (1,), True), 1.0 / cols)), t.mul(xh, b)) if centred else t.sub(g, t.mul(xh, b))
+    dx, dw = t.store(t.mul(inner, r)), t.store(t.mul(vdy, xh))
+    t.run()
+    _assert_held(t)
+    r64 = rstd.astype(np.float64) if centred else 1.0 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6)
+    h64, g64 = (x64 - mean) * r64, dy64 * w64
+    want = (g64 - (g64.mean(1, keepdims=True) if centred else 0.0) - h64 * (g64 * h64).mean(1, keepdims=True)) * r64
+    # sixteen halves of a unit in the last place of the terms' sizes: five roundings of a normalised element (of |x| + |mean|, that of the
+    # root among them), four of g and the differences, five of a mean (eight elements' sum, its rounding, the factor)
+    h = (np.abs(x64) + np.abs(mean)) * r64
+    size = (np.abs(g64) + np.abs(g64).mean(1, keepdims=True) + h * (np.abs(g64) * h).mean(1, keepdims=True)) * r64
+    assert (np.abs(t.output(dx) - want) <= 16 * 2.0 ** -24 * size).all()
+    assert (np.abs(t.output(dw) - dy64 * h64) <= 8 * 2.0 ** -24 * np.abs(dy64) * h).all()
