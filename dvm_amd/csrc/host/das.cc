@@ -242,7 +242,9 @@ std::string &VKernel::DisAssemble() {
       os << "entry cube " << kMemTypes[c->dtype] << " m=" << c->m << " n=" << c->n << " k=" << c->k << " trans_a=" << c->trans_a
          << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << DVM_CUBE_TILE_SIDE(c->tile) << " blocks="
          << ((c->epi_flags & VCF_SPLITK_COMBINE) ? static_cast<uint64_t>(c->tiles_m) * c->tiles_n * c->nb0 * c->nb1 : static_cast<uint64_t>(p.grid))
-         << " lds=" << p.lds_bytes << (c->fast ? (c->k % 64 != 0 ? " fast guarded-k-end" : " fast") : " guarded") << (c->tile == 3 ? " eight-waves" : "");
+         << " lds=" << p.lds_bytes << (c->fast ? " fast" : " guarded") << (c->tile == 3 ? " eight-waves" : "");
+      // (an operand whose rows are contiguous takes the ring in whole chunks of eight; its tiles over a ragged end that is none do not)
+      if (c->fast && ((c->trans_a && c->m % 8 != 0) || (!c->trans_b && c->n % 8 != 0))) os << " guarded-edge";
       if (c->epi_flags & VCF_PLAIN_STORE) os << " plain-store";
       else if (c->epi_flags & VCF_SLIM) os << " slim-epilogue";
       if (c->epi_flags & VCF_DUMP16) os << " tile-as-16-bit";
