@@ -372,7 +372,6 @@ static bool runs_hold(const VmParam &p) {
   return true;
 }
 
-// Checks one program blob against the launch it is to get and launches the interpreter kernel its entry type names.
 // The column build trusts its flag: the program is what VS_COLS says, the teams cover the kept index space, and the operands
 // lie where 128-bit accesses to whole elements reach them.
 static bool col_words_hold(const VmParam &p, uint32_t threads) {
@@ -414,6 +413,7 @@ static bool col_words_hold(const VmParam &p, uint32_t threads) {
   return false;
 }
 
+// Checks one program blob against the launch it is to get and launches the interpreter kernel its entry type names.
 static int launch_checked(const VmParam &p, uint32_t block_dim, uint32_t threads, uint32_t lds_bytes, void *stream, bool check_only = false) {
   if (block_dim == 0 || threads == 0 || threads > 1024 || (threads & 63u) != 0) {
     return static_cast<int>(hipErrorInvalidValue);

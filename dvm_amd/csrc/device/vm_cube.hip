@@ -71,8 +71,9 @@ __device__ __forceinline__ uint32_t tile_off(uint32_t row, uint32_t chunk) {
   return row * BK + ((chunk ^ ((row ^ (row >> 3)) & 7u)) << 3);
 }
 
-// Generic staging of one tile straight into local memory (edge tiles, odd leading dimensions, unaligned
-// operands, a k axis that is no multiple of 64). The unit is a run of 8 elements that are consecutive in memory:
+// Generic staging of one tile straight into local memory: operands that are no whole 16-byte chunks along their contiguous
+// axis (leading dimension, base address, extent), ragged tiles of an operand whose rows are contiguous and no multiple of 8,
+// and the two ends of a group's range along k. The unit is a run of 8 elements that are consecutive in memory:
 // 8 k of one row (k contiguous) or 8 rows at one k (rows contiguous); a run that lies inside the operand and is
 // 16-byte aligned (vec_ok: leading dimension a multiple of 8 and an aligned base) is one 128-bit load, any other
 // run goes element by element and reads as zero outside the operand. Slow next to the tile loops, correct for
@@ -125,7 +126,7 @@ __device__ __attribute__((noinline)) void stage_generic(uint16_t *tile, uint64_t
   }
 }
 
-// ---- the tile loop: stages of 32 or 64 k in a ring of buffers in local memory ---------------------------
+// ---- the tile loop: stages of 64 k in a ring of buffers in local memory ---------------------------
 // A stage holds BM rows x SK k of A and BN rows x SK k of B; NB stage buffers make a ring. While stage s is multiplied,
 // the direct loads of stages s+1 .. s+NB-2 are in flight and those of stage s+NB-1 are issued, a few at a time between
 // the MFMAs, into the buffer stage s-1 has just left. Both operand layouts are straight copies:

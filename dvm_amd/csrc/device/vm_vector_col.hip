@@ -73,7 +73,6 @@ __device__ __forceinline__ void col_rows(uint64_t at, uint64_t step, uint32_t le
       if (how1 != kNoSlot) col_row(r1, how1, x);
     }
   }
-#undef HDR
 }
 
 // Combines the partials of the lanes that stand along the rows: across the rows of a wave by shuffles, across the waves

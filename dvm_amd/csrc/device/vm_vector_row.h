@@ -377,7 +377,9 @@ __device__ __forceinline__ float row_one_unary(uint32_t sub, float x) {
 
 template <int UR, bool PLANES>
 __device__ __forceinline__ void vm_vector_row(const VmParam &p) {
-  if constexpr (UR == 4) {  // (residual RMSNorm bf16 [4490,1648] 14.9 us this way, 16.6 the other)
+  // (Four slabs are faster this way: residual RMSNorm bf16 [4490,1648] 14.8 us, 16.7 the other; over 172 softmaxes and residual
+  // norms of 300 to 8192 rows the other way is 2.7 % slower on average, 13 % at most, and 4 % faster at 300 x 13000.)
+  if constexpr (UR == 4) {
     const uint32_t rc = reinterpret_cast<const VVecHeader *>(p.w)->row_code;
     fetch_used_words(prog_lds, p.w, ((rc & 0xffffu) + (rc >> 16)) * 2);
   } else {

@@ -364,8 +364,11 @@ bool Compiler::SplitLongReduces() {
     const NDObject *load = nullptr;
     if (forced < 2 && !red[last] && k_->tuning_.vec_col != 0 && ReducesColumnsOfALoad(r, &load)) {
       // The column build gives a workgroup one 128-byte line of columns. In one launch: while the whole operand is at most
-      // 40 MB and a workgroup's share half a megabyte, and every reduce beside this one goes the same way. bf16 [4096,4096]
-      // over axis 0: 26 us in two launches, 17 in one; [4096,512] 17 and 10.
+      // 40 MB and a workgroup's share half a megabyte, and every reduce beside this one goes the same way. Measured on MI355X,
+      // sums over axis 0, us in one launch / on the same build in the parts that suit the size best: bf16 [4096,4096] 16.8 / 18.5,
+      // [2048,8192] 12.4 / 19.9, [4096,2048] 14.5 / 12.9, [4096,512] 11.6 / 10.8, fp32 [4096,2048] 14.7 / 14.9, [2048,4096]
+      // 11.5 / 17.7. More rows: bf16 [6000,2048] 18.7 / 13.9, [8192,1024] 22.4 / 12.7, fp32 [6000,512] 18.5 / 11.6. More bytes
+      // (49 to 67 MB, up to 4096 rows) would still gain from one launch, 17.4 to 19.7 / 21.6 to 23.6, and are shared all the same.
       bool alike = !load->strided || load->vstride_[load->rank() - 1] == 1, seen_kept = false;
       for (int d = 0; d < xr; ++d) {
         if (x->dim(d) == 1) continue;

@@ -87,8 +87,9 @@ enum {
 #define DVM_VEC_ROW_WORDS 64  // instruction words of a row program at most (one per lane of a wave)
 // slabs a lane the row build exists for, and the lanes a workgroup of that build may have
 #define DVM_VEC_ROW_OK(slabs) ((slabs) >= 1u && (slabs) <= 8u && (slabs) != 7u)
-// (over planes: not four, whose kernel would save 37 registers a lane to scratch memory and was the slowest of all that hold a
-// row, 22.9 us against 17.3 with three and 19.4 with eight at [24,256,28,28]; eight take a row of six to eight slabs there)
+// (over planes: not four, whose kernel would save 37 registers a lane to scratch memory and is the slowest of all that hold a row.
+// Batch-norm, us with four / with what is taken instead: [20,256,28,28] 20.5 / 15.9 (two), [20,512,28,28] 29.0 / 21.6 (eight),
+// [24,256,28,28] 22.9 / 17.3 (three); eight take a row of six to eight slabs there)
 #define DVM_VEC_PLANES_OK(slabs) (DVM_VEC_ROW_OK(slabs) && (slabs) != 4u)
 #define DVM_VEC_ROW_LANES(slabs) ((slabs) <= 4u ? 1024u : 512u)
 // elements from the first of a row's first plane to behind the last of its last one (byte offsets in 32 bits)
