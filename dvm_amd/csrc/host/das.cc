@@ -243,8 +243,10 @@ std::string &VKernel::DisAssemble() {
          << " trans_b=" << c->trans_b << " batch=" << c->nb0 << "x" << c->nb1 << " tile=" << DVM_CUBE_TILE_SIDE(c->tile) << " blocks="
          << ((c->epi_flags & VCF_SPLITK_COMBINE) ? static_cast<uint64_t>(c->tiles_m) * c->tiles_n * c->nb0 * c->nb1 : static_cast<uint64_t>(p.grid))
          << " lds=" << p.lds_bytes << (c->fast ? " fast" : " guarded") << (c->tile == 3 ? " eight-waves" : "");
+      // (a last stage that k does not fill: what lies past the end is outside the loads' range and reads as zeros)
+      if (c->fast && c->k % 64 != 0) os << " k-end-guarded-by-range";
       // (an operand whose rows are contiguous takes the ring in whole chunks of eight; its tiles over a ragged end that is none do not)
-      if (c->fast && ((c->trans_a && c->m % 8 != 0) || (!c->trans_b && c->n % 8 != 0))) os << " guarded-edge";
+      if (c->fast && ((c->trans_a && c->m % 8 != 0) || (!c->trans_b && c->n % 8 != 0))) os << " edge-by-element";
       if (c->epi_flags & VCF_PLAIN_STORE) os << " plain-store";
       else if (c->epi_flags & VCF_SLIM) os << " slim-epilogue";
       if (c->epi_flags & VCF_DUMP16) os << " tile-as-16-bit";

@@ -19,8 +19,10 @@ def test_three_sums_of_parts_share_a_compute_unit(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,ta,tb,route", [
-    (256, 256, 200, False, True, "fast"), (100, 72, 328, False, False, "fast"), (104, 72, 327, True, False, "fast"), (100, 77, 328, False, True, "fast"),
-    (100, 80, 328, True, True, "fast guarded-edge"), (104, 77, 328, True, False, "guarded"), (104, 80, 327, False, True, "guarded"), (104, 80, 327, True, True, "guarded")])
+    (256, 256, 192, False, True, "fast"), (256, 256, 200, False, True, "fast k-end"), (100, 72, 320, False, False, "fast"),
+    (104, 72, 327, True, False, "fast k-end"), (100, 77, 320, False, True, "fast"), (100, 80, 320, True, True, "fast edge"),
+    (100, 80, 328, True, True, "fast k-end edge"), (104, 77, 320, True, False, "guarded"), (104, 80, 327, False, True, "guarded"),
+    (104, 80, 327, True, True, "guarded")])
 def test_the_route_of_the_tiles(m, n, k, ta, tb, route):
     # a contiguous axis that is no multiple of eight: the leading dimension is none either, unless the operand is a window
     t = Tester("mix", run_mode="das")
@@ -31,5 +33,6 @@ def test_the_route_of_the_tiles(m, n, k, ta, tb, route):
         x = t.load(np.zeros((k, m) if ta else (m, k), np.float16))
     t.store(t.matmul(x, t.load(np.zeros((n, k) if tb else (k, n), np.float16)), ta, tb))
     t.codegen()
-    labels = re.search(r"^entry cube.* lds=\d+ (.*)$", t.das(), re.M).group(1)
-    assert labels.startswith(route) and ("guarded" in labels) == ("guarded" in route) and "guarded-k-end" not in labels, t.das()
+    labels = re.search(r"^entry cube.* lds=\d+ (.*)$", t.das(), re.M).group(1).split()
+    known = {"fast": "fast", "guarded": "guarded", "k-end-guarded-by-range": "k-end", "edge-by-element": "edge"}
+    assert [known[v] for v in labels if v in known] == route.split(), t.das()
