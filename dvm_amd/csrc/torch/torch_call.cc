@@ -178,16 +178,17 @@ PyObject *PlanRepeats(PyObject *self, PyObject *args) {
   END_HANDLE_TH_ERRORS
 }
 
-// record(load handles, outputs, store handles, many, workspace bytes): the call that `repeats` has just been asked about becomes
-// the plan. False when calls like it cannot go this way.
+// record(args, load handles, outputs, store handles, many, workspace bytes): the call that `repeats` has just been asked about
+// becomes the plan, unless another thread has asked about another one meanwhile. False when calls like it cannot go this way.
 PyObject *PlanRecord(PyObject *self, PyObject *pyargs) {
   HANDLE_TH_ERRORS
   Plan *p = reinterpret_cast<Plan *>(self);
-  PyObject *loads, *outs, *stores;
+  PyObject *args, *loads, *outs, *stores;
   int many = 0;
   long long ws_bytes = 0;
-  if (!PyArg_ParseTuple(pyargs, "O!O!O!pL", &PyList_Type, &loads, &PyList_Type, &outs, &PyList_Type, &stores, &many, &ws_bytes)) return nullptr;
+  if (!PyArg_ParseTuple(pyargs, "O!O!O!O!pL", &PyTuple_Type, &args, &PyList_Type, &loads, &PyList_Type, &outs, &PyList_Type, &stores, &many, &ws_bytes)) return nullptr;
   p->now->reset();
+  if (!Matches(*p->seen, DeviceOf(args), args, nullptr)) Py_RETURN_TRUE;
   auto r = std::make_shared<Recorded>();
   r->args = *p->seen;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(outs); ++i) {

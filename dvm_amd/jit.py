@@ -197,9 +197,10 @@ class _DeviceCall:
                 k._plan = False
                 return
             _raw_stream_of = self.torch._C._cuda_getCurrentRawStream
-        if not k._plan.repeats(tuple(self.args)):
+        args = tuple(self.args)
+        if not k._plan.repeats(args):
             return
-        if not k._plan.record([s.handle._h for s in k._slots if s.role == "tensor"], outs, [st._h for st in k._stores()[0]], many, k.workspace_bytes()):
+        if not k._plan.record(args, [s.handle._h for s in k._slots if s.role == "tensor"], outs, [st._h for st in k._stores()[0]], many, k.workspace_bytes()):
             k._plan = False
 
 

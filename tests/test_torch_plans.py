@@ -245,7 +245,11 @@ class Kernel:
     pass
 slow = type(scale._plan)(address(libc.usleep), address(libc.abs), 0, 300000)
 args = (x, 2.0)
-assert not slow.repeats(args) and slow.repeats(args) and slow.record([1], [x], [2], False, 0)
+assert not slow.repeats(args) and slow.repeats(args)
+# (another thread's call in between: its arguments are not recorded with this one's results)
+assert not slow.repeats((x[:1], 2.0)) and slow.record(args, [1], [x], [2], False, 0)
+assert slow.call(Kernel(), args, lambda device: 0) is None and slow.call(Kernel(), (x[:1], 2.0), lambda device: 0) is None
+assert not slow.repeats(args) and slow.repeats(args) and slow.record(args, [1], [x], [2], False, 0)
 before = beats[0]
 time.sleep(0.3)
 free = beats[0] - before
