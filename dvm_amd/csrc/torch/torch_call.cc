@@ -6,8 +6,8 @@
 // the call is: check them, allocate the outputs and the workspace from torch's caching allocator, write the addresses into the
 // compiled programs, launch. No address is kept from one call for the next, and whatever else changes the kernel
 // (dvm_rt_plan_stamp) makes the plan stale; any mismatch hands the call back to jit.py, which raises what there is to raise.
-// Measured on an MI355X's host, us a call from Python / from the plan: two fp32 tensors added 12.9 / 4.9, an Adam step on 64 x 64
-// (four tensors, two numbers, three results) 24.3 / 6.8; of that the launch itself takes 3.5.
+// Measured on an MI355X's host, us a call from Python / from the plan: two fp32 tensors added 12.9 / 4.4, an Adam step on 64 x 64
+// (four tensors, two numbers, three results) 24.3 / 6.0; of that the launch itself takes 3.5.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -58,7 +58,7 @@ struct Plan {
   void *rt;
   std::shared_ptr<const Recorded> *now;  // (empty: nothing recorded, or stale)
   std::vector<ArgSpec> *seen;            // arguments of the last call made from Python (empty: none that can be recorded)
-  std::mutex *launch;                    // one thread at a time writes addresses into the programs and launches them
+  std::recursive_mutex *launch;          // one thread at a time binds, generates code and launches, from here or from Python
 };
 
 bool IsPlainTensor(PyObject *o) { return THPVariable_CheckExact(o); }
@@ -98,7 +98,7 @@ PyObject *PlanNew(PyTypeObject *type, PyObject *args, PyObject *) {
   p->rt = reinterpret_cast<void *>(rt);
   p->now = new std::shared_ptr<const Recorded>();
   p->seen = new std::vector<ArgSpec>();
-  p->launch = new std::mutex();
+  p->launch = new std::recursive_mutex();
   return reinterpret_cast<PyObject *>(p);
 }
 
@@ -265,7 +265,7 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
       if (memory) workspace = made.back().data_ptr();
     }
     if (memory) {
-      const std::lock_guard<std::mutex> one(*p->launch);
+      const std::lock_guard<std::recursive_mutex> one(*p->launch);
       rc = p->rebind_run(p->rt, r->stamp, r->ios.data(), ptrs, np, workspace, raw);
     }
   }
@@ -300,7 +300,22 @@ PyObject *PlanCall(PyObject *self, PyObject *const *argv, Py_ssize_t argc) {
   END_HANDLE_TH_ERRORS
 }
 
+// hold() .. release(): a call from Python, which takes several steps, on a kernel that others may call from this plan
+PyObject *PlanHold(PyObject *self, PyObject *) {
+  HANDLE_TH_ERRORS
+  pybind11::gil_scoped_release no_gil;
+  reinterpret_cast<Plan *>(self)->launch->lock();
+  END_HANDLE_TH_ERRORS_RET(nullptr)
+  Py_RETURN_NONE;
+}
+PyObject *PlanRelease(PyObject *self, PyObject *) {
+  reinterpret_cast<Plan *>(self)->launch->unlock();
+  Py_RETURN_NONE;
+}
+
 PyMethodDef plan_methods[] = {
+    {"hold", PlanHold, METH_NOARGS, nullptr},
+    {"release", PlanRelease, METH_NOARGS, nullptr},
     {"repeats", PlanRepeats, METH_O, nullptr},
     {"record", PlanRecord, METH_VARARGS, nullptr},
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(PlanCall)), METH_FASTCALL, nullptr},

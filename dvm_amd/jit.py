@@ -77,10 +77,20 @@ class JitKernel(PyKernel):
         return (list(self._results) if many else [self._results]), many
 
     def __call__(self, *args, out=None):
-        if self._plan and out is None:
-            result = self._plan.call(self, args, _raw_stream_of)
+        plan = self._plan
+        if not plan:
+            return self._call_from_python(args, out)
+        if out is None:
+            result = plan.call(self, args, _raw_stream_of)
             if result is not None:
                 return result
+        plan.hold()  # (no other thread binds or launches this kernel meanwhile)
+        try:
+            return self._call_from_python(args, out)
+        finally:
+            plan.release()
+
+    def _call_from_python(self, args, out):
         if len(args) != len(self._slots):
             raise TypeError("kernel takes %d arguments, %d given" % (len(self._slots), len(args)))
         if any(_on_gpu(a) for a in args):

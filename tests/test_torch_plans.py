@@ -167,6 +167,7 @@ def step(k, p, g, lr):
 class Counting:  # the plan, and how often it is recorded and makes a call
     def __init__(self, plan):
         self.plan, self.recorded, self.called = plan, 0, 0
+        self.hold, self.release = plan.hold, plan.release
     def repeats(self, args):
         return self.plan.repeats(args)
     def record(self, *args):
@@ -282,6 +283,27 @@ threads = [threading.Thread(target=work, args=(n,)) for n in range(4)]
 [w.join(90) for w in threads]
 assert not any(w.is_alive() for w in threads)
 assert not failed, failed[:5]
+
+# shapes and numbers of their own: some calls come from the plan, some from Python
+failed = []
+def mixed(n):
+    try:
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            for i in range(200):
+                y = x[: 1 + (n + i // 5) % 3 * 20] + float(i)
+                f = 2.0 if i % 3 else float(n)
+                got = scale(y, f)
+                stream.synchronize()
+                if got.shape != y.shape or not torch.equal(got, y * f):
+                    failed.append((n, i))
+    except Exception as e:
+        failed.append(repr(e))
+threads = [threading.Thread(target=mixed, args=(n,)) for n in range(4)]
+[w.start() for w in threads]
+[w.join(90) for w in threads]
+assert not any(w.is_alive() for w in threads) and not failed, failed[:5]
 print("threads: ok")
 '''
 
